@@ -239,6 +239,7 @@ class MFMAConfig(Config):
         self.mfma_m, self.mfma_n, self.mfma_k = 32, 32, 16
         self.skinny = False      # small M: weight-streaming 16x16x32 kernel, K split over wavefronts
         self.stream = False      # M <= 64: W streamed through the LDS in 1 KiB row pieces, K sliced over workgroups
+        self.share = False       # M <= 128: every workgroup an equal number of columns (at most j blocks of 16) over the whole of K
         self.block_threads = 256
         self.stages = 0          # LDS stages of the load pipeline (0 = as many as the tile allows)
         self.split_k = 1         # workgroups that share a tile and split its K extent
@@ -267,7 +268,7 @@ class MFMAConfig(Config):
         return {"tile_shape": (self.tile_size_m, self.tile_size_n, self.tile_size_k),
                 "mfma_shape": (self.mfma_m, self.mfma_n, self.mfma_k), "i": self.i, "j": self.j,
                 "micro_shape": (self.micro_shape_x, self.micro_shape_y, self.micro_shape_k),
-                "skinny": self.skinny, "stream": self.stream, "block_threads": self.block_threads, "stages": self.stages,
+                "skinny": self.skinny, "stream": self.stream, "share": self.share, "block_threads": self.block_threads, "stages": self.stages,
                 "split_k": self.split_k, "acc_f16": self.acc_f16, "in_vec_len_a": self.in_vec_len_a, "in_vec_len_b": self.in_vec_len_b}
 
     def from_dict(self, dic: Dict) -> "MFMAConfig":
@@ -277,6 +278,7 @@ class MFMAConfig(Config):
         self.micro_shape_x, self.micro_shape_y, self.micro_shape_k = dic["micro_shape"]
         self.skinny = dic.get("skinny", False)
         self.stream = dic.get("stream", False)
+        self.share = dic.get("share", False)
         self.block_threads = dic.get("block_threads", 256)
         self.stages = dic.get("stages", 0)
         self.split_k = dic.get("split_k", 1)
@@ -288,6 +290,10 @@ class MFMAConfig(Config):
         if self.acc_f16:   # one kernel shape: 64x64 per workgroup, a k step of 16 per instruction
             c.variant, c.block, c.vec, c.unroll, c.split_k = _lib.GEMM_MFMA_ACC16, 256, 8, 1, 1
             c.tile[0], c.tile[1], c.tile[2] = 64, 64, 16
+            return c
+        if self.share:
+            c.variant, c.block, c.vec, c.unroll, c.split_k = _lib.GEMM_SHARE, 256, 8, 1, 1
+            c.tile[0], c.tile[1] = self.tile_size_m, self.tile_size_n
             return c
         c.variant = _lib.GEMM_SKINNY if self.skinny else _lib.GEMM_STREAM if self.stream else _lib.GEMM_MFMA
         c.block, c.vec = self.block_threads, 8

@@ -72,6 +72,14 @@ int launch_gemm_stream(const dtas_config& cfg, hipStream_t s, const half_t* A, c
 // 8-bit W (bytes [N][K], scales in ep.wscale): rows of A in {16, 32, 64}, K slices of 512 or 1024 (16 rows only)
 int launch_gemm_stream_q8(int rows_a, int k_slice, hipStream_t s, const half_t* A, const half_t* Wq, const GemmEpilogue& ep, void* C,
                           int64_t M, int64_t N, int64_t K);
+// ---- gemm_share.hip: every workgroup an equal number of columns (at most `cols`) over the whole of K, M <= rows; and whether
+// one of these kernels leads at a shape (cfg == NULL), with the one to take
+int launch_gemm_share(int rows, int cols, hipStream_t s, const half_t* A, const half_t* W, const GemmEpilogue& ep, void* C, int64_t M,
+                      int64_t N, int64_t K);
+int launch_gemm_share_q8(int rows, int cols, hipStream_t s, const half_t* A, const half_t* Wq, const GemmEpilogue& ep, void* C, int64_t M,
+                         int64_t N, int64_t K);
+bool share_leads(int64_t M, int64_t N, int64_t K, int* rows, int* cols);
+bool share_leads_q8(int64_t M, int64_t N, int64_t K, int* rows, int* cols);
 // DTAS_GEMM_MFMA_ACC16: the accumulator rounded to fp16 after every k step of 16 (cfg.vec 8: 16-byte operand loads, else elements)
 int launch_gemm_acc16(const dtas_config& cfg, hipStream_t s, const half_t* A, const half_t* W, const GemmEpilogue& ep, void* C,
                       int64_t M, int64_t N, int64_t K);
@@ -84,6 +92,19 @@ inline int stream_loop_stages(int bm, int bn) {
   if (bm == 16 && bn == 64) return 4;  // 160 KiB: one workgroup per CU
   if (bm == 16 && bn == 16) return 4;  // 64 KiB: two one-wavefront workgroups per CU
   return 0;
+}
+// the share kernel: the instantiated rows of A x columns, and its workgroups: a whole number of rounds of the chip, each
+// with N / workgroups columns (a W of few rows: at least 4 columns each)
+inline bool share_kernel_exists(int rows, int cols, bool q8) {
+  const bool narrow = cols == 16 || cols == 32 || cols == 48, any = narrow || cols == 64 || cols == 128;
+  if (rows == 16) return any && (q8 || cols != 48);
+  if (rows == 32 || rows == 48 || rows == 64) return any;
+  if (q8) return (rows == 80 && cols == 16) || (rows == 96 && (cols == 32 || cols == 48));
+  return (rows == 96 && narrow) || (rows == 128 && cols == 48);
+}
+inline int64_t share_grid(int64_t N, int cols) {
+  if (N <= 4 * kNumCU) return ceil_div(N, 4);
+  return kNumCU * ceil_div(N, static_cast<int64_t>(kNumCU) * cols);
 }
 // the instantiated W-streaming shapes: rows of A x columns x K slice
 inline bool stream_shape_ok(int bm, int bn, int bk) {

@@ -48,6 +48,16 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
       if (!stream_ok) return fail("gemm_q8: the W-streaming kernel needs K %% 256 == 0 and 16-byte aligned A, W and scales");
       return launch_gemm_stream_q8(bm, bk, s, a, w, ep, C, M, N, K);
     }
+    if (user && user->variant == DTAS_GEMM_SHARE) {
+      if (!share_kernel_exists(user->tile[0], user->tile[1], true) || user->block != 256)
+        return fail("gemm_q8: no share kernel for %d rows of A, %d columns per workgroup and %d threads", user->tile[0], user->tile[1], user->block);
+      if (M > user->tile[0]) return fail("gemm_q8: a share kernel of %d rows cannot hold M=%lld", user->tile[0], (long long)M);
+      if (!stream_ok) return fail("gemm_q8: the share kernel needs K %% 256 == 0 and 16-byte aligned A, W and scales");
+      return launch_gemm_share_q8(user->tile[0], user->tile[1], s, a, w, ep, C, M, N, K);
+    }
+    // up to 96 rows: every CU an equal share of W's rows, nothing handed over (share_leads_q8)
+    int rows = 0, cols = 0;
+    if (!user && stream_ok && N <= 0x7fffffff && share_leads_q8(M, N, K, &rows, &cols)) return launch_gemm_share_q8(rows, cols, s, a, w, ep, C, M, N, K);
     if (!user && stream_ok && M <= 32) {
       // measured at the model's shapes (M = 16: 10.1 against 25.6 us at 7680x2560, 14.9 against 92 at 2560x10240;
       // M = 32: 14.0 against 26.3 and 20.5 against 33.8).  512-element slices (three workgroups per CU) unless K is

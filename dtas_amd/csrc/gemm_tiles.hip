@@ -203,6 +203,19 @@ int describe_gemm(int64_t M, int64_t N, int64_t K, const dtas_config& cfg, int64
     la[6] = tn;
     return 0;
   }
+  if (cfg.variant == DTAS_GEMM_SHARE) {
+    if (!share_kernel_exists(cfg.tile[0], cfg.tile[1], false))
+      return fail("gemm: no share kernel for %d rows of A and %d columns per workgroup", cfg.tile[0], cfg.tile[1]);
+    if (M > cfg.tile[0]) return fail("gemm: a share kernel of %d rows cannot hold M=%lld", cfg.tile[0], (long long)M);
+    if (cfg.block != 256) return fail("gemm: the share kernel uses 256 threads, got %d", cfg.block);
+    if (K < 1 || K * 2 * 128 >= (int64_t{1} << 31)) return fail("gemm: K=%lld does not fit 32-bit offsets", (long long)K);
+    if (N > 0x7fffffff) return fail("gemm: too many columns");
+    la[0] = share_grid(N, cfg.tile[1]);
+    la[3] = 256;
+    la[5] = 1;
+    la[6] = la[0];
+    return 0;
+  }
   return fail("gemm: unknown variant %d", cfg.variant);
 }
 
@@ -293,9 +306,10 @@ extern "C" int dtas_gemm_f16_fused(const void* A, const void* W, const void* bia
   const bool vec_ok = K % 8 == 0 && aligned(A, 16) && aligned(W, 16);
   // two rows of A (the first bucket's table row is sized for 16): W streamed in whole rows, as the GEMV does
   if (!user && M == 2 && vec_ok) cfg = dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {2, N <= 2560 ? 1 : 2, 8}, 1, 0};
-  // three or four rows against a W of few rows: a row of W per wavefront fills the chip where 64-column tiles do not
-  // (4 x 2560 x 2560: 5.3 us against 7.6, 2560 x 10240: 14.1 / 18.5; level at 4096 x 4096, behind at 7680 x 2560: 11.5 / 10.1)
-  if (!user && (M == 3 || M == 4) && vec_ok && (N <= 2560 || (N <= 4096 && K <= 4096))) cfg = dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {4, 1, 8}, 1, 0};
+  // up to 128 rows of A: the share kernel where it leads (decided by M itself: what A costs it goes with M, and the table's
+  // row is sized for the end of its bucket)
+  int rows = 0, cols = 0;
+  if (!user && vec_ok && share_leads(M, N, K, &rows, &cols)) cfg = dtas_config{DTAS_GEMM_SHARE, 256, 8, 1, {rows, cols, 0}, 1, 0};
   if (cfg.vec == 8 && !vec_ok) cfg.vec = 1;  // K % 8 != 0 or odd pointers: element accesses
   int64_t la[7];
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;
@@ -308,6 +322,7 @@ extern "C" int dtas_gemm_f16_fused(const void* A, const void* W, const void* bia
   if (cfg.vec == 1) return launch_gemm_scalar("gemm", static_cast<unsigned>(la[0]), 1, s, a, w, b, c, M, N, K, false);
   if (cfg.variant == DTAS_GEMM_ROWS) return launch_gemm_rows(cfg, la, s, a, w, b, c, M, N, K);
   if (cfg.variant == DTAS_GEMM_SKINNY) return launch_gemm_skinny(cfg, la, s, a, w, b, c, M, N, K);
+  if (cfg.variant == DTAS_GEMM_SHARE) return launch_gemm_share(cfg.tile[0], cfg.tile[1], s, a, w, b, c, M, N, K);
   if (cfg.variant == DTAS_GEMM_STREAM) return launch_gemm_stream(cfg, s, a, w, b, c, M, N, K);
   return launch_tile_f16(cfg, s, a, w, b, c, M, N, K, 1);
 }

@@ -112,13 +112,18 @@ enum dtas_variant {
                              tile[2] = 256 is the looping form for a W with many rows: tile = {16, 16 | 64, 256}, a
                              workgroup owns its columns over the whole of K and walks it in segments of 256 through a
                              ring of four LDS stages; no workspace */
-  DTAS_GEMM_MFMA_ACC16 = 4 /* the reference's scheduled arithmetic: an fp16 accumulator updated once per k step of 16 by one
+  DTAS_GEMM_MFMA_ACC16 = 4, /* the reference's scheduled arithmetic: an fp16 accumulator updated once per k step of 16 by one
                              matrix-core instruction, as its wmma 16x16x16 kernels with a float16 "wmma.accumulator" do
                              (experiment/testIR/GEMM/m_n2560_k10240/wmma/16x16x16/i2j4_x7y2_in8.py:19,37): the 16 products
                              of a step are added to the accumulator at fp32 precision and the sum is rounded to fp16 before
                              the next step.  tile = {64, 64, 16}, block 256, vec 8 or 1, split_k 1 (the rounding order
                              admits no K split); any M; never the built-in choice.  A mode for comparing against the
                              reference's own numbers, not for speed: every step waits for its rounding */
+  DTAS_GEMM_SHARE = 5      /* M <= tile[0]: W streamed once, an equal number of columns (at most tile[1]) per workgroup over the
+                             whole of K, no workspace; block 256.  tile[0] x tile[1]: {16, 32, 48, 64} x {16, 32, 48, 64, 128}
+                             (16 x 48 excepted), 96 x {16, 32, 48}, 128 x 48; 8-bit weights: {16, 32, 48, 64} x {16, 32,
+                             48, 64, 128}, 80 x 16, 96 x {32, 48}.  With cfg == NULL the GEMM entry points take it up to
+                             128 rows (8-bit weights 96) wherever it leads at the M at hand, ahead of the bucket's row */
 };
 
 /* One row of a call table: the launch-relevant part of the reference's *Config classes
