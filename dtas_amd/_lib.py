@@ -144,6 +144,12 @@ def lib() -> ctypes.CDLL:
     return _lib
 
 
+def entry_addresses() -> dict:
+    """{entry point: its address in the loaded library}, as a C caller would link them."""
+    handle = lib()
+    return {name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in (*SIGNATURES, "dtas_last_error")}
+
+
 def last_error() -> str:
     return lib().dtas_last_error().decode("utf-8", "replace")
 

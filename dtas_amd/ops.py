@@ -5,6 +5,9 @@ experiment/dtas_tuned/elementwise/add/profile_add.py:26): the caller allocates e
 included; nothing is allocated or synchronised here.  Tensors must be contiguous device tensors; the
 kernel goes on torch's current stream.  ``cfg`` (a ``_lib.DtasConfig``) overrides the built-in bucket
 table.  torch is used for device memory and streams only.
+
+The ordinary call (plain contiguous device tensors that fit together, no ``cfg``) is checked and launched by
+``_fastcall`` (csrc/fastcall.cpp); the Python bodies below serve every other call and word every refusal.
 """
 from __future__ import annotations
 
@@ -14,7 +17,12 @@ from typing import Optional
 import torch
 
 from . import _lib
-from ._lib import DtasConfig, check, lib
+from ._lib import DtasConfig, DtasError, check
+
+try:
+    from . import _fastcall
+except ImportError as e:
+    raise ImportError("dtas_amd/_fastcall.so is missing or was built for another torch: build it with `make -C dtas_amd/csrc`") from e
 
 _ELT = {
     ("add", torch.float16): ("dtas_add_f16", _lib.OP_ADD_F16),
@@ -24,6 +32,19 @@ _ELT = {
     ("copy", torch.float32): ("dtas_copy_f32", _lib.OP_COPY_F32),
     ("copy", torch.int8): ("dtas_copy_i8", _lib.OP_COPY_I8),
 }
+
+
+_bound = None  # the library whose entry points _fastcall holds
+
+
+def lib() -> ctypes.CDLL:
+    """The loaded library.  The first call hands its entry points to ``_fastcall``, which refuses every call until then."""
+    global _bound
+    handle = _lib.lib()
+    if handle is not _bound:
+        _fastcall.bind(_lib.entry_addresses(), DtasError)
+        _bound = handle
+    return handle
 
 
 _raw_stream = getattr(torch._C, "_cuda_getCurrentRawStream", None)
@@ -63,6 +84,8 @@ def _rows_cols(t: torch.Tensor):
 
 def add(A: torch.Tensor, B: torch.Tensor, T_add: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """T_add = A + B, elementwise, fp16 / fp32 / int8 (int8 wraps)."""
+    if cfg is None and _fastcall.add(A, B, T_add):
+        return
     _dev(A, B, T_add)
     if not (A.dtype == B.dtype == T_add.dtype) or not (A.shape == B.shape == T_add.shape):
         raise ValueError("add: A, B, T_add must agree in dtype and shape")
@@ -73,6 +96,8 @@ def add(A: torch.Tensor, B: torch.Tensor, T_add: torch.Tensor, cfg: Optional[Dta
 
 def copy(A: torch.Tensor, B: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """B = A, bit for bit."""
+    if cfg is None and _fastcall.copy(A, B):
+        return
     _dev(A, B)
     if A.dtype != B.dtype or A.shape != B.shape:
         raise ValueError("copy: A and B must agree in dtype and shape")
@@ -83,6 +108,8 @@ def copy(A: torch.Tensor, B: torch.Tensor, cfg: Optional[DtasConfig] = None) -> 
 
 def cast(A: torch.Tensor, compute: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """compute = Cast(A): fp16 -> fp32 (exact) or fp32 -> fp16 (round to nearest even, overflow to inf)."""
+    if cfg is None and _fastcall.cast(A, compute):
+        return
     _dev(A, compute)
     if A.shape != compute.shape:
         raise ValueError("cast: shapes differ")
@@ -100,6 +127,8 @@ def cast(A: torch.Tensor, compute: torch.Tensor, cfg: Optional[DtasConfig] = Non
 def layer_norm(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, out: torch.Tensor, eps: float = 1e-5,
                cfg: Optional[DtasConfig] = None) -> None:
     """fused_layer_norm_cast1: fp32 x, gamma, beta -> fp16 out, over the last axis."""
+    if cfg is None and _fastcall.layer_norm(x, gamma, beta, out, eps):
+        return
     _dev(x, gamma, beta, out)
     n, H = _rows_cols(x)
     if x.dtype != torch.float32 or gamma.dtype != torch.float32 or beta.dtype != torch.float32 or out.dtype != torch.float16:
@@ -112,6 +141,8 @@ def layer_norm(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, out: to
 
 def layer_norm_f32(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, out: torch.Tensor, eps: float = 1e-5) -> None:
     """layer_norm / layer_norm1 (dolly-v2-3b-q0f16/before_dl.py:846-896): layer norm over the last axis, fp32 in and out."""
+    if _fastcall.layer_norm_f32(x, gamma, beta, out, eps):
+        return
     _dev(x, gamma, beta, out)
     if any(t.dtype != torch.float32 for t in (x, gamma, beta, out)) or out.shape != x.shape:
         raise ValueError("layer_norm_f32: expects fp32 tensors and an output of x's shape")
@@ -124,6 +155,8 @@ def layer_norm_f32(x: torch.Tensor, gamma: torch.Tensor, beta: torch.Tensor, out
 def rms_norm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, eps: float = 1e-5,
              cfg: Optional[DtasConfig] = None) -> None:
     """out = x * rsqrt(mean(x^2) + eps) * w over the last axis; fp16 in/out, fp32 arithmetic."""
+    if cfg is None and _fastcall.rms_norm(x, w, out, eps):
+        return
     _dev(x, w, out)
     n, H = _rows_cols(x)
     if x.dtype != torch.float16 or w.dtype != torch.float16 or out.dtype != torch.float16:
@@ -135,6 +168,8 @@ def rms_norm(x: torch.Tensor, w: torch.Tensor, out: torch.Tensor, eps: float = 1
 
 def softmax(A: torch.Tensor, out: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """fused_softmax_cast: softmax over the last axis, fp32 or fp16 in, fp16 out."""
+    if cfg is None and _fastcall.softmax(A, out):
+        return
     _dev(A, out)
     if out.dtype != torch.float16 or out.shape != A.shape:
         raise ValueError("softmax: out must be fp16 with A's shape")
@@ -155,6 +190,8 @@ def gemv(x: torch.Tensor, W: torch.Tensor, bias: Optional[torch.Tensor], y: torc
     (fused_NT_matmul10_add5); 1 ``(res1 + (mm + bias)) + res2`` (fused_NT_matmul8_add5_add7_add7,
     before_dl.py:408-439); 2 the same into an fp32 y (.._cast5, :442-480); 3 ``gelu(mm + bias)``
     (fused_NT_matmul9_add6_gelu1, :483-549)."""
+    if cfg is None and _fastcall.gemv(x, W, bias, y, epilogue, res1, res2):
+        return
     _dev(x, W, bias, y, res1, res2)
     N, K = W.shape
     if x.numel() != K or y.numel() != N or any(t is not None and t.numel() != N for t in (bias, res1, res2)):
@@ -172,6 +209,8 @@ def gemv(x: torch.Tensor, W: torch.Tensor, bias: Optional[torch.Tensor], y: torc
 
 def gemv_f32(x: torch.Tensor, W: torch.Tensor, y: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """y[N] = W[N,K] . x[K], all fp32: NT_matmul5 (dolly-v2-3b-q0f16/before_dl.py:8-19)."""
+    if cfg is None and _fastcall.gemv_f32(x, W, y):
+        return
     _dev(x, W, y)
     N, K = W.shape
     if x.numel() != K or y.numel() != N:
@@ -188,6 +227,8 @@ def gemm(A: torch.Tensor, W: torch.Tensor, bias: Optional[torch.Tensor], C: torc
     extent of A flattened.  epilogue (``_lib.EPI_*``): 0 ``+ bias``; 1 ``(res1 + (mm + bias)) + res2``;
     2 the same into an fp32 C; 3 ``gelu(mm + bias)`` -- each step rounded to fp16 as in the fused
     PrimFuncs (before_dl.py:163-318)."""
+    if cfg is None and _fastcall.gemm(A, W, bias, C, epilogue, res1, res2):
+        return
     _dev(A, W, bias, C, res1, res2)
     N, K = W.shape
     if A.shape[-1] != K or C.shape[-1] != N:
@@ -213,6 +254,8 @@ def attn_scores(Q: torch.Tensor, K: torch.Tensor, mask: torch.Tensor, out: torch
     """out[h,n,m] (fp32) = min(max(fp16(Q[h,n,:] . K[h,m,:]) * fp16(scale), -65504), mask[n,m]), each step an fp16
     value: fused_NT_matmul1_divide_maximum_minimum_cast2 (before_dl.py:116-160).  Q (..., heads, n, d),
     K (..., heads, m, d), mask (..., n, m) with leading extents of 1."""
+    if cfg is None and _fastcall.attn_scores(Q, K, mask, out, scale):
+        return
     _dev(Q, K, mask, out)
     heads, n, d = Q.shape[-3:]
     m = K.shape[-2]
@@ -230,6 +273,8 @@ def attn_pv(P: torch.Tensor, V: torch.Tensor, out: torch.Tensor, cfg: Optional[D
     """out[h,n,:] = sum_k P[h,n,k] * V[h,k,:], fp16 with fp32 accumulation: matmul8 (before_dl.py:915-929) and,
     with n = 1, matmul10 (:899-912).  P (..., heads, n, m), V (..., heads, m, d), out (..., heads, n, d) with
     leading extents of 1."""
+    if cfg is None and _fastcall.attn_pv(P, V, out):
+        return
     _dev(P, V, out)
     heads, n, m = P.shape[-3:]
     d = V.shape[-1]
@@ -254,6 +299,8 @@ def _q8_shapes(what: str, Wq: torch.Tensor, scale: torch.Tensor, scale_dtype=tor
 def decode_q8(Wq: torch.Tensor, scale: torch.Tensor, W: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """W[N,K] (fp16) = (fp16(byte) - 127) * scale[N, K/32]; element j of a row is byte j % 4 of word j / 4 of
     Wq[N, K/4]: fused_decode3 (dolly-v2-3b-q8f16_1/before_dl.py:335-343)."""
+    if cfg is None and _fastcall.decode_q8(Wq, scale, W):
+        return
     _dev(Wq, scale, W)
     N, K = _q8_shapes("decode_q8", Wq, scale)
     if W.dtype != torch.float16 or W.numel() != N * K:
@@ -265,6 +312,8 @@ def attn_mask(out: torch.Tensor) -> None:
     """out (..., n, m) fp16 = the causal mask of n query positions against m >= n key positions (65504 where a key
     may be seen, -65504 where not): fused_min_max_triu_te_broadcast_to + extend_te, and full for n = 1
     (dolly-v2-3b-q0f16/before_dl.py:642-658, :68-80, :83-93)."""
+    if _fastcall.attn_mask(out):
+        return
     _dev(out)
     n, m = out.shape[-2:]
     if out.dtype != torch.float16 or out.numel() != n * m:
@@ -275,6 +324,8 @@ def attn_mask(out: torch.Tensor) -> None:
 def softmax_temperature(logits: torch.Tensor, temperature: torch.Tensor, out: torch.Tensor) -> None:
     """softmax_with_temperature (dolly-v2-3b-q0f16/before_dl.py:4154-4161): out = softmax(logits / temperature) over
     the last axis, fp32 in and out; `temperature` is a 0-d (or one-element) fp32 device tensor."""
+    if _fastcall.softmax_temperature(logits, temperature, out):
+        return
     _dev(logits, temperature, out)
     if logits.dtype != torch.float32 or out.dtype != torch.float32 or temperature.dtype != torch.float32:
         raise ValueError("softmax_temperature: logits, temperature and out must be fp32")
@@ -305,6 +356,8 @@ def softmax_f32(A: torch.Tensor, out: torch.Tensor) -> None:
 def split3(A: torch.Tensor, out0: torch.Tensor, out1: torch.Tensor, out2: torch.Tensor) -> None:
     """split / fused_reshape7_split1 (dolly-v2-3b-q0f16/before_dl.py:1099-1125, :661-688): A (..., 3 d) fp16 cut into
     three (..., d) buffers along the last axis."""
+    if _fastcall.split3(A, out0, out1, out2):
+        return
     _dev(A, out0, out1, out2)
     d3 = A.shape[-1]
     if d3 % 3 != 0:
@@ -322,6 +375,8 @@ def split3(A: torch.Tensor, out0: torch.Tensor, out1: torch.Tensor, out2: torch.
 def swap_axes(A: torch.Tensor, out: torch.Tensor) -> None:
     """out (..., b, a, d) = A (..., a, b, d) with leading extents of 1, fp16: transpose6 / transpose7
     (dolly-v2-3b-q0f16/before_dl.py:1177-1203)."""
+    if _fastcall.swap_axes(A, out):
+        return
     _dev(A, out)
     a, b, d = A.shape[-3:]
     if A.dtype != torch.float16 or out.dtype != torch.float16 or A.numel() != a * b * d or tuple(out.shape[-3:]) != (b, a, d) \
@@ -335,6 +390,8 @@ def rotary(A: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, out: torch.Ten
     """rotary_embedding (dolly-v2-3b-q0f16/before_dl.py:1023-1035; rotary_embedding1 :1038-1047): A and out
     (..., n, heads, d) fp16 with leading extents of 1, cos / sin [max_pos, rot] fp16; position s of A takes the
     tables' row m + s - n (m = length of the whole sequence)."""
+    if cfg is None and _fastcall.rotary(A, cos, sin, out, m):
+        return
     _dev(A, cos, sin, out)
     if any(t.dtype != torch.float16 for t in (A, cos, sin, out)) or cos.dim() != 2 or cos.shape != sin.shape or A.dim() < 3:
         raise ValueError("rotary: expects fp16 A (..., n, heads, d) and fp16 tables [max_pos, rot]")
@@ -348,6 +405,8 @@ def rotary(A: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, out: torch.Ten
 def take(A: torch.Tensor, ids: torch.Tensor, out: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """out[n,H] = A[ids[i], :], the fp16 embedding lookup: take (dolly-v2-3b-q0f16/before_dl.py:1151-1163) and, one row,
     take1 (:1166-1174).  ids int32; values outside [0, V) are clipped to the nearest row."""
+    if cfg is None and _fastcall.take(A, ids, out):
+        return
     _dev(A, ids, out)
     if A.dim() != 2 or A.dtype != torch.float16 or ids.dtype != torch.int32 or out.dtype != torch.float16:
         raise ValueError("take: expects an fp16 table [V, H], int32 ids[n] and an fp16 output")
@@ -362,6 +421,8 @@ def take_q8(Wq: torch.Tensor, scale: torch.Tensor, ids: torch.Tensor, out: torch
     """out[n,K] (fp16) = rows ids[i] of decode_q8(Wq, scale), the embedding lookup of the 8-bit model:
     fused_fused_decode1_take1 (dolly-v2-3b-q8f16_1/before_dl.py:357-369) and, one row, fused_fused_decode1_take
     (:346-355).  ids int32; values outside [0, V) are clipped to the nearest row."""
+    if cfg is None and _fastcall.take_q8(Wq, scale, ids, out):
+        return
     _dev(Wq, scale, ids, out)
     V, K = _q8_shapes("take_q8", Wq, scale)
     n = ids.numel()
@@ -373,6 +434,8 @@ def take_q8(Wq: torch.Tensor, scale: torch.Tensor, ids: torch.Tensor, out: torch
 def gemv_q8_f32(x: torch.Tensor, Wq: torch.Tensor, scale: torch.Tensor, y: torch.Tensor, cfg: Optional[DtasConfig] = None) -> None:
     """fp32 y[N] = x[K] . W^T with W = float32(byte - 127) * scale[N, K/32] (fp32 scales), never written: the vocabulary
     projection of the 8-bit model, fused_fused_decode6_NT_matmul5 (dolly-v2-3b-q8f16_1/before_dl.py:640-657)."""
+    if cfg is None and _fastcall.gemv_q8_f32(x, Wq, scale, y):
+        return
     _dev(x, Wq, scale, y)
     N, K = _q8_shapes("gemv_q8_f32", Wq, scale, torch.float32)
     if x.numel() != K or y.numel() != N:
@@ -387,6 +450,8 @@ def gemv_q8(x: torch.Tensor, Wq: torch.Tensor, scale: torch.Tensor, bias: Option
     """y[N] = x[K] . decode_q8(Wq, scale)^T (+ bias[N]; ``_lib.EPI_BIAS_GELU``: then GELU), the weights dequantised
     in registers: fused_fused_decode2_fused_NT_matmul_add / fused_fused_decode4_fused_NT_matmul3_add2_gelu
     (dolly-v2-3b-q8f16_1/before_dl.py:401-426, :428-502)."""
+    if cfg is None and _fastcall.gemv_q8(x, Wq, scale, bias, y, epilogue):
+        return
     _dev(x, Wq, scale, bias, y)
     N, K = _q8_shapes("gemv_q8", Wq, scale)
     if x.numel() != K or y.numel() != N or (bias is not None and bias.numel() != N):
@@ -402,6 +467,8 @@ def gemm_q8(A: torch.Tensor, Wq: torch.Tensor, scale: torch.Tensor, bias: Option
             res2: Optional[torch.Tensor] = None) -> None:
     """C[M,N] = epilogue(A[M,K] . decode_q8(Wq, scale)^T), the weights dequantised on their way into the LDS: the
     dynamic-n q8f16_1 PrimFuncs (dolly-v2-3b-q8f16_1/before_dl.py:371-399, :504-581); epilogues as ``gemm``."""
+    if cfg is None and _fastcall.gemm_q8(A, Wq, scale, bias, C, epilogue, res1, res2):
+        return
     _dev(A, Wq, scale, bias, C, res1, res2)
     N, K = _q8_shapes("gemm_q8", Wq, scale)
     if A.shape[-1] != K or C.shape[-1] != N:
