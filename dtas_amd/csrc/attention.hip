@@ -365,6 +365,145 @@ __global__ void __launch_bounds__(256) attn_scores_pipe_kernel(const half_t* __r
   store_held();
 }
 
+// Scores whose rows are not whole 64-byte sectors (m % 16 != 0, or an output that is not sector-aligned).  Tiles cut every
+// row at the same columns, so the sector on each cut is written in two parts by two workgroups, and what the two L2s
+// cannot join is filled from memory first.  Here every row is cut at sector boundaries of its own: a workgroup takes 32
+// query rows and `chunk` keys (a multiple of 16, at most 480), computes 16 keys more, and writes of each row the whole
+// sectors that start in its chunk.  Only a row's two ends share a sector with its neighbours.
+//  * Q's fragments stay in registers, K's come straight from memory (5 KiB per 32 keys of 80, read in whole; the
+//    workgroups of a head share them in the L2), the next block's under the MFMAs of this one; no operand stages.
+//  * Q is the first MFMA operand, so that a lane holds one key of 16 rows, and a half-wavefront stores 32 neighbouring
+//    scores of a row; a row lies in the LDS at its distance from a 16-byte boundary of the output, so that four scores are
+//    one 8-byte LDS read, one (under-aligned) 8-byte read of the mask, requested before the products, and one aligned
+//    16-byte streaming store.  33 KiB of LDS: four workgroups per CU.
+// What bounds it: beside the stores, K passes through a CU's L1 once per 32 query rows.  32 heads of 80 against the tiles: 203 x 1031
+// 15.6 -> 13.3 us, 130 x 2049 18.0 -> 15.4.  Not kept: K through the LDS in 1 KiB loads (two workgroups per CU), that with 64 rows;
+// registers for three workgroups per CU; the mask under a row's ends loaded where it is used (a memory latency per end).
+template <int KS>
+__global__ void __launch_bounds__(256, 4) attn_scores_sector_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ Kmat,
+                                                                 const half_t* __restrict__ mask, float* __restrict__ out,
+                                                                 int64_t n, int64_t m, int64_t d, float scale, unsigned chunk,
+                                                                 unsigned tiles_m, unsigned tiles_n, unsigned heads, unsigned pinned) {
+  __shared__ __attribute__((aligned(16))) half_t rows[kSectorRows * kSectorPitch];
+  const unsigned t = threadIdx.x, l = t & 63u, wv = __builtin_amdgcn_readfirstlane(t >> 6);
+  // tile numbering as in attn_scores_kernel
+  const unsigned per_batch = tiles_m * tiles_n;
+  unsigned batch, pid;
+  if (pinned) {
+    const unsigned span_base = per_batch / kNumXCD, span_rem = per_batch % kNumXCD;
+    const unsigned xcd = blockIdx.x % kNumXCD, local = blockIdx.x / kNumXCD;
+    const unsigned span = span_base + (xcd < span_rem ? 1u : 0u), first = xcd * span_base + (xcd < span_rem ? xcd : span_rem);
+    if (local >= span * heads) return;  // (the shorter spans end earlier; uniform over the workgroup)
+    batch = __builtin_amdgcn_readfirstlane(local / span);
+    pid = __builtin_amdgcn_readfirstlane(first + local % span);
+  } else {
+    const unsigned gid = xcd_contiguous_id(blockIdx.x, per_batch * heads);
+    batch = __builtin_amdgcn_readfirstlane(gid / per_batch);
+    pid = __builtin_amdgcn_readfirstlane(gid % per_batch);
+  }
+  const unsigned tm = __builtin_amdgcn_readfirstlane(pid / tiles_n), tn = __builtin_amdgcn_readfirstlane(pid % tiles_n);
+  const int64_t m0 = static_cast<int64_t>(tm) * kSectorRows, c0 = static_cast<int64_t>(tn) * chunk;
+  const int rows_a = static_cast<int>(n - m0 < kSectorRows ? n - m0 : kSectorRows);
+  const int left = static_cast<int>(m - c0 < kSectorKeys ? m - c0 : kSectorKeys);   // keys from c0 on, as far as they count here
+  const bool last = c0 + chunk >= m;
+  const unsigned row_bytes = static_cast<unsigned>(d) * 2u;
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(Q + (static_cast<int64_t>(batch) * n + m0) * d, static_cast<unsigned>(rows_a) * row_bytes);
+  const __amdgpu_buffer_rsrc_t rw = make_rsrc(Kmat + (static_cast<int64_t>(batch) * m + c0) * d, static_cast<unsigned>(left) * row_bytes);
+
+  // fragments: lane l supplies row l & 31, 16-byte piece 2 ks + (l >> 5) (rows past the extents and pieces past d: zeros)
+  auto fragments = [&](const __amdgpu_buffer_rsrc_t& r, unsigned block, u32x4 (&f)[KS]) {
+    const unsigned at = (block * 32u + (l & 31u)) * row_bytes + (l >> 5) * 16u;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      f[ks] = __builtin_amdgcn_raw_buffer_load_b128(r, (2 * ks + (l >> 5)) * 8u < static_cast<unsigned>(d) ? at + ks * 32u : kOob, 0, 0);
+  };
+  u32x4 fq[KS], fk[KS];
+  fragments(ra, 0, fq);
+  fragments(rw, wv, fk);
+
+  // row r of the tile: its sectors begin at the columns (from c0) that are -lead(r) modulo 16
+  const unsigned base = static_cast<unsigned>(reinterpret_cast<uintptr_t>(out) >> 2) +
+                        static_cast<unsigned>((static_cast<int64_t>(batch) * n + m0) * m + c0), m_low = static_cast<unsigned>(m);
+  auto lead = [&](unsigned r) -> int { return static_cast<int>((base + r * m_low) & 15u); };
+  // wavefront w writes rows w, w + 4, ...: lane l the columns from 4 (l + 64 p) - lead % 4 on, in [lo, hi)
+  constexpr int kMine = kSectorRows / 4, kPasses = 2;
+  auto bounds = [&](int s, int& lo, int& hi) {
+    const int up = (16 - s) & 15;
+    lo = tn == 0 ? 0 : up;
+    hi = last || static_cast<int>(chunk) + up > left ? left : static_cast<int>(chunk) + up;
+  };
+  // a vector over a row's end reads into its neighbour, whose elements are not used; at the two ends of the mask it is moved inside
+  const int64_t mask_end = n * m - 4;
+  auto mask_at = [&](int64_t f) -> int64_t { return f < 0 ? 0 : f > mask_end ? mask_end : f; };
+  f16x4 mk[kMine][kPasses];
+#pragma unroll
+  for (int i = 0; i < kMine; ++i) {
+    const unsigned r = wv + 4u * i;
+    int lo, hi;
+    const int s = lead(r);
+    bounds(s, lo, hi);
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int col = 4 * static_cast<int>(l + 64 * p) - (s & 3);
+      mk[i][p] = f16x4{};
+      if (static_cast<int>(r) < rows_a && col + 4 > lo && col < hi)
+        mk[i][p] = *reinterpret_cast<const f16x4_a2*>(mask + mask_at((m0 + r) * m + c0 + col));
+    }
+  }
+
+  const int keys = last || static_cast<int>(chunk) + 15 > left ? left : static_cast<int>(chunk) + 15;
+  const unsigned blocks = static_cast<unsigned>((keys + 31) / 32);  // at most 16
+  for (unsigned b = wv; b < blocks; b += 4) {
+    u32x4 next[KS];
+    fragments(rw, b + 4, next);  // (past the last block: out of range, zeros)
+    f32x16 acc;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks)
+      acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fq[ks]), __builtin_bit_cast(f16x8, fk[ks]), acc, 0, 0, 0);
+    // acc[v] of lane l: row 8 (v / 4) + 4 (l >> 5) + v % 4, key l & 31 of the block
+    half_t* dst = rows + (4u * (l >> 5)) * kSectorPitch + b * 32u + (l & 31u);
+#pragma unroll
+    for (int v = 0; v < 16; ++v) dst[(8 * (v / 4) + v % 4) * kSectorPitch + (lead(v % 4) & 3)] = static_cast<half_t>(acc[v]);  // (lead modulo 4: rows 4 apart alike)
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) fk[ks] = next[ks];
+  }
+  __syncthreads();
+
+#pragma unroll
+  for (int i = 0; i < kMine; ++i) {
+    const unsigned r = wv + 4u * i;
+    if (static_cast<int>(r) >= rows_a) break;  // (uniform)
+    int lo, hi;
+    const int s = lead(r);
+    bounds(s, lo, hi);
+    float* dst = out + (static_cast<int64_t>(batch) * n + m0 + r) * m + c0;
+#pragma unroll
+    for (int p = 0; p < kPasses; ++p) {
+      const int group = static_cast<int>(l + 64 * p), col = 4 * group - (s & 3);
+      f16x4 hv = *reinterpret_cast<const f16x4*>(rows + r * kSectorPitch + 4 * group);
+      if (col >= lo && col + 4 <= hi) {
+        hv = scores_steps_vec(hv, scale, mk[i][p]);
+        __builtin_nontemporal_store(f32x4v{static_cast<float>(hv[0]), static_cast<float>(hv[1]), static_cast<float>(hv[2]), static_cast<float>(hv[3])},
+                                    reinterpret_cast<f32x4v*>(dst + col));
+      } else if (col + 4 > lo && col < hi) {  // a row's ends
+        f16x4 mv = mk[i][p];
+        const int64_t f = (m0 + r) * m + c0 + col;
+        if (f != mask_at(f)) {  // (the first or last row of the whole mask)
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (col + e >= lo && col + e < hi) mv[e] = mask[f + e];
+        }
+        hv = scores_steps_vec(hv, scale, mv);
+#pragma unroll
+        for (int e = 0; e < 4; ++e)
+          if (col + e >= lo && col + e < hi) dst[col + e] = static_cast<float>(hv[e]);
+      }
+    }
+  }
+}
+
 // P.V for a handful of query rows (decoding): out[h, r, :] = sum_k P[h, r, k] * V[h, k, :].
 // Workgroup = (head, 8 columns of V, R rows of P); thread t takes k = t, t + 256, ...: a 16-byte piece
 // of V's row k and P[h, r, k] of each row, eight k at a time with every load requested before the
@@ -668,6 +807,27 @@ extern "C" int dtas_attn_scores_f16_f32(const void* Q, const void* Kmat, const v
         hipLaunchKernelGGL(attn_scores_pipe_kernel<4>, dim3(static_cast<unsigned>(grid_p)), dim3(256), 0, static_cast<hipStream_t>(stream), q_, k_, m_,
                            static_cast<float*>(out), n, m, d, sc, tm, tn, static_cast<unsigned>(heads), pin);
       return check_launch("attn_scores");
+    }
+    // ... or every row is cut at sectors of its own (attn_scores_sector_kernel), for continuations of up to 256 rows.  32 heads
+    // of 80, tiles / own sectors, us: n x m = 203 x 703 12.1 / 11.7, 203 x 1031 15.6 / 13.3, 130 x 2049 18.0 / 15.4; a layer of 250
+    // rows behind 1501 keys 222.5 / 219.7.  Prompts: launches of scores alone gain more (2047 x 2047 208 / 128), but the softmax
+    // behind them then reads more from memory, and the layer gains nothing (1601: 636 / 642; 2047: 809 / 807).  Head
+    // dimensions of 64 and 128 pull more of K through the L1 than the tiles do (40 heads of 128, 1025 x 1025 57.6 / 98.9), and
+    // fewer workgroups than 1.75 per CU do not hide a workgroup's chain (65 x 481, 192 of them: 6.8 / 9.5)
+    const int64_t pieces = ceil_div(m, kSectorChunk), chunk = ceil_div(ceil_div(m, pieces), 16) * 16;
+    const int64_t tm_s = ceil_div(n, kSectorRows), tn_s = ceil_div(m, chunk), tiles_s = tm_s * tn_s;
+    if (!whole_sectors && d > 64 && d <= 80 && n <= 256 && m >= 700 && tiles_s * heads * 4 >= 7 * kNumCU) {
+      const bool pin = n * m >= (int64_t{1} << 21);
+      const int64_t wgs = pin ? kNumXCD * heads * ceil_div(tiles_s, kNumXCD) : tiles_s * heads;
+      if (wgs > 0x7fffffff) return fail("attn_scores: too many tiles");
+      auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(wgs)), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const half_t*>(Q),
+                           static_cast<const half_t*>(Kmat), static_cast<const half_t*>(mask), static_cast<float*>(out), n, m, d,
+                           static_cast<float>(static_cast<half_t>(scale)), static_cast<unsigned>(chunk), static_cast<unsigned>(tm_s),
+                           static_cast<unsigned>(tn_s), static_cast<unsigned>(heads), pin ? 1u : 0u);
+        return check_launch("attn_scores");
+      };
+      return launch(attn_scores_sector_kernel<5>);
     }
     const int64_t grid = !whole_sectors || total < 3 * kNumCU ? total : 3 * kNumCU;
     hipLaunchKernelGGL((attn_scores_kernel<128, 64>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, static_cast<hipStream_t>(stream),

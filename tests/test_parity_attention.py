@@ -52,6 +52,25 @@ def test_scores_builtin_other_head_dims(oracle, heads, n, m, d):
     _check(out.check(), q, k, mask, oracle)
 
 
+@pytest.mark.parametrize("heads,n,m,d,at", [(32, 225, 700, 80, 1), (32, 225, 960, 80, 4), (32, 256, 1201, 72, 2), (4, 256, 8193, 80, 3)])
+def test_scores_rows_cut_at_their_own_sectors(oracle, heads, n, m, d, at):
+    # rows that are no whole 64-byte sectors, or an output `at` floats off one: chunks of up to 480 keys whose edges move with
+    # the row (two to five of them; whole and partly filled blocks of 32 rows; head dimensions with and without an empty half
+    # k step; unequal spans per XCD from 2 M scores per head on).  Integer operands: every product and sum is exact, so the bits are the general kernel's
+    q, k, mask = _inputs(heads, n, m, d, n + m + d)
+    buf = torch.full((heads * n * m + at + 16,), -7.0, dtype=torch.float32, device="cuda")
+    out = buf[at:at + heads * n * m].view(heads, n, m)
+    ops.attn_scores(dev(q), dev(k), dev(mask), out, SCALE)
+    _check(out.cpu().numpy(), q, k, mask, oracle)
+    rng = np.random.default_rng(d)
+    qi, ki = (rng.integers(-4, 5, size=a.shape).astype(np.float16) for a in (q, k))
+    ops.attn_scores(dev(qi), dev(ki), dev(mask), out, SCALE)
+    want = torch.empty(heads, n, m, dtype=torch.float32, device="cuda")
+    ops.attn_scores(dev(qi), dev(ki), dev(mask), want, SCALE, cfg(variant=_lib.GEMM_MFMA, block=256, vec=8, unroll=2, tile=[64, 64, 64]))
+    assert torch.equal(out, want)
+    assert bool((buf[:at] == -7.0).all()) and bool((buf[at + heads * n * m:] == -7.0).all())
+
+
 @pytest.mark.parametrize("tile,block,stages", [((64, 64), 256, 2), ((64, 64), 256, 3), ((128, 128), 256, 2), ((128, 64), 256, 2),
                                                ((64, 128), 256, 2), ((256, 128), 256, 2), ((256, 256), 512, 2), ((256, 256), 256, 2)])
 @pytest.mark.parametrize("heads,n,m,d", [(3, 70, 131, 80), (2, 300, 260, 64), (1, 33, 7, 8)])
