@@ -379,6 +379,7 @@ __global__ void __launch_bounds__(256) attn_scores_pipe_kernel(const half_t* __r
 // What bounds it: beside the stores, K passes through a CU's L1 once per 32 query rows.  32 heads of 80 against the tiles: 203 x 1031
 // 15.6 -> 13.3 us, 130 x 2049 18.0 -> 15.4.  Not kept: K through the LDS in 1 KiB loads (two workgroups per CU), that with 64 rows;
 // registers for three workgroups per CU; the mask under a row's ends loaded where it is used (a memory latency per end).
+constexpr int kSectorRows = 32, kSectorKeys = 512, kSectorChunk = 480, kSectorPitch = kSectorKeys + 4;  // KS: k steps of 16 that hold the head dimension
 template <int KS>
 __global__ void __launch_bounds__(256, 4) attn_scores_sector_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ Kmat,
                                                                  const half_t* __restrict__ mask, float* __restrict__ out,
