@@ -122,8 +122,11 @@ __global__ void __launch_bounds__(256) gemm_share_kernel(const half_t* __restric
       __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(stage + S::kWBytes + (i * 4 + wv) * 1024), 16, at,
                                                static_cast<int>((i / kAPat) * 16u * row_bytes + seg * S::kARow), 0, 0);
     }
-    if constexpr (Q8)
-      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(stage + S::kWBytes + S::kABytes + wv * 1024), 16, off_s, static_cast<int>(seg * S::kScaleRow), 0, 0);
+    if constexpr (Q8) {
+      // (a piece past K would be the next row's first scales, which may be anything: inf x the zeros there is NaN)
+      const unsigned at = tail && k0 + (l % kPieces) * 256u >= K ? kOob : off_s;
+      __builtin_amdgcn_raw_ptr_buffer_load_lds(rs, (lds_ptr_t)(stage + S::kWBytes + S::kABytes + wv * 1024), 16, at, static_cast<int>(seg * S::kScaleRow), 0, 0);
+    }
   };
 #pragma unroll
   for (int p = 0; p < NSTG - 1; ++p)

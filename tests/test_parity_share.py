@@ -59,6 +59,25 @@ def test_share_kernels_on_8_bit_weights(oracle, rows, cols, kind, less, N_of, K)
     _check(out.check(), oracle.c.gemm_fused(a, w, bias, r1 if add2 else None, r2 if add2 else None, kind, threads=8), r1 if add2 else None, r2)
 
 
+@pytest.mark.parametrize("rows,cols", [(16, 16), (16, 32), (16, 48), (32, 16), (32, 32), (32, 48), (0, 0)])
+@pytest.mark.parametrize("K", [256, 768, 1280])
+@pytest.mark.parametrize("bad", [600.0, float("inf"), float("nan")])
+def test_the_scales_behind_a_row_stay_its_neighbours(oracle, rows, cols, K, bad):
+    # K ends inside a segment of 512: the 16 bytes behind a row's scales are the next row's, here too large for fp16 times a byte,
+    # infinite or NaN.  Only that row's column may show it (0, 0: what runs without a config)
+    M, N = rows or 29, 256 * (cols or 16) - 3
+    a, bias, _, _, rng = _inputs(M, N, K, K + rows)
+    wq = rng.integers(0, 2 ** 32, (N, K // 4), dtype=np.uint32)
+    scale = (rng.random((N, K // 32)) * 4e-4 + 1e-4).astype(np.float16)
+    good = np.arange(N) % 3 != 2
+    scale[~good] = bad
+    out = Guarded((M, N), torch.float16)
+    share = cfg(variant=_lib.GEMM_SHARE, tile=[rows, cols, 0]) if rows else None
+    ops.gemm_q8(dev(a), dev(wq.view(np.int32)), dev(scale), dev(bias), out.t, share)
+    want = oracle.c.gemm_fused(a, oracle.c.decode_q8(wq[good], scale[good]), np.ascontiguousarray(bias[good]), None, None, 0, threads=8)
+    _check(out.check()[:, good], want, None, None)
+
+
 @pytest.mark.parametrize("M", [3, 5, 16, 17, 33, 64, 65, 96, 128])
 @pytest.mark.parametrize("N,K", [(2560, 2560), (7680, 2560), (2560, 10240), (10240, 520), (257, 256), (17000, 2048)])
 def test_what_runs_without_a_config_either_side_of_the_line(oracle, M, N, K):
