@@ -80,6 +80,7 @@ SIGNATURES = {
     "dtas_init": [],
     "dtas_select_bucket": [_ci, _i64, _i64, _i64, ctypes.POINTER(DtasLaunchInfo)],
     "dtas_describe_launch": [_ci, _i64, _i64, _i64, _cfg, ctypes.POINTER(DtasLaunchInfo)],
+    "dtas_builtin_gemm": [_ci, _i64, _i64, _i64, ctypes.POINTER(DtasLaunchInfo)],
     "dtas_add_f16": [_vp, _vp, _vp, _i64, _i64, _cfg, _vp],
     "dtas_add_f32": [_vp, _vp, _vp, _i64, _i64, _cfg, _vp],
     "dtas_add_i8": [_vp, _vp, _vp, _i64, _i64, _cfg, _vp],
@@ -168,4 +169,11 @@ def select_bucket(op: int, n: int, d0: int = 0, d1: int = 0) -> DtasLaunchInfo:
 def describe_launch(op: int, n: int, d0: int, d1: int, cfg: DtasConfig) -> DtasLaunchInfo:
     info = DtasLaunchInfo()
     check(lib().dtas_describe_launch(op, n, d0, d1, ctypes.byref(cfg), ctypes.byref(info)), "dtas_describe_launch")
+    return info
+
+
+def builtin_gemm(M: int, N: int, K: int, q8: bool = False) -> DtasLaunchInfo:
+    """What a GEMM call without a config runs (``select_bucket`` reports the bucket table's row)."""
+    info = DtasLaunchInfo()
+    check(lib().dtas_builtin_gemm(int(q8), M, N, K, ctypes.byref(info)), "dtas_builtin_gemm")
     return info

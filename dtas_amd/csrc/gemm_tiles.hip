@@ -259,7 +259,42 @@ int launch_tile_f16(const dtas_config& cfg, hipStream_t s, const half_t* a, cons
   return fail("gemm: no MFMA kernel for tile %dx%d", bm, bn);
 }
 
+// What a call without a config runs: the bucket's row, or ahead of it a kernel chosen by M itself (what A costs it goes
+// with M, and the row is sized for the end of its bucket).  vec_ok: 16-byte loads of A and W are possible.
+dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok) {
+  // two rows of A (the first bucket's table row is sized for 16): W streamed in whole rows, as the GEMV does
+  if (M == 2 && vec_ok) return dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {2, N <= 2560 ? 1 : 2, 8}, 1, 0};
+  // up to 128 rows of A: the share kernel where it leads
+  int rows = 0, cols = 0;
+  if (vec_ok && share_leads(M, N, K, &rows, &cols)) return dtas_config{DTAS_GEMM_SHARE, 256, 8, 1, {rows, cols, 0}, 1, 0};
+  return builtin_config(DTAS_OP_GEMM_F16, M, N, K).cfg;
+}
+
 }  // namespace dtas
+
+extern "C" int dtas_builtin_gemm(int weights_8bit, int64_t M, int64_t N, int64_t K, dtas_launch_info* out) {
+  using namespace dtas;
+  clear_error();
+  if (!out) return fail("dtas_builtin_gemm: out is NULL");
+  if (M < 2 || N < 1 || K < 1) return fail("dtas_builtin_gemm: M >= 2, N >= 1 and K >= 1 wanted (one row is the GEMV), got %lld, %lld, %lld", (long long)M, (long long)N, (long long)K);
+  memset(out, 0, sizeof(*out));
+  out->index = -1;
+  out->table_row = -1;
+  const char* what = "gemm";
+  if (weights_8bit) {
+    if (K % 32 != 0) return fail("dtas_builtin_gemm: K must be a multiple of the scale group, 32 (K=%lld)", (long long)K);
+    what = "gemm_q8";
+    if (builtin_gemm_q8(M, N, K, K % 256 == 0, &out->config)) {
+      snprintf(out->name, sizeof(out->name), "%s", what);
+      return 0;  // (launch_args stay zero: the 8-bit kernels' grids are their launchers')
+    }
+    what = "decode_q8 + gemm";
+  }
+  snprintf(out->name, sizeof(out->name), "%s", what);
+  out->config = builtin_gemm(M, N, K, K % 8 == 0);
+  if (K % 8 != 0) out->config.vec = 1;
+  return describe_gemm(M, N, K, out->config, out->launch_args);
+}
 
 extern "C" int dtas_gemm_f16(const void* A, const void* W, const void* bias, void* C, int64_t M, int64_t N, int64_t K,
                              const dtas_config* user, void* stream) {
@@ -302,14 +337,8 @@ extern "C" int dtas_gemm_f16_fused(const void* A, const void* W, const void* bia
   if (!user && M == 1) return dtas_gemv_f16_fused(A, W, bias, res1, res2, C, N, K, epilogue, nullptr, stream);
   const GemmEpilogue ep = {static_cast<const half_t*>(bias), static_cast<const half_t*>(res1),
                            static_cast<const half_t*>(res2), epilogue, out_bytes == 4 ? 1 : 0, 0.f, 0, 0, 0, 0};
-  dtas_config cfg = user ? *user : builtin_config(DTAS_OP_GEMM_F16, M, N, K).cfg;
   const bool vec_ok = K % 8 == 0 && aligned(A, 16) && aligned(W, 16);
-  // two rows of A (the first bucket's table row is sized for 16): W streamed in whole rows, as the GEMV does
-  if (!user && M == 2 && vec_ok) cfg = dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {2, N <= 2560 ? 1 : 2, 8}, 1, 0};
-  // up to 128 rows of A: the share kernel where it leads (decided by M itself: what A costs it goes with M, and the table's
-  // row is sized for the end of its bucket)
-  int rows = 0, cols = 0;
-  if (!user && vec_ok && share_leads(M, N, K, &rows, &cols)) cfg = dtas_config{DTAS_GEMM_SHARE, 256, 8, 1, {rows, cols, 0}, 1, 0};
+  dtas_config cfg = user ? *user : builtin_gemm(M, N, K, vec_ok);
   if (cfg.vec == 8 && !vec_ok) cfg.vec = 1;  // K % 8 != 0 or odd pointers: element accesses
   int64_t la[7];
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;

@@ -167,13 +167,21 @@ const char* dtas_last_error(void);
  * static scratch array of dtas_gemm_f16_static there.  Optional: every entry point works without it. */
 int dtas_init(void);
 
-/* The built-in bucket table: which config a call with these extents uses.
+/* The built-in bucket table: the row that a call with these extents falls in, and its config.  A call without a config
+ * runs it, but for the GEMM of up to 128 rows, which may take a kernel chosen by M itself ahead of its row:
+ * dtas_builtin_gemm names what runs.
  * n = the dynamic extent (rows n; softmax: cols when dynamic; GEMM: M), d0/d1 = static extents
  * (elementwise/norm: H, 0; softmax: rows, cols; GEMV: N, K; GEMM: N, K). */
 int dtas_select_bucket(int op, int64_t n, int64_t d0, int64_t d1, dtas_launch_info* out);
 /* Resolve launch_args for an explicit config (used by tuners to inspect candidates). */
 int dtas_describe_launch(int op, int64_t n, int64_t d0, int64_t d1, const dtas_config* cfg,
                          dtas_launch_info* out);
+
+/* What dtas_gemm_f16, dtas_gemm_f16_fused and dtas_gemm_f16_static (weights_8bit = 0) or dtas_gemm_q8_f16_fused (1) run
+ * without a config for M >= 2 rows (one row is the GEMV) and operands at 16-byte boundaries: out->config, and for fp16 weights
+ * the launch_args.  out->name "decode_q8 + gemm": the 8-bit weights are widened into a buffer first, and the config is that
+ * of the fp16 GEMM behind it.  The other fields are not used (index, table_row = -1). */
+int dtas_builtin_gemm(int weights_8bit, int64_t M, int64_t N, int64_t K, dtas_launch_info* out);
 
 /* ---- elementwise: tuning_test/tune_ele_add.py:10-22, tune_ele_copy.py:10-21,
  *      tune_cast.py:10-21; dtype variants under experiment/dtas_tuned/elementwise/ ------- */

@@ -52,6 +52,29 @@ def test_select_bucket_uses_labelled_ranges():
     assert _lib.select_bucket(_lib.OP_GEMM_F16, 100000, 4096, 4096).index == 511
 
 
+def test_builtin_gemm_names_what_runs_without_a_config():
+    # ahead of the bucket's row: a kernel chosen by M itself
+    share = _lib.builtin_gemm(16, 4096, 4096)
+    assert (share.config.variant, list(share.config.tile)) == (_lib.GEMM_SHARE, [16, 16, 0]) and list(share.launch_args)[:4] == [256, 1, 1, 256]
+    assert _lib.builtin_gemm(2, 4096, 4096).config.variant == _lib.GEMM_ROWS
+    # ... and the row where none leads
+    for M, N, K in ((129, 4096, 4096), (300, 7680, 2560), (96, 4096, 4096)):
+        assert _lib.builtin_gemm(M, N, K).config.to_dict() == _lib.select_bucket(_lib.OP_GEMM_F16, M, N, K).config.to_dict()
+    assert _lib.builtin_gemm(5, 100, 101).config.vec == 1
+    # 8-bit weights: share, W-streaming, tiles, and the dequantiser in front of the fp16 GEMM
+    q8 = lambda *e: _lib.builtin_gemm(*e, q8=True)
+    assert q8(16, 2560, 2560).config.variant == _lib.GEMM_SHARE and q8(16, 100, 256).config.variant == _lib.GEMM_STREAM
+    assert (q8(203, 7680, 2560).config.variant, q8(203, 7680, 2560).name) == (_lib.GEMM_MFMA, b"gemm_q8")
+    assert q8(2048, 7680, 2560).name == b"decode_q8 + gemm"
+    assert q8(2048, 7680, 2560).config.to_dict() == _lib.builtin_gemm(2048, 7680, 2560).config.to_dict()
+    assert q8(16, 2560, 2528).config.variant == _lib.GEMM_MFMA    # (K % 256 != 0: not the kernels that stream the bytes)
+    for bad in ((1, 64, 64), (2, 0, 64), (2, 64, 0)):
+        with pytest.raises(_lib.DtasError, match="one row is the GEMV"):
+            _lib.builtin_gemm(*bad)
+    with pytest.raises(_lib.DtasError, match="scale group"):
+        q8(16, 64, 40)
+
+
 def test_select_bucket_table_rows_are_monotone_and_merged():
     rows, last = [], None
     for n in range(1, 8193, 16):
