@@ -282,6 +282,7 @@ static bool share_shape(bool q8, int64_t M, int64_t N, int* rows, int* cols) {
 // against 10240 x 2560 21.7 / 26.7, 7680 x 2560 19.0 / 17.8.
 bool share_leads(int64_t M, int64_t N, int64_t K, int* rows, int* cols) {
   if (M < 3 || M > 128 || N < 256 || K < 256 || !share_shape(false, M, N, rows, cols)) return false;
+  if (N > 0x7fffffff || K * 2 * 128 >= (int64_t{1} << 31)) return false;  // (describe_gemm refuses these; other kernels hold them)
   const double m = static_cast<double>(M), w_mb = 2e-6 * static_cast<double>(N) * static_cast<double>(K);
   const double a_kb = 2e-3 * m * static_cast<double>(K), w_cu_kb = w_mb * 1e3 / kNumCU;
   const bool wide = *cols == 128;

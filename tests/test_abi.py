@@ -75,6 +75,14 @@ def test_builtin_gemm_names_what_runs_without_a_config():
         q8(16, 64, 40)
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 2048, 1 << 23), (16, 2560, 1 << 23), (64, 50280, (1 << 23) + 8), (3, 1 << 31, 256)])
+def test_builtin_gemm_names_the_share_kernel_only_where_it_can_run(M, N, K):
+    # one step below the limit of its 32-bit offsets, at it and beyond; describe_launch is what the launch checks
+    assert _lib.describe_launch(_lib.OP_GEMM_F16, M, 4096, (1 << 23) - 8, _lib.DtasConfig.from_dict(
+        {"variant": _lib.GEMM_SHARE, "block": 256, "vec": 8, "unroll": 1, "tile": [16 if M <= 16 else 64, 16, 0]}))
+    assert _lib.builtin_gemm(M, N, K).config.variant != _lib.GEMM_SHARE
+
+
 def test_select_bucket_table_rows_are_monotone_and_merged():
     rows, last = [], None
     for n in range(1, 8193, 16):
