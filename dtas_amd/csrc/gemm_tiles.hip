@@ -264,6 +264,12 @@ int launch_tile_f16(const dtas_config& cfg, hipStream_t s, const half_t* a, cons
 dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok) {
   // two rows of A (the first bucket's table row is sized for 16): W streamed in whole rows, as the GEMV does
   if (M == 2 && vec_ok) return dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {2, N <= 2560 ? 1 : 2, 8}, 1, 0};
+  // three or four rows: the row kernel, a row of W per wavefront, against a W too small or too short for the share kernel
+  // (3 x 64 x 256, 200 x 520, 255 x 4096, 4096 x 128: 3.1, 3.5, 5.7, 4.0 us against 4.1, 4.6, 7.3, 4.6; with long rows the other
+  // way round: 128 x 10240 9.5 / 8.0), and against long rows of W that are few (1024 x 8192 9.2 / 9.8, 2048 x 11008 0.90 of the
+  // share kernel's time; level at 2560 rows: 10240 0.99; behind for shorter ones, 1024 x 1024 3.9 / 3.8, 2560 x 2560 1.03)
+  const bool few_rows = N < 256 ? K < 8192 : K < 256 ? N <= 4096 : N < 2560 && K >= 6144;
+  if ((M == 3 || M == 4) && vec_ok && few_rows) return dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {4, 1, 8}, 1, 0};
   // up to 128 rows of A: the share kernel where it leads
   int rows = 0, cols = 0;
   if (vec_ok && share_leads(M, N, K, &rows, &cols)) return dtas_config{DTAS_GEMM_SHARE, 256, 8, 1, {rows, cols, 0}, 1, 0};

@@ -75,6 +75,16 @@ def test_builtin_gemm_names_what_runs_without_a_config():
         q8(16, 64, 40)
 
 
+@pytest.mark.parametrize("M", [3, 4])
+def test_three_and_four_rows_keep_the_row_kernel_where_the_share_kernel_is_behind(M):
+    variant = lambda N, K: _lib.builtin_gemm(M, N, K).config.variant
+    for N, K in ((64, 256), (255, 8184), (200, 520), (2560, 128), (4096, 248), (300, 6144), (2559, 10240), (1024, 8192)):
+        assert variant(N, K) == _lib.GEMM_ROWS, (N, K)
+    for N, K in ((255, 8192), (4097, 248), (256, 256), (2559, 6136), (2560, 10240), (2560, 2560)):
+        assert variant(N, K) != _lib.GEMM_ROWS, (N, K)
+    assert _lib.builtin_gemm(5, 200, 520).config.variant != _lib.GEMM_ROWS
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 2048, 1 << 23), (16, 2560, 1 << 23), (64, 50280, (1 << 23) + 8), (3, 1 << 31, 256)])
 def test_builtin_gemm_names_the_share_kernel_only_where_it_can_run(M, N, K):
     # one step below the limit of its 32-bit offsets, at it and beyond; describe_launch is what the launch checks

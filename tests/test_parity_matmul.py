@@ -322,8 +322,12 @@ def test_gemm_row_kernel_every_variant(oracle, mv, r, block, N, K):
 
 @pytest.mark.parametrize("M", [3, 4])
 def test_gemm_three_and_four_rows_against_few_rows_of_w_take_the_row_kernel(oracle, M):
-    # built-in: the row kernel up to 2560 rows of W (or 4096 x 4096), the tiles beyond; every epilogue
-    for kind, N, K in ((0, 2560, 2560), (1, 2560, 10240), (2, 4096, 4096), (3, 1000, 520), (0, 7680, 2560)):
+    # built-in: the row kernel against a W of fewer than 256 rows or columns and against few long rows, other kernels beyond;
+    # every epilogue
+    for kind, N, K in ((0, 200, 520), (1, 255, 4096), (2, 64, 256), (3, 4096, 128), (3, 2048, 6144), (1, 300, 10240)):
+        assert _lib.builtin_gemm(M, N, K).config.variant == _lib.GEMM_ROWS
+    for kind, N, K in ((0, 200, 520), (1, 255, 4096), (2, 64, 256), (3, 4096, 128), (3, 2048, 6144), (1, 300, 10240),
+                       (0, 2560, 2560), (1, 2560, 10240), (2, 4096, 4096), (3, 1000, 520), (0, 7680, 2560)):
         a, w, bias, r1, r2 = _fused_inputs(M, N, K, 50 + kind + M)
         res = (dev(r1), dev(r2)) if kind in (1, 2) else (None, None)
         out = Guarded((1, M, N), torch.float32 if kind == 2 else torch.float16)
