@@ -273,25 +273,40 @@ static bool share_shape(bool q8, int64_t M, int64_t N, int* rows, int* cols) {
   return share_kernel_exists(*rows, *cols, q8);
 }
 
-// fp16 weights.  Two estimates in us, fitted to sweeps of 3 .. 128 rows against 25 shapes of W from 1024 x 1024 to 50280 x
-// 2560 (W from memory).  Share: 3.3 + the root of the squares of what W costs from memory (6.6 TB/s; 5.4 with 128 columns)
-// and what A and the CU's part of W cost through its L1 (65 KB/us, 55 where the segments are short: 128 columns, or more
-// than 64 rows).  The other kernels: 6.5 us + W at 5.5 TB/s + 0.03 per row (wide W: x the rounds of 64-column tiles over
-// their exact number), and 8.5 us + W at 4.2 TB/s beyond 64 rows.  What the line separates, share / others: 64 rows against
-// 4096 x 4096 13.7 / 13.5, 48 rows 12.1 / 13.2; 32 rows against 4096 x 11008 25.3 / 24.0, 17 rows 22.3 / 23.5; 128 rows
-// against 10240 x 2560 21.7 / 26.7, 7680 x 2560 19.0 / 17.8.
+// fp16 weights.  Two estimates in us, fitted to sweeps of 3 .. 128 rows against W of 300 .. 50280 rows and 256 .. 14336
+// columns (W from memory).  Share: 3.3 + the root of the squares of what W costs from memory (6.6 TB/s; 5.4 with 128
+// columns) and what A and the CU's part of W cost through its L1 (65 KB/us, 55 where the segments are short: 128 columns, or
+// more than 64 rows).  The other kernels: 6.5 us + W at 5.5 TB/s + 0.03 per row (wide W: x the rounds of 64-column tiles over
+// their exact number), and beyond 64 rows 8.5 us + W at 4.2 TB/s, 8.1 + 4.5 TB/s where their tiles split K evenly (up to 4096
+// columns, and long K).  What the line separates, share / others: 64 rows against 4096 x 4096 13.7 / 13.5, 48 rows 12.1 / 13.2; 32
+// rows against 4096 x 11008 25.3 / 24.0, 17 rows 22.3 / 23.5; 128 rows against 10240 x 2560 21.7 / 26.7, 7680 x 2560 19.0 / 17.8.
+// What the estimates do not see, share / others:
+//  * few long rows of W: a workgroup's segments follow one another at 0.8 .. 1.2 us per 1024 of K, while the W-streaming kernel
+//    deals K out in slices -- 8 rows against 300 x 14336 14.1 / 8.4, 1024 x 8192 9.5 / 8.6, 17 rows against 512 x 8192 12.3 / 9.3.
+//    Its workgroups must fit one round; with 256 of them the share kernel is level (2048 x 8192) and beyond it ahead (0.7);
+//  * rows of W 20 or 28 KiB apart (K = 10240, 14336): 33 rows against 5120 x 10240 30.4 / 26.6, 65 against 8192 x 10240 55.3 / 44.6, 5
+//    against 8192 x 14336 50.5 / 45.9; not at 12288 (0.82), and not beyond 8192 rows of W (11008: 0.80);
+//  * wide W whose rows are short (17 rows against 50280 x 256 12.8 / 11.7), or a power of two long and no fewer than 7/8 of a
+//    round of 128-column tiles, which then run as if in whole rounds (48 rows against 28672 x 4096 1.05, x 2560 0.87);
+//  * more than 64 rows against short rows of a W beyond 8192 (128 rows against 11008 x 256 8.2 / 6.7,
+//    x 1024 13.2 / 12.4, 10240 x 1536 16.3 / 19.4; 80 rows against 11008 x 512 1.03, 10240 x 1024 0.93).
 bool share_leads(int64_t M, int64_t N, int64_t K, int* rows, int* cols) {
   if (M < 3 || M > 128 || N < 256 || K < 256 || !share_shape(false, M, N, rows, cols)) return false;
   if (N > 0x7fffffff || K * 2 * 128 >= (int64_t{1} << 31)) return false;  // (describe_gemm refuses these; other kernels hold them)
+  const bool wide = *cols == 128;
+  if (wide && ((K < 2048 && M > 32) || (K <= 512 && M > 16 && N > 32768))) return false;  // (28672 x 1024: 48 rows 15.6 / 15.5 us, 64 rows 16.7 / 15.9)
+  if (*cols == 48 && M > 64 && K < (M > 96 ? 1536 : 1024)) return false;
+  if (M <= 32 && ceil_div(N, 64) * ceil_div(K, M <= 16 ? 1024 : 512) <= 240 && (K >= 8192 || (K >= 6144 && N < 1024))) return false;
   const double m = static_cast<double>(M), w_mb = 2e-6 * static_cast<double>(N) * static_cast<double>(K);
   const double a_kb = 2e-3 * m * static_cast<double>(K), w_cu_kb = w_mb * 1e3 / kNumCU;
-  const bool wide = *cols == 128;
-  if (wide && K < 2048 && M > 32) return false;  // (28672 x 1024: 48 rows 15.6 / 15.5 us, 64 rows 16.7 / 15.9)
   const double hbm = w_mb / (wide ? 5.4 : 6.6), l1 = (a_kb + w_cu_kb) / (wide || M > 64 ? 55.0 : 65.0);
-  const double share = 3.3 + sqrt(hbm * hbm + l1 * l1);
-  const double tiles = static_cast<double>(ceil_div(N, 64)) / kNumCU;
-  const double waste = wide ? static_cast<double>(ceil_div(ceil_div(N, 64), kNumCU)) / tiles : 1.0;
-  const double others = M <= 64 ? 6.5 + w_mb / 5.5 * waste + 0.03 * m : 8.5 + w_mb / 4.2 + 0.02 * (m - 64.0);
+  const double pitch = K > 8192 && K % 4096 == 2048 && N > (M < 32 ? 6144 : 4096) && N <= 8192 ? 1.2 : 1.0;
+  const double share = 3.3 + pitch * sqrt(hbm * hbm + l1 * l1);
+  const int64_t t64 = ceil_div(N, 64), t128 = ceil_div(N, 128);
+  const bool whole = (K & (K - 1)) == 0 && t128 <= kNumCU && t128 * 8 >= 7 * kNumCU;
+  const double waste = wide && !whole ? static_cast<double>(ceil_div(t64, kNumCU) * kNumCU) / static_cast<double>(t64) : 1.0;
+  const bool even = N <= 4096 || (N <= 10240 && K > 5120);
+  const double others = M <= 64 ? 6.5 + w_mb / 5.5 * waste + 0.03 * m : (even ? 8.1 + w_mb / 4.5 : 8.5 + w_mb / 4.2) + 0.02 * (m - 64.0);
   return share < others;
 }
 

@@ -85,6 +85,20 @@ def test_three_and_four_rows_keep_the_row_kernel_where_the_share_kernel_is_behin
     assert _lib.builtin_gemm(5, 200, 520).config.variant != _lib.GEMM_ROWS
 
 
+# rows against N x K: (share kernel, another) on each side of every line of the built-in choice, measured on both
+FP16_LINES = [((16, 2048, 8192), (16, 1024, 8192)), ((8, 1024, 6144), (8, 768, 7168)), ((17, 1024, 8192), (17, 512, 8192)),
+              ((5, 8192, 11008), (40, 8192, 10240)), ((8, 6144, 10240), (65, 8192, 10240)), ((33, 11008, 10240), (33, 5120, 10240)),
+              ((5, 7680, 12288), (40, 7680, 14336)), ((16, 50280, 512), (17, 50280, 512)), ((48, 28672, 2560), (48, 28672, 4096)),
+              ((80, 10240, 1024), (80, 10240, 512)), ((128, 10240, 1536), (128, 11008, 1024)), ((65, 7680, 2560), (80, 2560, 2560)),
+              ((17, 2560, 10240), (33, 2560, 10240))]
+
+
+@pytest.mark.parametrize("leads,behind", FP16_LINES)
+def test_where_the_share_kernel_is_chosen_for_fp16_weights(leads, behind):
+    assert _lib.builtin_gemm(*leads).config.variant == _lib.GEMM_SHARE
+    assert _lib.builtin_gemm(*behind).config.to_dict() == _lib.select_bucket(_lib.OP_GEMM_F16, *behind).config.to_dict()
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 2048, 1 << 23), (16, 2560, 1 << 23), (64, 50280, (1 << 23) + 8), (3, 1 << 31, 256)])
 def test_builtin_gemm_names_the_share_kernel_only_where_it_can_run(M, N, K):
     # one step below the limit of its 32-bit offsets, at it and beyond; describe_launch is what the launch checks
