@@ -313,9 +313,25 @@ bool share_leads(int64_t M, int64_t N, int64_t K, int* rows, int* cols) {
 // 8-bit weights: the other kernels widen every weight once per row of tiles, so the share kernel leads until the rows of A
 // that each CU pulls in (2 M K bytes) outgrow both 660 KB and 6.5 times its part of W: 2560 x 10240, 32 rows 18.8 us
 // against 19.4, 48 rows 24.5 / 21.2; 4096 x 11008, 48 rows 27.0 / 28.6, 64 rows 33.2 / 29.3; 7680 x 2560, 96 rows 18.2 / 19.7,
-// 128 rows (no kernel) 21.2 / 20.8.
+// 128 rows (no kernel) 21.2 / 20.8.  And not, from a sweep of 2 .. 96 rows against W of 300 .. 50280 rows and 256 .. 14336 columns
+// (W from memory, share / others):
+//  * against few long rows of W, which the W-streaming kernel and the tiles take in slices of K while a workgroup here walks
+//    them whole: 16 rows against 300 x 14336 18.7 / 8.3, 1024 x 8192 11.8 / 8.7, 1024 x 4096 7.5 / 7.3, 2048 x 2560 0.84, 2560 x 10240
+//    0.99; 48 rows against 1024 x 6144 15.7 / 13.5, 2560 x 9216 21.5 / 19.7, 3072 x 10240 0.88; 64 rows against 1536 x 4096 1.07,
+//    2048 x 5120 0.95, 6144 x 10240 1.05, 7680 x 10240 0.93.  The fewest rows of W, by the rows of A and K:
+//  * more than 64 rows: 80 against 8192 x 8192 1.06, 5120 x 4096 1.05, 2048 x 4096 1.05, but 10240 x 5120 0.95, 4096 x 4096
+//    0.92, any W of up to 3328 columns 0.64 .. 1.03, and beyond 10240 rows of W 0.67 .. 0.91;
+//  * against a wide W of up to 512 columns (128 columns per workgroup): 8 rows against 50280 x 512 12.8 / 9.9, 17 rows against 28672
+//    x 512 1.09, 20480 x 256 0.85, 64 rows against 32000 x 512 11.7 / 9.8; more than 32 rows of A against more than 32768 rows of W
+//    are the exception: what is left there writes the weights out in fp16 first (50280 x 512 17.3 / 32.4).
 bool share_leads_q8(int64_t M, int64_t N, int64_t K, int* rows, int* cols) {
   if (M > 96 || N < 256 || !share_shape(true, M, N, rows, cols)) return false;
+  if (K <= 512 && N > (M <= 16 ? 64 : 80) * kNumCU && (M <= 32 || N <= 32768)) return false;
+  if (M > 64) return K < 3584 || N > 10240 || (K < 6144 && N > 5120) || (K < 5120 && N > 2048 && N <= 4096);
+  const int64_t least = M <= 32   ? (K >= 8192 ? 2560 : K >= 6144 ? 1536 : K >= 3328 ? 1024 : 0)
+                        : M <= 48 ? (K >= 9216 ? 3072 : K >= 6144 ? 1536 : K >= 4096 ? 1024 : 0)
+                                  : (K >= 9216 ? 6145 : K >= 3584 ? 2048 : 0);
+  if (N < least) return false;
   const double a_kb = 2e-3 * static_cast<double>(M) * static_cast<double>(K);
   const double w_cu_kb = 1.0625e-3 * static_cast<double>(N) * static_cast<double>(K) / kNumCU;
   return a_kb <= 660.0 || a_kb <= 6.5 * w_cu_kb;

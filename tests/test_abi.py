@@ -99,6 +99,20 @@ def test_where_the_share_kernel_is_chosen_for_fp16_weights(leads, behind):
     assert _lib.builtin_gemm(*behind).config.to_dict() == _lib.select_bucket(_lib.OP_GEMM_F16, *behind).config.to_dict()
 
 
+Q8_LINES = [((16, 1024, 4096), (16, 768, 4096)), ((32, 1536, 6144), (2, 1535, 7168)), ((16, 2560, 10240), (16, 2048, 8192)),
+            ((16, 300, 3072), (16, 300, 3328)), ((48, 1024, 4096), (48, 768, 4096)), ((33, 1536, 8192), (48, 1280, 6144)),
+            ((33, 3072, 9216), (33, 2560, 10240)), ((64, 2048, 5120), (64, 1536, 4096)), ((64, 7680, 10240), (64, 6144, 10240)),
+            ((80, 2560, 3328), (80, 1536, 3584)), ((80, 4096, 4096), (65, 5120, 4096)), ((96, 10240, 5120), (80, 8192, 8192)),
+            ((96, 11008, 8192), (96, 10240, 8192)), ((8, 50280, 768), (8, 50280, 512)), ((64, 50280, 512), (64, 32000, 512)),
+            ((17, 20480, 256), (17, 28672, 512))]
+
+
+@pytest.mark.parametrize("leads,behind", Q8_LINES)
+def test_where_the_share_kernel_is_chosen_for_8_bit_weights(leads, behind):
+    assert _lib.builtin_gemm(*leads, q8=True).config.variant == _lib.GEMM_SHARE
+    assert _lib.builtin_gemm(*behind, q8=True).config.variant != _lib.GEMM_SHARE
+
+
 @pytest.mark.parametrize("M,N,K", [(3, 2048, 1 << 23), (16, 2560, 1 << 23), (64, 50280, (1 << 23) + 8), (3, 1 << 31, 256)])
 def test_builtin_gemm_names_the_share_kernel_only_where_it_can_run(M, N, K):
     # one step below the limit of its 32-bit offsets, at it and beyond; describe_launch is what the launch checks
