@@ -85,11 +85,17 @@ template <class F, class... A>
 PyObject* launch(const char* name, F fn, A... args) {
   void* stream = c10::hip::getCurrentHIPStream().stream();
   int rc;
+  bool thrown = false;
   Py_BEGIN_ALLOW_THREADS
-  rc = fn(args..., stream);
+  try {  // (nothing may leave this block but through its end, which takes the GIL again)
+    rc = fn(args..., stream);
+  } catch (...) {
+    rc = -1;
+    thrown = true;
+  }
   Py_END_ALLOW_THREADS
   if (rc == 0) Py_RETURN_TRUE;
-  PyErr_Format(g_error, "%s: %s", name, p_dtas_last_error());
+  PyErr_Format(g_error, "%s: %s", name, thrown ? "a C++ exception left the library" : p_dtas_last_error());
   return nullptr;
 }
 #define DTAS_CALL(name, ...) launch(#name, p_##name, __VA_ARGS__)

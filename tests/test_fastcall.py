@@ -1,5 +1,6 @@
 """The natively checked call (csrc/fastcall.cpp) and the Python body behind it are one function: what the first accepts
 gives the same bits as the second, and what the second refuses the first leaves to it."""
+import ctypes
 import os
 import subprocess
 import sys
@@ -111,3 +112,23 @@ def test_refusals_stay_the_bodys():
     with pytest.raises(_lib.DtasError, match="gemv"):
         ops.gemv(h(64), h(32, 64), h(32), h(32), epilogue=9)
     ops.copy(h(0, 8), h(0, 8))  # empty: no launch, no error
+
+
+@pytest.mark.gpu
+def test_an_exception_of_the_library_comes_back_with_the_gil(tmp_path):
+    ops.lib()
+    (tmp_path / "throws.cpp").write_text('extern "C" int throws(const void*, void*, long, long, const void*, void*) { throw 1; }')
+    subprocess.run(["g++", "-shared", "-fPIC", "-o", str(tmp_path / "throws.so"), str(tmp_path / "throws.cpp")], check=True)
+    throws = ctypes.CDLL(str(tmp_path / "throws.so")).throws
+    a = torch.ones(4, 8, device="cuda", dtype=torch.float16)
+    addresses = _lib.entry_addresses()
+    try:
+        _fastcall.bind({**addresses, "dtas_copy_f16": ctypes.cast(throws, ctypes.c_void_p).value}, _lib.DtasError)
+        for _ in range(3):
+            with pytest.raises(_lib.DtasError, match="dtas_copy_f16: a C\\+\\+ exception"):
+                ops.copy(a, a.clone())
+    finally:
+        _fastcall.bind(addresses, _lib.DtasError)
+    b = torch.zeros_like(a)
+    ops.copy(a, b)
+    assert torch.equal(a, b)
