@@ -7,11 +7,13 @@ kernel goes on torch's current stream.  ``cfg`` (a ``_lib.DtasConfig``) override
 table.  torch is used for device memory and streams only.
 
 The ordinary call (plain contiguous device tensors that fit together, no ``cfg``) is checked and launched by
-``_fastcall`` (csrc/fastcall.cpp); the Python bodies below serve every other call and word every refusal.
+``_fastcall`` (csrc/fastcall.cpp); the Python bodies below serve every other call, word every refusal, and serve every
+call where ``_fastcall`` is missing or was built for another torch.
 """
 from __future__ import annotations
 
 import ctypes
+import warnings
 from typing import Optional
 
 import torch
@@ -19,10 +21,34 @@ import torch
 from . import _lib
 from ._lib import DtasConfig, DtasError, check
 
-try:
-    from . import _fastcall
-except ImportError as e:
-    raise ImportError("dtas_amd/_fastcall.so is missing or was built for another torch: build it with `make -C dtas_amd/csrc`") from e
+
+class _NoFastcall:
+    """Stands in for ``_fastcall`` where it cannot be used: every call is left to its Python body."""
+
+    _built_for = None
+
+    def __getattr__(self, name):
+        return lambda *args: None if name == "bind" else False
+
+
+def _load_fastcall():
+    """``_fastcall`` if it was built for this torch (it reads tensors in place), else the bodies below on their own: the same
+    kernels, about 2 us more host time per call."""
+    try:
+        from . import _fastcall as built
+    except ImportError as e:
+        why = str(e)
+    else:
+        here = f"{torch.__version__} {torch.version.git_version}"
+        if getattr(built, "_built_for", None) == here:
+            return built
+        why = f"built for torch {getattr(built, '_built_for', 'unknown')}, this is {here}"
+    warnings.warn(f"dtas_amd checks its calls in Python, without dtas_amd/_fastcall ({why}); `make -C dtas_amd/csrc` builds it",
+                  RuntimeWarning, stacklevel=3)
+    return _NoFastcall()
+
+
+_fastcall = _load_fastcall()
 
 _ELT = {
     ("add", torch.float16): ("dtas_add_f16", _lib.OP_ADD_F16),

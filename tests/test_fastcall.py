@@ -26,6 +26,32 @@ def test_nothing_is_accepted_before_the_library_is_bound():
     assert subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True).stdout.strip() == "ok"
 
 
+@pytest.mark.parametrize("there", ["None", "types.ModuleType('dtas_amd._fastcall')",
+                                   "types.SimpleNamespace(_built_for='1.0 other', add=lambda *a: 1 / 0, bind=lambda *a: 1 / 0)"])
+def test_missing_or_built_for_another_torch_the_bodies_serve_every_call(there):
+    code = f"""
+import sys, types, warnings
+import torch
+sys.modules["dtas_amd._fastcall"] = {there}
+with warnings.catch_warnings(record=True) as w:
+    warnings.simplefilter("always")
+    from dtas_amd import ops
+assert [x.category for x in w if "_fastcall" in str(x.message)] == [RuntimeWarning], w
+ops.lib()
+a = torch.zeros(2, 8, dtype=torch.float16)
+try:
+    ops.add(a, a, a)
+except ValueError as e:
+    print(e)
+"""
+    done = subprocess.run([sys.executable, "-c", code], cwd=ROOT, capture_output=True, text=True)
+    assert "no CPU path" in done.stdout, done.stderr
+
+
+def test_built_for_this_torch():
+    assert ops._fastcall is _fastcall and _fastcall._built_for == f"{torch.__version__} {torch.version.git_version}"
+
+
 def _calls():
     """(name, positional arguments, index of each output) over forms that the bodies accept."""
     g = torch.Generator(device="cuda").manual_seed(3)
