@@ -379,8 +379,8 @@ __global__ void __launch_bounds__(256) attn_scores_pipe_kernel(const half_t* __r
 // What bounds it: beside the stores, K passes through a CU's L1 once per 32 query rows.  32 heads of 80 against the tiles: 203 x 1031
 // 15.6 -> 13.3 us, 130 x 2049 18.0 -> 15.4.  Not kept: K through the LDS in 1 KiB loads (two workgroups per CU), that with 64 rows;
 // registers for three workgroups per CU; the mask under a row's ends loaded where it is used (a memory latency per end).
-constexpr int kSectorRows = 32, kSectorKeys = 512, kSectorChunk = 480, kSectorPitch = kSectorKeys + 4;  // KS: k steps of 16 that hold the head dimension
-template <int KS>
+constexpr int kSectorRows = 32, kSectorKeys = 512, kSectorChunk = 480, kSectorPitch = kSectorKeys + 4;
+constexpr int kSectorSteps = 5;  // k steps of 16: head dimensions of 65 .. 80
 __global__ void __launch_bounds__(256, 4) attn_scores_sector_kernel(const half_t* __restrict__ Q, const half_t* __restrict__ Kmat,
                                                                  const half_t* __restrict__ mask, float* __restrict__ out,
                                                                  int64_t n, int64_t m, int64_t d, float scale, unsigned chunk,
@@ -412,13 +412,13 @@ __global__ void __launch_bounds__(256, 4) attn_scores_sector_kernel(const half_t
   const __amdgpu_buffer_rsrc_t rw = make_rsrc(Kmat + (static_cast<int64_t>(batch) * m + c0) * d, static_cast<unsigned>(left) * row_bytes);
 
   // fragments: lane l supplies row l & 31, 16-byte piece 2 ks + (l >> 5) (rows past the extents and pieces past d: zeros)
-  auto fragments = [&](const __amdgpu_buffer_rsrc_t& r, unsigned block, u32x4 (&f)[KS]) {
+  auto fragments = [&](const __amdgpu_buffer_rsrc_t& r, unsigned block, u32x4 (&f)[kSectorSteps]) {
     const unsigned at = (block * 32u + (l & 31u)) * row_bytes + (l >> 5) * 16u;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int ks = 0; ks < kSectorSteps; ++ks)
       f[ks] = __builtin_amdgcn_raw_buffer_load_b128(r, (2 * ks + (l >> 5)) * 8u < static_cast<unsigned>(d) ? at + ks * 32u : kOob, 0, 0);
   };
-  u32x4 fq[KS], fk[KS];
+  u32x4 fq[kSectorSteps], fk[kSectorSteps];
   fragments(ra, 0, fq);
   fragments(rw, wv, fk);
 
@@ -455,20 +455,20 @@ __global__ void __launch_bounds__(256, 4) attn_scores_sector_kernel(const half_t
   const int keys = last || static_cast<int>(chunk) + 15 > left ? left : static_cast<int>(chunk) + 15;
   const unsigned blocks = static_cast<unsigned>((keys + 31) / 32);  // at most 16
   for (unsigned b = wv; b < blocks; b += 4) {
-    u32x4 next[KS];
+    u32x4 next[kSectorSteps];
     fragments(rw, b + 4, next);  // (past the last block: out of range, zeros)
     f32x16 acc;
 #pragma unroll
     for (int v = 0; v < 16; ++v) acc[v] = 0.f;
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks)
+    for (int ks = 0; ks < kSectorSteps; ++ks)
       acc = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, fq[ks]), __builtin_bit_cast(f16x8, fk[ks]), acc, 0, 0, 0);
     // acc[v] of lane l: row 8 (v / 4) + 4 (l >> 5) + v % 4, key l & 31 of the block
     half_t* dst = rows + (4u * (l >> 5)) * kSectorPitch + b * 32u + (l & 31u);
 #pragma unroll
     for (int v = 0; v < 16; ++v) dst[(8 * (v / 4) + v % 4) * kSectorPitch + (lead(v % 4) & 3)] = static_cast<half_t>(acc[v]);  // (lead modulo 4: rows 4 apart alike)
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) fk[ks] = next[ks];
+    for (int ks = 0; ks < kSectorSteps; ++ks) fk[ks] = next[ks];
   }
   __syncthreads();
 
@@ -809,26 +809,27 @@ extern "C" int dtas_attn_scores_f16_f32(const void* Q, const void* Kmat, const v
                            static_cast<float*>(out), n, m, d, sc, tm, tn, static_cast<unsigned>(heads), pin);
       return check_launch("attn_scores");
     }
-    // ... or every row is cut at sectors of its own (attn_scores_sector_kernel), for continuations of up to 256 rows.  32 heads
-    // of 80, tiles / own sectors, us: n x m = 203 x 703 12.1 / 11.7, 203 x 1031 15.6 / 13.3, 130 x 2049 18.0 / 15.4; a layer of 250
-    // rows behind 1501 keys 222.5 / 219.7.  Prompts: launches of scores alone gain more (2047 x 2047 208 / 128), but the softmax
-    // behind them then reads more from memory, and the layer gains nothing (1601: 636 / 642; 2047: 809 / 807).  Head
-    // dimensions of 64 and 128 pull more of K through the L1 than the tiles do (40 heads of 128, 1025 x 1025 57.6 / 98.9), and
-    // fewer workgroups than 1.75 per CU do not hide a workgroup's chain (65 x 481, 192 of them: 6.8 / 9.5)
+    // ... or every row is cut at sectors of its own (attn_scores_sector_kernel), for continuations of up to 256 rows.  Tiles / own
+    // sectors, us, head dimension 80; in brackets with the softmax that reads them behind:
+    //  * keys: 32 heads, 203 x 601 11.2 / 12.0 (20.9 / 20.0), 256 x 601 11.8 / 11.9 (22.7 / 22.2); 203 x 703 12.6 / 12.3 (23.2 / 20.3), 256 x
+    //    703 13.2 / 12.0 (24.8 / 24.0), 203 x 1031 15.7 / 13.8 (26.5 / 25.4), 130 x 2049 17.5 / 15.7 (29.3 / 27.4), 256 x 4095 49.5 / 37.3;
+    //  * workgroups per CU, whose chains have to hide one another: 1.5, 32 heads, 65 x 1531 11.1 / 12.0, 100 x 1301 11.4 / 11.9, 24 heads,
+    //    225 x 777 11.6 / 12.4; 1.75 and more, 32 heads, 203 x 777 14.0 / 12.5, 130 x 1031 13.8 / 11.8, 65 x 2049 13.1 / 11.9;
+    //  * rows: 64 heads, 225 x 1031 23.6 / 25.5 (41.5 / 42.8), 225 x 1301 26.5 / 28.9 (48.3 / 49.9), and level beyond 8192 rows in all with
+    //    32 heads (400 x 1031 21.9 / 22.4, 512 x 1301 30.6 / 29.2).  Prompts: launches of scores alone gain more (2047 x 2047 208 /
+    //    128), the layer around them nothing (1601: 636 / 642; 2047: 809 / 807).
+    // Head dimensions of 64 and 128 pull more of K through the L1 than the tiles do (40 heads of 128, 1025 x 1025 57.6 / 98.9)
     const int64_t pieces = ceil_div(m, kSectorChunk), chunk = ceil_div(ceil_div(m, pieces), 16) * 16;
     const int64_t tm_s = ceil_div(n, kSectorRows), tn_s = ceil_div(m, chunk), tiles_s = tm_s * tn_s;
-    if (!whole_sectors && d > 64 && d <= 80 && n <= 256 && m >= 700 && tiles_s * heads * 4 >= 7 * kNumCU) {
+    if (!whole_sectors && d > 64 && d <= 16 * kSectorSteps && n <= 256 && n * heads <= 8192 && m >= 700 && tiles_s * heads * 4 >= 7 * kNumCU) {
       const bool pin = n * m >= (int64_t{1} << 21);
       const int64_t wgs = pin ? kNumXCD * heads * ceil_div(tiles_s, kNumXCD) : tiles_s * heads;
       if (wgs > 0x7fffffff) return fail("attn_scores: too many tiles");
-      auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, dim3(static_cast<unsigned>(wgs)), dim3(256), 0, static_cast<hipStream_t>(stream), static_cast<const half_t*>(Q),
-                           static_cast<const half_t*>(Kmat), static_cast<const half_t*>(mask), static_cast<float*>(out), n, m, d,
-                           static_cast<float>(static_cast<half_t>(scale)), static_cast<unsigned>(chunk), static_cast<unsigned>(tm_s),
-                           static_cast<unsigned>(tn_s), static_cast<unsigned>(heads), pin ? 1u : 0u);
-        return check_launch("attn_scores");
-      };
-      return launch(attn_scores_sector_kernel<5>);
+      hipLaunchKernelGGL(attn_scores_sector_kernel, dim3(static_cast<unsigned>(wgs)), dim3(256), 0, static_cast<hipStream_t>(stream),
+                         static_cast<const half_t*>(Q), static_cast<const half_t*>(Kmat), static_cast<const half_t*>(mask), static_cast<float*>(out), n,
+                         m, d, static_cast<float>(static_cast<half_t>(scale)), static_cast<unsigned>(chunk), static_cast<unsigned>(tm_s),
+                         static_cast<unsigned>(tn_s), static_cast<unsigned>(heads), pin ? 1u : 0u);
+      return check_launch("attn_scores");
     }
     const int64_t grid = !whole_sectors || total < 3 * kNumCU ? total : 3 * kNumCU;
     hipLaunchKernelGGL((attn_scores_kernel<128, 64>), dim3(static_cast<unsigned>(grid)), dim3(256), 0, static_cast<hipStream_t>(stream),
