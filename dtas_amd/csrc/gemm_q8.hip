@@ -20,15 +20,15 @@ bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, dtas_confi
   }
   // the W-streaming kernel, which widens the bytes on their way from the LDS into the MFMA
   if (stream_ok && M <= 32) {
-    // measured at the model's shapes (M = 16: 10.1 against 25.6 us at 7680x2560, 14.9 against 92 at 2560x10240;
-    // M = 32: 14.0 against 26.3 and 20.5 against 33.8).  512-element slices (three workgroups per CU) unless K is
-    // long: from 16 slices on the hand-over of the partial sums costs more than the second workgroup hides
+    // what the share kernel leaves to it, against the best of the tiles, W from memory: 8 rows against 300 x 14336 8.5 us / 20.3, 16
+    // against 1024 x 8192 8.9 / 15.9, 32 against 1024 x 8192 12.3 / 16.1, 768 x 4096 8.6 / 12.1.  512-element slices (three workgroups
+    // per CU) unless K is long: from 16 slices on the hand-over of the partial sums costs more than the second
+    // workgroup hides (1024-element slices / 512: 16 rows against 512 x 4096 7.5 / 6.8, 2048 x 8192 10.6 / 12.6)
     cfg = dtas_config{DTAS_GEMM_STREAM, 256, 8, 1, {M > 16 ? 32 : 16, 64, M <= 16 && K >= 8192 ? 1024 : 512}, 1, 0};
     return true;
   }
-  // up to 64 rows only while its workgroups (64 columns x 512 of K each) run in one round: 48 rows against 2560 x 2560 /
-  // 2048 x 4096 / 4096 x 2048 11.3 / 12.1 / 10.6 us where the tiles take 11.8 / 12.8 / 11.5, but 16.4 / 16.5 / 21.2 against
-  // 13.0 / 12.5 / 15.5 at 3072 x 3072 / 4096 x 2560 / 4096 x 4096
+  // up to 64 rows only while its workgroups (64 columns x 512 of K each) run in one round: 48 rows against 512 x 4096 / 1024 x
+  // 6144 / 1024 x 8192 10.7 / 13.9 / 15.9 us where the best of the tiles takes 11.7 / 14.5 / 16.2, but 19.5 against 16.3 at 1088 x 8192
   if (stream_ok && M <= 64 && ceil_div(N, 64) * ceil_div(K, 512) <= kNumCU) {
     cfg = dtas_config{DTAS_GEMM_STREAM, 256, 8, 1, {64, 64, 512}, 1, 0};
     return true;

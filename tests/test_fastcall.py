@@ -115,8 +115,10 @@ def test_same_results_as_the_body(monkeypatch):
         for i in outs:
             args[i].zero_()
         slow = [a.as_subclass(_Subclass) if isinstance(a, torch.Tensor) else a for a in args]
-        getattr(ops, name)(*slow)
-        assert took == [True], name
+        with monkeypatch.context() as m:
+            m.setattr(ops._fastcall, name, lambda *a: took.append(fast(*a)) or took[-1])
+            getattr(ops, name)(*slow)
+        assert took == [True, False], name   # (the second time the body computed it)
         for i, g in zip(outs, got):
             assert g.count_nonzero() > 0 and torch.equal(args[i].contiguous().view(torch.uint8) if args[i].dim() else args[i], g.view(torch.uint8) if g.dim() else g), name
         seen.add(name)

@@ -219,7 +219,8 @@ def test_gemm_looping_streaming_tiles(oracle, cols, N, K):
 
 
 def test_gemm_looping_streaming_tile_is_the_choice_for_many_rows_of_w_exact_and_refuses_what_it_cannot_hold(oracle):
-    # what cfg = NULL runs for M <= 16 against 4096 < N <= 16384 rows of W with K <= 4096
+    # the table's row (a tuned module's: without a config the share kernel leads here) for M <= 16 against 4096 < N <= 16384
+    # rows of W with K <= 4096
     for N, K, tile, block in ((7680, 2560, [16, 16, 256], 64), (8192, 4096, [16, 16, 256], 64), (11008, 4096, [16, 64, 256], 256),
                               (10240, 2560, [16, 64, 256], 256)):
         got = _lib.select_bucket(_lib.OP_GEMM_F16, 16, N, K).config
@@ -260,11 +261,12 @@ def test_gemm_fused_epilogues_looping_streaming_tile(oracle, kind, cols, M, N, K
 def test_gemm_streaming_tile_is_reproducible_exact_and_refuses_what_it_cannot_hold(oracle):
     M, N, K = 16, 4096, 4096
     a, w = _inputs(M, N, K, 5)
-    assert _lib.select_bucket(_lib.OP_GEMM_F16, M, N, K).config.variant == _lib.GEMM_STREAM   # what cfg = NULL runs here
+    row = _lib.select_bucket(_lib.OP_GEMM_F16, M, N, K).config   # (a tuned module's; without a config the share kernel leads here)
+    assert row.variant == _lib.GEMM_STREAM and K // row.tile[2] == 4
     runs = []
     for _ in range(3):
         out = Guarded((M, N), torch.float16)
-        ops.gemm(dev(a), dev(w), None, out.t)
+        ops.gemm(dev(a), dev(w), None, out.t, row)
         runs.append(out.check())
     assert all(np.array_equal(r.view(np.uint16), runs[0].view(np.uint16)) for r in runs)   # slices are added in slice order
     _check(runs[0], oracle.c.gemm(a, w, threads=8), oracle.np64.gemm(a, w))

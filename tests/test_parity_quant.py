@@ -267,10 +267,12 @@ def test_gemm_q8_at_the_models_shapes(oracle, M, N, K, kind):
 
 
 @pytest.mark.parametrize("M", [33, 48, 64])
-@pytest.mark.parametrize("N,K", [(2048, 4096), (4096, 2048), (3072, 3072), (4096, 2560), (4096, 4096)])
-def test_gemm_q8_33_to_64_rows_either_side_of_one_round_of_the_streaming_form(oracle, M, N, K):
-    # 64 columns x 512 of K per workgroup: the first two shapes are one round of the chip (the W-streaming kernel),
-    # the others more (the tiles with K in parts)
+@pytest.mark.parametrize("N,K,variant", [(768, 4096, _lib.GEMM_STREAM), (1024, 8192, _lib.GEMM_STREAM), (1088, 8192, _lib.GEMM_MFMA),
+                                         (2560, 10240, _lib.GEMM_MFMA), (2048, 4096, _lib.GEMM_SHARE), (4096, 2560, _lib.GEMM_SHARE)])
+def test_gemm_q8_33_to_64_rows_either_side_of_one_round_of_the_streaming_form(oracle, M, N, K, variant):
+    # 64 columns x 512 of K per workgroup: the first two shapes are at most one round of the chip (the W-streaming kernel),
+    # the next two more (the tiles with K in parts); with more rows of W, or shorter ones, the share kernel comes first
+    assert _lib.builtin_gemm(M, N, K, q8=True).config.variant == variant
     rng = np.random.default_rng(M + N + K)
     wq, scale = _weights(N, K, N + K + 1)
     a = rng.standard_normal((M, K)).astype(np.float16)
@@ -304,7 +306,9 @@ def test_gemm_q8_streaming_tiles(oracle, kind, rows, cols, kslice, M, N, K):
 
 
 def test_gemm_q8_streaming_is_the_choice_for_few_rows_exact_and_reproducible(oracle):
-    # one-hot rows of A return decoded columns of W bit for bit, through the route cfg = NULL takes for M <= 16
+    # one-hot rows of A return decoded columns of W bit for bit, through the route cfg = NULL takes for M <= 16 against fewer rows
+    # of W than the share kernel takes
+    assert _lib.builtin_gemm(7, 200, 1280, q8=True).config.variant == _lib.GEMM_STREAM
     wq, scale = _weights(200, 1280, 3)
     w = oracle.c.decode_q8(wq, scale)
     ks = (0, 7, 31, 32, 511, 512, 1279)
@@ -321,7 +325,7 @@ def test_gemm_q8_streaming_is_the_choice_for_few_rows_exact_and_reproducible(ora
     runs = []
     for _ in range(3):
         out = Guarded((16, 2560), torch.float16)
-        ops.gemm_q8(dev(a), _words(wq), dev(scale), None, out.t)
+        ops.gemm_q8(dev(a), _words(wq), dev(scale), None, out.t, cfg(variant=_lib.GEMM_STREAM, tile=[16, 64, 512]))
         runs.append(out.check())
     assert all(np.array_equal(r.view(np.uint16), runs[0].view(np.uint16)) for r in runs)
     _check_gemm_q8(runs[0], a, wq, scale, None, None, None, 0, oracle)

@@ -78,9 +78,11 @@ def test_the_scales_behind_a_row_stay_its_neighbours(oracle, rows, cols, K, bad)
     _check(out.check()[:, good], want, None, None)
 
 
+# the rows of A up to which the share kernel is chosen
 @pytest.mark.parametrize("M", [3, 5, 16, 17, 33, 64, 65, 96, 128])
-@pytest.mark.parametrize("N,K", [(2560, 2560), (7680, 2560), (2560, 10240), (10240, 520), (257, 256), (17000, 2048)])
-def test_what_runs_without_a_config_either_side_of_the_line(oracle, M, N, K):
+@pytest.mark.parametrize("N,K,up_to", [(2560, 2560, 65), (7680, 2560, 96), (2560, 10240, 17), (10240, 520, 64), (257, 256, 96), (17000, 2048, 64)])
+def test_what_runs_without_a_config_either_side_of_the_line(oracle, M, N, K, up_to):
+    assert (_lib.builtin_gemm(M, N, K).config.variant == _lib.GEMM_SHARE) == (M <= up_to)
     a, bias, _, _, rng = _inputs(M, N, K, M + N)
     w = (rng.standard_normal((N, K)) * 0.05).astype(np.float16)
     out = Guarded((M, N), torch.float16)

@@ -81,10 +81,14 @@ def test_static_scratch_gemm_refuses_what_the_array_cannot_hold():
 
 def test_static_scratch_gemm_on_the_w_streaming_kernel():
     L = _lib.lib()
-    # 16 rows against 4096 x 4096: the built-in row is the W-streaming kernel, whose K slices meet in the scratch as well
+    # the W-streaming kernel, whose K slices meet in the scratch as well: 16 rows against 4096 x 4096 by the table's row, and
+    # against 1024 x 8192 without a config
     small = _problem(16, 4096, 4096, 5)
-    assert _lib.select_bucket(_lib.OP_GEMM_F16, 16, 4096, 4096).config.variant == _lib.GEMM_STREAM
-    assert_bits_equal(_run(L.dtas_gemm_f16_static, *small, None), _run(L.dtas_gemm_f16, *small, None))
+    row = _lib.select_bucket(_lib.OP_GEMM_F16, 16, 4096, 4096).config
+    assert row.variant == _lib.GEMM_STREAM and _lib.builtin_gemm(16, 1024, 8192).config.variant == _lib.GEMM_STREAM
+    assert_bits_equal(_run(L.dtas_gemm_f16_static, *small, row), _run(L.dtas_gemm_f16, *small, row))
+    long = _problem(16, 1024, 8192, 6)
+    assert_bits_equal(_run(L.dtas_gemm_f16_static, *long, None), _run(L.dtas_gemm_f16, *long, None))
 
 
 def test_static_scratch_gemm_allocates_no_device_memory():
