@@ -239,7 +239,7 @@ class MFMAConfig(Config):
         self.mfma_m, self.mfma_n, self.mfma_k = 32, 32, 16
         self.skinny = False      # small M: weight-streaming 16x16x32 kernel, K split over wavefronts
         self.stream = False      # M <= 64: W streamed through the LDS in 1 KiB row pieces, K sliced over workgroups
-        self.share = False       # M <= 128: every workgroup an equal number of columns (at most j blocks of 16) over the whole of K
+        self.share = False       # M <= 128: every workgroup an equal number of columns (at most tile_size_n) over the whole of K
         self.block_threads = 256
         self.stages = 0          # LDS stages of the load pipeline (0 = as many as the tile allows)
         self.split_k = 1         # workgroups that share a tile and split its K extent

@@ -366,8 +366,9 @@ __global__ void __launch_bounds__(256) attn_scores_pipe_kernel(const half_t* __r
 }
 
 // Scores whose rows are not whole 64-byte sectors (m % 16 != 0, or an output that is not sector-aligned).  Tiles cut every
-// row at the same columns, so the sector on each cut is written in two parts by two workgroups, and what the two L2s
-// cannot join is filled from memory first.  Here every row is cut at sector boundaries of its own: a workgroup takes 32
+// row at the same columns, so the sector on each cut is written in two parts by two workgroups: 1.5 write requests per sector
+// at the L2s (203 x 1031), and on larger outputs fills from memory (1025 x 1025: 50 MB).  Here every row is cut at sector
+// boundaries of its own, 1.09 requests per sector: a workgroup takes 32
 // query rows and `chunk` keys (a multiple of 16, at most 480), computes 16 keys more, and writes of each row the whole
 // sectors that start in its chunk.  Only a row's two ends share a sector with its neighbours.
 //  * Q's fragments stay in registers, K's come straight from memory (5 KiB per 32 keys of 80, read in whole; the
@@ -376,8 +377,8 @@ __global__ void __launch_bounds__(256) attn_scores_pipe_kernel(const half_t* __r
 //    scores of a row; a row lies in the LDS at its distance from a 16-byte boundary of the output, so that four scores are
 //    one 8-byte LDS read, one (under-aligned) 8-byte read of the mask, requested before the products, and one aligned
 //    16-byte streaming store.  33 KiB of LDS: four workgroups per CU.
-// What bounds it: beside the stores, K passes through a CU's L1 once per 32 query rows.  32 heads of 80 against the tiles: 203 x 1031
-// 15.6 -> 13.3 us, 130 x 2049 18.0 -> 15.4.  Not kept: K through the LDS in 1 KiB loads (two workgroups per CU), that with 64 rows;
+// What bounds it: beside the stores, K passes through a CU's L1 once per 32 query rows (68 MB for 27 MB of scores at 203 x 1031; the
+// wavefronts' cycles fall by a quarter).  32 heads of 80 against the tiles: 203 x 1031 15.6 -> 13.3 us, 130 x 2049 18.0 -> 15.4.  Not kept: K through the LDS in 1 KiB loads (two workgroups per CU), that with 64 rows;
 // registers for three workgroups per CU; the mask under a row's ends loaded where it is used (a memory latency per end).
 constexpr int kSectorRows = 32, kSectorKeys = 512, kSectorChunk = 480, kSectorPitch = kSectorKeys + 4;
 constexpr int kSectorSteps = 5;  // k steps of 16: head dimensions of 65 .. 80

@@ -19,8 +19,9 @@ namespace {
 //    8-bit weight widened) once per workgroup; their sums meet in the LDS at the end, added in wavefront order.
 // Measured with W from memory, us, before / now: 17 rows against 7680 x 2560, 10240 x 2560, 2560 x 10240, 2560 x 2560 13.1 / 9.8,
 // 16.5 / 12.0, 19.3 / 16.3, 8.7 / 6.5; 48 rows against 11008 x 4096, 4096 x 4096 26.0 / 20.5, 13.2 / 12.1; 8-bit weights, 48
-// rows against 7680 x 2560, 10240 x 2560 17.1 / 10.8, 17.9 / 12.5 (6.0 TB/s of W at best, where the fp16 GEMV takes 8.5
-// and 10.0 us of the first two).
+// rows against 7680 x 2560, 10240 x 2560 17.1 / 10.8, 17.9 / 12.5 (5.0 TB/s of W at 16 rows against 11008 x 4096, where the
+// fp16 GEMV takes 14.7 us and this 17.9).  What bounds it: memory delivers W once (17 rows against 10240 x 2560: 53 MB fetched for 52),
+// and a CU pulls A in beside it -- 48 rows against 11008 x 4096: 101 MB of A for 90 of W, 35 KB/us per CU at 890 cycles a request.
 // In the LDS the 16-byte chunk c of row r sits in slot c ^ f(r), f(r) = 2 (r & 7) + ((r >> 3) & 1), and lane groups 0..3 of a
 // fragment read take chunks 0, 2, 1, 3 of the k step (both operands alike): the 16 rows of a lane group fall into 16 bank groups.
 // W is the first MFMA operand: register v of lane l is row l & 15 of C, column 4 (l >> 4) + v of a 16x16 block, so that a

@@ -183,8 +183,9 @@ class MFMAConfigEmiter(BaseConfigEmiter):
                 c.i, c.j, c.micro_shape_x, c.micro_shape_y, c.micro_shape_k = 1, cols // 16, rows // 16, 1, kslice // 32
                 c.mfma_m, c.mfma_n, c.mfma_k = 16, 16, 32
                 stream.append(c)
-        # the share kernel: every workgroup N / (number of CUs) columns over the whole of K (the library takes it for a call
-        # without a config wherever it leads at the M at hand; the table's rows, which a first candidate equals, do not name it)
+        # the share kernel: every workgroup N / (number of CUs) columns over the whole of K.  The second candidate: the library
+        # takes it for a call without a config where it leads at the M at hand (libdtas: share_leads), a line that the table's
+        # rows, which a first candidate equals, do not draw -- only a timed tuning finds it here
         share: List[MFMAConfig] = []
         rows, cols = self.share_shape(m_hi, N)
         if rows:
@@ -256,7 +257,8 @@ class MFMAConfigEmiter(BaseConfigEmiter):
 
     def share_shape(self, m_hi: int, N: int) -> Tuple[int, int]:
         """(rows of A, columns per workgroup) of the share kernel for m_hi rows, (0, 0) where there is none: the rows rounded
-        up to a kernel's, the fewest columns that give every CU one workgroup (libdtas: share_shape)."""
+        up to a kernel's, the fewest columns that give every CU one workgroup (libdtas: share_shape; a host test keeps the
+        two alike)."""
         per_cu = -(-N // self.arch.num_sm)
         rows = next((r for r in (16, 32, 48, 64, 96, 128) if m_hi <= r), 0)
         if rows == 16:

@@ -213,8 +213,8 @@ def _first_candidate(func, ranges):
 
 @pytest.mark.parametrize("N,K", [(4096, 4096), (11008, 4096), (4096, 11008), (2560, 10240), (4096, 1024), (1024, 1024), (8192, 8192)])
 def test_gemm_emitter_leads_with_the_librarys_builtin_choice(N, K):
-    # the closed-form policy exists twice (C tables for cfg == NULL, Python emitter for the tuner's
-    # first candidate): they must not drift apart
+    # the closed-form policy of the table's rows exists twice (the C tables, the Python emitter for the tuner's first
+    # candidate): they must not drift apart
     func = pf.fused_NT_matmul_add_gemm(N, K, bias=True)
     for m_hi in (16, 32, 48, 64, 128, 256, 512, 1024, 2048, 4096, 8192):
         want = _lib.select_bucket(_lib.OP_GEMM_F16, m_hi, N, K).config.to_dict()
@@ -223,6 +223,17 @@ def test_gemm_emitter_leads_with_the_librarys_builtin_choice(N, K):
         if want["variant"] == _lib.GEMM_MFMA and want["block"] == 512:
             keys = ("variant", "block", "tile", "split_k")   # the 8-wavefront ring loops have no stage count
         assert {k: got[k] for k in keys} == {k: want[k] for k in keys}, (m_hi, got, want)
+
+
+@pytest.mark.parametrize("N", [256, 1000, 4096, 4097, 8192, 8193, 12288, 14336, 14337, 16384, 16385, 50280])
+def test_gemm_emitter_names_the_share_kernel_that_the_library_would_take(N):
+    from dtas_amd.policy import MFMAConfigEmiter
+    emiter = MFMAConfigEmiter(FuncInfo(pf.fused_NT_matmul_add_gemm(N, 2560, bias=True)), MI355X())
+    for m_hi in (16, 32, 48, 64, 96, 128):
+        for K in (256, 512, 1024, 2048, 2560, 4096):
+            c = _lib.builtin_gemm(m_hi, N, K).config
+            if c.variant == _lib.GEMM_SHARE:
+                assert emiter.share_shape(m_hi, N) == tuple(c.tile[:2]), (m_hi, K)
 
 
 def test_reduction_emitters_lead_with_the_librarys_builtin_choice():
