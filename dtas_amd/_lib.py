@@ -117,6 +117,9 @@ SIGNATURES = {
     "dtas_gemm_q8_f16_fused": [_vp, _vp, _vp, _vp, _vp, _vp, _vp, _i64, _i64, _i64, ctypes.c_int32, _cfg, _vp],
 }
 
+# entry points that builds of this ABI version from before them lack: such a build (DTAS_LIBRARY) serves everything else
+LATER = {"dtas_builtin_gemm"}
+
 _lib = None
 
 
@@ -134,6 +137,8 @@ def lib() -> ctypes.CDLL:
                 "(hipcc --offload-arch=gfx950); dtas_amd has no fallback path")
         handle = ctypes.CDLL(LIB_PATH)
         for name, argtypes in SIGNATURES.items():
+            if name in LATER and not hasattr(handle, name):
+                continue
             fn = getattr(handle, name)
             fn.argtypes = argtypes
             fn.restype = ctypes.c_int
@@ -148,7 +153,8 @@ def lib() -> ctypes.CDLL:
 def entry_addresses() -> dict:
     """{entry point: its address in the loaded library}, as a C caller would link them."""
     handle = lib()
-    return {name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in (*SIGNATURES, "dtas_last_error")}
+    return {name: ctypes.cast(getattr(handle, name), ctypes.c_void_p).value for name in (*SIGNATURES, "dtas_last_error")
+            if name not in LATER or hasattr(handle, name)}
 
 
 def last_error() -> str:

@@ -27,6 +27,16 @@ def test_library_exports_every_declared_symbol():
     assert set(names) == set(_lib.SIGNATURES) | {"dtas_last_error"}
 
 
+def test_a_build_without_a_later_entry_point_loads(monkeypatch):
+    monkeypatch.setattr(_lib, "_lib", None)
+    monkeypatch.setitem(_lib.SIGNATURES, "dtas_not_yet", [])
+    with pytest.raises(AttributeError):
+        _lib.lib()
+    monkeypatch.setattr(_lib, "LATER", {"dtas_not_yet"})
+    assert _lib.lib().dtas_abi_version() == _lib.ABI_VERSION
+    assert "dtas_not_yet" not in _lib.entry_addresses() and "dtas_builtin_gemm" in _lib.entry_addresses()
+
+
 def test_abi_version_and_struct_layout():
     assert _lib.lib().dtas_abi_version() == _lib.ABI_VERSION
     assert ctypes.sizeof(_lib.DtasConfig) == 40          # 8 x int32 + int64
