@@ -71,6 +71,26 @@ def test_scores_rows_cut_at_their_own_sectors(oracle, heads, n, m, d, at):
     assert bool((buf[:at] == -7.0).all()) and bool((buf[at + heads * n * m:] == -7.0).all())
 
 
+@pytest.mark.parametrize("bad", [float("inf"), float("-inf"), float("nan")])
+def test_scores_rows_cut_at_their_own_sectors_with_non_finite_keys(oracle, bad):
+    # a key at each end of a chunk and the last one, a query in the last partly filled block; the mask's own infinities
+    heads, n, m, d = 32, 225, 1031, 72
+    q, k, mask = _inputs(heads, n, m, d, 7)
+    keys = [0, 351, 352, 703, 704, 1030]
+    k[:, keys, d - 1] = bad
+    q[:, 224, 0] = bad
+    mask[:, 17], mask[3, 500] = np.float16(np.inf), np.float16(-np.inf)
+    out = Guarded((heads, n, m), torch.float32)
+    ops.attn_scores(dev(q), dev(k), dev(mask), out.t, SCALE)
+    got = out.check()
+    good = np.setdiff1d(np.arange(m), keys)
+    want = oracle.c.attn_scores(*(np.ascontiguousarray(a) for a in (q[:, :224], k[:, good], mask[:224][:, good])), SCALE, threads=8)
+    got = got[:, :224][:, :, good]
+    fin = np.isfinite(want)     # (-inf under the mask's -inf, and nowhere else)
+    assert np.array_equal(got[~fin], want[~fin]) and not fin.all()
+    assert (np.abs(got[fin].astype(np.float64) - want[fin]) <= 1e-3 + 2.0 ** -9 * np.abs(want[fin])).all()
+
+
 @pytest.mark.parametrize("tile,block,stages", [((64, 64), 256, 2), ((64, 64), 256, 3), ((128, 128), 256, 2), ((128, 64), 256, 2),
                                                ((64, 128), 256, 2), ((256, 128), 256, 2), ((256, 256), 512, 2), ((256, 256), 256, 2)])
 @pytest.mark.parametrize("heads,n,m,d", [(3, 70, 131, 80), (2, 300, 260, 64), (1, 33, 7, 8)])

@@ -78,6 +78,24 @@ def test_the_scales_behind_a_row_stay_its_neighbours(oracle, rows, cols, K, bad)
     _check(out.check()[:, good], want, None, None)
 
 
+@pytest.mark.parametrize("rows,cols", [(16, 16), (32, 48), (64, 128), (96, 32), (128, 48)])
+@pytest.mark.parametrize("bad", [65504.0, float("inf"), float("nan")])
+def test_non_finite_rows_and_columns_stay_where_they_are(oracle, rows, cols, bad):
+    # the last element of K, the last rows of A and of a workgroup's columns: what lies behind them is read as zero, and zero times
+    # any of these would be seen
+    M, N, K = rows - 3, 256 * cols - 5, 520
+    a, bias, _, _, rng = _inputs(M, N, K, rows + cols)
+    w = (rng.standard_normal((N, K)) * 0.05).astype(np.float16)
+    a[M - 1, K - 1] = a[0, 0] = a[M // 2, 256] = bad
+    w[cols - 1::cols, K - 1] = bad
+    w[N - 1, 0] = bad
+    r, c = np.isfinite(a).all(1) & (np.abs(a) < 6e4).all(1), np.isfinite(w).all(1) & (np.abs(w) < 6e4).all(1)
+    out = Guarded((M, N), torch.float16)
+    ops.gemm(dev(a), dev(w), dev(bias), out.t, cfg(variant=_lib.GEMM_SHARE, tile=[rows, cols, 0]))
+    want = oracle.c.gemm_fused(a[r], w[c], np.ascontiguousarray(bias[c]), None, None, 0, threads=8)
+    _check(np.ascontiguousarray(out.check()[r][:, c]), want, None, None)
+
+
 # the rows of A up to which the share kernel is chosen
 @pytest.mark.parametrize("M", [3, 5, 16, 17, 33, 64, 65, 96, 128])
 @pytest.mark.parametrize("N,K,up_to", [(2560, 2560, 65), (7680, 2560, 96), (2560, 10240, 17), (10240, 520, 64), (257, 256, 96), (17000, 2048, 64)])
