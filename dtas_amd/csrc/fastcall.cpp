@@ -1,7 +1,8 @@
 // The ordinary case of every entry point of dtas_amd.ops, checked and launched natively: tensors in, one library call out.
-// A call of three rows of 4096 costs the host 3.7 us here (copy, RMSNorm), hardly more than the launch (the library's entry
-// point through ctypes, pointers at hand: 3.8), and 5.9 / 6.4 us through the checks, pointers and extents in Python; a decode
-// layer of 19 launches is bound by just that (one layer at 127 keys 110 -> 74 us).
+// A call of three rows of 4096 costs the host 2.9 .. 3.7 us here (copy, RMSNorm; which of the two goes with the core that the
+// process got), no more than the launch (the library's entry point through ctypes, pointers at hand: 3.1 .. 3.8), and 5.3 .. 6.4
+// us through the checks, pointers and extents in Python; a decode layer of 19 launches is bound by just that (one layer at
+// 127 keys 110 -> 72 .. 75 us).
 // Each function takes the arguments of the `ops` function of its name (without `cfg`) and returns True after the launch.
 // For whatever is not the ordinary case -- another type of object, a tensor that is not a plain contiguous one on the
 // device, any check that does not hold, an extent of zero, a torch-function mode -- it does nothing and returns False:
