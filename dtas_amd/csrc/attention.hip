@@ -854,6 +854,8 @@ extern "C" int dtas_attn_scores_f16_f32(const void* Q, const void* Kmat, const v
   if (cfg.split_k > 1) return fail("attn_scores: K is the head dimension, it is not split");
   int64_t la[7];
   if (describe_gemm(n, m, d, cfg, la) != 0) return -1;
+  if (cfg.block == 512 && cfg.tile[0] != 192 && cfg.tile[0] + cfg.tile[1] != 384 && cfg.tile[0] + cfg.tile[1] != 512)
+    return fail("attn_scores: the %dx%d MFMA kernel does not come with 512 threads", cfg.tile[0], cfg.tile[1]);
   GemmEpilogue ep = {nullptr, static_cast<const half_t*>(mask), nullptr, kEpiScores, 1,
                      static_cast<float>(static_cast<half_t>(scale)), n * d, m * d, n * m, 0, 1,
                      // a mask beyond an L2's reach (4 MiB) is kept in place, one part per XCD; below that
@@ -1103,6 +1105,7 @@ extern "C" int dtas_attn_pv_f16(const void* P, const void* V, void* out, int64_t
   int64_t la[7];
   if (describe_gemm(n, d, m, cfg, la) != 0) return -1;   // (also: no more LDS stages than the tile allows)
   const int bm = cfg.tile[0], bn = cfg.tile[1];
+  if (bm == 128 && bn <= 128 && cfg.block != 256) return fail("attn_pv: the %dx%d MFMA kernel uses 256 threads, got %d", bm, bn, cfg.block);
   const int ns = cfg.unroll >= 2 ? cfg.unroll : 2;
   ep.lda = m;
   ep.k_tail = static_cast<unsigned>(m - m_main);

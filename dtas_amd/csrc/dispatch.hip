@@ -192,7 +192,8 @@ dtas_config gemv_policy(int64_t N, int64_t K) {
   return make(DTAS_GEMV_SPLITK, 256, 8, 2, 1);
 }
 
-// GEMM: a cost model fitted to sweeps of every tile x stage count x K split over M on an MI355X.
+// GEMM: more than 128 rows: tile8_policy (gemm_tiles.hip).  Up to 128 rows: a cost model fitted to sweeps of every tile x
+// stage count x K split over M on an MI355X.
 // A candidate's time is (rounds of workgroups over the chip) x (time of one k tile) x (k tiles):
 //  * time of one k tile with every CU busy: 256x256 1.50 us, 256x128 (8 wavefronts) 1.00 us, 128x128
 //    0.665 us with 4 stages (one workgroup per CU) or 1.14 us per round of two per CU with 2 stages;
@@ -220,6 +221,8 @@ double gemm_rounds(double wgs, double slots) {
 dtas_config gemm_policy(int64_t M_hi, int64_t N, int64_t K) {
   const int64_t n = N > 0 ? N : 1, k = K > 0 ? K : 1;
   const int64_t ktiles = ceil_div(k, 64);
+  dtas_config wide;
+  if (M_hi > 128 && tile8_policy(M_hi, n, k, true, true, &wide)) return wide;
   GemmChoice best = {1e30, 64, 64, 256, 4, 1};
   auto consider = [&](double us, int bm, int bn, int block, int stages, int split) {
     if (us < best.us) best = {us, bm, bn, block, stages, split};

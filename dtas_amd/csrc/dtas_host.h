@@ -60,5 +60,7 @@ int resolve_static_scratch(void** out);
 // split_k = 0 on the 8-wavefront 256x256 GEMM tile: how the tiles of a last, partly filled round are shared.
 // *unsplit tiles (whole rounds of the chip) get one workgroup each, the rest *nsplit workgroups each (1 = none).
 void tail_split_256(int64_t M, int64_t N, int64_t K, int* nsplit, unsigned* unsplit);
+// the tile of a GEMM of more than 128 rows, and the parts of K; false: none holds the extents
+bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table, dtas_config* out);
 
 }  // namespace dtas

@@ -143,6 +143,7 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
   int64_t la[7];
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;
   const int bm = cfg.tile[0], bn = cfg.tile[1];
+  if (bm == 128 && bn <= 128 && cfg.block != 256) return fail("gemm_q8: the %dx%d MFMA kernel uses 256 threads, got %d", bm, bn, cfg.block);
   if (bm == 256 && bn == 128 && cfg.unroll == 3) return launch_mfma<256, 128, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);
   if (bm == 128 && bn == 128 && cfg.unroll == 3) return launch_mfma<128, 128, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);
   if (bm == 64 && bn == 64 && cfg.unroll == 2) return launch_mfma<64, 64, 2, 2, 2, false, true>(s, a, w, ep, C, M, N, K, sk);

@@ -17,6 +17,12 @@
 namespace dtas {
 namespace {
 
+constexpr int largest_divisor(int n, int limit) {
+  int d = n < limit ? n : limit;
+  while (n % d != 0) --d;
+  return d;
+}
+
 // WT: W is given k-major ([K][N], N contiguous -- the V operand of attention's P.V); its tiles sit in the LDS as they lie
 // in memory (the same direct-to-LDS loads and pipelines as a row-major W) and the MFMA fragments are read with the
 // transposing LDS read ds_read_b64_tr_b16 (4 wavefronts only).
@@ -37,17 +43,18 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   constexpr int LA = BM / 8 / NW, LB = BN / 8 / NW;  // 1 KiB block loads per wavefront per k tile
   constexpr int kABytes = BM * kRowBytes, kStage = (BM + BN) * kRowBytes;
   static_assert(NW % 2 == 0 && LA >= 1 && LB >= 1 && MT >= 1 && NT >= 1, "tile / wavefront split");
-  static_assert(NS >= 2 && NS <= 4 && (NW != 8 || NS == 2), "stage count");
+  static_assert(NS >= 2 && NS <= (M16 ? 6 : 4), "stage count");
   static_assert((NS - 1) * (LA + LB) <= 63, "outstanding loads must fit the vmcnt field");
   constexpr bool WREG = WQ;  // W tiles pass through registers (dequantised), not the direct-to-LDS path
   static_assert(!WREG || (NS <= 3 && NW == 4), "the register W path is written for two or three stages and 4 wavefronts");
   static_assert(!(WT && WQ), "k-major 8-bit weights are not served");
   static_assert(!WT || (NW == 4 && BN >= 64), "the k-major W path is written for the 4-wavefront 32x32x16 loops");
   static_assert(M16 == (NW == 8) && (!M16 || !WREG), "8 wavefronts run the 16x16x32 loop, and only they");
-  // 256x256 and every 8-wavefront tile: a ring of 5 operand units, each the larger operand's rows of a k tile
-  constexpr bool kRing = BM + BN == 512 || M16;
+  // 256x256 and the 8-wavefront tiles on two stages: a ring of 5 operand units, each the larger operand's rows of a k tile
+  constexpr bool kRing = M16 ? NS == 2 : BM + BN == 512;
   constexpr int kRingUnit = (BM > BN ? BM : BN) * kRowBytes;
-  constexpr int kLdsAlloc = kRing ? 5 * kRingUnit : NS * kStage;
+  constexpr int kStagesA = !M16 || NS * kStage <= kLdsBytes ? NS : 2;  // (8 wavefronts: W's stages are NS, A's what the LDS leaves)
+  constexpr int kLdsAlloc = kRing ? 5 * kRingUnit : kStagesA * kABytes + NS * BN * kRowBytes;
   static_assert(BM * BN * 2 <= kLdsAlloc, "epilogue staging must fit the operand stages");
   static_assert(kLdsAlloc <= kLdsBytes, "stages exceed the LDS");
   __shared__ __attribute__((aligned(1024))) char lds[kLdsAlloc];
@@ -383,12 +390,18 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     //  * loads are whole 128-byte lines (half lines cost the L2 path twice the requests), and the barrier sits
     //    where every wavefront holds all fragments of the tile in registers, so both units of tile kt are free
     //    from that barrier on.
-    // The whole LDS is a ring of five 32 KiB operand units, A(0) W(0) A(1) W(1) A(2) ...: unit u sits in slot u % 5;
+    // NS = 2: the whole LDS is a ring of five 32 KiB operand units, A(0) W(0) A(1) W(1) A(2) ...: unit u sits in slot u % 5;
     // a k tile is two k32 steps.
     // (a 256x128 or 128x256 tile leaves half of every other slot unused)
+    // NS >= 3: NS stages of W and kStagesA of A.  The ring requests W one k tile ahead, 1.5 us on 256x256, which is time enough;
+    // a smaller tile's k tile is shorter than a trip to memory, and with W from HBM it waited for it: 192x128 0.88 us per k tile on the
+    // ring, 0.67 with W three and A two k tiles ahead (1024 x 4096 x 4096 53.1 -> 42.3 us), 256x128 0.98 -> 0.86 (1025 x 2560 x 10240 in
+    // two parts 76.5 -> 68.9), 192x256 with two stages of A and three of W 1.28 -> 1.12 (1025 x 7680 x 2560 52.9 -> 47.3).  More stages than these
+    // gain nothing (96x128 with 5, 128x64 with 6): then it is the rate at which lines that miss the L2 come in.
     constexpr int kUnit = kRingUnit;
     constexpr int kLoadsA = BM / 32, kLoadsW = BN / 32;  // 1 KiB block loads per wavefront and unit
-    static_assert(5 * kUnit <= kLdsAlloc && BM % 32 == 0 && BN % 32 == 0, "ring exceeds the LDS");
+    static_assert((!kRing || 5 * kUnit <= kLdsAlloc) && BM % 32 == 0 && BN % 32 == 0, "ring exceeds the LDS");
+    constexpr int kFirstW = kRing ? kUnit : kStagesA * kABytes;  // where W(0) sits
     auto wrap5 = [](int v) { return v >= 5 ? v - 5 : v; };
     const bool hi = wv >= 4;
     if (hi) __builtin_amdgcn_s_setprio(0); else __builtin_amdgcn_s_setprio(2);
@@ -420,7 +433,38 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     for (int ks = 0; ks < 2; ++ks) rd16[ks] = lds_chunk_offset(l & 15u, 4u * ks + (((l >> 4) & 1u) << 1 | (l >> 5)));
     const unsigned a_frag = wm * WTM * 128u, b_frag = wn * WTN * 128u;
     f16x8 ga[2][MT16], gb[2][NT16];
-    if (hi) {
+    // stages: A(kt) in A stage kt % kStagesA, W(kt) in W stage kt % NS.  Wavefronts 4-7 load right behind the barrier, which
+    // is as early as a stage is free: W, or with two stages of A the operand that has no time to lose, A.  0-3 load the
+    // other one behind their MFMAs as on the ring (kLoLate; half a k tile earlier measured 2-15 % slower on 128x256, level on 256x128),
+    // or, W in three stages, between their two steps: it is then a k tile and a half ahead.
+    constexpr bool hi_w = kStagesA >= 3;
+    constexpr int kHiStages = hi_w ? NS : kStagesA, kLoStages = hi_w ? kStagesA : NS;
+    constexpr int kHiLoads = hi_w ? kLoadsW : kLoadsA, kLoLoads = hi_w ? kLoadsA : kLoadsW;
+    constexpr int kWBase = kStagesA * kABytes;
+    constexpr bool kLoLate = hi_w;
+    auto fetch_a = [&](int stage, unsigned voff) {
+      char* base = lds + stage * kABytes + (wv & 3u) * 1024;
+#pragma unroll
+      for (int q = 0; q < kLoadsA; ++q) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(base + q * 4096), 16, voff, q * g16_step, 0, DTAS_GEMM_LOAD_AUX);
+    };
+    auto fetch_w = [&](int stage, unsigned voff) {
+      char* base = lds + kWBase + stage * (BN * kRowBytes) + (wv & 3u) * 1024;
+#pragma unroll
+      for (int q = 0; q < kLoadsW; ++q) __builtin_amdgcn_raw_ptr_buffer_load_lds(rw, (lds_ptr_t)(base + q * 4096), 16, voff, q * g16_step, 0, DTAS_GEMM_LOAD_AUX);
+    };
+    auto fetch_hi = [&](int stage, unsigned voff) { if constexpr (hi_w) fetch_w(stage, voff); else fetch_a(stage, voff); };
+    auto fetch_lo = [&](int stage, unsigned voff) { if constexpr (hi_w) fetch_a(stage, voff); else fetch_w(stage, voff); };
+    if constexpr (!kRing) {
+      if (hi) {
+#pragma unroll
+        for (int p = 0; p < kHiStages; ++p) fetch_hi(p, lane_off16(p));
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((kHiStages - 1) * kHiLoads));
+      } else {
+#pragma unroll
+        for (int p = 0; p < kLoStages; ++p) fetch_lo(p, lane_off16(p));
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((kLoStages - 1) * kLoLoads));
+      }
+    } else if (hi) {
       fetch16(1, lane_off16(0));
       fetch16(3, lane_off16(1));
       __builtin_amdgcn_s_waitcnt(waitcnt_imm(kLoadsW));
@@ -433,7 +477,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     __builtin_amdgcn_s_barrier();
     DTAS_SCHED_FENCE();
 #pragma unroll
-    for (int j = 0; j < NT16; ++j) gb[0][j] = *reinterpret_cast<const f16x8*>(lds + kUnit + b_frag + j * 2048 + rd16[0]);
+    for (int j = 0; j < NT16; ++j) gb[0][j] = *reinterpret_cast<const f16x8*>(lds + kFirstW + b_frag + j * 2048 + rd16[0]);
 #pragma unroll
     for (int i = 0; i < MT16; ++i) ga[0][i] = *reinterpret_cast<const f16x8*>(lds + a_frag + i * 2048 + rd16[0]);
     DTAS_SCHED_FENCE();
@@ -458,8 +502,30 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
         }
     };
     static_assert(kReadEvery * (MT16 + NT16) <= MT16 * NT16, "fragment reads must fit between the MFMAs of a step");
+    if constexpr (!kRing) {
+      static_assert((NS - 1) * (kLoadsA > kLoadsW ? kLoadsA : kLoadsW) <= 63, "outstanding loads must fit the vmcnt field");
+      int sa = 0, sw = 0;  // stages of A(kt), W(kt)
+      for (int kt = 0; kt < ktiles; ++kt) {
+        const int na = sa + 1 == kStagesA ? 0 : sa + 1, nw = sw + 1 == NS ? 0 : sw + 1;
+        step16(0, lds + sa * kABytes, lds + kWBase + sw * (BN * kRowBytes), 1);
+        if (kLoLate && !hi && kt > 0) fetch_lo(sa == 0 ? kStagesA - 1 : sa - 1, lane_off16(kt + kLoStages - 1));
+        // every fragment of tile kt is in registers and tile kt+1 has landed (later tiles may be in flight)
+        if (hi) __builtin_amdgcn_s_waitcnt(waitcnt_imm((kHiStages - 2) * kHiLoads)); else __builtin_amdgcn_s_waitcnt(waitcnt_imm((kLoStages - 2) * kLoLoads));
+        DTAS_SCHED_FENCE();
+        __builtin_amdgcn_s_barrier();
+        DTAS_SCHED_FENCE();
+        // the stages of tile kt are free: wavefronts 4-7 request now, 0-3 after their MFMAs of the step
+        if (hi) fetch_hi(hi_w ? sw : sa, lane_off16(kt + kHiStages));
+        DTAS_SCHED_FENCE();
+        step16(1, lds + na * kABytes, lds + kWBase + nw * (BN * kRowBytes), 0);
+        if (!kLoLate && !hi) fetch_lo(sw, lane_off16(kt + kLoStages));
+        DTAS_SCHED_FENCE();
+        sa = na;
+        sw = nw;
+      }
+    }
     int slot_a = 0, slot_w = 1;  // slots of A(kt), W(kt)
-    for (int kt = 0; kt < ktiles; ++kt) {
+    for (int kt = 0; kRing && kt < ktiles; ++kt) {
       const char* pa = lds + slot_a * kUnit;
       const char* pw = lds + slot_w * kUnit;
       const int next_a = wrap5(slot_a + 2), next_w = wrap5(slot_w + 2);
@@ -905,7 +971,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     constexpr int kPasses = WTM / kRowsPerPass;
     // as many as the registers hold (kVecC / 2 per vector): 128 registers for one operand, 64 each for two
     constexpr int kWant = (KIND == DTAS_EPI_BIAS_GELU ? 16 : kAdd2 ? 64 : kUseR1 ? 128 : 16) / kVecC;
-    constexpr int G = kPasses <= kWant ? kPasses : kPasses % kWant == 0 ? kWant : (kPasses % 8 == 0 && kWant >= 8 ? 8 : (kPasses % 4 == 0 && kWant >= 4 ? 4 : 1));
+    constexpr int G = largest_divisor(kPasses, kWant);
 #pragma unroll 1
     for (int p0 = 0; p0 < kPasses; p0 += G) {
       cvec_t r1v[G] = {}, r2v[G] = {};

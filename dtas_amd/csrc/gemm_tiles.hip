@@ -32,7 +32,9 @@
 //              and the card is power-limited on random operands), a whole k32 step of fragments in
 //              registers, one barrier per k tile; wavefronts w and w+4 share a SIMD, the older one
 //              wins the MFMA pipe, and each requests its share of the next units while the other
-//              multiplies (a wavefront that issues a load stalls until the load path takes it).
+//              multiplies (a wavefront that issues a load stalls until the load path takes it).  What the loads run
+//              ahead by decides the smaller of these tiles: with W from memory a k tile of 192x128 takes 0.88 us when
+//              it is requested one k tile ahead and 0.67 when two or three are in flight.
 //   epilogue : accumulators -> fp16 -> wavefront-private LDS region (xor-swizzled 8-byte
 //              slots) -> coalesced stores of whole tile rows (8 bytes per lane, 16 on the
 //              8-wavefront tiles) with the bias added on the way out.
@@ -56,6 +58,21 @@ namespace {
 inline int mfma_threads(int bm, int bn) { return bm == 256 && bn == 256 ? 512 : 256; }
 // LDS stages a launch uses unless told otherwise: 2 for 256x256, 3 for 256x128, 4 below that
 inline int mfma_max_stages(int bm, int bn) { return bm + bn >= 512 ? 2 : bm + bn >= 384 ? 3 : 4; }
+
+// The tiles that 8 wavefronts serve with stages of their own, and how many of W (0: none): as many k tiles ahead as the LDS
+// holds, at most three.  192x256 and 224x256 have three stages of W and two of A (the kernel's kStagesA): W is what
+// comes from memory.
+int tile8_stages(int bm, int bn) {
+  if (bn == 256) return bm == 96 || bm == 128 || bm == 160 || bm == 192 || bm == 224 ? 3 : 0;
+  if (bn == 128) return bm == 224 || bm == 256 ? 3 : bm == 96 || bm == 128 || bm == 160 || bm == 192 ? 4 : 0;
+  return bn == 64 && bm == 128 ? 4 : 0;
+}
+// ... and the ones that also come as a ring of five operand units (cfg.unroll == 2), each the larger operand's rows of a k tile
+bool tile8_ring(int bm, int bn) { return (bn == 256 && (bm == 128 || bm == 192)) || (bn == 128 && (bm == 192 || bm == 256)); }
+int tile8_lds(int bm, int bn) {
+  const int ns = tile8_stages(bm, bn);
+  return ((ns * (bm + bn) * kRowBytes <= kLdsBytes ? ns : 2) * bm + ns * bn) * kRowBytes;
+}
 
 }  // namespace
 
@@ -106,25 +123,26 @@ int describe_gemm(int64_t M, int64_t N, int64_t K, const dtas_config& cfg, int64
   if (cfg.vec != 8) return fail("gemm: vector width must be 8 (128 bit) or 1, got %d", cfg.vec);
   if (cfg.variant == DTAS_GEMM_MFMA) {
     const int bm = cfg.tile[0], bn = cfg.tile[1];
-    // tiles of 192 rows (8 wavefronts only): between the others in size, for tile counts that fill the chip better
-    const bool with_192 = bm == 192 && (bn == 256 || bn == 128);  // (192 columns: the epilogue's lane map wants wavefront tiles of 64 columns)
+    // tiles of 96, 160, 192 and 224 rows (8 wavefronts only): between the others in size, for tile counts that fill the chip
+    // better (192 columns: the epilogue's lane map wants wavefront tiles of 32, 64 or 128 columns)
+    const bool between = (bm == 96 || bm == 160 || bm == 192 || bm == 224) && (bn == 256 || bn == 128);
     const bool known = (bm == 256 && bn == 256) || (bm == 256 && bn == 128) || (bm == 128 && bn == 256) ||
                        (bm == 128 && bn == 128) || (bm == 64 && bn == 128) || (bm == 128 && bn == 64) ||
-                       (bm == 64 && bn == 64) || with_192;
+                       (bm == 64 && bn == 64) || between;
     if (!known || cfg.tile[2] != kBK) return fail("gemm: no MFMA kernel for tile %dx%dx%d", bm, bn, cfg.tile[2]);
-    // 256x256 comes as 8 wavefronts (two per SIMD, 128x64 each) or 4 (one per SIMD, 128x128 each); 256x128 and
-    // 128x256 as 4 wavefronts on whole-tile stages or 8 (64x64 each) on the 16x16x32 ring loop (128x128 on that
-    // loop, 64x32 per wavefront, measured slower than on 4 wavefronts at every M: not instantiated)
+    // 256x256 comes as 8 wavefronts (two per SIMD, 128x64 each) or 4 (one per SIMD, 128x128 each); 256x128, 128x256,
+    // 128x128 and 128x64 as 4 wavefronts or 8
     const bool four_waves = bm == 256 && bn == 256 && cfg.block == 256;
-    const bool eight_waves = (bm + bn == 384 || with_192) && cfg.block == 512;
-    if (with_192 && !eight_waves) return fail("gemm: the %dx%d MFMA kernel uses 512 threads, got %d", bm, bn, cfg.block);
+    const bool eight_waves = tile8_stages(bm, bn) != 0 && cfg.block == 512;
+    if (between && !eight_waves) return fail("gemm: the %dx%d MFMA kernel uses 512 threads, got %d", bm, bn, cfg.block);
     if (cfg.block != mfma_threads(bm, bn) && !four_waves && !eight_waves)
       return fail("gemm: the %dx%d MFMA kernel uses %d threads, got %d", bm, bn, mfma_threads(bm, bn), cfg.block);
     if (K * 2 * (bm > bn ? bm : bn) >= (int64_t{1} << 31)) return fail("gemm: K=%lld too large for 32-bit tile offsets", (long long)K);
     const int64_t tm = ceil_div(M, bm), tn = ceil_div(N, bn);
     if (tm * tn > 0x7fffffff) return fail("gemm: too many tiles");
     // cfg.unroll = LDS stages (the depth of the load pipeline); 0 or 1 = as many as fit
-    const int max_stages = with_192 ? 2 : mfma_max_stages(bm, bn);
+    // (8 wavefronts: 0 or 1 = the stages that tile8_stages says; 2 on 192, 256 or 128 x 256 = the ring of five operand units)
+    const int max_stages = bm == 192 ? 2 : eight_waves ? tile8_stages(bm, bn) : mfma_max_stages(bm, bn);
     if (cfg.unroll < 0 || cfg.unroll > max_stages)
       return fail("gemm: the %dx%d tile holds at most %d LDS stages, got %d", bm, bn, max_stages, cfg.unroll);
     int nsplit = cfg.split_k < 1 ? 1 : cfg.split_k;
@@ -135,9 +153,9 @@ int describe_gemm(int64_t M, int64_t N, int64_t K, const dtas_config& cfg, int64
     if (tm * tn * nsplit > 0x7fffffff) return fail("gemm: too many workgroups");
     la[0] = unsplit + (tm * tn - unsplit) * nsplit;
     la[3] = four_waves ? 256 : eight_waves ? 512 : mfma_threads(bm, bn);
-    // 256x256 and the 8-wavefront tiles: a ring of five operand units; else whole-tile stages
-    la[4] = (bm == 256 && bn == 256) || eight_waves ? 5 * (bm > bn ? bm : bn) * kRowBytes
-                                                    : (cfg.unroll >= 2 ? cfg.unroll : mfma_max_stages(bm, bn)) * (bm + bn) * kRowBytes;
+    if ((bm == 256 && bn == 256) || (eight_waves && cfg.unroll == 2 && tile8_ring(bm, bn))) la[4] = 5 * (bm > bn ? bm : bn) * kRowBytes;
+    else if (eight_waves) la[4] = tile8_lds(bm, bn);
+    else la[4] = (cfg.unroll >= 2 ? cfg.unroll : mfma_max_stages(bm, bn)) * (bm + bn) * kRowBytes;
     la[5] = tm;
     la[6] = tn;
     return 0;
@@ -234,11 +252,26 @@ int launch_tile_f16(const dtas_config& cfg, hipStream_t s, const half_t* a, cons
     if (cfg.split_k == 0 && batch == 1) tail_split_256(M, N, K, &split, &unsplit);  // (split_k >= 1: that split for every tile)
     return launch_mfma<256, 256, 2, 4, 2, false, false, true>(s, a, w, b, c, M, N, K, split, batch, unsplit);
   }
-  if (cfg.block == 512) {  // 8 wavefronts on the 16x16x32 ring loop
-    if (bm == 256 && bn == 128) return launch_mfma<256, 128, 4, 2, 2, false, false, true>(s, a, w, b, c, M, N, K, sk, batch);
-    if (bm == 128 && bn == 256) return launch_mfma<128, 256, 2, 4, 2, false, false, true>(s, a, w, b, c, M, N, K, sk, batch);
-    if (bm == 192 && bn == 256) return launch_mfma<192, 256, 2, 4, 2, false, false, true>(s, a, w, b, c, M, N, K, sk, batch);
-    if (bm == 192 && bn == 128) return launch_mfma<192, 128, 4, 2, 2, false, false, true>(s, a, w, b, c, M, N, K, sk, batch);
+  if (cfg.block == 512) {  // 8 wavefronts on the 16x16x32 loop
+#define DTAS_TILE8(BM_, BN_, WM_, WN_, NS_) \
+    if (bm == BM_ && bn == BN_ && (NS_ > 2 || (ns == 2 && tile8_ring(bm, bn)))) return launch_mfma<BM_, BN_, WM_, WN_, NS_, false, false, true>(s, a, w, b, c, M, N, K, sk, batch)
+    DTAS_TILE8(256, 128, 4, 2, 2);  // the rings of two stages: by a config only, but for 192x256 (tile8_policy)
+    DTAS_TILE8(128, 256, 2, 4, 2);
+    DTAS_TILE8(192, 256, 2, 4, 2);
+    DTAS_TILE8(192, 128, 4, 2, 2);
+    DTAS_TILE8(128, 64, 4, 2, 4);
+    DTAS_TILE8(96, 128, 2, 4, 4);
+    DTAS_TILE8(128, 128, 4, 2, 4);
+    DTAS_TILE8(160, 128, 2, 4, 4);
+    DTAS_TILE8(192, 128, 4, 2, 4);
+    DTAS_TILE8(224, 128, 2, 4, 3);
+    DTAS_TILE8(256, 128, 4, 2, 3);
+    DTAS_TILE8(96, 256, 2, 4, 3);
+    DTAS_TILE8(128, 256, 2, 4, 3);
+    DTAS_TILE8(160, 256, 2, 4, 3);
+    DTAS_TILE8(192, 256, 2, 4, 3);
+    DTAS_TILE8(224, 256, 2, 4, 3);
+#undef DTAS_TILE8
   }
   if (bm == 256 && bn == 128) return ns == 2 ? launch_mfma<256, 128, 2, 2, 2>(s, a, w, b, c, M, N, K, sk, batch)
                                              : launch_mfma<256, 128, 2, 2, 3>(s, a, w, b, c, M, N, K, sk, batch);
@@ -259,9 +292,95 @@ int launch_tile_f16(const dtas_config& cfg, hipStream_t s, const half_t* a, cons
   return fail("gemm: no MFMA kernel for tile %dx%d", bm, bn);
 }
 
+// Beyond 128 rows: the tile, and the parts of K.  A candidate's time is
+//   rounds of the chip x (a + b x k tiles of a part), a partly filled round at b x (r + (1 - r) x its share of the chip),
+//   + w x workgroups per CU + h0 + h1 x parts + h2 x (share of the chip)^4 where K is split (the hand-over of the partial tiles),
+// with b growing with 1 / (tile rows of the grid) (fewer workgroups share what W costs to bring in), falling with the rows past M
+// in the tiles (nothing is loaded for them), and x pitch where W's rows lie 5, 6, 10, .. KiB apart.  (64x64, of which a CU holds
+// several, at r + (1 - r) x its share up to one per CU and at 0.75 per workgroup of the fullest CU beyond.)  Fitted to 600 sizes (M =
+// 129 .. 8192 against 26 W of 512 x 2048 .. 50280 x 2560, W from memory) x up to 40 configurations each; h0 of the 8-wavefront tiles 1.8 us
+// above the fit and 64x64's hand-over as before the fit: in a layer, where other kernels run in between, a hand-over costs more than
+// in a loop over one kernel (140 x 2560 x 10240 in 3 parts of 128x64 33.9 us there, 27.5 in the loop; 64x64 in 2 parts 30.0 / 29.1).
+// In the bucket table (`in_table`): the tiles marked so, K in up to 4 parts of 8 k tiles or more (1.03 of the best
+// configuration's time on average); for a call without a config also the tiles between them, where no more than a fifth of
+// their rows lie past M or they make at most three rows of tiles, and up to 6 parts of 6 k tiles (1.012; over 260 random sizes
+// 0.93 of the time before these kernels).
+struct Tile8Cost {
+  int bm, bn, block, stages;
+  bool in_table;
+  double a, b, w, r, h0, h1, h2, pitch, few, pad;
+};
+constexpr Tile8Cost kTile8Cost[] = {
+    {64, 64, 256, 4, true, 3.74, 0.243, 0.42, 0.71, 1, 1, 0.3, 1.03, 0.8, 0.16},
+    {128, 64, 512, 0, true, 4.02, 0.326, 0, 0.69, 3.14, 0.57, 0.51, 1.08, 0.65, 0.71},
+    {96, 128, 512, 0, false, 3.9, 0.435, 0, 0.68, 2.66, 0.96, 1.87, 1.12, 0.8, 0.53},
+    {128, 128, 512, 0, true, 4.06, 0.501, 0.21, 0.62, 2.59, 1.2, 2.98, 1.11, 0.8, 0.74},
+    {160, 128, 512, 0, false, 4.58, 0.599, 0, 0.64, 2.97, 1.41, 3.14, 1.1, 0.54, 0.71},
+    {192, 128, 512, 0, true, 4.52, 0.673, 0.49, 0.65, 2.68, 1.81, 3.93, 1.08, 0.46, 0.66},
+    {224, 128, 512, 0, false, 4.2, 0.755, 1.33, 0.63, 2.51, 2.3, 2.67, 1.06, 0.36, 0.59},
+    {256, 128, 512, 0, true, 4.1, 0.827, 1.96, 0.66, 2.03, 2.65, 3.96, 1.06, 0.26, 0.52},
+    {96, 256, 512, 0, false, 3.85, 0.717, 0.83, 0.7, 3.49, 1.73, 2.44, 1.16, 0.8, 0.16},
+    {128, 256, 512, 0, false, 3.71, 0.835, 2.06, 0.66, 3.25, 2.39, 3.21, 1.15, 0.71, 0.48},
+    {160, 256, 512, 0, false, 5.21, 1.02, 0.65, 0.57, 2.21, 3.07, 3.96, 1.11, 0.49, 0.48},
+    {192, 256, 512, 0, true, 5.19, 1.152, 2.05, 0.59, 2.39, 3.56, 3.96, 1.11, 0.37, 0.33},
+    {224, 256, 512, 0, false, 5.85, 1.317, 1.9, 0.56, 1.66, 4.2, 4.84, 1.05, 0.3, 0.36},
+    {256, 256, 512, 2, true, 6.98, 1.505, 0.41, 0.48, -4, 5.88, 5, 1.02, 0.28, 0.34},
+};
+bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table, dtas_config* out) {
+  const int64_t ktiles = ceil_div(K, kBK);
+  const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
+  double best = 1e300;
+  for (const Tile8Cost& c : kTile8Cost) {
+    if (!c.in_table && (in_table || (ceil_div(M, c.bm) > 3 && M * 5 < ceil_div(M, c.bm) * c.bm * 4))) continue;
+    if (K * 2 * (c.bm > c.bn ? c.bm : c.bn) >= (int64_t{1} << 31)) continue;  // (32-bit tile offsets, describe_gemm)
+    const int64_t tm = ceil_div(M, c.bm), tn = ceil_div(N, c.bn), tiles = tm * tn;
+    if (tiles > 0x7fffffff / 8) continue;
+    const bool whole_rounds = c.bm == 256 && c.bn == 256;  // its split is of the last round's tiles (tail_split_256)
+    const int64_t slots = c.bm * c.bn <= 64 * 64 ? 2 * kNumCU : kNumCU;
+    const double b = c.b * (odd_pitch ? c.pitch : 1.0) *
+                     (1.0 + c.few / static_cast<double>(tm) - c.pad * (1.0 - static_cast<double>(M) / static_cast<double>(tm * c.bm)));
+    for (int parts = 1; parts <= (in_table ? 4 : 6); ++parts) {
+      int last_parts = parts;
+      unsigned unsplit = 0;
+      if (whole_rounds) {
+        tail_split_256(M, N, K, &last_parts, &unsplit);
+        // (inside dtas_gemm_f16_static: only as many partial tiles as there is room for)
+        if (!may_split || (!in_table && t_fixed_scratch && (tiles - unsplit) * last_parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) last_parts = 1;
+      } else if (parts > 1 && (!may_split || tiles * parts > slots || ktiles / parts < (in_table ? 8 : 6) ||
+                               tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) {
+        break;  // (no more partial tiles than dtas_gemm_f16_static has room for)
+      }
+      const bool tail = whole_rounds && last_parts > 1;
+      const int64_t wgs = whole_rounds ? tiles : tiles * parts, full = wgs / slots, rem = wgs % slots;
+      const double steps = static_cast<double>(whole_rounds ? ktiles : ceil_div(ktiles, parts));
+      const double share = static_cast<double>(wgs) / kNumCU;
+      double us = static_cast<double>(full) * (c.a + b * steps) + c.w * share;
+      const double fill = static_cast<double>(whole_rounds ? rem * last_parts : rem) / static_cast<double>(slots);
+      if (slots > kNumCU)  // (64x64: two or more workgroups share a CU)
+        us = c.a + b * steps * (wgs <= kNumCU ? c.r + (1.0 - c.r) * share : 0.75 * static_cast<double>(ceil_div(wgs, kNumCU))) + c.w * share;
+      else if (rem > 0) us += c.a + b * (whole_rounds ? static_cast<double>(ceil_div(ktiles, last_parts)) : steps) * (c.r + (1.0 - c.r) * fill);
+      if (last_parts > 1) {
+        const double crowd = whole_rounds ? fill : share;
+        us += c.h0 + c.h1 * last_parts + c.h2 * crowd * crowd * crowd * crowd;
+      }
+      if (us < best) {
+        best = us;
+        *out = dtas_config{DTAS_GEMM_MFMA, c.block, 8, c.stages, {c.bm, c.bn, kBK}, tail ? 0 : parts, 0};
+      }
+      if (whole_rounds) break;
+    }
+  }
+  // 192x256 against rows of W a multiple of 4 KiB apart: W in three stages and A in two, requested in the middle of a k tile,
+  // falls behind the ring of two (700 x 11008 x 4096 78.2 / 71.8 us, 1025 x 8192 x 2048 41.1 / 38.4; ahead elsewhere: 1400 x
+  // 4096 x 11008 152 / 178, 1025 x 7680 x 2560 50.7 / 53.9)
+  if (out->tile[0] == 192 && out->tile[1] == 256 && out->split_k == 1 && K % 2048 == 0) out->unroll = 2;
+  return best < 1e300;
+}
+
 // What a call without a config runs: the bucket's row, or ahead of it a kernel chosen by M itself (what A costs it goes
 // with M, and the row is sized for the end of its bucket).  vec_ok: 16-byte loads of A and W are possible.
-dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok) {
+// may_split: partial tiles have a place to go (what needs none otherwise).
+dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok, bool may_split) {
   // two rows of A (the first bucket's table row is sized for 16): W streamed in whole rows, as the GEMV does
   if (M == 2 && vec_ok) return dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {2, N <= 2560 ? 1 : 2, 8}, 1, 0};
   // three or four rows: the row kernel, a row of W per wavefront, against a W too small or too short for the share kernel
@@ -273,6 +392,8 @@ dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok) {
   // up to 128 rows of A: the share kernel where it leads
   int rows = 0, cols = 0;
   if (vec_ok && share_leads(M, N, K, &rows, &cols)) return dtas_config{DTAS_GEMM_SHARE, 256, 8, 1, {rows, cols, 0}, 1, 0};
+  dtas_config cfg;
+  if (M > 128 && vec_ok && tile8_policy(M, N, K, may_split, false, &cfg)) return cfg;
   return builtin_config(DTAS_OP_GEMM_F16, M, N, K).cfg;
 }
 
@@ -297,7 +418,7 @@ extern "C" int dtas_builtin_gemm(int weights_8bit, int64_t M, int64_t N, int64_t
     what = "decode_q8 + gemm";
   }
   snprintf(out->name, sizeof(out->name), "%s", what);
-  out->config = builtin_gemm(M, N, K, K % 8 == 0);
+  out->config = builtin_gemm(M, N, K, K % 8 == 0, true);
   if (K % 8 != 0) out->config.vec = 1;
   return describe_gemm(M, N, K, out->config, out->launch_args);
 }
@@ -344,7 +465,13 @@ extern "C" int dtas_gemm_f16_fused(const void* A, const void* W, const void* bia
   const GemmEpilogue ep = {static_cast<const half_t*>(bias), static_cast<const half_t*>(res1),
                            static_cast<const half_t*>(res2), epilogue, out_bytes == 4 ? 1 : 0, 0.f, 0, 0, 0, 0};
   const bool vec_ok = K % 8 == 0 && aligned(A, 16) && aligned(W, 16);
-  dtas_config cfg = user ? *user : builtin_gemm(M, N, K, vec_ok);
+  dtas_config cfg = user ? *user : builtin_gemm(M, N, K, vec_ok, true);
+  // a first call under capture cannot allocate the workspace: whole tiles then
+  if (!user && M > 128 && vec_ok && cfg.split_k > 1) {
+    const size_t tiles = static_cast<size_t>(ceil_div(M, cfg.tile[0]) * ceil_div(N, cfg.tile[1]));
+    if (!split_scratch_at_hand(static_cast<hipStream_t>(stream), tiles * cfg.split_k * cfg.tile[0] * cfg.tile[1] * 4, tiles))
+      cfg = builtin_gemm(M, N, K, vec_ok, false);
+  }
   if (cfg.vec == 8 && !vec_ok) cfg.vec = 1;  // K % 8 != 0 or odd pointers: element accesses
   int64_t la[7];
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;

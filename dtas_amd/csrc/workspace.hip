@@ -170,6 +170,22 @@ int split_scratch(hipStream_t s, size_t bytes, size_t split_tiles, int nsplit, f
   return split_workspace(s, bytes, split_tiles, partials, arrivals);
 }
 
+// Whether split_scratch would find room without allocating, or may allocate: false only while `s` is being captured.
+bool split_scratch_at_hand(hipStream_t s, size_t bytes, size_t split_tiles) {
+  if (t_fixed_scratch) return true;
+  std::lock_guard<std::recursive_mutex> lock(g_ws_mutex);
+  int dev = 0;
+  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices)
+    for (const StreamWorkspace& w : g_ws[dev].slot)
+      if (w.used && w.stream == s && w.partial_bytes >= bytes && w.tiles >= split_tiles) return true;
+  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {  // (the default stream, while another one is captured: as before, the allocation says)
+    (void)hipGetLastError();
+    return true;
+  }
+  return capturing == hipStreamCaptureStatusNone;
+}
+
 // The device address of the static scratch array on the current device.  hipGetSymbolAddress is asked once per
 // device, with that device current (each GPU holds its own copy of the array at its own address).
 int resolve_static_scratch(void** out) {

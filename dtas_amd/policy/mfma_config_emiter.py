@@ -5,7 +5,7 @@ enumerate block tiles as i x j wavefronts of micro_x x micro_y matrix-core block
 those that do not fit shared memory / registers (:46-70) and rank by a roofline estimate in which a
 tile's throughput is min(matrix-core peak, bandwidth * flops-per-byte of the tile) and the job costs
 ceil(tiles / SMs) rounds (:148-262).  The candidate set is what libdtas_gfx950.so has kernels for:
-MFMA tiles from 64x64 to 256x256 (16x16x32 on the largest, 32x32x16 below) with 2 to 4 LDS stages, with K split over up to 4 workgroups
+MFMA tiles from 64x64 to 256x256 (16x16x32 on 8 wavefronts, 32x32x16 on 4) with 2 to 4 LDS stages, with K split over up to 4 workgroups
 per tile when M x N yields few tiles, plus, for M <= 64, the weight-streaming 16x16x32 kernel whose
 wavefronts split K.  The order is the one on-GPU sweeps favoured;
 with a GPU present the Engine times the top-k anyway.
@@ -15,13 +15,36 @@ from typing import List, Tuple
 from ..common.config import MFMAConfig, Range
 from .base_config_emiter import BaseConfigEmiter
 
-# (micro_x, micro_y) per wavefront of the 2x2-wavefront kernels (the 256x256 tile runs 2x4 wavefronts)
-_TILES = [(4, 4), (3, 4), (4, 2), (3, 2), (2, 4), (2, 2), (1, 2), (2, 1), (1, 1)]
+# (micro_x, micro_y) per wavefront of the 2x2-wavefront kernels
+_TILES = [(4, 2), (2, 4), (2, 2), (1, 2), (2, 1), (1, 1)]
+# the 8-wavefront kernels: tile -> (wavefronts along M, along N)
+_TILES8 = {(256, 256): (2, 4), (224, 256): (2, 4), (192, 256): (2, 4), (160, 256): (2, 4), (128, 256): (2, 4), (96, 256): (2, 4),
+           (256, 128): (4, 2), (224, 128): (2, 4), (192, 128): (4, 2), (160, 128): (2, 4), (128, 128): (4, 2), (96, 128): (2, 4), (128, 64): (4, 2)}
+# the library's cost model beyond 128 rows (libdtas: kTile8Cost): tile, threads, stages, whether the table's rows name it, and
+# a, b, w, r, h0, h1, h2, pitch, few, pad
+_COST8 = [
+    (64, 64, 256, 4, True, 3.74, 0.243, 0.42, 0.71, 1, 1, 0.3, 1.03, 0.8, 0.16),
+    (128, 64, 512, 0, True, 4.02, 0.326, 0, 0.69, 3.14, 0.57, 0.51, 1.08, 0.65, 0.71),
+    (96, 128, 512, 0, False, 3.9, 0.435, 0, 0.68, 2.66, 0.96, 1.87, 1.12, 0.8, 0.53),
+    (128, 128, 512, 0, True, 4.06, 0.501, 0.21, 0.62, 2.59, 1.2, 2.98, 1.11, 0.8, 0.74),
+    (160, 128, 512, 0, False, 4.58, 0.599, 0, 0.64, 2.97, 1.41, 3.14, 1.1, 0.54, 0.71),
+    (192, 128, 512, 0, True, 4.52, 0.673, 0.49, 0.65, 2.68, 1.81, 3.93, 1.08, 0.46, 0.66),
+    (224, 128, 512, 0, False, 4.2, 0.755, 1.33, 0.63, 2.51, 2.3, 2.67, 1.06, 0.36, 0.59),
+    (256, 128, 512, 0, True, 4.1, 0.827, 1.96, 0.66, 2.03, 2.65, 3.96, 1.06, 0.26, 0.52),
+    (96, 256, 512, 0, False, 3.85, 0.717, 0.83, 0.7, 3.49, 1.73, 2.44, 1.16, 0.8, 0.16),
+    (128, 256, 512, 0, False, 3.71, 0.835, 2.06, 0.66, 3.25, 2.39, 3.21, 1.15, 0.71, 0.48),
+    (160, 256, 512, 0, False, 5.21, 1.02, 0.65, 0.57, 2.21, 3.07, 3.96, 1.11, 0.49, 0.48),
+    (192, 256, 512, 0, True, 5.19, 1.152, 2.05, 0.59, 2.39, 3.56, 3.96, 1.11, 0.37, 0.33),
+    (224, 256, 512, 0, False, 5.85, 1.317, 1.9, 0.56, 1.66, 4.2, 4.84, 1.05, 0.3, 0.36),
+    (256, 256, 512, 2, True, 6.98, 1.505, 0.41, 0.48, -4, 5.88, 5, 1.02, 0.28, 0.34),
+]
 _LDS = 160 * 1024
 
 
 class MFMAConfigEmiter(BaseConfigEmiter):
     def check_valid(self, c: MFMAConfig) -> bool:
+        if c.block_threads == 512:   # the 8-wavefront kernels are built to fit
+            return (c.tile_size_m, c.tile_size_n) in _TILES8
         stages = c.stages or 2
         lds = stages * (c.tile_size_m + c.tile_size_n) * c.tile_size_k * 2  # fp16 stages of the load pipeline
         acc = c.micro_shape_x * c.micro_shape_y * 16                         # fp32 accumulators per lane
@@ -29,11 +52,57 @@ class MFMAConfigEmiter(BaseConfigEmiter):
 
     @staticmethod
     def max_stages(tile_m: int, tile_n: int) -> int:
-        return 2 if tile_m + tile_n >= 512 or tile_m == 192 else 3 if tile_m + tile_n >= 384 else 4
+        return 2 if tile_m + tile_n >= 512 else 3 if tile_m + tile_n >= 384 else 4
+
+    def tile8_policy(self, M: int, N: int, K: int):
+        """(tile_m, tile_n, stages, split_k, threads) of the table's row beyond 128 rows: the cost model of the library's
+        tile8_policy, over the tiles and splits the table's rows name (a host test keeps the two alike)."""
+        cdiv = lambda a, b: -(-a // b)
+        cus, ktiles = self.arch.num_sm, cdiv(K, 64)
+        odd_pitch = K % 1024 == 0 and (K // 1024) & (K // 1024 - 1) != 0
+        best_us, best = 1e300, None
+        for bm, bn, threads, stages, in_table, a, b0, w, r, h0, h1, h2, pitch, few, pad in _COST8:
+            if not in_table or K * 2 * max(bm, bn) >= 1 << 31:
+                continue
+            tm = cdiv(M, bm)
+            tiles = tm * cdiv(N, bn)
+            if tiles > 0x7fffffff // 8:
+                continue
+            whole_rounds = bm == 256 and bn == 256
+            slots = 2 * cus if bm * bn <= 64 * 64 else cus
+            b = b0 * (pitch if odd_pitch else 1.0) * (1.0 + few / float(tm) - pad * (1.0 - float(M) / float(tm * bm)))
+            for parts in range(1, 5):
+                last_parts = parts
+                if whole_rounds:
+                    last_parts, _ = self.tail_split_256(M, N, K)
+                elif parts > 1 and (tiles * parts > slots or ktiles // parts < 8 or tiles * parts * bm * bn * 4 > 32 << 20):
+                    break
+                tail = whole_rounds and last_parts > 1
+                wgs = tiles if whole_rounds else tiles * parts
+                full, rem = divmod(wgs, slots)
+                steps = float(ktiles if whole_rounds else cdiv(ktiles, parts))
+                share = float(wgs) / cus
+                us = float(full) * (a + b * steps) + w * share
+                fill = float(rem * last_parts if whole_rounds else rem) / float(slots)
+                if slots > cus:     # (64x64: two or more workgroups share a CU)
+                    us = a + b * steps * (r + (1.0 - r) * share if wgs <= cus else 0.75 * float(cdiv(wgs, cus))) + w * share
+                elif rem > 0:
+                    us += a + b * (float(cdiv(ktiles, last_parts)) if whole_rounds else steps) * (r + (1.0 - r) * fill)
+                if last_parts > 1:
+                    crowd = fill if whole_rounds else share
+                    us += h0 + h1 * last_parts + h2 * crowd * crowd * crowd * crowd
+                if us < best_us:
+                    best_us, best = us, (bm, bn, stages, 0 if tail else parts, threads)
+                if whole_rounds:
+                    break
+        if best and best[:2] == (192, 256) and best[3] == 1 and K % 2048 == 0:
+            best = (192, 256, 2, 1, 512)
+        self._model_us = best_us
+        return best
 
     def preferred(self, m_hi: int, N: int, K: int = 4096):
-        """(tile_m, tile_n, stages, split_k) under the cost model fitted to sweeps on an MI355X (the same
-        one the library's built-in table uses): time = rounds of workgroups over the chip x time of one
+        """(tile_m, tile_n, stages, split_k, threads) under the cost models fitted to sweeps on an MI355X (the same
+        ones the library's built-in table uses).  Beyond 128 rows: tile8_policy.  Up to 128 rows: time = rounds of workgroups over the chip x time of one
         k tile x k tiles.  One k tile with every CU busy: 256x256 see below, 256x128 (8 wavefronts of 64x64) 1.00 us,
         128x128 0.665 us (4 stages, one workgroup per CU) or 1.14 us per round of two per CU (2 stages);
         a partly filled last round costs 0.55 + 0.45 * fill of a full one (0.8 + 0.2 * fill for 128x128 with 4 stages
@@ -45,6 +114,10 @@ class MFMAConfigEmiter(BaseConfigEmiter):
         more (~4.5 us per partial tile: 512 x 5120 x 13824 in 3 parts 86.8 us against 98.2 for 256x256, 640 x 4096 x 8192 in 2 parts
         63.8 against 67.3).  No candidate is faster than W (2NK bytes) streams through it: 3.1 .. 4.3 TB/s
         by tile, measured with 64 rows against a 50280 x 2560 W."""
+        if m_hi > 128:
+            wide = self.tile8_policy(m_hi, N, K)
+            if wide:
+                return wide
         cdiv = lambda a, b: -(-a // b)
         cus = self.arch.num_sm
         ktiles = cdiv(K, 64)
@@ -103,7 +176,8 @@ class MFMAConfigEmiter(BaseConfigEmiter):
             if c[0] < best[0]:
                 best = c
         self._model_us = best[0]
-        return best[1]
+        tm, tn, stages, split = best[1]
+        return tm, tn, stages, split, 512 if stages == 2 and (tm, tn) in ((256, 256), (192, 256), (256, 128), (192, 128)) else 256
 
     def tail_split_256(self, M: int, N: int, K: int):
         """(parts, tiles left whole) for split_k = 0 on the 8-wavefront 256x256 tile: whole rounds of the chip
@@ -214,40 +288,39 @@ class MFMAConfigEmiter(BaseConfigEmiter):
                 out.append(c)
         pref = self.preferred(m_hi, N, K)
         scored = []
+        shapes: List[MFMAConfig] = []
+        for (tm, tn), (wm, wn) in _TILES8.items():
+            # stages 0: what the LDS holds; 2: the ring of the largest tile, which 192x256 comes with too
+            for st in ((2,) if (tm, tn) == (256, 256) else (0, 2) if (tm, tn) == (192, 256) else (0,)):
+                c = MFMAConfig()
+                c.i, c.j, c.micro_shape_x, c.micro_shape_y, c.micro_shape_k = wm, wn, tm // wm // 16, tn // wn // 16, 2
+                c.mfma_m, c.mfma_n, c.mfma_k, c.block_threads, c.stages = 16, 16, 32, 512, st
+                shapes.append(c)
         for mx, my in _TILES:
             base = MFMAConfig()
             base.micro_shape_x, base.micro_shape_y = mx, my
-            tm, tn = base.tile_size_m, base.tile_size_n
-            for stages in range(2, self.max_stages(tm, tn) + 1):
+            for stages in range(2, self.max_stages(base.tile_size_m, base.tile_size_n) + 1):
                 c = MFMAConfig()
                 c.micro_shape_x, c.micro_shape_y, c.stages = mx, my, stages
-                if (mx, my) == (4, 4):
-                    # the 256x256 kernel runs 2x4 wavefronts of 128x64 (two per SIMD)
-                    c.i, c.j, c.micro_shape_x, c.micro_shape_y, c.block_threads = 2, 4, 4, 2, 512
-                if (mx, my) == (3, 4):
-                    # 192x256: 2x4 wavefronts of 96x64 on the same ring loop
-                    c.i, c.j, c.micro_shape_x, c.micro_shape_y, c.block_threads = 2, 4, 3, 2, 512
-                if (mx, my) == (3, 2):
-                    # 192x128: 4x2 wavefronts of 48x64 (16x16x32 blocks) on the ring loop; the vocabulary's 32-wide micro
-                    # blocks do not express 48 rows, so the 2x2 shape stands for the tile's extents
-                    c.block_threads = 512
-                if (mx, my) == (4, 2) and stages == 2:
-                    # 256x128 with two "stages": 4x2 wavefronts of 64x64 on the ring loop of the 256x256 kernel
-                    c.i, c.j, c.micro_shape_x, c.micro_shape_y, c.block_threads = 4, 2, 2, 2, 512
-                if not self.check_valid(c):
-                    continue
-                tiles = -(-m_hi // tm) * -(-N // tn)
-                c.num_wave = -(-tiles // self.arch.num_sm)
-                splits = [1] + [sk for sk in (2, 3, 4) if tiles * sk <= 4 * self.arch.num_sm and -(-K // 64) // sk >= 8]
-                if c.block_threads == 512 and (tm, tn) == (256, 256):
-                    splits = [0] + splits   # 0: only the tiles of a partly filled last round are split
-                for sk in splits:
-                    cs = MFMAConfig().from_dict(c.to_dict())
-                    cs.split_k, cs.num_wave = sk, -(-tiles * sk // self.arch.num_sm)
-                    # rank: the measured preference first, then by distance in tile area, split and stage count
-                    rank = (0 if (tm, tn, stages, sk) == pref else 1, abs(tm * tn - pref[0] * pref[1]),
-                            abs(sk - pref[3]), abs(stages - pref[2]))
-                    scored.append((rank, cs))
+                shapes.append(c)
+        for c in shapes:
+            tm, tn, stages = c.tile_size_m, c.tile_size_n, c.stages
+            if not self.check_valid(c):
+                continue
+            tiles = -(-m_hi // tm) * -(-N // tn)
+            c.num_wave = -(-tiles // self.arch.num_sm)
+            splits = [1] + [sk for sk in (2, 3, 4) if tiles * sk <= 4 * self.arch.num_sm and -(-K // 64) // sk >= 8]
+            if c.block_threads == 512 and (tm, tn) == (256, 256):
+                splits = [0] + splits   # 0: only the tiles of a partly filled last round are split
+            for sk in splits:
+                cs = MFMAConfig().from_dict(c.to_dict())
+                cs.split_k, cs.num_wave = sk, -(-tiles * sk // self.arch.num_sm)
+                # rank: the measured preference first, then by distance in tile area, split and stage count
+                first = (tm, tn, sk, c.block_threads) == (pref[0], pref[1], pref[3], pref[4]) and \
+                    (stages == pref[2] or (c.block_threads == 512 and (tm, tn) != (192, 256)))
+                rank = (0 if first else 1, abs(tm * tn - pref[0] * pref[1]),
+                        abs(sk - pref[3]), abs(stages - pref[2]), abs(c.block_threads - pref[4]))
+                scored.append((rank, cs))
         mfma = [c for _, c in sorted(scored, key=lambda t: t[0])]
         # the W-streaming kernel leads only where it beats the best MFMA candidate under the model
         out = (out + mfma) if self.prefers_skinny(m_hi, N, K) else (mfma[:1] + out + mfma[1:])

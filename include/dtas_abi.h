@@ -97,11 +97,11 @@ enum dtas_variant {
                              (experiment/testIR/GEMV/m1n2560k10240/IR/5wt.py:11-92): for results bit-identical to
                              that kernel's arithmetic; block 256 (8 rows per workgroup), vec 8 or 1 */
   /* GEMM (python/dtas/schedule/tir_wmma.py:20-222) */
-  DTAS_GEMM_MFMA = 0,     /* LDS-tiled MFMA, tile = tile[0] x tile[1] x 64 with tile[0], tile[1] in {64, 128, 256}
-                             (64x256 and 256x64 excepted); block 256 (4 wavefronts), or 512 (8 wavefronts, 16x16x32
-                             MFMA, a ring of five operand units instead of `unroll` stages) for 256x256, 256x128
-                             and 128x256; 256x256 takes either.  192x256 and 192x128 exist with block 512 and
-                             unroll 2 only */
+  DTAS_GEMM_MFMA = 0,     /* LDS-tiled MFMA, tile = tile[0] x tile[1] x 64.  block 256 (4 wavefronts): tile[0], tile[1] in
+                             {64, 128, 256} (64x256 and 256x64 excepted) on `unroll` stages.  block 512 (8 wavefronts,
+                             16x16x32 MFMA): 256x256 on a ring of five operand units; {96, 128, 160, 192, 224} x 256,
+                             {96, 128, 160, 192, 224, 256} x 128 and 128x64 on as many stages as the LDS holds (unroll 0),
+                             {128, 192} x 256 and {192, 256} x 128 also on the ring (unroll 2) */
   DTAS_GEMM_SKINNY = 1,   /* small M: weight-streaming MFMA 16x16x32, split over N and K */
   DTAS_GEMM_ROWS = 2,     /* M <= 4: W streamed once in whole rows (tile[1] per wavefront) against tile[0] >= M
                              rows of A on the vector ALU; tile = {2|4, 1|2|4, 8}, block 64 / 128 / 256 */

@@ -1,0 +1,128 @@
+"""GPU parity of the 8-wavefront GEMM tiles: every tile and stage count on sizes at its edges, whole and with K in parts, with
+every epilogue; and what a call of more than 128 rows without a config runs."""
+import numpy as np
+import pytest
+import torch
+
+from dtas_amd import _lib, ops
+from gpu_util import Guarded, assert_bits_equal, cfg, dev
+
+RTOL, ATOL = 1e-2, 2e-3
+# (rows, columns, k tiles of W that the LDS holds; 2: the ring of five operand units)
+TILES = [(128, 64, 4), (96, 128, 4), (128, 128, 4), (160, 128, 4), (192, 128, 4), (224, 128, 3), (256, 128, 3), (96, 256, 3), (128, 256, 3),
+         (160, 256, 3), (192, 256, 3), (192, 256, 2), (224, 256, 3), (256, 256, 2)]
+
+
+def _check(got, oracle_out, f64):
+    got = got.astype(np.float64)
+    assert np.isfinite(got).all()
+    assert (np.abs(got - f64) <= ATOL + RTOL * np.abs(f64)).all()
+    # against the oracle (same fp32 arithmetic, another summation order): about one fp16 ulp
+    want = oracle_out.astype(np.float64)
+    assert (np.abs(got - want) <= 1e-3 + 2.0 ** -9 * np.abs(want)).all()
+
+
+def _inputs(M, N, K, seed):
+    rng = np.random.default_rng(seed)
+    return (rng.standard_normal((M, K)).astype(np.float16), (rng.standard_normal((N, K)) * 0.02).astype(np.float16),
+            rng.uniform(-1, 1, N).astype(np.float16))
+
+
+def _cfg(bm, bn, stages, split=1):
+    return cfg(variant=_lib.GEMM_MFMA, block=512, vec=8, unroll=2 if stages == 2 else 0, tile=[bm, bn, 64], split_k=split)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn,stages", TILES)
+def test_every_tile_at_its_edges(oracle, bm, bn, stages):
+    # one row and column either side of whole tiles; one k tile, as many as there are stages and a chunk more, and one fewer
+    for M, N, K, split in ((3, 5, 8, 1), (bm - 1, bn + 1, 64, 1), (bm + 1, 2 * bn - 1, 64 * stages + 8, 1), (2 * bm, bn, 64 * (stages + 1), 1),
+                           (bm + 33, bn + 8, 64 * (stages - 1) - 8, 1), (bm + 7, bn + 9, 1096, 3), (2 * bm - 5, bn, 2048, 6)):
+        a, w, bias = _inputs(M, N, K, M + N + K)
+        out = Guarded((M, N), torch.float16)
+        ops.gemm(dev(a), dev(w), dev(bias), out.t, _cfg(bm, bn, stages, split))
+        _check(out.check(), oracle.c.gemm(a, w, bias, threads=8), oracle.np64.gemm(a, w, bias))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn,stages", TILES)
+@pytest.mark.parametrize("epilogue", [_lib.EPI_BIAS_ADD2, _lib.EPI_BIAS_ADD2_CAST_F32, _lib.EPI_BIAS_GELU])
+def test_every_epilogue_of_every_tile(bm, bn, stages, epilogue):
+    # the epilogues act on the product rounded to fp16: the same bits as on 64x64 tiles, whose k order is the same
+    M, N, K = bm + 5, bn + 12, 200
+    a, w, bias = (dev(x) for x in _inputs(M, N, K, bm + bn))
+    g = torch.Generator(device="cuda").manual_seed(1)
+    res = [torch.randn(M, N, device="cuda", generator=g).half() for _ in range(2)] if epilogue != _lib.EPI_BIAS_GELU else [None, None]
+    plain = cfg(variant=_lib.GEMM_MFMA, block=256, vec=8, unroll=2, tile=[64, 64, 64])
+    mm, mm8 = (torch.empty(M, N, dtype=torch.float16, device="cuda") for _ in range(2))
+    ops.gemm(a, w, None, mm, plain)
+    ops.gemm(a, w, None, mm8, _cfg(bm, bn, stages))
+    same = mm == mm8    # (16x16x32 and 32x32x16 products are added in another order: a last bit may differ)
+    assert float(same.float().mean()) > 0.98
+    outs = []
+    for c in (plain, _cfg(bm, bn, stages)):
+        out = Guarded((M, N), torch.float32 if epilogue == _lib.EPI_BIAS_ADD2_CAST_F32 else torch.float16)
+        ops.gemm(a, w, bias, out.t, c, epilogue=epilogue, res1=res[0], res2=res[1])
+        outs.append(out.check())
+    keep = same.cpu().numpy()
+    assert_bits_equal(outs[0][keep], outs[1][keep])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(129, 4096, 1024), (203, 2560, 2560), (300, 520, 4096), (385, 7680, 520), (600, 1000, 264), (1025, 2560, 2560),
+                                   (1150, 100, 72), (200, 7, 8), (700, 2048, 10240), (897, 2560, 2048)])
+def test_what_runs_without_a_config(oracle, M, N, K):
+    a, w, bias = _inputs(M, N, K, M + N + K)
+    out = Guarded((M, N), torch.float16)
+    ops.gemm(dev(a), dev(w), dev(bias), out.t)
+    got = out.check()
+    named = Guarded((M, N), torch.float16)
+    ops.gemm(dev(a), dev(w), dev(bias), named.t, _lib.builtin_gemm(M, N, K).config)
+    assert_bits_equal(got, named.check())
+    rows = np.linspace(0, M - 1, min(M, 64)).astype(int)
+    _check(got[rows], oracle.c.gemm(a[rows], w, bias, threads=8), oracle.np64.gemm(a[rows], w, bias))
+
+
+@pytest.mark.gpu
+def test_a_first_call_under_capture_splits_nothing():
+    # a stream without a workspace that is being captured: whole tiles instead of an allocation
+    M, N, K = 200, 2560, 10240
+    assert _lib.builtin_gemm(M, N, K).config.split_k > 1
+    a, w, _ = (dev(x) for x in _inputs(M, N, K, 1))
+    eager, out = (torch.zeros(M, N, dtype=torch.float16, device="cuda") for _ in range(2))
+    ops.gemm(a, w, None, eager)
+    stream = torch.cuda.Stream()
+    graph = torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.gemm(a, w, None, out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        assert float((out.float() - eager.float()).abs().max()) <= 2.0 ** -9 * float(eager.float().abs().max())
+        ops.gemm(a, w, None, eager)
+
+
+def test_every_tile_describes_its_launch_and_nothing_else_is_taken():
+    for bm, bn, stages in TILES:
+        info = _lib.describe_launch(_lib.OP_GEMM_F16, 1000, 3000, 4096, _lib.DtasConfig.from_dict(
+            {"variant": _lib.GEMM_MFMA, "block": 512, "vec": 8, "unroll": 2 if stages == 2 else 0, "tile": [bm, bn, 64], "split_k": 1}))
+        assert list(info.launch_args)[:4] == [-(-1000 // bm) * -(-3000 // bn), 1, 1, 512] and info.launch_args[4] <= 160 * 1024
+    for bm, bn, block, stages in ((96, 128, 256, 4), (160, 256, 256, 3), (64, 128, 512, 2), (64, 64, 512, 2), (96, 64, 512, 4), (320, 128, 512, 2), (96, 128, 512, 5)):
+        with pytest.raises(_lib.DtasError):
+            _lib.describe_launch(_lib.OP_GEMM_F16, 1000, 3000, 4096, _lib.DtasConfig.from_dict(
+                {"variant": _lib.GEMM_MFMA, "block": block, "vec": 8, "unroll": stages, "tile": [bm, bn, 64], "split_k": 1}))
+
+
+@pytest.mark.parametrize("seed", range(4))
+def test_a_call_without_a_config_names_a_launchable_kernel(seed):
+    # partial tiles never outgrow the room that a caller who cannot allocate has, as in the rows before
+    rng = np.random.default_rng(seed)
+    for _ in range(500):
+        M, N, K = int(rng.integers(129, 8192)), int(2 ** rng.uniform(0, 17)), 8 * int(2 ** rng.uniform(0, 11))
+        info = _lib.builtin_gemm(M, N, K)
+        c = info.config
+        assert list(_lib.describe_launch(_lib.OP_GEMM_F16, M, N, K, c).launch_args) == list(info.launch_args), (M, N, K)
+        if c.split_k > 1:
+            assert info.launch_args[0] * c.tile[0] * c.tile[1] * 4 <= 32 << 20 and -(-K // 64) // c.split_k >= 6, (M, N, K)
