@@ -7,9 +7,59 @@
 #include "gemm_tile_kernel.h"
 
 namespace dtas {
+namespace {
+// The tiles that dequantise in their W path, by the estimate of tile8_policy (the 4-wavefront tiles, of which a CU holds several:
+// at r + (1 - r) x share of the chip up to one workgroup per CU, and at 0.75 (64x64) or 0.85 (128x64) per workgroup of the fullest
+// CU beyond).  Fitted to 300 sizes (65 .. 2048 rows against fourteen W of 2048 x 768 .. 14336 x 4096, W from memory) x up to 30 configurations:
+// 1.003 of the best one's time at 100 .. 1100 rows, 0.85 .. 0.91 of the time of the 4-wavefront tiles that ran before (203 x 10240 x 2560
+// 34.7 -> 28.0 us, 512 x 7680 x 2560 36.4 -> 30.3, 700 x 2560 x 10240 71.5 -> 55.4); h0 of the 8-wavefront tiles 1.5 us above the fit, as there.
+struct TileQ8Cost {
+  int bm, bn, block, stages;
+  double a, b, w, r, h0, h1, h2, pitch, few, pad;
+};
+constexpr TileQ8Cost kTileQ8Cost[] = {
+    {64, 64, 256, 3, 4.53, 0.333, 0, 0.96, 0.85, 0.53, 0.04, 1, 0.48, 0.14},
+    {128, 64, 256, 3, 4.69, 0.474, 0.19, 0.86, 1.23, 0.67, 0.46, 1.02, 0.11, 0.05},
+    {96, 128, 512, 0, 4.72, 0.508, 0.35, 0.8, 2.45, 0.89, 0.55, 1.02, 0.37, 0.11},
+    {128, 128, 512, 0, 4.3, 0.57, 0.64, 0.75, 2.76, 1.15, 0.91, 1.01, 0.3, 0.17},
+    {160, 128, 512, 0, 3.74, 0.689, 1.35, 0.83, 2.92, 1.46, 1.13, 1.02, 0.15, 0.12},
+    {192, 128, 512, 0, 4.9, 0.789, 0, 0.73, 2.73, 1.87, 1.5, 1.01, 0.09, 0.15},
+    {256, 128, 512, 0, 4.95, 1.015, 0, 0.71, 2.92, 2.41, 1.98, 0.99, 0, 0.14},
+};
+double tile_q8_policy(int64_t M, int64_t N, int64_t K, bool may_split, dtas_config* out) {
+  const int64_t ktiles = ceil_div(K, kBK);
+  const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
+  double best = 1e300;
+  for (const TileQ8Cost& c : kTileQ8Cost) {
+    const int64_t tm = ceil_div(M, c.bm), tn = ceil_div(N, c.bn), tiles = tm * tn, limit = c.block == 256 ? 2 * kNumCU : kNumCU;
+    if (tiles > 0x7fffffff / 8) continue;
+    const double b = c.b * (odd_pitch ? c.pitch : 1.0) *
+                     (1.0 + c.few / static_cast<double>(tm) - c.pad * (1.0 - static_cast<double>(M) / static_cast<double>(tm * c.bm)));
+    for (int parts = 1; parts <= 8; ++parts) {
+      // (K <= 768: a launch is mostly its start, and a hand-over costs what the shorter loop saves: 128 x 2048 x 768 8.6 us whole, 11.3 in three)
+      if (parts > 1 && (!may_split || ktiles <= 12 || tiles * parts > limit || ktiles / parts < (c.block == 256 ? 4 : 6) ||
+                        tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) break;
+      const int64_t wgs = tiles * parts, full = wgs / kNumCU, rem = wgs % kNumCU;
+      const double steps = static_cast<double>(ceil_div(ktiles, parts)), share = static_cast<double>(wgs) / kNumCU;
+      double us = c.w * share;
+      if (c.block == 256)
+        us += c.a + b * steps * (wgs <= kNumCU ? c.r + (1.0 - c.r) * share : (c.bm == 64 ? 0.75 : 0.85) * static_cast<double>(ceil_div(wgs, kNumCU)));
+      else
+        us += static_cast<double>(full) * (c.a + b * steps) + (rem > 0 ? c.a + b * steps * (c.r + (1.0 - c.r) * static_cast<double>(rem) / kNumCU) : 0.0);
+      if (parts > 1) us += c.h0 + c.h1 * parts + c.h2 * share * share * share * share;
+      if (us < best) {
+        best = us;
+        *out = dtas_config{DTAS_GEMM_MFMA, c.block, 8, c.stages, {c.bm, c.bn, kBK}, parts, 0};
+      }
+    }
+  }
+  return best;
+}
+}  // namespace
+
 // What a call without a config runs; false: the dequantiser into a library-owned buffer, then the fp16 GEMM.  stream_ok: the
-// kernels that stream the bytes of W can take the call (16-byte aligned operands, K % 256 == 0, K < 2^24).
-bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, dtas_config* out) {
+// kernels that stream the bytes of W can take the call (16-byte aligned operands, K % 256 == 0, K < 2^24); vec_ok: the tiles can.
+bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_ok, bool may_split, dtas_config* out) {
   dtas_config& cfg = *out;
   // Few rows of A: the launch is one read of the bytes of W.
   // up to 96 rows: every CU an equal share of W's rows, nothing handed over (share_leads_q8)
@@ -33,44 +83,18 @@ bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, dtas_confi
     cfg = dtas_config{DTAS_GEMM_STREAM, 256, 8, 1, {64, 64, 512}, 1, 0};
     return true;
   }
-  // Two routes.  (1) Dequantising in the W path of the tile kernel: no intermediate, W read once per row of tiles as
-  // bytes; a plain burst pipeline on 4 wavefronts, with K split over workgroups while the tiles leave CUs idle.
-  // (2) The dequantiser into a library-owned fp16 buffer, then the fp16 GEMM with everything its table offers: 3 more
-  // bytes per weight through memory (9-14 us at the model's shapes), worth it once the GEMM itself is long.
-  // Measured at the model's shapes with rotating weights, us, route 1 (tile, K parts) / route 2 / the fp16 GEMM on
-  // fp16 weights: 7680x2560, M = 64 / 128 / 256 / 512 / 1024: 16.4 (64x64, 4) / 28.0 / 14.3, 21.9 (64x64, 3) / 29.6 /
-  // 17.7, 26.8 (128x128, 2) / 33.6 / 25.3, 38.6 (128x128, 1) / 41.4 / 33.4, 58.8 / 52.6 / 43.3; 10240x2560, M = 64 / 128 /
-  // 256 / 512: 19.5 / 29.9 / 18.7, 24.2 (128x128, 3) / 34.7 / 26.0, 35.1 / 40.5 / 33.3, 56.4 / 48.8 / 39.6; 2560x10240,
-  // M = 64 / 256 / 512 / 1024: 25.7 (64x64, 8) / 34.0 / 22.6, 37.4 (128x128, 6) / 44.1 / 38.5, 52.9 / 57.3 / 50.0, 87.9 /
-  // 76.0 / 66.8.  So route 1 up to 512 rows while 128x128 tiles fit the chip in one round; 64x64 tiles (two stages, ~2
-  // workgroups per CU wanted) up to 128 rows unless they already number more than the CUs, 128x128 (three stages, one
-  // per CU) beyond; K parts to fill the chip, each at least 4 k tiles.  A cfg selects route 1 with its own tile and split.
-  const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128), t64 = ceil_div(M, 64) * ceil_div(N, 64), ktiles = ceil_div(K, kBK);
-  if (M > 512 || t128 > kNumCU) return false;
-  // three tiles of three stages -- 64x64 (three workgroups per CU), 128x64 (two), 128x128 (one) -- with K in 1 .. 8 parts of
-  // 4 k tiles or more: us = start + (k tiles per part) x (cost of one, growing with the workgroups on the chip) + a
-  // hand-over per part, fitted to a sweep of the model's shapes at M = 96 .. 512 with the weights streamed from memory
-  // (2560 x 2560, M = 256: 64x64 in 3 parts 15.4 us, 22 before; 10240 x 2560, M = 192: 64x64 28.3, 34 before; within 10 % of
-  // the best of 36 configurations on the sweep's 24 shapes, 3 % on average)
-  const int64_t t12864 = ceil_div(M, 128) * ceil_div(N, 64);
-  // (rows 5, 6, 10, ... KiB of fp16 apart: a loaded chip takes a k tile of the 128x64 tile 20-25 % longer -- 2560 x 10240,
-  // M = 512 in 3 parts: 58.6 us where the fit without it says 47.6, 128x128 53.6)
-  const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
-  double best = 1e30;
+  // Two routes.  (1) Dequantising in the W path of the tile kernel: no intermediate, W read once per row of tiles as bytes.
+  // (2) The dequantiser into a library-owned fp16 buffer, then the fp16 GEMM with every tile it has: ~5 us and 3 more bytes per
+  // weight through memory, worth it once the GEMM itself is long (7680 x 2560: from ~1300 rows, 10240 x 2560 ~900).  Its time
+  // against the fit's 300 sizes: 5.3 us + 0.415 per million weights + 0.907 of the fp16 GEMM's estimate (W comes from the cache); the
+  // lesser of the two estimates is the lesser time to 0.1 %.
   cfg = dtas_config{DTAS_GEMM_MFMA, 256, 8, 3, {128, 128, kBK}, 1, 0};
-  for (int parts = 1; parts <= 8; ++parts) {
-    if (parts > 1 && ktiles / parts < 4) break;
-    const double steps = static_cast<double>(ceil_div(ktiles, parts));
-    const double w64 = static_cast<double>(t64 * parts), w12864 = static_cast<double>(t12864 * parts), w128 = static_cast<double>(t128 * parts);
-    const double us64 = w64 <= 512 ? 4.4 + (0.30 + 0.26 * w64 / 480.0) * steps + 1.33 * (parts - 1) : 1e30;
-    const double b12864 = 0.18 + 0.69 * (odd_pitch ? 1.35 : 1.0) * w12864 / 480.0;
-    const double us12864 = w12864 <= 512 ? 8.4 + (b12864 < 0.44 ? 0.44 : b12864) * steps + 1.5 * (parts - 1) : 1e30;
-    const double us128 = w128 <= kNumCU ? 9.2 + (0.373 + 0.45 * w128 / 480.0) * steps + 1.87 * (parts - 1) : 1e30;
-    if (us64 < best) best = us64, cfg.tile[0] = 64, cfg.tile[1] = 64, cfg.split_k = parts;
-    if (us12864 < best) best = us12864, cfg.tile[0] = 128, cfg.tile[1] = 64, cfg.split_k = parts;
-    if (us128 < best) best = us128, cfg.tile[0] = 128, cfg.tile[1] = 128, cfg.split_k = parts;
-  }
-  return true;
+  const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128);
+  if (!vec_ok) return M <= 512 && t128 <= kNumCU;  // (the element kernel, or the two passes, whose second can run on whole vectors)
+  const double us = tile_q8_policy(M, N, K, may_split, &cfg);
+  dtas_config wide;
+  double us16 = 0.;
+  return !(M > 128 && tile8_policy(M, N, K, true, false, &wide, &us16) && 5.3 + 0.415e-6 * static_cast<double>(N) * static_cast<double>(K) + 0.907 * us16 < us);
 }
 }  // namespace dtas
 
@@ -100,16 +124,22 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
     return dtas_gemv_q8_f16(A, Wq, scale, bias, C, N, K, epilogue, nullptr, stream);
   GemmEpilogue ep = {static_cast<const half_t*>(bias), static_cast<const half_t*>(res1), static_cast<const half_t*>(res2),
                      epilogue, out_bytes == 4 ? 1 : 0, 0.f, 0, 0, 0, 0, 1, 0, static_cast<const half_t*>(scale)};
+  const bool vec_ok = aligned(A, 16) && aligned(Wq, 16) && aligned(scale, 2) && N * K < (int64_t{1} << 32) && K > 0;
   const bool stream_ok = K > 0 && K % 256 == 0 && aligned(A, 16) && aligned(Wq, 16) && aligned(scale, 16) && K < (int64_t{1} << 24);
   dtas_config cfg;
   if (user) {
     cfg = *user;
-  } else if (!builtin_gemm_q8(M, N, K, stream_ok, &cfg)) {
+  } else if (!builtin_gemm_q8(M, N, K, stream_ok, vec_ok, true, &cfg)) {
     void* wbuf = nullptr;
     std::lock_guard<std::recursive_mutex> ws_lock(g_ws_mutex);  // until both launches are enqueued
     if (operand_workspace(static_cast<hipStream_t>(stream), static_cast<size_t>(N) * K * 2, &wbuf) != 0) return -1;
     if (dtas_decode_q8_f16(Wq, scale, wbuf, N, K, nullptr, stream) != 0) return -1;
     return dtas_gemm_f16_fused(A, wbuf, bias, res1, res2, C, M, N, K, epilogue, nullptr, stream);
+  } else if (cfg.variant == DTAS_GEMM_MFMA && cfg.split_k > 1) {
+    // a first call under capture cannot allocate the workspace: whole tiles then
+    const size_t tiles = static_cast<size_t>(ceil_div(M, cfg.tile[0]) * ceil_div(N, cfg.tile[1]));
+    if (!split_scratch_at_hand(static_cast<hipStream_t>(stream), tiles * cfg.split_k * cfg.tile[0] * cfg.tile[1] * 4, tiles))
+      (void)tile_q8_policy(M, N, K, false, &cfg);
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const half_t* a = static_cast<const half_t*>(A);
@@ -130,7 +160,6 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
     if (!stream_ok) return fail("gemm_q8: the share kernel needs K %% 256 == 0 and 16-byte aligned A, W and scales");
     return launch_gemm_share_q8(cfg.tile[0], cfg.tile[1], s, a, w, ep, C, M, N, K);
   }
-  const bool vec_ok = aligned(A, 16) && aligned(Wq, 16) && aligned(scale, 2) && N * K < (int64_t{1} << 32) && K > 0;
   if (cfg.vec == 8 && !vec_ok) cfg.vec = 1;
   if (cfg.vec == 1) {
     int64_t grid = ceil_div(M * N, 256);
@@ -143,6 +172,13 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
   int64_t la[7];
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;
   const int bm = cfg.tile[0], bn = cfg.tile[1];
+  if (cfg.block == 512 && bn == 128 && cfg.unroll == 0) {
+    if (bm == 96) return launch_mfma<96, 128, 2, 4, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
+    if (bm == 128) return launch_mfma<128, 128, 4, 2, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
+    if (bm == 160) return launch_mfma<160, 128, 2, 4, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
+    if (bm == 192) return launch_mfma<192, 128, 4, 2, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
+    if (bm == 256) return launch_mfma<256, 128, 4, 2, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
+  }
   if (bm == 128 && bn <= 128 && cfg.block != 256) return fail("gemm_q8: the %dx%d MFMA kernel uses 256 threads, got %d", bm, bn, cfg.block);
   if (bm == 256 && bn == 128 && cfg.unroll == 3) return launch_mfma<256, 128, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);
   if (bm == 128 && bn == 128 && cfg.unroll == 3) return launch_mfma<128, 128, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);
@@ -150,5 +186,5 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
   if (bm == 128 && bn == 64 && cfg.unroll == 3) return launch_mfma<128, 64, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);
   if (bm == 64 && bn == 64 && cfg.unroll == 3) return launch_mfma<64, 64, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);
   if (bm == 64 && bn == 128 && cfg.unroll == 3) return launch_mfma<64, 128, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);
-  return fail("gemm_q8: 8-bit weights come with tiles 256x128, 128x128, 128x64, 64x128 (three stages) and 64x64 (two or three), got %dx%d with %d", bm, bn, cfg.unroll);
+  return fail("gemm_q8: 8-bit weights come with tiles 256x128, 128x128, 128x64, 64x128 (three stages) and 64x64 (two or three), and with 512 threads {96, 128, 160, 192, 256} x 128 (unroll 0), got %dx%d with %d", bm, bn, cfg.unroll);
 }

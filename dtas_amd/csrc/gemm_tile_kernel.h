@@ -46,15 +46,18 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   static_assert(NS >= 2 && NS <= (M16 ? 6 : 4), "stage count");
   static_assert((NS - 1) * (LA + LB) <= 63, "outstanding loads must fit the vmcnt field");
   constexpr bool WREG = WQ;  // W tiles pass through registers (dequantised), not the direct-to-LDS path
-  static_assert(!WREG || (NS <= 3 && NW == 4), "the register W path is written for two or three stages and 4 wavefronts");
+  static_assert(!WREG || M16 || (NS <= 3 && NW == 4), "the register W path on 4 wavefronts is written for two or three stages");
+  static_assert(!(WQ && M16) || (NS >= 3 && BN == 128), "8-bit W on 8 wavefronts: a 16-byte piece of W per lane and k tile");
   static_assert(!(WT && WQ), "k-major 8-bit weights are not served");
   static_assert(!WT || (NW == 4 && BN >= 64), "the k-major W path is written for the 4-wavefront 32x32x16 loops");
-  static_assert(M16 == (NW == 8) && (!M16 || !WREG), "8 wavefronts run the 16x16x32 loop, and only they");
+  static_assert(M16 == (NW == 8), "8 wavefronts run the 16x16x32 loop, and only they");
   // 256x256 and the 8-wavefront tiles on two stages: a ring of 5 operand units, each the larger operand's rows of a k tile
   constexpr bool kRing = M16 ? NS == 2 : BM + BN == 512;
   constexpr int kRingUnit = (BM > BN ? BM : BN) * kRowBytes;
   constexpr int kStagesA = !M16 || NS * kStage <= kLdsBytes ? NS : 2;  // (8 wavefronts: W's stages are NS, A's what the LDS leaves)
-  constexpr int kLdsAlloc = kRing ? 5 * kRingUnit : kStagesA * kABytes + NS * BN * kRowBytes;
+  // 8-bit W on 8 wavefronts: NS stages of A, its rows rounded up to whole loads of every wavefront, and two of (fp16) W
+  constexpr int kQLoadsA = (BM + 63) / 64, kQStageA = kQLoadsA * 64 * kRowBytes;
+  constexpr int kLdsAlloc = kRing ? 5 * kRingUnit : WQ && M16 ? NS * kQStageA + 2 * BN * kRowBytes : kStagesA * kABytes + NS * BN * kRowBytes;
   static_assert(BM * BN * 2 <= kLdsAlloc, "epilogue staging must fit the operand stages");
   static_assert(kLdsAlloc <= kLdsBytes, "stages exceed the LDS");
   __shared__ __attribute__((aligned(1024))) char lds[kLdsAlloc];
@@ -227,7 +230,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   // The pieces come through buffer loads (out of range -> zeros), so every lane issues the same number of loads per tile
   // whatever its rows: the waits below count them.  Every row of the tile is written every time (rows past N as zeros).
   constexpr int kWtItems = WREG ? 4 * BN / (64 * NW) : 1;
-  constexpr int kWtSlots = WREG ? NS - 1 : 1;  // register sets: one per tile in flight
+  constexpr int kWtSlots = WREG ? (M16 ? 3 : NS - 1) : 1;  // register sets: one per tile in flight
   constexpr int kWtLoads = 2 * kWtItems;  // per lane and tile: a piece and its scale per item
   u32x4 wt_reg[kWtSlots][kWtItems][1];
   unsigned short wq_scale[kWtSlots][kWtItems];
@@ -239,14 +242,13 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     for (int i = 0; i < kWtItems; ++i) {
       const unsigned item = t + i * 64 * NW, r = item >> 2, c4 = item & 3u;
       const int64_t row = n0 + r, k = static_cast<int64_t>(kt_abs(kt)) * kBK + c4 * 16;
-      const bool in = row < N && k < K;  // K % 32 == 0: a piece and its scale group are all-in or all-out
+      const bool in = row < N && k < K && (!M16 || kt < ktiles);  // K % 32 == 0: a piece and its scale group are all-in or all-out
       wt_reg[SLOT][i][0] = __builtin_amdgcn_raw_buffer_load_b128(rv, in ? static_cast<unsigned>(row * K + k) : kOob, 0, 0);
       wq_scale[SLOT][i] = __builtin_amdgcn_raw_buffer_load_b16(rs, in ? static_cast<unsigned>((row * (K >> 5) + (k >> 5)) * 2) : kOob, 0, 0);
     }
   };
-  auto wt_commit = [&](int kt, auto slot_tag) {
+  auto wt_commit_at = [&](char* base, auto slot_tag) {
     constexpr int SLOT = decltype(slot_tag)::value;
-    char* base = lds + (kt % NS) * kStage + kABytes;
 #pragma unroll
     for (int i = 0; i < kWtItems; ++i) {
       const unsigned item = t + i * 64 * NW, r = item >> 2, c4 = item & 3u;
@@ -265,6 +267,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       *reinterpret_cast<u32x4*>(base + lds_chunk_offset(r, 2 * c4 + 1)) = out[1];
     }
   };
+
+  auto wt_commit = [&](int kt, auto slot_tag) { wt_commit_at(lds + (kt % NS) * kStage + kABytes, slot_tag); };
 
   f16x8 fa[2][MT], fb[2][NT];
   auto read_a = [&](int set, int i, const char* stage, int ks) {
@@ -318,7 +322,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     }
   };
 
-  if constexpr (WREG) {
+  if constexpr (WREG && !M16) {
     // ---- W through registers (k-major or 8-bit): NS stages, NS-1 tiles requested ahead (W pieces to registers, then the A blocks
     // to the LDS, so the loads of a tile are contiguous in the order they complete in).  This path
     // is bound by the bytes of A in flight, not by MFMA issue: loads go out in one burst per tile.
@@ -401,7 +405,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     constexpr int kUnit = kRingUnit;
     constexpr int kLoadsA = BM / 32, kLoadsW = BN / 32;  // 1 KiB block loads per wavefront and unit
     static_assert((!kRing || 5 * kUnit <= kLdsAlloc) && BM % 32 == 0 && BN % 32 == 0, "ring exceeds the LDS");
-    constexpr int kFirstW = kRing ? kUnit : kStagesA * kABytes;  // where W(0) sits
+    constexpr int kFirstW = kRing ? kUnit : WQ ? NS * kQStageA : kStagesA * kABytes;  // where W(0) sits
     auto wrap5 = [](int v) { return v >= 5 ? v - 5 : v; };
     const bool hi = wv >= 4;
     if (hi) __builtin_amdgcn_s_setprio(0); else __builtin_amdgcn_s_setprio(2);
@@ -454,7 +458,28 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     };
     auto fetch_hi = [&](int stage, unsigned voff) { if constexpr (hi_w) fetch_w(stage, voff); else fetch_a(stage, voff); };
     auto fetch_lo = [&](int stage, unsigned voff) { if constexpr (hi_w) fetch_a(stage, voff); else fetch_w(stage, voff); };
-    if constexpr (!kRing) {
+    [[maybe_unused]] auto a_off_q = [&](int kt) -> unsigned {
+      return static_cast<int64_t>(kt_abs(kt)) * kBK + c_in * 8 < K && kt < ktiles ? g_off + static_cast<unsigned>(kt_abs(kt)) * kRowBytes : kOob;
+    };
+    [[maybe_unused]] auto fetch_a_q = [&](int stage, int kt) {  // (rows past the tile are past the descriptor's range: zeros, nothing is loaded)
+      const unsigned off = a_off_q(kt);
+      char* base = lds + stage * kQStageA + wv * 1024;
+#pragma unroll
+      for (int q = 0; q < kQLoadsA; ++q) __builtin_amdgcn_raw_ptr_buffer_load_lds(ra, (lds_ptr_t)(base + q * NW * 1024), 16, off, q * g_step, 0, DTAS_GEMM_LOAD_AUX);
+    };
+    if constexpr (WQ) {
+      wt_load(0, std::integral_constant<int, 0>{});
+      wt_load(1, std::integral_constant<int, 1>{});
+      wt_load(2, std::integral_constant<int, 2>{});
+      DTAS_SCHED_FENCE();
+#pragma unroll
+      for (int p = 0; p < NS - 1; ++p) fetch_a_q(p, p);
+      DTAS_SCHED_FENCE();
+      wt_commit_at(lds + NS * kQStageA, std::integral_constant<int, 0>{});
+      wt_load(3, std::integral_constant<int, 0>{});
+      DTAS_SCHED_FENCE();
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA + 2));
+    } else if constexpr (!kRing) {
       if (hi) {
 #pragma unroll
         for (int p = 0; p < kHiStages; ++p) fetch_hi(p, lane_off16(p));
@@ -502,7 +527,39 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
         }
     };
     static_assert(kReadEvery * (MT16 + NT16) <= MT16 * NT16, "fragment reads must fit between the MFMAs of a step");
-    if constexpr (!kRing) {
+    if constexpr (WQ) {
+      // ---- 8-bit W on 8 wavefronts.  Every wavefront does the same: its blocks of A NS - 1 k tiles ahead, straight to the LDS, and
+      // a 16-byte piece of W per lane (16 weights and their scale) three k tiles ahead of the stage it is dequantised into,
+      // one k tile before it is multiplied; the dequantiser's instructions issue under the MFMAs of the step before.
+      static_assert((NS - 2) * kQLoadsA + 4 <= 63, "outstanding loads must fit the vmcnt field");
+      char* const w0 = lds + NS * kQStageA;
+      int sa = 0;  // stage of A(kt)
+      auto q_tile = [&](int kt, auto slot_tag) {  // (slot of W(kt + 1))
+        const int na = sa + 1 == NS ? 0 : sa + 1;
+        char* const wc = w0 + (kt & 1) * (BN * kRowBytes);
+        char* const w_next = w0 + ((kt & 1) ^ 1) * (BN * kRowBytes);
+        fetch_a_q(sa == 0 ? NS - 1 : sa - 1, kt + NS - 1);  // into the stage that tile kt-1 left at the previous barrier
+        DTAS_SCHED_FENCE();
+        step16(0, lds + sa * kQStageA, wc, 1);
+        wt_commit_at(w_next, slot_tag);                          // W(kt+1), into the stage that W(kt-1) left
+        wt_load(kt + 4, slot_tag);
+        DTAS_SCHED_FENCE();
+        // A(kt+1) has landed: behind it were requested A(kt+2) .. A(kt+NS-1) and two or more k tiles' pieces of W
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA + 4));
+        __builtin_amdgcn_s_barrier();
+        DTAS_SCHED_FENCE();
+        step16(1, lds + na * kQStageA, w_next, 0);
+        sa = na;
+      };
+      int kt = 0;
+      for (; kt + 2 < ktiles; kt += 3) {
+        q_tile(kt, std::integral_constant<int, 1>{});
+        q_tile(kt + 1, std::integral_constant<int, 2>{});
+        q_tile(kt + 2, std::integral_constant<int, 0>{});
+      }
+      if (kt < ktiles) q_tile(kt, std::integral_constant<int, 1>{});
+      if (kt + 1 < ktiles) q_tile(kt + 1, std::integral_constant<int, 2>{});
+    } else if constexpr (!kRing) {
       static_assert((NS - 1) * (kLoadsA > kLoadsW ? kLoadsA : kLoadsW) <= 63, "outstanding loads must fit the vmcnt field");
       int sa = 0, sw = 0;  // stages of A(kt), W(kt)
       for (int kt = 0; kt < ktiles; ++kt) {
@@ -525,7 +582,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       }
     }
     int slot_a = 0, slot_w = 1;  // slots of A(kt), W(kt)
-    for (int kt = 0; kRing && kt < ktiles; ++kt) {
+    for (int kt = 0; kRing && !WQ && kt < ktiles; ++kt) {
       const char* pa = lds + slot_a * kUnit;
       const char* pw = lds + slot_w * kUnit;
       const int next_a = wrap5(slot_a + 2), next_w = wrap5(slot_w + 2);

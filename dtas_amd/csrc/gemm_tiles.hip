@@ -326,7 +326,7 @@ constexpr Tile8Cost kTile8Cost[] = {
     {224, 256, 512, 0, false, 5.85, 1.317, 1.9, 0.56, 1.66, 4.2, 4.84, 1.05, 0.3, 0.36},
     {256, 256, 512, 2, true, 6.98, 1.505, 0.41, 0.48, -4, 5.88, 5, 1.02, 0.28, 0.34},
 };
-bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table, dtas_config* out) {
+bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table, dtas_config* out, double* us_out) {
   const int64_t ktiles = ceil_div(K, kBK);
   const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
   double best = 1e300;
@@ -374,6 +374,7 @@ bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table
   // falls behind the ring of two (700 x 11008 x 4096 78.2 / 71.8 us, 1025 x 8192 x 2048 41.1 / 38.4; ahead elsewhere: 1400 x
   // 4096 x 11008 152 / 178, 1025 x 7680 x 2560 50.7 / 53.9)
   if (out->tile[0] == 192 && out->tile[1] == 256 && out->split_k == 1 && K % 2048 == 0) out->unroll = 2;
+  if (us_out) *us_out = best;
   return best < 1e300;
 }
 
@@ -411,7 +412,7 @@ extern "C" int dtas_builtin_gemm(int weights_8bit, int64_t M, int64_t N, int64_t
   if (weights_8bit) {
     if (K % 32 != 0) return fail("dtas_builtin_gemm: K must be a multiple of the scale group, 32 (K=%lld)", (long long)K);
     what = "gemm_q8";
-    if (builtin_gemm_q8(M, N, K, K % 256 == 0, &out->config)) {
+    if (builtin_gemm_q8(M, N, K, K % 256 == 0, N < (int64_t{1} << 32) / K, true, &out->config)) {
       snprintf(out->name, sizeof(out->name), "%s", what);
       return 0;  // (launch_args stay zero: the 8-bit kernels' grids are their launchers')
     }

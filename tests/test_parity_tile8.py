@@ -83,6 +83,53 @@ def test_what_runs_without_a_config(oracle, M, N, K):
     _check(got[rows], oracle.c.gemm(a[rows], w, bias, threads=8), oracle.np64.gemm(a[rows], w, bias))
 
 
+Q8_TILES = [(96, 128), (128, 128), (160, 128), (192, 128), (256, 128)]
+
+
+def _q8(N, K, seed):
+    rng = np.random.default_rng(seed)
+    return rng.integers(0, 2 ** 32, (N, K // 4), dtype=np.uint32), (rng.random((N, K // 32)) * 0.0008 + 0.0002).astype(np.float16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn", Q8_TILES)
+def test_every_8_bit_tile_at_its_edges(oracle, bm, bn):
+    # k tiles: half of one, fewer than the loads run ahead, a whole number of the loop's three, one and two more; K in parts
+    for M, N, K, split in ((3, 5, 32, 1), (bm - 1, bn + 1, 64, 1), (bm + 1, 2 * bn - 1, 224, 1), (2 * bm, bn, 384, 1), (bm + 33, bn + 8, 448, 1),
+                           (bm + 7, bn + 9, 1056, 3), (bm - 5, bn, 2080, 6)):
+        a, _, bias = _inputs(M, N, K, M + N + K)
+        wq, scale = _q8(N, K, M + K)
+        w = oracle.c.decode_q8(wq, scale, threads=8)
+        out = Guarded((M, N), torch.float16)
+        ops.gemm_q8(dev(a), torch.from_numpy(wq.view(np.int32)).cuda(), dev(scale), dev(bias), out.t, _cfg(bm, bn, 0, split))
+        _check(out.check(), oracle.c.gemm(a, w, bias, threads=8), oracle.np64.gemm(a, w, bias))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("epilogue", [_lib.EPI_BIAS, _lib.EPI_BIAS_ADD2, _lib.EPI_BIAS_ADD2_CAST_F32, _lib.EPI_BIAS_GELU])
+@pytest.mark.parametrize("M,N,K", [(97, 2560, 2560), (130, 768, 1024), (203, 520, 2080), (320, 2560, 10240), (450, 7680, 320), (700, 10240, 256), (900, 1000, 4096)])
+def test_8_bit_weights_without_a_config(M, N, K, epilogue):
+    # against the fp16 GEMM on the dequantised weights, which are the same numbers: another order of the fp32 sums can move the
+    # rounding of the product and of the up to three steps behind it by an fp16 ulp each, 2^-10 of what is added up there, S
+    # at most -- the result itself may be small where residuals cancel it -- and the GELU's slope stays below 1.13: 2^-8 S
+    a, _, bias = (dev(x) for x in _inputs(M, N, K, M + N))
+    wq, scale = _q8(N, K, N + K)
+    words, scale = torch.from_numpy(wq.view(np.int32)).cuda(), dev(scale)
+    w = torch.empty(N, K, dtype=torch.float16, device="cuda")
+    ops.decode_q8(words, scale, w)
+    g = torch.Generator(device="cuda").manual_seed(1)
+    res = [torch.randn(M, N, device="cuda", generator=g).half() for _ in range(2)] if epilogue in (_lib.EPI_BIAS_ADD2, _lib.EPI_BIAS_ADD2_CAST_F32) else [None, None]
+    kind = torch.float32 if epilogue == _lib.EPI_BIAS_ADD2_CAST_F32 else torch.float16
+    out, want = Guarded((M, N), kind), torch.empty(M, N, dtype=kind, device="cuda")
+    ops.gemm_q8(a, words, scale, bias, out.t, None, epilogue, *res)
+    ops.gemm(a, w, bias, want, cfg(variant=_lib.GEMM_MFMA, block=256, vec=8, unroll=2, tile=[64, 64, 64]), epilogue, *res)
+    mm = torch.empty(M, N, dtype=torch.float16, device="cuda")
+    ops.gemm(a, w, None, mm, cfg(variant=_lib.GEMM_MFMA, block=256, vec=8, unroll=2, tile=[64, 64, 64]))
+    S = sum(t.double().abs() for t in (mm, bias.expand(M, N), *(r for r in res if r is not None))).cpu().numpy()
+    got, want = out.check().astype(np.float64), want.cpu().numpy().astype(np.float64)
+    assert (np.abs(got - want) <= 2.0 ** -8 * S).all()
+
+
 @pytest.mark.gpu
 def test_a_first_call_under_capture_splits_nothing():
     # a stream without a workspace that is being captured: whole tiles instead of an allocation
