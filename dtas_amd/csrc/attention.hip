@@ -628,21 +628,28 @@ __global__ void __launch_bounds__(1024) attn_scores_rows_kernel(const half_t* __
 // workgroups on the chip).  A head's V is m rows of d fp16 = d / 8 16-byte pieces each, contiguous in memory: thread t of
 // 1024 takes piece t % (d / 8) of the rows t / (d / 8), + rows-per-pass, ... -- consecutive threads read consecutive
 // 16 bytes, a wavefront 1 KiB, eight passes in flight -- and multiplies each piece with its row's P.  The 8 sums of a
-// thread are those of its 8 columns; threads with the same piece index meet in the LDS and are added in thread order.
+// thread are those of its 8 columns; threads with the same piece index meet in the LDS, where block / cols threads add an
+// equal part of a column each (one thread per column, 51 .. 102 sums one after the other: 0.3 .. 1.0 us more, 2048 keys
+// with 16 columns per workgroup 8.9 -> 7.2).  What bounds it: how fast a CU pulls its part of V in, whole 128-byte lines,
+// 50 KB/us of them from memory.  Workgroups that share a head's lines are neighbours on an XCD and read them through its L2.
 __global__ void __launch_bounds__(1024) attn_pv_whole_row_kernel(const half_t* __restrict__ P, const half_t* __restrict__ V,
                                                                 half_t* __restrict__ out, int64_t n, int64_t m, int64_t d, unsigned cols,
-                                                                unsigned nsplit, float* __restrict__ ws, unsigned* __restrict__ arrivals) {
-  __shared__ float red[1024][8];
+                                                                unsigned inv_cols, unsigned nsplit, float* __restrict__ ws, unsigned* __restrict__ arrivals) {
+  __shared__ float red[1024][8], sums[1024];
   __shared__ unsigned is_last;
   // (cols < d: the workgroups of a (head, row) share the pieces of a key, cols / 8 consecutive ones each)
   const unsigned row_chunks = static_cast<unsigned>(d / 8), chunks = cols / 8, groups = row_chunks / chunks;
-  const unsigned per_pass = blockDim.x / chunks, t = threadIdx.x;
-  const int64_t h = blockIdx.x / groups, r = blockIdx.y;
-  const unsigned first = (blockIdx.x % groups) * chunks;
+  // (inv_cols = ceil(2^20 / cols): (x inv_cols) >> 20 is x / cols up to 1024, (8 x inv_cols) >> 20 is x / chunks; divided
+  // out a launch against few keys takes 5 .. 8 % longer: 8 heads of 256, 2 rows, 50 keys 4.3 us, so 4.0)
+  const unsigned per_pass = (8u * blockDim.x * inv_cols) >> 20, t = threadIdx.x;
+  const unsigned id = groups == 1 ? blockIdx.x : xcd_contiguous_id(blockIdx.x, gridDim.x);
+  const unsigned head = groups == 1 ? id : id / groups;
+  const int64_t h = head, r = blockIdx.y;
+  const unsigned first = (id - head * groups) * chunks;
   const half_t* p = P + (h * n + r) * m;
   const u32x4* v = reinterpret_cast<const u32x4*>(V + h * m * d) + first;
   const bool active = t < per_pass * chunks;
-  const unsigned row0 = t / chunks;
+  const unsigned row0 = (8u * t * inv_cols) >> 20;
   float acc[8];
 #pragma unroll
   for (int e = 0; e < 8; ++e) acc[e] = 0.f;
@@ -661,7 +668,7 @@ __global__ void __launch_bounds__(1024) attn_pv_whole_row_kernel(const half_t* _
         const int64_t k = k0 + static_cast<int64_t>(u) * per_pass;
         // (piece index of thread t in pass u: t + u * per_pass * chunks -- the passes continue where the last thread stopped)
         // (one row: V is read this once and streamed past the caches; more rows: their workgroups share it)
-        vraw[u] = k >= k_hi ? zero : n == 1 ? load_stream(v + k * row_chunks + (t - row0 * chunks)) : v[k * row_chunks + (t - row0 * chunks)];
+        vraw[u] = k >= k_hi ? zero : n == 1 && groups == 1 ? load_stream(v + k * row_chunks + (t - row0 * chunks)) : v[k * row_chunks + (t - row0 * chunks)];
         pk[u] = k < k_hi ? p[k] : static_cast<half_t>(0.f);
       }
 #pragma unroll
@@ -676,22 +683,18 @@ __global__ void __launch_bounds__(1024) attn_pv_whole_row_kernel(const half_t* _
 #pragma unroll
   for (int e = 0; e < 8; ++e) red[t][e] = active ? acc[e] : 0.f;
   __syncthreads();
-  // column j of the row: piece j / 8, element j % 8, summed over the per_pass threads that hold that piece
-  const bool holds = t < chunks * 8u;
+  // column j of the row: piece j / 8, element j % 8, held by per_pass threads; block / cols threads add an equal part of
+  // them each, the first adds the parts up in their order
+  const unsigned parts = (blockDim.x * inv_cols) >> 20, part = (t * inv_cols) >> 20, j = t - part * cols;
+  const bool holds = t < cols;
   float sum = 0.f;
-  if (holds) {
-    const unsigned c = t >> 3, e = t & 7u;
-    float s0 = 0.f, s1 = 0.f, s2 = 0.f, s3 = 0.f;
-    unsigned q = 0;
-    for (; q + 3 < per_pass; q += 4) {
-      s0 += red[(q + 0) * chunks + c][e];
-      s1 += red[(q + 1) * chunks + c][e];
-      s2 += red[(q + 2) * chunks + c][e];
-      s3 += red[(q + 3) * chunks + c][e];
-    }
-    for (; q < per_pass; ++q) s0 += red[q * chunks + c][e];
-    sum = (s0 + s1) + (s2 + s3);
+  if (part < parts) {
+    for (unsigned q = part; q < per_pass; q += parts) sum += red[q * chunks + (j >> 3)][j & 7u];
+    sums[t] = sum;
   }
+  __syncthreads();
+  if (holds)
+    for (unsigned i = 1; i < parts; ++i) sum += sums[i * cols + t];
   if (nsplit > 1) {
     const size_t tile = static_cast<size_t>(blockIdx.y) * gridDim.x + blockIdx.x;  // (row, head, columns)
     float* tile_ws = ws + tile * nsplit * cols;
@@ -939,19 +942,44 @@ extern "C" int dtas_attn_pv_f16(const void* P, const void* V, void* out, int64_t
       // are too few to pull V in)
       const int64_t pieces = d / 8;
       const int halves = pieces % 2 == 0 && heads * n * 2 <= kNumCU ? 2 : 1;
-      // many keys (from ~3000) and room on the chip for several workgroups per (head, row): the workgroups share the keys,
-      // a run each, and meet in the split-K workspace (1 row against 4096 / 8192 keys in 8 runs 11.8 / 15.0 us, the row
-      // kernel 16.8 / 30.6; 2 rows in 4 runs 12.1 / 16.9 against 16.5 / 28.0; 4 rows in 2 runs 15.1 / 23.8 against 16.3 /
-      // 28.0 in halves / on the tiles; up to 2048 keys the hand-over costs more than it saves: 8.2 against 7.1)
-      int runs = 1;
+      // many keys and room on the chip for several workgroups per (head, row): the workgroups share the keys, a run each, and
+      // meet in the split-K workspace.  Half of the pieces of a key each where that leaves two to four runs: 32 heads of 80,
+      // V from memory, 1 row against 2304 .. 6000 keys in halves and 4 runs 9.3 / 9.8 (3001) / 10.7 (4096) / 11.8 us, whole
+      // in 8 runs 10.7 / 11.0 / 11.9 / 13.0, without runs 9.5 / 10.8 / 13.5; 2 rows against 2500 / 4096 9.7 / 12.1, 11.0 /
+      // 13.6 without; 16 heads of 64 against 2500 8.2 / 9.3; up to 2048 keys level or behind, and one row in 2 runs only from
+      // 3072 (40 heads of 80 against 2304 10.3 / 9.6 without).
+      int runs = 1, half_runs = 1;
       while (heads * n * runs * 2 <= kNumCU && runs < 8) runs *= 2;
+      while (pieces % 2 == 0 && heads * n * half_runs * 4 <= kNumCU && half_runs < 4) half_runs *= 2;
+      const bool in_halves = half_runs == 4 || (half_runs == 2 && heads * n * 4 >= 3 * kNumCU / 4);  // (40 heads of 80 against 3500 keys: whole in 4 runs 11.8, halves in 2 12.2)
+      if (in_halves) runs = half_runs;
+      const int64_t run_cols = in_halves ? d / 2 : d;
+      bool in_runs = runs >= 2 && pieces <= 128 && m >= 3072;
+      if (!in_runs && in_halves && m >= 2304 && (runs == 4 || n >= 2))  // (without a workspace under capture: one of the forms below)
+        in_runs = split_scratch_at_hand(static_cast<hipStream_t>(stream), static_cast<size_t>(heads * n * d * runs) * sizeof(float), static_cast<size_t>(2 * heads * n));
+      // one row, more of the row kernel's workgroups (a piece each) than CUs: the fewest pieces per workgroup with which
+      // every CU has at most one.  A 16-byte piece costs a CU's L1 its whole 128-byte line, and the CU with two such
+      // workgroups ends last.  V from memory, us, 32 heads of 80: 1024 / 2048 / 2250 keys 6.4 / 8.6 / 9.2, the row kernel
+      // 6.6 / 9.9 / 11.2; 32 heads of 128 6.8 / 10.0, 7.3 / 12.1; 40 of 128 (4 pieces) against 300 / 600 / 2048 5.1 / 6.0 /
+      // 10.8, 5.1 / 7.0 / 13.5; 64 of 80 (5) 7.7 / 11.2, 8.1 / 14.0; 96 of 128 (8) against 300 / 2048 5.6 / 15.4, 8.5 / 18.5.
+      // Fewer keys are level or lose by the sums' longer way through the LDS (32 heads of 80: 600 keys 5.4 / 5.2).
+      int64_t shared_pieces = 1;
+      if (n == 1 && heads * pieces > kNumCU && heads <= kNumCU) {
+        shared_pieces = 2;
+        while (shared_pieces < pieces && (pieces % shared_pieces != 0 || heads * (pieces / shared_pieces) > kNumCU)) ++shared_pieces;
+        if (shared_pieces > 128 || m < (shared_pieces == 2 ? 800 : 384)) shared_pieces = 1;
+        if (shared_pieces == pieces && heads < 3 * kNumCU / 4 && m * d > 200000) shared_pieces = 1;  // (160 heads of 128, 3000 keys: 32.4 / 30.8; 730 of 80: 9.2 / 12.2)
+      }
       // (a workgroup's sweep of V, keys x head dimension, is what the whole-row forms pay for: the limits below are the 3072 /
       // 6144 / 4096 keys of 80 they were measured at -- 8 rows against 8192 keys, 16 heads of 128, in 2 runs: 33.2 us, the tiles 18.8)
       const int64_t md = m * d, kMd = 80;
-      const double whole_row_runs_us = 7.0 + 5e-5 * static_cast<double>(ceil_div(m, runs) * d) + 0.5 * runs;  // (4 rows of 128 against 4096 keys in 2 runs: 20.7 us, the tiles 16.0; 4 rows of 80 against 8192: 23.4 / 19.2)
-      if (m >= 3072 && runs >= 2 && pieces <= 128 && (!mfma_ok || whole_row_runs_us <= mfma_us)) {
+      const double whole_row_runs_us = 7.0 + 5e-5 * static_cast<double>(ceil_div(m, runs) * run_cols) + 0.5 * runs;  // (4 rows of 128 against 4096 keys in 2 runs: 20.7 us, the tiles 16.0; 4 rows of 80 against 8192: 23.4 / 19.2)
+      if (in_runs && (!mfma_ok || whole_row_runs_us <= mfma_us)) {
         rows = true;
-        cfg = dtas_config{DTAS_GEMM_SKINNY, 1024, 8, 1, {1, 8, static_cast<int32_t>(d)}, runs, 0};
+        cfg = dtas_config{DTAS_GEMM_SKINNY, 1024, 8, 1, {1, 8, static_cast<int32_t>(run_cols)}, runs, 0};
+      } else if (shared_pieces > 1) {
+        rows = true;
+        cfg = dtas_config{DTAS_GEMM_SKINNY, shared_pieces == 2 ? 512 : 1024, 8, 1, {1, 8, static_cast<int32_t>(shared_pieces * 8)}, 1, 0};
       } else if (n >= 2 && n <= 8 && heads * n <= kNumCU && pieces <= 128 && (md < (halves == 2 ? 6144 : 3072) * kMd || !mfma_ok)) {
         rows = true;
         cfg = dtas_config{DTAS_GEMM_SKINNY, 1024, 8, 1, {1, 8, static_cast<int32_t>(d / halves)}, 1, 0};
@@ -1080,7 +1108,8 @@ extern "C" int dtas_attn_pv_f16(const void* P, const void* V, void* out, int64_t
     std::unique_lock<std::recursive_mutex> ws_lock;  // held until the launch is enqueued
     if (nsplit > 1 && split_scratch(s, tiles * nsplit * cols * sizeof(float), tiles, nsplit, &partials, &arrivals, &ws_lock) != 0) return -1;
     hipLaunchKernelGGL(attn_pv_whole_row_kernel, dim3(static_cast<unsigned>(heads * (d / cols)), static_cast<unsigned>(n), static_cast<unsigned>(nsplit)),
-                       dim3(cfg.block), 0, s, a, w, c, n, m, d, static_cast<unsigned>(cols), static_cast<unsigned>(nsplit), partials, arrivals);
+                       dim3(cfg.block), 0, s, a, w, c, n, m, d, static_cast<unsigned>(cols),
+                       ((1u << 20) + static_cast<unsigned>(cols) - 1u) / static_cast<unsigned>(cols), static_cast<unsigned>(nsplit), partials, arrivals);
     return check_launch("attn_pv");
   }
   if (cfg.variant == DTAS_GEMM_SKINNY) {

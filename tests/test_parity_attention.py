@@ -508,3 +508,44 @@ def test_decode_attention_against_the_prefill_kernels_and_properties(oracle, n):
     want = oracle.c.attn_pv(p[:2].cpu().numpy(), v[:2].cpu().numpy(), threads=8).astype(np.float64)
     got = o[:2].cpu().numpy().astype(np.float64)
     assert (np.abs(got - want) <= 1e-4 + 2.0 ** -9 * np.abs(want)).all()
+
+
+@pytest.mark.parametrize("heads,n,m,d", [
+    (32, 1, 799, 80), (32, 1, 800, 80), (32, 1, 2303, 80), (32, 1, 2304, 80), (32, 1, 3071, 80), (33, 1, 1025, 80),   # two pieces per workgroup; runs in halves
+    (40, 1, 383, 128), (40, 1, 384, 128), (64, 1, 515, 80), (96, 1, 387, 128), (29, 1, 801, 72),                      # four, five, eight, three
+    (256, 1, 390, 16), (256, 1, 385, 64), (257, 1, 385, 24), (160, 1, 1251, 160), (160, 1, 400, 160),                 # whole heads and none
+    (32, 2, 2304, 80), (16, 4, 2311, 64), (40, 1, 3072, 80), (12, 1, 2304, 64), (3, 2, 2500, 8), (24, 1, 3073, 120)]) # runs: in halves, whole
+def test_pv_few_rows_shared_columns_and_runs(oracle, heads, n, m, d):
+    p, v = _pv_inputs(heads, n, m, d, heads + m)
+    out = Guarded((heads, n, d), torch.float16)
+    ops.attn_pv(dev(p), dev(v), out.t)
+    _check_pv(out.check(), p, v, oracle)
+
+
+@pytest.mark.parametrize("heads,block,cols,d,runs", [(3, 512, 16, 80, 1), (2, 256, 256, 256, 3), (5, 512, 24, 72, 2), (2, 1024, 1024, 1024, 1), (1, 512, 512, 512, 5),
+                                                     (4, 1024, 8, 80, 4)])
+def test_pv_whole_row_kernel_sums_every_column_once(heads, block, cols, d, runs):
+    # exact on small integers, whatever the number of threads that share a column (down to one) and of keys (down to none)
+    rng = np.random.default_rng(block + cols)
+    for m in (1, 7, 129, 1000):
+        p, v = rng.integers(0, 2, size=(heads, 2, m)).astype(np.float16), rng.integers(-1, 2, size=(heads, m, d)).astype(np.float16)
+        out = Guarded((heads, 2, d), torch.float16)
+        ops.attn_pv(dev(p), dev(v), out.t, cfg(variant=_lib.GEMM_SKINNY, block=block, vec=8, unroll=1, tile=[1, 8, cols], split_k=runs))
+        assert np.array_equal(out.check().astype(np.float64), np.einsum("hnm,hmd->hnd", p.astype(np.float64), v.astype(np.float64)))
+
+
+def test_pv_first_call_under_capture_needs_no_workspace_below_3072_keys():
+    p, v = (dev(x) for x in _pv_inputs(32, 1, 2400, 80, 3))
+    eager, out = (torch.zeros(32, 1, 80, dtype=torch.float16, device="cuda") for _ in range(2))
+    ops.attn_pv(p, v, eager)
+    stream, graph = torch.cuda.Stream(), torch.cuda.CUDAGraph()
+    torch.cuda.synchronize()
+    with torch.cuda.graph(graph, stream=stream):
+        ops.attn_pv(p, v, out)
+    for _ in range(3):
+        out.zero_()
+        graph.replay()
+        torch.cuda.synchronize()
+        # (two orders of fp32 sums, each within 2^-23 per addition, then rounded to fp16: at most an ulp apart)
+        assert ((out.float() - eager.float()).abs() <= 2.0 ** -10 * eager.float().abs() + 2.0 ** -12 * float(eager.float().abs().max())).all()
+        ops.attn_pv(p, v, eager)
