@@ -392,14 +392,16 @@ int dtas_gemv_q8_f32(const void* x, const void* Wq, const void* scale, void* y, 
 /* dtas_gemm_q8_f16_fused: C[M,N] = epilogue(A[M,K] . W^T) with W dequantised on its way into the LDS, never
  * written: the dynamic-n forms fused_fused_decode2_fused_NT_matmul6_add4 (:371-399), ..decode4.._matmul9_add6_gelu1
  * (:504-581), ..decode5.._matmul4_add1; epilogues as dtas_gemm_f16_fused.  cfg, when given: a DTAS_GEMM_MFMA row
- * with tile {256,128,64}, {128,128,64}, {128,64,64} or {64,128,64} and unroll 3, or {64,64,64} and unroll 2 or 3; or a DTAS_GEMM_STREAM row
+ * with tile {256,128,64}, {128,128,64}, {128,64,64} or {64,128,64} and unroll 3, {64,64,64} and unroll 2 or 3, or block 512,
+ * unroll 0 and tile {96 | 128 | 160 | 192 | 256,128,64}; or a DTAS_GEMM_STREAM row
  * (block 256, tile {16,64,512}, {16,64,1024}, {32,64,512} or {64,64,512}; M <= tile[0]; K % 256 == 0; 16-byte
  * aligned A, Wq and scale): the W-streaming kernel on the bytes of W, widened between the LDS and the MFMA; its K
  * slices meet in the split-K workspace.  A DTAS_GEMM_MFMA row may carry split_k in [1, 16]: that many workgroups share
  * a tile and meet in the split-K workspace as in dtas_gemm_f16.  One row with a bias or GELU epilogue goes to
  * dtas_gemv_q8_f16.  With cfg == NULL: M <= 32 (M <= 64 while N / 64 x K / 512 workgroups fit one round of the chip) takes the W-streaming kernel where it
- * applies; up to 512 rows, while 128x128 tiles fit the chip in one round, the tile kernel dequantises in its W path
- * (64x64, 128x64 or 128x128 tiles of three stages with K in 1 .. 8 parts, by a fitted cost model); beyond that the two-pass route:
+ * applies; beyond that the tile kernel dequantises in its W path (64x64 and 128x64 tiles of three stages or the 512-thread
+ * tiles, K in 1 .. 8 parts with at most 32 MiB of partial tiles, or whole on a captured stream without a workspace) until a fitted
+ * cost model puts the two-pass route ahead, at 800 .. 1300 rows for most W:
  * dtas_decode_q8_f16 into a per-device fp16 buffer of its own (allocated on first use, grown on demand, at most
  * 1 GiB; same sharing rule as the split-K workspace), then dtas_gemm_f16_fused. */
 int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void* scale, const void* bias,
