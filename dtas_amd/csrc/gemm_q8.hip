@@ -135,11 +135,8 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
     if (operand_workspace(static_cast<hipStream_t>(stream), static_cast<size_t>(N) * K * 2, &wbuf) != 0) return -1;
     if (dtas_decode_q8_f16(Wq, scale, wbuf, N, K, nullptr, stream) != 0) return -1;
     return dtas_gemm_f16_fused(A, wbuf, bias, res1, res2, C, M, N, K, epilogue, nullptr, stream);
-  } else if (cfg.variant == DTAS_GEMM_MFMA && cfg.split_k > 1) {
-    // a first call under capture cannot allocate the workspace: whole tiles then
-    const size_t tiles = static_cast<size_t>(ceil_div(M, cfg.tile[0]) * ceil_div(N, cfg.tile[1]));
-    if (!split_scratch_at_hand(static_cast<hipStream_t>(stream), tiles * cfg.split_k * cfg.tile[0] * cfg.tile[1] * 4, tiles))
-      (void)tile_q8_policy(M, N, K, false, &cfg);
+  } else if (!gemm_scratch_at_hand(static_cast<hipStream_t>(stream), M, N, K, cfg)) {
+    (void)tile_q8_policy(M, N, K, false, &cfg);  // a first call under capture cannot allocate the workspace: whole tiles then
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const half_t* a = static_cast<const half_t*>(A);

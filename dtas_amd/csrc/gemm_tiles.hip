@@ -378,6 +378,19 @@ bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table
   return best < 1e300;
 }
 
+// Whether the partial tiles of `cfg` have a place to go on stream `s` (true where it splits nothing; split_k == 0 on the
+// 8-wavefront 256x256 tile splits the last round's).
+bool gemm_scratch_at_hand(hipStream_t s, int64_t M, int64_t N, int64_t K, const dtas_config& cfg) {
+  if (cfg.variant != DTAS_GEMM_MFMA) return true;
+  const int64_t tile = static_cast<int64_t>(cfg.tile[0]) * cfg.tile[1];
+  int nsplit = cfg.split_k;
+  unsigned unsplit = 0;
+  if (cfg.split_k == 0 && cfg.block == 512 && cfg.tile[0] == 256 && cfg.tile[1] == 256) tail_split_256(M, N, K, &nsplit, &unsplit);
+  if (nsplit <= 1) return true;
+  const size_t split_tiles = static_cast<size_t>(ceil_div(M, cfg.tile[0]) * ceil_div(N, cfg.tile[1]) - unsplit);
+  return split_scratch_at_hand(s, split_tiles * nsplit * tile * sizeof(float), split_tiles);
+}
+
 // What a call without a config runs: the bucket's row, or ahead of it a kernel chosen by M itself (what A costs it goes
 // with M, and the row is sized for the end of its bucket).  vec_ok: 16-byte loads of A and W are possible.
 // may_split: partial tiles have a place to go (what needs none otherwise).
@@ -468,11 +481,7 @@ extern "C" int dtas_gemm_f16_fused(const void* A, const void* W, const void* bia
   const bool vec_ok = K % 8 == 0 && aligned(A, 16) && aligned(W, 16);
   dtas_config cfg = user ? *user : builtin_gemm(M, N, K, vec_ok, true);
   // a first call under capture cannot allocate the workspace: whole tiles then
-  if (!user && M > 128 && vec_ok && cfg.split_k > 1) {
-    const size_t tiles = static_cast<size_t>(ceil_div(M, cfg.tile[0]) * ceil_div(N, cfg.tile[1]));
-    if (!split_scratch_at_hand(static_cast<hipStream_t>(stream), tiles * cfg.split_k * cfg.tile[0] * cfg.tile[1] * 4, tiles))
-      cfg = builtin_gemm(M, N, K, vec_ok, false);
-  }
+  if (!user && M > 128 && vec_ok && !gemm_scratch_at_hand(static_cast<hipStream_t>(stream), M, N, K, cfg)) cfg = builtin_gemm(M, N, K, vec_ok, false);
   if (cfg.vec == 8 && !vec_ok) cfg.vec = 1;  // K % 8 != 0 or odd pointers: element accesses
   int64_t la[7];
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;
