@@ -31,6 +31,7 @@ double tile_q8_policy(int64_t M, int64_t N, int64_t K, bool may_split, dtas_conf
   const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
   double best = 1e300;
   for (const TileQ8Cost& c : kTileQ8Cost) {
+    if (K * 2 * (c.bm > c.bn ? c.bm : c.bn) >= (int64_t{1} << 31)) continue;  // (32-bit tile offsets, describe_gemm)
     const int64_t tm = ceil_div(M, c.bm), tn = ceil_div(N, c.bn), tiles = tm * tn, limit = c.block == 256 ? 2 * kNumCU : kNumCU;
     if (tiles > 0x7fffffff / 8) continue;
     const double b = c.b * (odd_pitch ? c.pitch : 1.0) *

@@ -425,7 +425,7 @@ extern "C" int dtas_builtin_gemm(int weights_8bit, int64_t M, int64_t N, int64_t
   if (weights_8bit) {
     if (K % 32 != 0) return fail("dtas_builtin_gemm: K must be a multiple of the scale group, 32 (K=%lld)", (long long)K);
     what = "gemm_q8";
-    if (builtin_gemm_q8(M, N, K, K % 256 == 0, N < (int64_t{1} << 32) / K, true, &out->config)) {
+    if (builtin_gemm_q8(M, N, K, K % 256 == 0, N <= ((int64_t{1} << 32) - 1) / K, true, &out->config)) {
       snprintf(out->name, sizeof(out->name), "%s", what);
       return 0;  // (launch_args stay zero: the 8-bit kernels' grids are their launchers')
     }

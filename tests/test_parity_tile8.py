@@ -228,3 +228,11 @@ def test_a_call_without_a_config_names_a_launchable_kernel(seed):
         assert list(_lib.describe_launch(_lib.OP_GEMM_F16, M, N, K, c).launch_args) == list(info.launch_args), (M, N, K)
         if c.split_k > 1:
             assert info.launch_args[0] * c.tile[0] * c.tile[1] * 4 <= 32 << 20 and -(-K // 64) // c.split_k >= 6, (M, N, K)
+
+
+@pytest.mark.parametrize("M,N,K", [(1960, 611, 6003008), (1358, 500, 7290176), (1424, 426, 9246144), (2203, 257, 11799328), (70, 200, 16777184)])
+def test_an_8_bit_call_without_a_config_names_a_tile_that_holds_its_rows(M, N, K):
+    # a tile's rows are addressed with 32-bit offsets: from K = 4.2 million the taller tiles no longer hold them, the 64-row one up to 2^24
+    info = _lib.builtin_gemm(M, N, K, q8=True)
+    if info.name == b"gemm_q8":     # (otherwise the two passes, whose fp16 tile dtas_builtin_gemm describes by itself)
+        _lib.describe_launch(_lib.OP_GEMM_F16, M, N, K, info.config)
