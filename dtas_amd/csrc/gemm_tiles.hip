@@ -370,12 +370,13 @@ bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table
       if (whole_rounds) break;
     }
   }
+  if (us_out) *us_out = best;
+  if (best == 1e300) return false;  // (nothing was written to *out)
   // 192x256 against rows of W a multiple of 4 KiB apart: W in three stages and A in two, requested in the middle of a k tile,
   // falls behind the ring of two (700 x 11008 x 4096 78.2 / 71.8 us, 1025 x 8192 x 2048 41.1 / 38.4; ahead elsewhere: 1400 x
   // 4096 x 11008 152 / 178, 1025 x 7680 x 2560 50.7 / 53.9)
   if (out->tile[0] == 192 && out->tile[1] == 256 && out->split_k == 1 && K % 2048 == 0) out->unroll = 2;
-  if (us_out) *us_out = best;
-  return best < 1e300;
+  return true;
 }
 
 // Whether the partial tiles of `cfg` have a place to go on stream `s` (true where it splits nothing; split_k == 0 on the

@@ -236,3 +236,9 @@ def test_an_8_bit_call_without_a_config_names_a_tile_that_holds_its_rows(M, N, K
     info = _lib.builtin_gemm(M, N, K, q8=True)
     if info.name == b"gemm_q8":     # (otherwise the two passes, whose fp16 tile dtas_builtin_gemm describes by itself)
         _lib.describe_launch(_lib.OP_GEMM_F16, M, N, K, info.config)
+
+
+def test_a_k_that_no_tile_holds_is_refused():
+    for K in (1 << 24, 1 << 25):
+        with pytest.raises(_lib.DtasError, match="too large"):
+            _lib.builtin_gemm(300, 64, K)
