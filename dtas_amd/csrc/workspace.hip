@@ -20,15 +20,16 @@ namespace {
 //  * the split-K workspace: nsplit fp32 partial tiles per shared output tile and one arrival counter per tile
 //    (zero between launches: the last arriver of a tile re-arms it);
 //  * the operand buffer: the fp16 copy of an 8-bit weight matrix (dtas_gemm_q8_f16_fused's two-pass route).
-// Allocated on first use by a stream and grown on demand -- the only allocations in the library.  Launches on one
-// stream are ordered by it and share its set; launches on different streams use different sets, so they may overlap.
-// g_ws_mutex is held from the lookup until the launches that use the set are enqueued: a set is never grown (freed
-// and re-allocated: hipFree waits for the device, hence for every launch that may still use it) between a lookup
-// and its launch, also with several host threads.  At most kMaxWsStreams streams per device hold a set; beyond
-// that the set used longest ago is released first.
+// Allocated on first use by a stream and grown on demand -- the only allocations in the library.  A buffer that
+// was outgrown stays until its set is released: a recorded graph, or a launch that still runs, may hold its address.  Each one
+// is at least twice the one before it while the limit allows, so what is kept stays below twice what is in use.  Launches on
+// one stream are ordered by it and share its set; launches on different streams use different sets, so they may overlap.
+// g_ws_mutex is held from the lookup until the launches that use the set are enqueued, also with several host threads.
+// At most kMaxWsStreams streams per device hold a set; beyond that the set used longest ago is released first.
 constexpr size_t kMaxSplitWsBytes = size_t{1} << 30;
 constexpr int kMaxDevices = 64;
 constexpr int kMaxWsStreams = 16;
+constexpr int kMaxOutgrown = 40;  // (32 or 64 MiB doubled up to 1 GiB, 16 KiB of counters up to 2^31 tiles: 28 in all)
 struct StreamWorkspace {
   bool used = false;
   hipStream_t stream = nullptr;
@@ -39,6 +40,8 @@ struct StreamWorkspace {
   size_t tiles = 0;
   void* operand = nullptr;
   size_t operand_bytes = 0;
+  void* outgrown[kMaxOutgrown] = {};
+  int outgrown_count = 0;
 };
 struct DeviceWorkspaces {
   StreamWorkspace slot[kMaxWsStreams];
@@ -54,9 +57,32 @@ __global__ void zero_u32_kernel(unsigned* p, size_t count) {
 int release_workspace(StreamWorkspace& w) {
   // kernels of earlier launches may still use the buffers: hipFree waits for the device
   if (w.partials && hipFree(w.partials) != hipSuccess) return fail("workspace: hipFree of the split-K partials failed");
+  w.partials = nullptr;
   if (w.arrivals && hipFree(w.arrivals) != hipSuccess) return fail("workspace: hipFree of the split-K counters failed");
+  w.arrivals = nullptr;
   if (w.operand && hipFree(w.operand) != hipSuccess) return fail("workspace: hipFree of the operand buffer failed");
+  w.operand = nullptr;
+  for (; w.outgrown_count > 0; --w.outgrown_count)
+    if (hipFree(w.outgrown[w.outgrown_count - 1]) != hipSuccess) return fail("workspace: hipFree of an outgrown buffer failed");
   w = StreamWorkspace{};
+  return 0;
+}
+
+// A buffer of `need` bytes or more in the place of *buffer (of `have` bytes, none at first), at least twice as large while
+// that stays within `limit`.
+int grow(StreamWorkspace& w, void** buffer, size_t* have, size_t need, size_t first, size_t limit) {
+  size_t want = need > 2 * *have ? need : 2 * *have;
+  if (want < first) want = first;
+  if (want > limit) want = limit;
+  if (*buffer && w.outgrown_count == kMaxOutgrown) return fail("workspace: outgrown too often");
+  void* fresh = nullptr;
+  if (hipMalloc(&fresh, want) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail("workspace: cannot allocate %zu bytes", want);
+  }
+  if (*buffer) w.outgrown[w.outgrown_count++] = *buffer;
+  *buffer = fresh;
+  *have = want;
   return 0;
 }
 
@@ -90,32 +116,21 @@ int stream_workspace(hipStream_t stream, StreamWorkspace** out) {
 int split_workspace(hipStream_t stream, size_t partial_bytes, size_t tiles, float** partials, unsigned** arrivals) {
   StreamWorkspace* w = nullptr;
   if (stream_workspace(stream, &w) != 0) return -1;
-  if (partial_bytes > w->partial_bytes) {
-    if (w->partials && hipFree(w->partials) != hipSuccess) return fail("gemm: hipFree of the split-K workspace failed");
-    w->partials = nullptr;
-    w->partial_bytes = 0;
-    const size_t want = partial_bytes < (size_t{32} << 20) ? (size_t{32} << 20) : partial_bytes;
-    if (hipMalloc(reinterpret_cast<void**>(&w->partials), want) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail("gemm: cannot allocate %zu bytes of split-K workspace", want);
-    }
-    w->partial_bytes = want;
-  }
+  if (partial_bytes > w->partial_bytes &&
+      grow(*w, reinterpret_cast<void**>(&w->partials), &w->partial_bytes, partial_bytes, size_t{32} << 20, kMaxSplitWsBytes) != 0)
+    return -1;
   if (tiles > w->tiles) {
-    if (w->arrivals && hipFree(w->arrivals) != hipSuccess) return fail("gemm: hipFree of the split-K counters failed");
-    w->arrivals = nullptr;
-    w->tiles = 0;
-    const size_t want = tiles < 4096 ? 4096 : tiles;
-    if (hipMalloc(reinterpret_cast<void**>(&w->arrivals), want * sizeof(unsigned)) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail("gemm: cannot allocate the split-K arrival counters");
-    }
+    void* counters = w->arrivals;
+    size_t bytes = w->tiles * sizeof(unsigned);
+    w->tiles = 0;  // (until they are cleared)
+    if (grow(*w, &counters, &bytes, tiles * sizeof(unsigned), 4096 * sizeof(unsigned), SIZE_MAX) != 0) return -1;
+    w->arrivals = static_cast<unsigned*>(counters);
     // cleared on the stream that will use them (a clear on the default stream is not ordered with a non-blocking
     // stream), and by a kernel: a memset node recorded into a caller's graph is what a fill kernel avoids
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(want), 256))), dim3(256), 0, stream,
-                       w->arrivals, want);
+    const size_t count = bytes / sizeof(unsigned);
+    hipLaunchKernelGGL(zero_u32_kernel, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(count), 256))), dim3(256), 0, stream, w->arrivals, count);
     if (check_launch("gemm") != 0) return -1;
-    w->tiles = want;
+    w->tiles = bytes / sizeof(unsigned);
   }
   *partials = w->partials;
   *arrivals = w->arrivals;
@@ -131,18 +146,8 @@ std::mutex g_static_scratch_mutex;
 int operand_workspace(hipStream_t stream, size_t bytes, void** out) {
   StreamWorkspace* w = nullptr;
   if (stream_workspace(stream, &w) != 0) return -1;
-  if (bytes > w->operand_bytes) {
-    if (bytes > kMaxSplitWsBytes) return fail("operand buffer: a rewritten operand needs %zu bytes (limit %zu)", bytes, kMaxSplitWsBytes);
-    if (w->operand && hipFree(w->operand) != hipSuccess) return fail("operand buffer: hipFree failed");
-    w->operand = nullptr;
-    w->operand_bytes = 0;
-    const size_t want = bytes < (size_t{64} << 20) ? (size_t{64} << 20) : bytes;
-    if (hipMalloc(&w->operand, want) != hipSuccess) {
-      (void)hipGetLastError();
-      return fail("operand buffer: cannot allocate %zu bytes", want);
-    }
-    w->operand_bytes = want;
-  }
+  if (bytes > kMaxSplitWsBytes) return fail("operand buffer: a rewritten operand needs %zu bytes (limit %zu)", bytes, kMaxSplitWsBytes);
+  if (bytes > w->operand_bytes && grow(*w, &w->operand, &w->operand_bytes, bytes, size_t{64} << 20, kMaxSplitWsBytes) != 0) return -1;
   *out = w->operand;
   return 0;
 }

@@ -23,14 +23,14 @@
  *    dtas_gemm_f16 with K split over workgroups (split_k > 1, 0 on the 256x256 tile, or the
  *    W-streaming kernel, also behind dtas_gemm_q8_f16_fused for few rows; the built-in table chooses
  *    these when M x N leaves CUs idle) keeps fp32 partial tiles in a workspace that the
- *    library allocates on first use and grows on demand (32 MiB at first, at most 1 GiB; growing
- *    waits for the device).  There is one workspace per (device, stream): launches on one stream are
+ *    library allocates on first use and grows on demand (32 MiB at first, at least twice as much
+ *    when it grows, at most 1 GiB).  There is one workspace per (device, stream): launches on one stream are
  *    ordered by it, launches on different streams use different workspaces and may overlap; the
  *    library holds its lock from looking a workspace up to enqueueing the launch, so host threads may
  *    share a stream.  At most 16 streams per device hold one (the one used longest ago is released
  *    first, which waits for the device).  A recorded HIP graph holds the workspace's address: the
- *    first split launch on a stream, and any launch that makes its workspace grow, belong before the
- *    recording.  A cfg with split_k = 1 uses none; dtas_gemm_f16_static
+ *    first split launch on a stream belongs before the recording; what a workspace outgrows is kept until
+ *    the stream's workspace is released.  A cfg with split_k = 1 uses none; dtas_gemm_f16_static
  *    never allocates.  dtas_gemm_q8_f16_fused keeps a second buffer of that kind
  *    (an fp16 copy of the weights it was given) under the same rules;
  *  - `cfg` selects the kernel variant and launch shape explicitly (what one row of the
