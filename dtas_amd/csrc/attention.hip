@@ -954,9 +954,7 @@ extern "C" int dtas_attn_pv_f16(const void* P, const void* V, void* out, int64_t
       const bool in_halves = half_runs == 4 || (half_runs == 2 && heads * n * 4 >= 3 * kNumCU / 4);  // (40 heads of 80 against 3500 keys: whole in 4 runs 11.8, halves in 2 12.2)
       if (in_halves) runs = half_runs;
       const int64_t run_cols = in_halves ? d / 2 : d;
-      bool in_runs = runs >= 2 && pieces <= 128 && m >= 3072;
-      if (!in_runs && in_halves && m >= 2304 && (runs == 4 || n >= 2))  // (without a workspace under capture: one of the forms below)
-        in_runs = split_scratch_at_hand(static_cast<hipStream_t>(stream), static_cast<size_t>(heads * n * d * runs) * sizeof(float), static_cast<size_t>(2 * heads * n));
+      const bool in_runs = runs >= 2 && pieces <= 128 && (m >= 3072 || (in_halves && m >= 2304 && (runs == 4 || n >= 2)));
       // one row, more of the row kernel's workgroups (a piece each) than CUs: the fewest pieces per workgroup with which
       // every CU has at most one.  A 16-byte piece costs a CU's L1 its whole 128-byte line, and the CU with two such
       // workgroups ends last.  V from memory, us, 32 heads of 80: 1024 / 2048 / 2250 keys 6.4 / 8.6 / 9.2, the row kernel

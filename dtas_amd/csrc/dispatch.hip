@@ -222,7 +222,7 @@ dtas_config gemm_policy(int64_t M_hi, int64_t N, int64_t K) {
   const int64_t n = N > 0 ? N : 1, k = K > 0 ? K : 1;
   const int64_t ktiles = ceil_div(k, 64);
   dtas_config wide;
-  if (M_hi > 128 && tile8_policy(M_hi, n, k, true, true, &wide)) return wide;
+  if (M_hi > 128 && tile8_policy(M_hi, n, k, true, &wide)) return wide;
   GemmChoice best = {1e30, 64, 64, 256, 4, 1};
   auto consider = [&](double us, int bm, int bn, int block, int stages, int split) {
     if (us < best.us) best = {us, bm, bn, block, stages, split};

@@ -61,6 +61,6 @@ int resolve_static_scratch(void** out);
 // *unsplit tiles (whole rounds of the chip) get one workgroup each, the rest *nsplit workgroups each (1 = none).
 void tail_split_256(int64_t M, int64_t N, int64_t K, int* nsplit, unsigned* unsplit);
 // the tile of a GEMM of more than 128 rows, and the parts of K; false: none holds the extents
-bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table, dtas_config* out, double* us = nullptr);
+bool tile8_policy(int64_t M, int64_t N, int64_t K, bool in_table, dtas_config* out, double* us = nullptr);
 
 }  // namespace dtas

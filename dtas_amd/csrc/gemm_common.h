@@ -44,7 +44,6 @@ extern std::recursive_mutex g_ws_mutex;
 // (the caller keeps it until its kernel is enqueued).
 int split_scratch(hipStream_t s, size_t bytes, size_t split_tiles, int nsplit, float** partials, unsigned** arrivals,
                   std::unique_lock<std::recursive_mutex>* lock);
-bool split_scratch_at_hand(hipStream_t s, size_t bytes, size_t split_tiles);
 // The stream's buffer for a rewritten operand (g_ws_mutex held by the caller until the launches that use it are enqueued).
 int operand_workspace(hipStream_t stream, size_t bytes, void** out);
 // Where a launch that splits K keeps its partial tiles when the caller must not allocate: set (per host thread) by
@@ -82,9 +81,8 @@ int launch_gemm_share_q8(int rows, int cols, hipStream_t s, const half_t* A, con
 bool share_leads(int64_t M, int64_t N, int64_t K, int* rows, int* cols);
 bool share_leads_q8(int64_t M, int64_t N, int64_t K, int* rows, int* cols);
 // ---- what a call without a config runs: gemm_tiles.hip; gemm_q8.hip (false: the dequantiser into a buffer, then the fp16 GEMM)
-dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok, bool may_split);
-bool gemm_scratch_at_hand(hipStream_t s, int64_t M, int64_t N, int64_t K, const dtas_config& cfg);
-bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_ok, bool may_split, dtas_config* cfg);
+dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok);
+bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_ok, dtas_config* cfg);
 // DTAS_GEMM_MFMA_ACC16: the accumulator rounded to fp16 after every k step of 16 (cfg.vec 8: 16-byte operand loads, else elements)
 int launch_gemm_acc16(const dtas_config& cfg, hipStream_t s, const half_t* A, const half_t* W, const GemmEpilogue& ep, void* C,
                       int64_t M, int64_t N, int64_t K);

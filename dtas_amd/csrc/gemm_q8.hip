@@ -26,7 +26,7 @@ constexpr TileQ8Cost kTileQ8Cost[] = {
     {192, 128, 512, 0, 4.9, 0.789, 0, 0.73, 2.73, 1.87, 1.5, 1.01, 0.09, 0.15},
     {256, 128, 512, 0, 4.95, 1.015, 0, 0.71, 2.92, 2.41, 1.98, 0.99, 0, 0.14},
 };
-double tile_q8_policy(int64_t M, int64_t N, int64_t K, bool may_split, dtas_config* out) {
+double tile_q8_policy(int64_t M, int64_t N, int64_t K, dtas_config* out) {
   const int64_t ktiles = ceil_div(K, kBK);
   const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
   double best = 1e300;
@@ -38,7 +38,7 @@ double tile_q8_policy(int64_t M, int64_t N, int64_t K, bool may_split, dtas_conf
                      (1.0 + c.few / static_cast<double>(tm) - c.pad * (1.0 - static_cast<double>(M) / static_cast<double>(tm * c.bm)));
     for (int parts = 1; parts <= 8; ++parts) {
       // (K <= 768: a launch is mostly its start, and a hand-over costs what the shorter loop saves: 128 x 2048 x 768 8.6 us whole, 11.3 in three)
-      if (parts > 1 && (!may_split || ktiles <= 12 || tiles * parts > limit || ktiles / parts < (c.block == 256 ? 4 : 6) ||
+      if (parts > 1 && (ktiles <= 12 || tiles * parts > limit || ktiles / parts < (c.block == 256 ? 4 : 6) ||
                         tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) break;
       const int64_t wgs = tiles * parts, full = wgs / kNumCU, rem = wgs % kNumCU;
       const double steps = static_cast<double>(ceil_div(ktiles, parts)), share = static_cast<double>(wgs) / kNumCU;
@@ -60,7 +60,7 @@ double tile_q8_policy(int64_t M, int64_t N, int64_t K, bool may_split, dtas_conf
 
 // What a call without a config runs; false: the dequantiser into a library-owned buffer, then the fp16 GEMM.  stream_ok: the
 // kernels that stream the bytes of W can take the call (16-byte aligned operands, K % 256 == 0, K < 2^24); vec_ok: the tiles can.
-bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_ok, bool may_split, dtas_config* out) {
+bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_ok, dtas_config* out) {
   dtas_config& cfg = *out;
   // Few rows of A: the launch is one read of the bytes of W.
   // up to 96 rows: every CU an equal share of W's rows, nothing handed over (share_leads_q8)
@@ -92,10 +92,10 @@ bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_o
   cfg = dtas_config{DTAS_GEMM_MFMA, 256, 8, 3, {128, 128, kBK}, 1, 0};
   const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128);
   if (!vec_ok) return M <= 512 && t128 <= kNumCU;  // (the element kernel, or the two passes, whose second can run on whole vectors)
-  const double us = tile_q8_policy(M, N, K, may_split, &cfg);
+  const double us = tile_q8_policy(M, N, K, &cfg);
   dtas_config wide;
   double us16 = 0.;
-  return !(M > 128 && tile8_policy(M, N, K, true, false, &wide, &us16) && 5.3 + 0.415e-6 * static_cast<double>(N) * static_cast<double>(K) + 0.907 * us16 < us);
+  return !(M > 128 && tile8_policy(M, N, K, false, &wide, &us16) && 5.3 + 0.415e-6 * static_cast<double>(N) * static_cast<double>(K) + 0.907 * us16 < us);
 }
 }  // namespace dtas
 
@@ -130,14 +130,12 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
   dtas_config cfg;
   if (user) {
     cfg = *user;
-  } else if (!builtin_gemm_q8(M, N, K, stream_ok, vec_ok, true, &cfg)) {
+  } else if (!builtin_gemm_q8(M, N, K, stream_ok, vec_ok, &cfg)) {
     void* wbuf = nullptr;
     std::lock_guard<std::recursive_mutex> ws_lock(g_ws_mutex);  // until both launches are enqueued
     if (operand_workspace(static_cast<hipStream_t>(stream), static_cast<size_t>(N) * K * 2, &wbuf) != 0) return -1;
     if (dtas_decode_q8_f16(Wq, scale, wbuf, N, K, nullptr, stream) != 0) return -1;
     return dtas_gemm_f16_fused(A, wbuf, bias, res1, res2, C, M, N, K, epilogue, nullptr, stream);
-  } else if (!gemm_scratch_at_hand(static_cast<hipStream_t>(stream), M, N, K, cfg)) {
-    (void)tile_q8_policy(M, N, K, false, &cfg);  // a first call under capture cannot allocate the workspace: whole tiles then
   }
   hipStream_t s = static_cast<hipStream_t>(stream);
   const half_t* a = static_cast<const half_t*>(A);

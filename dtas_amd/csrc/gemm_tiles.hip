@@ -326,7 +326,7 @@ constexpr Tile8Cost kTile8Cost[] = {
     {224, 256, 512, 0, false, 5.85, 1.317, 1.9, 0.56, 1.66, 4.2, 4.84, 1.05, 0.3, 0.36},
     {256, 256, 512, 2, true, 6.98, 1.505, 0.41, 0.48, -4, 5.88, 5, 1.02, 0.28, 0.34},
 };
-bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table, dtas_config* out, double* us_out) {
+bool tile8_policy(int64_t M, int64_t N, int64_t K, bool in_table, dtas_config* out, double* us_out) {
   const int64_t ktiles = ceil_div(K, kBK);
   const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
   double best = 1e300;
@@ -345,8 +345,8 @@ bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table
       if (whole_rounds) {
         tail_split_256(M, N, K, &last_parts, &unsplit);
         // (inside dtas_gemm_f16_static: only as many partial tiles as there is room for)
-        if (!may_split || (!in_table && t_fixed_scratch && (tiles - unsplit) * last_parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) last_parts = 1;
-      } else if (parts > 1 && (!may_split || tiles * parts > slots || ktiles / parts < (in_table ? 8 : 6) ||
+        if (!in_table && t_fixed_scratch && (tiles - unsplit) * last_parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES) last_parts = 1;
+      } else if (parts > 1 && (tiles * parts > slots || ktiles / parts < (in_table ? 8 : 6) ||
                                tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) {
         break;  // (no more partial tiles than dtas_gemm_f16_static has room for)
       }
@@ -379,23 +379,9 @@ bool tile8_policy(int64_t M, int64_t N, int64_t K, bool may_split, bool in_table
   return true;
 }
 
-// Whether the partial tiles of `cfg` have a place to go on stream `s` (true where it splits nothing; split_k == 0 on the
-// 8-wavefront 256x256 tile splits the last round's).
-bool gemm_scratch_at_hand(hipStream_t s, int64_t M, int64_t N, int64_t K, const dtas_config& cfg) {
-  if (cfg.variant != DTAS_GEMM_MFMA) return true;
-  const int64_t tile = static_cast<int64_t>(cfg.tile[0]) * cfg.tile[1];
-  int nsplit = cfg.split_k;
-  unsigned unsplit = 0;
-  if (cfg.split_k == 0 && cfg.block == 512 && cfg.tile[0] == 256 && cfg.tile[1] == 256) tail_split_256(M, N, K, &nsplit, &unsplit);
-  if (nsplit <= 1) return true;
-  const size_t split_tiles = static_cast<size_t>(ceil_div(M, cfg.tile[0]) * ceil_div(N, cfg.tile[1]) - unsplit);
-  return split_scratch_at_hand(s, split_tiles * nsplit * tile * sizeof(float), split_tiles);
-}
-
 // What a call without a config runs: the bucket's row, or ahead of it a kernel chosen by M itself (what A costs it goes
 // with M, and the row is sized for the end of its bucket).  vec_ok: 16-byte loads of A and W are possible.
-// may_split: partial tiles have a place to go (what needs none otherwise).
-dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok, bool may_split) {
+dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok) {
   // two rows of A (the first bucket's table row is sized for 16): W streamed in whole rows, as the GEMV does
   if (M == 2 && vec_ok) return dtas_config{DTAS_GEMM_ROWS, 64, 8, 1, {2, N <= 2560 ? 1 : 2, 8}, 1, 0};
   // three or four rows: the row kernel, a row of W per wavefront, against a W too small or too short for the share kernel
@@ -408,7 +394,7 @@ dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok, bool may_
   int rows = 0, cols = 0;
   if (vec_ok && share_leads(M, N, K, &rows, &cols)) return dtas_config{DTAS_GEMM_SHARE, 256, 8, 1, {rows, cols, 0}, 1, 0};
   dtas_config cfg;
-  if (M > 128 && vec_ok && tile8_policy(M, N, K, may_split, false, &cfg)) return cfg;
+  if (M > 128 && vec_ok && tile8_policy(M, N, K, false, &cfg)) return cfg;
   return builtin_config(DTAS_OP_GEMM_F16, M, N, K).cfg;
 }
 
@@ -426,14 +412,14 @@ extern "C" int dtas_builtin_gemm(int weights_8bit, int64_t M, int64_t N, int64_t
   if (weights_8bit) {
     if (K % 32 != 0) return fail("dtas_builtin_gemm: K must be a multiple of the scale group, 32 (K=%lld)", (long long)K);
     what = "gemm_q8";
-    if (builtin_gemm_q8(M, N, K, K % 256 == 0, N <= ((int64_t{1} << 32) - 1) / K, true, &out->config)) {
+    if (builtin_gemm_q8(M, N, K, K % 256 == 0, N <= ((int64_t{1} << 32) - 1) / K, &out->config)) {
       snprintf(out->name, sizeof(out->name), "%s", what);
       return 0;  // (launch_args stay zero: the 8-bit kernels' grids are their launchers')
     }
     what = "decode_q8 + gemm";
   }
   snprintf(out->name, sizeof(out->name), "%s", what);
-  out->config = builtin_gemm(M, N, K, K % 8 == 0, true);
+  out->config = builtin_gemm(M, N, K, K % 8 == 0);
   if (K % 8 != 0) out->config.vec = 1;
   return describe_gemm(M, N, K, out->config, out->launch_args);
 }
@@ -480,9 +466,7 @@ extern "C" int dtas_gemm_f16_fused(const void* A, const void* W, const void* bia
   const GemmEpilogue ep = {static_cast<const half_t*>(bias), static_cast<const half_t*>(res1),
                            static_cast<const half_t*>(res2), epilogue, out_bytes == 4 ? 1 : 0, 0.f, 0, 0, 0, 0};
   const bool vec_ok = K % 8 == 0 && aligned(A, 16) && aligned(W, 16);
-  dtas_config cfg = user ? *user : builtin_gemm(M, N, K, vec_ok, true);
-  // a first call under capture cannot allocate the workspace: whole tiles then
-  if (!user && M > 128 && vec_ok && !gemm_scratch_at_hand(static_cast<hipStream_t>(stream), M, N, K, cfg)) cfg = builtin_gemm(M, N, K, vec_ok, false);
+  dtas_config cfg = user ? *user : builtin_gemm(M, N, K, vec_ok);
   if (cfg.vec == 8 && !vec_ok) cfg.vec = 1;  // K % 8 != 0 or odd pointers: element accesses
   int64_t la[7];
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;

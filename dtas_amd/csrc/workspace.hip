@@ -20,7 +20,8 @@ namespace {
 //  * the split-K workspace: nsplit fp32 partial tiles per shared output tile and one arrival counter per tile
 //    (zero between launches: the last arriver of a tile re-arms it);
 //  * the operand buffer: the fp16 copy of an 8-bit weight matrix (dtas_gemm_q8_f16_fused's two-pass route).
-// Allocated on first use by a stream and grown on demand -- the only allocations in the library.  A buffer that
+// Allocated on first use by a stream and grown on demand -- the only allocations in the library -- also while the stream is
+// being captured, so that a call takes the same kernel, and gives the same bits, eagerly and from a graph.  A buffer that
 // was outgrown stays until its set is released: a recorded graph, or a launch that still runs, may hold its address.  Each one
 // is at least twice the one before it while the limit allows, so what is kept stays below twice what is in use.  Launches on
 // one stream are ordered by it and share its set; launches on different streams use different sets, so they may overlap.
@@ -54,7 +55,16 @@ __global__ void zero_u32_kernel(unsigned* p, size_t count) {
   if (i < count) p[i] = 0u;
 }
 
+// Allocating and releasing are no work of a stream, but in the capture mode that a thread starts with they are an error, and
+// the end of the capture, while any stream is being captured.  (tried under all three modes of capture: no part of the graph)
+struct RelaxedCapture {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+  ~RelaxedCapture() { (void)hipThreadExchangeStreamCaptureMode(&mode); }
+};
+
 int release_workspace(StreamWorkspace& w) {
+  RelaxedCapture relaxed;
   // kernels of earlier launches may still use the buffers: hipFree waits for the device
   if (w.partials && hipFree(w.partials) != hipSuccess) return fail("workspace: hipFree of the split-K partials failed");
   w.partials = nullptr;
@@ -75,6 +85,7 @@ int grow(StreamWorkspace& w, void** buffer, size_t* have, size_t need, size_t fi
   if (want < first) want = first;
   if (want > limit) want = limit;
   if (*buffer && w.outgrown_count == kMaxOutgrown) return fail("workspace: outgrown too often");
+  RelaxedCapture relaxed;
   void* fresh = nullptr;
   if (hipMalloc(&fresh, want) != hipSuccess) {
     (void)hipGetLastError();
@@ -113,6 +124,22 @@ int stream_workspace(hipStream_t stream, StreamWorkspace** out) {
   return 0;
 }
 
+// Arrival counters start at zero.  Cleared by a kernel (a memset recorded into a caller's graph is what a fill kernel avoids) on a
+// stream of its own, and waited for: recorded on a stream that is being captured it would run with the graph, not now.
+int clear_counters(unsigned* counters, size_t count) {
+  RelaxedCapture relaxed;
+  hipStream_t own = nullptr;
+  if (hipStreamCreateWithFlags(&own, hipStreamNonBlocking) != hipSuccess) {
+    (void)hipGetLastError();
+    return fail("gemm: no stream to clear the split-K counters on");
+  }
+  hipLaunchKernelGGL(zero_u32_kernel, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(count), 256))), dim3(256), 0, own, counters, count);
+  int rc = check_launch("gemm");
+  if (hipStreamSynchronize(own) != hipSuccess && rc == 0) rc = fail("gemm: clearing the split-K counters failed");
+  (void)hipStreamDestroy(own);
+  return rc;
+}
+
 int split_workspace(hipStream_t stream, size_t partial_bytes, size_t tiles, float** partials, unsigned** arrivals) {
   StreamWorkspace* w = nullptr;
   if (stream_workspace(stream, &w) != 0) return -1;
@@ -125,11 +152,7 @@ int split_workspace(hipStream_t stream, size_t partial_bytes, size_t tiles, floa
     w->tiles = 0;  // (until they are cleared)
     if (grow(*w, &counters, &bytes, tiles * sizeof(unsigned), 4096 * sizeof(unsigned), SIZE_MAX) != 0) return -1;
     w->arrivals = static_cast<unsigned*>(counters);
-    // cleared on the stream that will use them (a clear on the default stream is not ordered with a non-blocking
-    // stream), and by a kernel: a memset node recorded into a caller's graph is what a fill kernel avoids
-    const size_t count = bytes / sizeof(unsigned);
-    hipLaunchKernelGGL(zero_u32_kernel, dim3(static_cast<unsigned>(ceil_div(static_cast<int64_t>(count), 256))), dim3(256), 0, stream, w->arrivals, count);
-    if (check_launch("gemm") != 0) return -1;
+    if (clear_counters(w->arrivals, bytes / sizeof(unsigned)) != 0) return -1;
     w->tiles = bytes / sizeof(unsigned);
   }
   *partials = w->partials;
@@ -173,22 +196,6 @@ int split_scratch(hipStream_t s, size_t bytes, size_t split_tiles, int nsplit, f
   if (bytes > kMaxSplitWsBytes) return fail("gemm: split_k %d needs %zu bytes of workspace (limit %zu)", nsplit, bytes, kMaxSplitWsBytes);
   *lock = std::unique_lock<std::recursive_mutex>(g_ws_mutex);
   return split_workspace(s, bytes, split_tiles, partials, arrivals);
-}
-
-// Whether split_scratch would find room without allocating, or may allocate: false only while `s` is being captured.
-bool split_scratch_at_hand(hipStream_t s, size_t bytes, size_t split_tiles) {
-  if (t_fixed_scratch) return true;
-  std::lock_guard<std::recursive_mutex> lock(g_ws_mutex);
-  int dev = 0;
-  if (hipGetDevice(&dev) == hipSuccess && dev >= 0 && dev < kMaxDevices)
-    for (const StreamWorkspace& w : g_ws[dev].slot)
-      if (w.used && w.stream == s && w.partial_bytes >= bytes && w.tiles >= split_tiles) return true;
-  hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-  if (hipStreamIsCapturing(s, &capturing) != hipSuccess) {  // (the default stream, while another one is captured: as before, the allocation says)
-    (void)hipGetLastError();
-    return true;
-  }
-  return capturing == hipStreamCaptureStatusNone;
 }
 
 // The device address of the static scratch array on the current device.  hipGetSymbolAddress is asked once per

@@ -28,9 +28,11 @@
  *    ordered by it, launches on different streams use different workspaces and may overlap; the
  *    library holds its lock from looking a workspace up to enqueueing the launch, so host threads may
  *    share a stream.  At most 16 streams per device hold one (the one used longest ago is released
- *    first, which waits for the device).  A recorded HIP graph holds the workspace's address: the
- *    first split launch on a stream belongs before the recording; what a workspace outgrows is kept until
- *    the stream's workspace is released.  A cfg with split_k = 1 uses none; dtas_gemm_f16_static
+ *    first, which waits for the device).  All of this also while the stream is being captured: a call
+ *    runs the same kernels, and gives the same bits, eagerly and from a graph.  A recorded graph holds
+ *    the workspace's address: what a workspace outgrew is kept until the stream's workspace is released
+ *    (as the seventeenth stream's takes its place), and a replay must not overlap other launches that
+ *    use the workspace of the stream it was recorded on.  A cfg with split_k = 1 uses none; dtas_gemm_f16_static
  *    never allocates.  dtas_gemm_q8_f16_fused keeps a second buffer of that kind
  *    (an fp16 copy of the weights it was given) under the same rules;
  *  - `cfg` selects the kernel variant and launch shape explicitly (what one row of the
@@ -400,7 +402,7 @@ int dtas_gemv_q8_f32(const void* x, const void* Wq, const void* scale, void* y, 
  * a tile and meet in the split-K workspace as in dtas_gemm_f16.  One row with a bias or GELU epilogue goes to
  * dtas_gemv_q8_f16.  With cfg == NULL: M <= 32 (M <= 64 while N / 64 x K / 512 workgroups fit one round of the chip) takes the W-streaming kernel where it
  * applies; beyond that the tile kernel dequantises in its W path (64x64 and 128x64 tiles of three stages or the 512-thread
- * tiles, K in 1 .. 8 parts with at most 32 MiB of partial tiles, or whole on a captured stream without a workspace) until a fitted
+ * tiles, K in 1 .. 8 parts with at most 32 MiB of partial tiles) until a fitted
  * cost model puts the two-pass route ahead, at 800 .. 1300 rows for most W:
  * dtas_decode_q8_f16 into a per-device fp16 buffer of its own (allocated on first use, grown on demand, at most
  * 1 GiB; same sharing rule as the split-K workspace), then dtas_gemm_f16_fused. */

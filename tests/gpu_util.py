@@ -1,7 +1,5 @@
 """Helpers of the GPU parity tests: seeded inputs made on the CPU (so the oracle and the kernel see
 the same bits), guard bands around device outputs, explicit call-table rows."""
-import ctypes
-
 import numpy as np
 import torch
 
@@ -51,25 +49,3 @@ def assert_bits_equal(got: np.ndarray, want: np.ndarray, nan_ok: bool = False) -
     else:
         bad = np.nonzero(bits(got).ravel() != bits(want).ravel())[0]
         assert bad.size == 0, f"{bad.size} elements differ, first at {bad[:5]}: {got.ravel()[bad[:5]]} vs {want.ravel()[bad[:5]]}"
-
-
-def new_stream():
-    """A stream that no workspace belongs to: torch's own come from a pool, where an earlier test may have had this one."""
-    handle = ctypes.c_void_p()
-    assert _lib.lib().hipStreamCreateWithFlags(ctypes.byref(handle), 1) == 0   # (found in the runtime that the library is linked to; 1: non-blocking)
-    return torch.cuda.ExternalStream(handle.value)
-
-
-def replays_of(stream, launch, out, replays=3):
-    """What three replays of a graph recorded on `stream` leave in `out`, an eager launch on another stream in between."""
-    graph, got = torch.cuda.CUDAGraph(), []
-    torch.cuda.synchronize()
-    with torch.cuda.graph(graph, stream=stream):
-        launch()
-    for _ in range(replays):
-        out.zero_()
-        graph.replay()
-        torch.cuda.synchronize()
-        got.append(out.cpu().numpy())
-        launch()
-    return got

@@ -5,7 +5,7 @@ import pytest
 import torch
 
 from dtas_amd import _lib, ops
-from gpu_util import Guarded, assert_bits_equal, cfg, dev, new_stream, replays_of
+from gpu_util import Guarded, assert_bits_equal, cfg, dev
 
 RTOL, ATOL = 1e-2, 2e-3
 # (rows, columns, k tiles of W that the LDS holds; 2: the ring of five operand units)
@@ -128,82 +128,6 @@ def test_8_bit_weights_without_a_config(M, N, K, epilogue):
     S = sum(t.double().abs() for t in (mm, bias.expand(M, N), *(r for r in res if r is not None))).cpu().numpy()
     got, want = out.check().astype(np.float64), want.cpu().numpy().astype(np.float64)
     assert (np.abs(got - want) <= 2.0 ** -8 * S).all()
-
-
-@pytest.mark.gpu
-def test_a_first_call_under_capture_splits_nothing():
-    # a stream without a workspace that is being captured: whole tiles instead of an allocation
-    M, N, K = 200, 2560, 10240
-    assert _lib.builtin_gemm(M, N, K).config.split_k > 1
-    a, w, _ = (dev(x) for x in _inputs(M, N, K, 1))
-    eager, out = (torch.zeros(M, N, dtype=torch.float16, device="cuda") for _ in range(2))
-    ops.gemm(a, w, None, eager)
-    stream = torch.cuda.Stream()
-    graph = torch.cuda.CUDAGraph()
-    torch.cuda.synchronize()
-    with torch.cuda.graph(graph, stream=stream):
-        ops.gemm(a, w, None, out)
-    for _ in range(3):
-        out.zero_()
-        graph.replay()
-        torch.cuda.synchronize()
-        assert float((out.float() - eager.float()).abs().max()) <= 2.0 ** -9 * float(eager.float().abs().max())
-        ops.gemm(a, w, None, eager)
-
-
-def _last_round_split(N, K):
-    """The most rows up to 6000 whose call without a config splits only the last round of 256x256 tiles (split_k 0), over
-    more partial tiles than the 32 MiB that the first launch of a stream allocates."""
-    for M in range(6000, 1000, -1):
-        info = _lib.builtin_gemm(M, N, K)
-        tiles = -(-M // 256) * -(-N // 256)
-        if info.config.split_k == 0 and (info.launch_args[0] - tiles + tiles % 256) * 256 * 256 * 4 > 32 << 20 and info.launch_args[0] > tiles:
-            return M
-    raise AssertionError("no size splits its last round")
-
-
-def _whole(run, M, N, *configs):
-    """The results of whole tiles: those of 8 wavefronts all add along K in one order, those of 4 in another."""
-    outs = [torch.zeros(M, N, dtype=torch.float16, device="cuda") for _ in configs]
-    for out, c in zip(outs, configs):
-        run(out, c)
-    return [out.cpu().numpy() for out in outs]
-
-
-@pytest.mark.gpu
-@pytest.mark.parametrize("tail,room", [(False, "none"), (True, "none"), (True, "too small")])
-def test_a_first_call_under_capture_runs_whole_tiles(tail, room):
-    # also where only the last round of 256x256 tiles is split, and on a stream whose workspace would have to grow
-    N, K = (4096, 11008) if tail else (2560, 10240)
-    M = _last_round_split(N, K) if tail else 200
-    c = _lib.builtin_gemm(M, N, K).config
-    assert tail or c.split_k > 1
-    a, w, _ = (dev(x) for x in _inputs(M, N, K, 1))
-    out, split_up = (torch.zeros(M, N, dtype=torch.float16, device="cuda") for _ in range(2))
-    ops.gemm(a, w, None, split_up, c)
-    whole = _whole(lambda out, c: ops.gemm(a, w, None, out, c), M, N, _cfg(128, 128, 4), cfg(variant=_lib.GEMM_MFMA, unroll=4, tile=[64, 64, 64]))
-    stream = new_stream()
-    if room == "too small":
-        torch.cuda.synchronize()
-        with torch.cuda.stream(stream):
-            ops.gemm(a[:200], w, None, out[:200], _cfg(128, 64, 4, 2))
-    for got in replays_of(stream, lambda: ops.gemm(a, w, None, out), out):
-        assert any(np.array_equal(got, x) for x in whole) and not np.array_equal(got, split_up.cpu().numpy())
-
-
-@pytest.mark.gpu
-def test_a_first_8_bit_call_under_capture_runs_whole_tiles():
-    M, N, K = 203, 2560, 10240
-    c = _lib.builtin_gemm(M, N, K, q8=True).config
-    assert c.variant == _lib.GEMM_MFMA and c.split_k > 1
-    a, _, bias = (dev(x) for x in _inputs(M, N, K, 2))
-    wq, scale = _q8(N, K, 3)
-    words, scale = torch.from_numpy(wq.view(np.int32)).cuda(), dev(scale)
-    out, split_up = (torch.zeros(M, N, dtype=torch.float16, device="cuda") for _ in range(2))
-    ops.gemm_q8(a, words, scale, bias, split_up, c)
-    whole = _whole(lambda out, c: ops.gemm_q8(a, words, scale, bias, out, c), M, N, _cfg(128, 128, 0), cfg(variant=_lib.GEMM_MFMA, unroll=3, tile=[64, 64, 64]))
-    for got in replays_of(new_stream(), lambda: ops.gemm_q8(a, words, scale, bias, out), out):
-        assert any(np.array_equal(got, x) for x in whole) and not np.array_equal(got, split_up.cpu().numpy())
 
 
 def test_every_tile_describes_its_launch_and_nothing_else_is_taken():
