@@ -195,16 +195,15 @@ dtas_config gemv_policy(int64_t N, int64_t K) {
 // GEMM: more than 128 rows: tile8_policy (gemm_tiles.hip).  Up to 128 rows: a cost model fitted to sweeps of every tile x
 // stage count x K split over M on an MI355X.
 // A candidate's time is (rounds of workgroups over the chip) x (time of one k tile) x (k tiles):
-//  * time of one k tile with every CU busy: 256x256 1.50 us, 256x128 (8 wavefronts) 1.00 us, 128x128
-//    0.665 us with 4 stages (one workgroup per CU) or 1.14 us per round of two per CU with 2 stages;
+//  * time of one k tile with every CU busy: 128x128 0.665 us with 4 stages (one workgroup per CU) or 1.14 us per round of two
+//    per CU with 2 stages;
 //  * a partly filled last round is faster than a full one: x (0.55 + 0.45 * fill); 128x128 with 4
 //    stages in a single round gains less: x (0.8 + 0.2 * fill);
 //  * 64x64: 0.33 us per k tile up to 256 workgroups, x 0.82 * (workgroups on the fullest CU) beyond;
 //  * 128x64 (4 stages, one workgroup per CU at most): 0.47 us per k tile whatever the fill;
 //  * few tiles: K split over up to 4 workgroups per tile, each partial tile costing the last
 //    workgroup ~4 us (128x128), ~2.5 us (128x64), ~1 us (64x64; 2.5 us with more than one per CU)
-//    to add up; 256x128 splits while its workgroups fit one round and each keeps 32 k tiles or
-//    more (~4.5 us per partial tile: 512 x 5120 x 13824 in 3 parts 86.8 us against 98.2 for 256x256, 640 x 4096 x 8192 in 2 parts 63.8 against 67.3);
+//    to add up;
 //  * a floor: W (2NK bytes) streams at 3.1 .. 4.3 TB/s depending on the tile (few rows against a very wide W);
 //  * M <= 32: the W-streaming SKINNY kernel, whose time grows with N*K (about 3.5 TB/s of W).
 struct GemmChoice {
@@ -231,49 +230,8 @@ dtas_config gemm_policy(int64_t M_hi, int64_t N, int64_t K) {
   const double kt = static_cast<double>(ktiles);
   // no candidate is faster than it streams W: TB/s measured at M = 64 against a 50280 x 2560 W
   const double w_mb = 2.0 * static_cast<double>(n) * static_cast<double>(k) * 1e-6;
-  // (candidates that all sit on the floor are told apart by their own estimates: 256 x 32000 x 4096, 125 tiles of 256x256
-  // 89.0 us, 250 of 256x128 74.4)
+  // (candidates that all sit on the floor are told apart by their own estimates)
   auto floored = [&](double us, double tbs) { return (us > w_mb / tbs ? us : w_mb / tbs) + 1e-3 * us; };
-  auto relief = [](double fill) { return fill <= 0.5 ? 0.63 : 0.63 + 0.74 * (fill - 0.5); };
-  {
-    // 256x256 on 8 wavefronts (16x16x32 MFMA): a round of the chip costs ~8 us plus 1.50 us per k tile with every CU
-    // busy; with half of the CUs or fewer busy the card clocks higher and a k tile takes 0.63 of that, linearly in
-    // between.  split_k = 0: the tiles of a partly filled last round are shared by 2..4 workgroups each
-    // (tail_split_256), which costs ~15 / 18 / 21 us to combine the partial tiles.
-    const int64_t tiles = static_cast<int64_t>(tiles_of(256, 256));
-    const int64_t full = tiles / kNumCU, rem = tiles % kNumCU;
-    double us = static_cast<double>(full) * (8.0 + 1.50 * kt);
-    if (rem > 0) {
-      int split = 1;
-      unsigned unsplit = 0;
-      tail_split_256(M_hi, n, k, &split, &unsplit);
-      if (split >= 2)
-        us += 8.0 + 1.50 * static_cast<double>(ceil_div(ktiles, split)) * relief(static_cast<double>(rem * split) / kNumCU) + 12.0 + 3.0 * (split - 1);
-      else
-        us += 8.0 + 1.50 * kt * relief(static_cast<double>(rem) / kNumCU);
-    }
-    consider(floored(us, 3.5), 256, 256, 512, 2, 0);
-  }
-  {
-    // 192x256 on 8 wavefronts (96x64 each, the same loop): 1.18 us per k tile with every CU busy -- as many flops per us
-    // as 256x256 -- and the same relief in a partly filled round; there for the tile counts it fills the chip better
-    // with (M = 4096 against N = 2560: 220 tiles where 256x256 makes 160, 196 against 219 us at K = 10240; 3072 x 4096:
-    // 256 tiles against 192; 2048 x 10240: 440 against 320)
-    const int64_t tiles = static_cast<int64_t>(tiles_of(192, 256));
-    const int64_t full = tiles / kNumCU, rem = tiles % kNumCU;
-    double us = static_cast<double>(full) * (8.0 + 1.18 * kt);
-    if (rem > 0) us += 8.0 + 1.18 * kt * relief(static_cast<double>(rem) / kNumCU);
-    consider(floored(us, 3.5), 192, 256, 512, 2, 1);
-  }
-  // 256x128 on 8 wavefronts (64x64 each, the 16x16x32 ring loop): 1.00 us per k tile against 1.045 us on 4 wavefronts
-  consider(floored(gemm_rounds(tiles_of(256, 128), kNumCU) * 1.0 * kt, 3.5), 256, 128, 512, 2, 1);
-  // 192x128 on 8 wavefronts (48x64 each), where its tiles fill three quarters of the chip or more in one round: ~6 us plus
-  // 0.66 us per k tile (2048 x 2560 x 2560: 220 tiles, 29.8 us against 32.6 for the 160 tiles of 256x128; 1536 x 4096 x 4096:
-  // 48.2 against 49.7).  With fewer tiles the split tiles are ahead of what this model says of them (1024 x 2560 x 4096:
-  // 37.0 against 31.3), a second round costs it more than its share (1536 x 11008 x 4096: 164 against 145), and past 64 k
-  // tiles each one takes it 0.8 us (1536 x 4096 x 11008: 144 against 138 for 256x256)
-  if (tiles_of(192, 128) <= kNumCU && tiles_of(192, 128) * 4 >= 3 * kNumCU && kt <= 64)
-    consider(floored(6.0 + gemm_rounds(tiles_of(192, 128), kNumCU) * 0.66 * kt, 3.5), 192, 128, 512, 2, 1);
   consider(floored(gemm_rounds(tiles_of(128, 128), 2 * kNumCU) * 1.14 * kt, 3.1), 128, 128, 256, 2, 1);
   for (int split = 1; split <= 4; ++split) {
     // (K <= 1024: a launch is mostly its start, and a hand-over costs what the shorter loop saves: 512 x 1024 x 1024 7.8 us whole, 8.6 in two parts)
@@ -283,9 +241,6 @@ dtas_config gemm_policy(int64_t M_hi, int64_t N, int64_t K) {
     if (split == 1 || t128 <= kNumCU)
       consider(floored((t128 <= kNumCU ? 0.8 + 0.2 * t128 / kNumCU : gemm_rounds(t128, kNumCU)) * 0.665 * steps + (split > 1 ? 4.0 * split : 0.0), split > 1 ? 3.5 : 4.1), 128, 128, 256, 4, split);   // (in K parts W streams slower: 128 x 14336 x 4096 in two parts 39.1 us, 3.0 TB/s)
     consider(floored((t64 <= kNumCU ? 1.0 : 0.82 * static_cast<double>(ceil_div(static_cast<int64_t>(t64), kNumCU))) * 0.33 * steps + (split > 1 ? (t64 <= kNumCU ? 1.0 : 2.5) * split : 0.0), 4.3), 64, 64, 256, 4, split);
-    const double t256128 = tiles_of(256, 128) * split;
-    if (split > 1 && steps >= 32 && t256128 <= kNumCU)
-      consider(floored(gemm_rounds(t256128, kNumCU) * 1.0 * steps + 4.5 * split, 3.5), 256, 128, 512, 2, split);
     const double t12864 = tiles_of(128, 64) * split;
     if (t12864 <= kNumCU)
       consider(floored(0.47 * steps + (split > 1 ? 2.5 * split : 0.0), 3.8), 128, 64, 256, 4, split);   // (128 x 8192 x 8192 in two parts: 38.4 us, 3.5 TB/s of W)

@@ -102,17 +102,13 @@ class MFMAConfigEmiter(BaseConfigEmiter):
 
     def preferred(self, m_hi: int, N: int, K: int = 4096):
         """(tile_m, tile_n, stages, split_k, threads) under the cost models fitted to sweeps on an MI355X (the same
-        ones the library's built-in table uses).  Beyond 128 rows: tile8_policy.  Up to 128 rows: time = rounds of workgroups over the chip x time of one
-        k tile x k tiles.  One k tile with every CU busy: 256x256 see below, 256x128 (8 wavefronts of 64x64) 1.00 us,
-        128x128 0.665 us (4 stages, one workgroup per CU) or 1.14 us per round of two per CU (2 stages);
-        a partly filled last round costs 0.55 + 0.45 * fill of a full one (0.8 + 0.2 * fill for 128x128 with 4 stages
-        in a single round); 64x64 0.33 us per k tile up to
-        one workgroup per CU, x 0.82 * (workgroups on the fullest CU) beyond; with few tiles K is split over up
-        to 4 workgroups per tile at ~4 us (128x128) / ~1 us (64x64; 2.5 us with more than one per CU) per partial
-        tile; 128x64 (4 stages, at most one workgroup per CU) 0.47 us per k tile whatever the fill and ~2.5 us
-        per partial tile; 256x128 splits too while its workgroups fit one round and each keeps 32 k tiles or
-        more (~4.5 us per partial tile: 512 x 5120 x 13824 in 3 parts 86.8 us against 98.2 for 256x256, 640 x 4096 x 8192 in 2 parts
-        63.8 against 67.3).  No candidate is faster than W (2NK bytes) streams through it: 3.1 .. 4.3 TB/s
+        ones the library's built-in table uses).  Beyond 128 rows: tile8_policy.  Up to 128 rows: time = rounds of workgroups
+        over the chip x time of one k tile x k tiles.  One k tile with every CU busy: 128x128 0.665 us (4 stages, one workgroup
+        per CU) or 1.14 us per round of two per CU (2 stages); a partly filled round costs 0.55 + 0.45 * fill of a full
+        one (0.8 + 0.2 * fill for 128x128 with 4 stages in a single round); 64x64 0.33 us per k tile up to one workgroup per CU,
+        x 0.82 * (workgroups on the fullest CU) beyond; with few tiles K is split over up to 4 workgroups per tile at ~4 us
+        (128x128) / ~1 us (64x64; 2.5 us with more than one per CU) per partial tile; 128x64 (4 stages, at most one workgroup
+        per CU) 0.47 us per k tile whatever the fill and ~2.5 us per partial tile.  No candidate is faster than W (2NK bytes) streams through it: 3.1 .. 4.3 TB/s
         by tile, measured with 64 rows against a 50280 x 2560 W."""
         if m_hi > 128:
             wide = self.tile8_policy(m_hi, N, K)
@@ -130,30 +126,7 @@ class MFMAConfigEmiter(BaseConfigEmiter):
         w_mb = 2.0 * float(N) * float(K) * 1e-6
         # W streams at 3.1 .. 4.3 TB/s, by tile; candidates that all sit on that floor are told apart by their own estimates
         floored = lambda us, tbs: (us if us > w_mb / tbs else w_mb / tbs) + 1e-3 * us
-        # 256x256 on 8 wavefronts: ~8 us per round of the chip plus 1.50 us per k tile with every CU busy, 0.63 of that
-        # with half of the CUs or fewer busy (the card clocks higher), linear in between; split_k = 0: the tiles of
-        # a partly filled last round are shared by 2..4 workgroups each (~15 / 18 / 21 us to combine)
-        t256 = tiles(256, 256)
-        full, rem = divmod(t256, cus)
-        relief = lambda fill: 0.63 if fill <= 0.5 else 0.63 + 0.74 * (fill - 0.5)
-        us256 = full * (8.0 + 1.50 * ktiles)
-        if rem:
-            split, _ = self.tail_split_256(m_hi, N, K)
-            if split >= 2:
-                us256 += 8.0 + 1.50 * cdiv(ktiles, split) * relief(rem * split / cus) + 12.0 + 3.0 * (split - 1)
-            else:
-                us256 += 8.0 + 1.50 * ktiles * relief(rem / cus)
-        # 192x256 on 8 wavefronts (96x64 each): 1.18 us per k tile with every CU busy, the same relief
-        full192, rem192 = divmod(tiles(192, 256), cus)
-        us192 = full192 * (8.0 + 1.18 * ktiles) + ((8.0 + 1.18 * ktiles * relief(rem192 / cus)) if rem192 else 0.0)
-        cands = [(floored(us256, 3.5), (256, 256, 2, 0)),
-                 (floored(us192, 3.5), (192, 256, 2, 1)),
-                 (floored(rounds(tiles(256, 128), cus) * 1.0 * ktiles, 3.5), (256, 128, 2, 1))]
-        # 192x128 on 8 wavefronts (48x64 each), one round that fills three quarters of the chip or more: ~6 us plus
-        # 0.66 us per k tile up to 64 of them
-        if 3 * cus <= 4 * tiles(192, 128) <= 4 * cus and ktiles <= 64:
-            cands.append((floored(6.0 + rounds(tiles(192, 128), cus) * 0.66 * ktiles, 3.5), (192, 128, 2, 1)))
-        cands.append((floored(rounds(tiles(128, 128), 2 * cus) * 1.14 * ktiles, 3.1), (128, 128, 2, 1)))
+        cands = [(floored(rounds(tiles(128, 128), 2 * cus) * 1.14 * ktiles, 3.1), (128, 128, 2, 1))]
         for split in (1, 2, 3, 4):
             if split > 1 and (ktiles // split < 8 or ktiles <= 16):    # (K <= 1024: a hand-over costs what the shorter loop saves)
                 continue
@@ -165,9 +138,6 @@ class MFMAConfigEmiter(BaseConfigEmiter):
             cands.append((floored((1.0 if t64 <= cus else 0.82 * -(-int(t64) // cus)) * 0.33 * steps
                                   + ((1.0 if t64 <= cus else 2.5) * split if split > 1 else 0.0), 4.3),
                           (64, 64, 4, split)))
-            t256128 = tiles(256, 128) * split
-            if split > 1 and steps >= 32 and t256128 <= cus:
-                cands.append((floored(rounds(t256128, cus) * 1.0 * steps + 4.5 * split, 3.5), (256, 128, 2, split)))
             t12864 = tiles(128, 64) * split
             if t12864 <= cus:
                 cands.append((floored(0.47 * steps + (2.5 * split if split > 1 else 0.0), 3.8), (128, 64, 4, split)))
@@ -177,7 +147,7 @@ class MFMAConfigEmiter(BaseConfigEmiter):
                 best = c
         self._model_us = best[0]
         tm, tn, stages, split = best[1]
-        return tm, tn, stages, split, 512 if stages == 2 and (tm, tn) in ((256, 256), (192, 256), (256, 128), (192, 128)) else 256
+        return tm, tn, stages, split, 256
 
     def tail_split_256(self, M: int, N: int, K: int):
         """(parts, tiles left whole) for split_k = 0 on the 8-wavefront 256x256 tile: whole rounds of the chip
