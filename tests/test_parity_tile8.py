@@ -130,6 +130,81 @@ def test_8_bit_weights_without_a_config(M, N, K, epilogue):
     assert (np.abs(got - want) <= 2.0 ** -8 * S).all()
 
 
+def _among_nans(t):
+    """The same elements in a buffer that holds NaN before and behind them (200 rows of them behind)."""
+    flat = torch.full((t.numel() + 200 * t.shape[-1] + 512,), float("nan"), dtype=t.dtype, device="cuda")
+    flat[512:512 + t.numel()] = t.reshape(-1)
+    return flat[512:512 + t.numel()].view(t.shape)
+
+
+def _check_non_finite(run, a, N):
+    """What lies around the operands reaches no result; NaN and infinities in the last rows of A and W reach their row and
+    column and no other element: every other one has the bits it has without them."""
+    M = a.shape[0]
+    clean = run(_among_nans(a))
+    assert np.isfinite(clean.astype(np.float64)).all()
+    bad = a.clone()
+    bad[M - 1, a.shape[1] - 1] = float("nan")
+    bad[0, 0] = float("inf")
+    got = run(_among_nans(bad), True)
+    assert np.isnan(got[M - 1]).all() and np.isnan(got[:, N - 1]).all() and not np.isfinite(got[0].astype(np.float64)).any()
+    assert_bits_equal(got[1:M - 1, :N - 1], clean[1:M - 1, :N - 1])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn,stages", TILES)
+def test_non_finite_operands_at_the_edges_of_every_tile(bm, bn, stages):
+    # (K = 200: the last k tile is a chunk of 8 wide, the next row's elements and what lies behind the last row follow it)
+    for M, N, K, split in ((bm + 3, bn + 5, 200, 1), (bm - 7, 2 * bn - 3, 1096, 2)):
+        a, w, _ = (dev(x) for x in _inputs(M, N, K, M))
+
+        def run(a, poison=False):
+            wn = w.clone()
+            if poison:
+                wn[N - 1, K - 1] = float("nan")
+            out = Guarded((M, N), torch.float16)
+            ops.gemm(a, _among_nans(wn), None, out.t, _cfg(bm, bn, stages, split))
+            return out.check()
+
+        _check_non_finite(run, a, N)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn", Q8_TILES)
+def test_non_finite_operands_at_the_edges_of_every_8_bit_tile(bm, bn):
+    # (tiles of 96 and 160 rows load A in whole 64-row steps: the rows in between are past the tile and must not be read)
+    for M, N, K, split in ((bm + 3, bn + 5, 224, 1), (2 * bm - 7, bn - 3, 1120, 2)):
+        a = dev(_inputs(M, N, K, M)[0])
+        wq, scale = _q8(N, K, M)
+        words, scale = torch.from_numpy(wq.view(np.int32)).cuda(), dev(scale)
+
+        def run(a, poison=False):
+            sn = scale.clone()
+            if poison:
+                sn[N - 1, K // 32 - 1] = float("nan")
+            out = Guarded((M, N), torch.float16)
+            ops.gemm_q8(a, words, _among_nans(sn), None, out.t, _cfg(bm, bn, 0, split))
+            return out.check()
+
+        _check_non_finite(run, a, N)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("q8,bm,bn,stages", [(False, *t) for t in TILES] + [(True, bm, bn, 0) for bm, bn in Q8_TILES])
+def test_a_part_of_k_without_a_k_tile(oracle, q8, bm, bn, stages):
+    # 5 k tiles in 4 parts of 2: the last part has none and adds zeros
+    M, N, K = bm + 9, bn + 7, 288
+    a, w, bias = _inputs(M, N, K, bm * bn)
+    out = Guarded((M, N), torch.float16)
+    if q8:
+        wq, scale = _q8(N, K, bm)
+        w = oracle.c.decode_q8(wq, scale, threads=8)
+        ops.gemm_q8(dev(a), torch.from_numpy(wq.view(np.int32)).cuda(), dev(scale), dev(bias), out.t, _cfg(bm, bn, 0, 4))
+    else:
+        ops.gemm(dev(a), dev(w), dev(bias), out.t, _cfg(bm, bn, stages, 4))
+    _check(out.check(), oracle.c.gemm(a, w, bias, threads=8), oracle.np64.gemm(a, w, bias))
+
+
 def test_every_tile_describes_its_launch_and_nothing_else_is_taken():
     for bm, bn, stages in TILES:
         info = _lib.describe_launch(_lib.OP_GEMM_F16, 1000, 3000, 4096, _lib.DtasConfig.from_dict(
