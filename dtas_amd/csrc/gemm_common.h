@@ -80,6 +80,15 @@ int launch_gemm_share_q8(int rows, int cols, hipStream_t s, const half_t* A, con
                          int64_t N, int64_t K);
 bool share_leads(int64_t M, int64_t N, int64_t K, int* rows, int* cols);
 bool share_leads_q8(int64_t M, int64_t N, int64_t K, int* rows, int* cols);
+// ---- the pitch of A's and W's rows (K fp16 elements), as the tiles' cost models see it.  us per k tile beside K + 64, operands from
+// memory, 2048 x 4096 x K on 256x128 / 1024 x 4096 x K on 128x128: rows 3, 5, 6, 10, 12, 20, 24 KiB apart 1.04 / 0.61 (K = 5120), 0.97 / 0.59 (6144), 1.00 /
+// 0.61 (10240) where others take 0.85 .. 0.89 / 0.54 .. 0.57, a power of two 0.83 / 0.51: few memory channels serve one k tile, or many.
+enum RowPitch { kPitchPlain, kPitchSlow, kPitchPow2 };
+inline RowPitch row_pitch(int64_t K) {
+  const int64_t odd = K > 0 ? K >> __builtin_ctzll(static_cast<unsigned long long>(K)) : 0;
+  if (odd == 1 && K >= 2048) return kPitchPow2;
+  return K % 512 == 0 && (odd == 3 || odd == 5) ? kPitchSlow : kPitchPlain;
+}
 // ---- what a call without a config runs: gemm_tiles.hip; gemm_q8.hip (false: the dequantiser into a buffer, then the fp16 GEMM)
 dtas_config builtin_gemm(int64_t M, int64_t N, int64_t K, bool vec_ok);
 bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_ok, dtas_config* cfg);

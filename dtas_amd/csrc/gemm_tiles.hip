@@ -49,6 +49,8 @@
 // The kernels for few rows of A (SKINNY, STREAM, ROWS) are in gemm_stream.hip, the attention kernels in attention.hip,
 // the 8-bit-weight entry point in gemm_q8.hip, the split-K workspace in workspace.hip; the tile kernel itself is the
 // template in gemm_tile_kernel.h.
+#include <utility>
+
 #include "gemm_tile_kernel.h"
 
 namespace dtas {
@@ -255,7 +257,7 @@ int launch_tile_f16(const dtas_config& cfg, hipStream_t s, const half_t* a, cons
   if (cfg.block == 512) {  // 8 wavefronts on the 16x16x32 loop
 #define DTAS_TILE8(BM_, BN_, WM_, WN_, NS_) \
     if (bm == BM_ && bn == BN_ && (NS_ > 2 || (ns == 2 && tile8_ring(bm, bn)))) return launch_mfma<BM_, BN_, WM_, WN_, NS_, false, false, true>(s, a, w, b, c, M, N, K, sk, batch)
-    DTAS_TILE8(256, 128, 4, 2, 2);  // the rings of two stages: by a config only, but for 192x256 (tile8_policy)
+    DTAS_TILE8(256, 128, 4, 2, 2);  // the rings of two stages: by a config only, but for 192x256 (kTile8Cost)
     DTAS_TILE8(128, 256, 2, 4, 2);
     DTAS_TILE8(192, 256, 2, 4, 2);
     DTAS_TILE8(192, 128, 4, 2, 2);
@@ -296,87 +298,115 @@ int launch_tile_f16(const dtas_config& cfg, hipStream_t s, const half_t* a, cons
 //   rounds of the chip x (a + b x k tiles of a part), a partly filled round at b x (r + (1 - r) x its share of the chip),
 //   + w x workgroups per CU + h0 + h1 x parts + h2 x (share of the chip)^4 where K is split (the hand-over of the partial tiles),
 // with b growing with 1 / (tile rows of the grid) (fewer workgroups share what W costs to bring in), falling with the rows past M
-// in the tiles (nothing is loaded for them), and x pitch where W's rows lie 5, 6, 10, .. KiB apart.  (64x64, of which a CU holds
-// several, at r + (1 - r) x its share up to one per CU and at 0.75 per workgroup of the fullest CU beyond.)  Fitted to 600 sizes (M =
-// 129 .. 8192 against 26 W of 512 x 2048 .. 50280 x 2560, W from memory) x up to 40 configurations each; h0 of the 8-wavefront tiles 1.8 us
-// above the fit and 64x64's hand-over as before the fit: in a layer, where other kernels run in between, a hand-over costs more than
-// in a loop over one kernel (140 x 2560 x 10240 in 3 parts of 128x64 33.9 us there, 27.5 in the loop; 64x64 in 2 parts 30.0 / 29.1).
-// In the bucket table (`in_table`): the tiles marked so, K in up to 4 parts of 8 k tiles or more (1.03 of the best
-// configuration's time on average); for a call without a config also the tiles between them, where no more than a fifth of
-// their rows lie past M or they make at most three rows of tiles, and up to 6 parts of 6 k tiles (1.012; over 260 random sizes
-// 0.93 of the time before these kernels).
+// in the tiles (nothing is loaded for them), and x pitch or pow2 by K's row_pitch.  (64x64, of which a CU holds
+// several, at r + (1 - r) x its share up to one per CU and at 0.75 per workgroup of the fullest CU beyond.)
+// Fitted to 537 sizes (M = 129 .. 8192 against 27 W of 512 x 2048 .. 50280 x 2560) x up to 14 configurations each, A, W and C all
+// taken from memory: that is what a launch between other kernels costs.  With one A kept for all launches the staged tiles look
+// up to 13 % better than in a pass (2048 x 4096 x 11008: 256x128 whole 150 us so and 169 with A from memory, 256x256 with the tiles
+// in two parts 155 either way, and a pass of three products 14 us shorter with the latter; 150 x 2560 x 10240: 128x64 in three
+// parts 26 / 34, 64x64 in two 29 / 30, a layer 3.6 us shorter).
+// In the bucket table (`in_table`): the tiles marked so, K in up to 4 parts of 8 k tiles or more (1.036 of the best configuration's time on
+// average).  For a call without a config also the tiles between them, where no more than a fifth of their rows lie past M or
+// they make at most three rows of tiles, and up to 6 parts of 6 k tiles: 1.007 (1.026 with the fit to one A).  Up to two rows of tiles
+// those take K in parts only if they are ahead by 0.46 us a part: what is nearer is left to the table's tile (0.001 of the time).
 struct Tile8Cost {
   int bm, bn, block, stages;
   bool in_table;
-  double a, b, w, r, h0, h1, h2, pitch, few, pad;
+  double a, b, w, r, h0, h1, h2, pitch, pow2, few, pad;
 };
 constexpr Tile8Cost kTile8Cost[] = {
-    {64, 64, 256, 4, true, 3.74, 0.243, 0.42, 0.71, 1, 1, 0.3, 1.03, 0.8, 0.16},
-    {128, 64, 512, 0, true, 4.02, 0.326, 0, 0.69, 3.14, 0.57, 0.51, 1.08, 0.65, 0.71},
-    {96, 128, 512, 0, false, 3.9, 0.435, 0, 0.68, 2.66, 0.96, 1.87, 1.12, 0.8, 0.53},
-    {128, 128, 512, 0, true, 4.06, 0.501, 0.21, 0.62, 2.59, 1.2, 2.98, 1.11, 0.8, 0.74},
-    {160, 128, 512, 0, false, 4.58, 0.599, 0, 0.64, 2.97, 1.41, 3.14, 1.1, 0.54, 0.71},
-    {192, 128, 512, 0, true, 4.52, 0.673, 0.49, 0.65, 2.68, 1.81, 3.93, 1.08, 0.46, 0.66},
-    {224, 128, 512, 0, false, 4.2, 0.755, 1.33, 0.63, 2.51, 2.3, 2.67, 1.06, 0.36, 0.59},
-    {256, 128, 512, 0, true, 4.1, 0.827, 1.96, 0.66, 2.03, 2.65, 3.96, 1.06, 0.26, 0.52},
-    {96, 256, 512, 0, false, 3.85, 0.717, 0.83, 0.7, 3.49, 1.73, 2.44, 1.16, 0.8, 0.16},
-    {128, 256, 512, 0, false, 3.71, 0.835, 2.06, 0.66, 3.25, 2.39, 3.21, 1.15, 0.71, 0.48},
-    {160, 256, 512, 0, false, 5.21, 1.02, 0.65, 0.57, 2.21, 3.07, 3.96, 1.11, 0.49, 0.48},
-    {192, 256, 512, 0, true, 5.19, 1.152, 2.05, 0.59, 2.39, 3.56, 3.96, 1.11, 0.37, 0.33},
-    {224, 256, 512, 0, false, 5.85, 1.317, 1.9, 0.56, 1.66, 4.2, 4.84, 1.05, 0.3, 0.36},
-    {256, 256, 512, 2, true, 6.98, 1.505, 0.41, 0.48, -4, 5.88, 5, 1.02, 0.28, 0.34},
+    {64, 64, 256, 4, true, 3.57, 0.29, 0.478, 0.717, 0.524, 0.734, 0.129, 1.088, 1.009, 0.574, 0.47},
+    {128, 64, 512, 0, true, 2.631, 0.403, 1.476, 0.909, 2.034, 0.637, 0.653, 1.108, 0.961, 0.203, 0.153},
+    {96, 128, 512, 0, false, 3.519, 0.476, 0.746, 0.809, 1.266, 0.975, 1.735, 1.107, 0.98, 0.614, 0.623},
+    {128, 128, 512, 0, true, 3.291, 0.544, 1.551, 0.823, 0.877, 1.463, 2.133, 1.071, 0.951, 0.485, 0.404},
+    {160, 128, 512, 0, false, 3.721, 0.611, 0.409, 0.902, 1.024, 1.727, 4.122, 1.08, 0.968, 0.377, 0.217},
+    {192, 128, 512, 0, true, 4.008, 0.677, 0.586, 0.909, 1.074, 2.066, 5.196, 1.085, 0.974, 0.301, 0.201},
+    {224, 128, 512, 0, false, 4.428, 0.766, 0, 0.849, 2.076, 2.391, 3.818, 1.088, 0.968, 0.232, 0.231},
+    {256, 128, 512, 0, true, 5.651, 0.874, 0, 0.737, 1.586, 2.705, 3.646, 1.051, 0.932, 0.223, 0.316},
+    {96, 256, 512, 0, false, 3.125, 0.722, 1.919, 0.88, 1.049, 1.981, 2.592, 1.096, 0.96, 0.948, 0.41},
+    {128, 256, 512, 0, false, 5.289, 0.846, 0, 0.692, 0.862, 2.651, 2.37, 1.081, 0.954, 0.889, 0.566},
+    {160, 256, 512, 0, false, 5.914, 0.99, 0.447, 0.675, -0.599, 3.146, 6.082, 1.054, 0.979, 0.584, 0.593},
+    {192, 256, 512, 0, true, 7.283, 1.152, 0.273, 0.69, 0.249, 2.667, 7.583, 1.039, 0.966, 0.497, 0.537},
+    {224, 256, 512, 0, false, 7.123, 1.294, 0.808, 0.652, 1.88, 2.796, 4.098, 1.025, 0.983, 0.407, 0.415},
+    {256, 256, 512, 2, true, 8.473, 1.449, 0.41, 0.613, -1.316, 4.31, 8.162, 1.011, 0.984, 0.311, 0.395},
+    {192, 256, 512, 2, true, 6.715, 1.142, 0.592, 0.663, 2.39, 3.56, 3.96, 1.063, 0.96, 0.508, 0.209},
 };
-bool tile8_policy(int64_t M, int64_t N, int64_t K, bool in_table, dtas_config* out, double* us_out) {
-  const int64_t ktiles = ceil_div(K, kBK);
-  const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
-  double best = 1e300;
-  for (const Tile8Cost& c : kTile8Cost) {
-    if (!c.in_table && (in_table || (ceil_div(M, c.bm) > 3 && M * 5 < ceil_div(M, c.bm) * c.bm * 4))) continue;
-    if (K * 2 * (c.bm > c.bn ? c.bm : c.bn) >= (int64_t{1} << 31)) continue;  // (32-bit tile offsets, describe_gemm)
-    const int64_t tm = ceil_div(M, c.bm), tn = ceil_div(N, c.bn), tiles = tm * tn;
-    if (tiles > 0x7fffffff / 8) continue;
-    const bool whole_rounds = c.bm == 256 && c.bn == 256;  // its split is of the last round's tiles (tail_split_256)
-    const int64_t slots = c.bm * c.bn <= 64 * 64 ? 2 * kNumCU : kNumCU;
-    const double b = c.b * (odd_pitch ? c.pitch : 1.0) *
-                     (1.0 + c.few / static_cast<double>(tm) - c.pad * (1.0 - static_cast<double>(M) / static_cast<double>(tm * c.bm)));
-    for (int parts = 1; parts <= (in_table ? 4 : 6); ++parts) {
-      int last_parts = parts;
-      unsigned unsplit = 0;
-      if (whole_rounds) {
-        tail_split_256(M, N, K, &last_parts, &unsplit);
-        // (inside dtas_gemm_f16_static: only as many partial tiles as there is room for)
-        if (!in_table && t_fixed_scratch && (tiles - unsplit) * last_parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES) last_parts = 1;
-      } else if (parts > 1 && (tiles * parts > slots || ktiles / parts < (in_table ? 8 : 6) ||
-                               tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) {
-        break;  // (no more partial tiles than dtas_gemm_f16_static has room for)
-      }
-      const bool tail = whole_rounds && last_parts > 1;
-      const int64_t wgs = whole_rounds ? tiles : tiles * parts, full = wgs / slots, rem = wgs % slots;
-      const double steps = static_cast<double>(whole_rounds ? ktiles : ceil_div(ktiles, parts));
-      const double share = static_cast<double>(wgs) / kNumCU;
-      double us = static_cast<double>(full) * (c.a + b * steps) + c.w * share;
-      const double fill = static_cast<double>(whole_rounds ? rem * last_parts : rem) / static_cast<double>(slots);
-      if (slots > kNumCU)  // (64x64: two or more workgroups share a CU)
-        us = c.a + b * steps * (wgs <= kNumCU ? c.r + (1.0 - c.r) * share : 0.75 * static_cast<double>(ceil_div(wgs, kNumCU))) + c.w * share;
-      else if (rem > 0) us += c.a + b * (whole_rounds ? static_cast<double>(ceil_div(ktiles, last_parts)) : steps) * (c.r + (1.0 - c.r) * fill);
-      if (last_parts > 1) {
-        const double crowd = whole_rounds ? fill : share;
-        us += c.h0 + c.h1 * last_parts + c.h2 * crowd * crowd * crowd * crowd;
-      }
-      if (us < best) {
-        best = us;
-        *out = dtas_config{DTAS_GEMM_MFMA, c.block, 8, c.stages, {c.bm, c.bn, kBK}, tail ? 0 : parts, 0};
-      }
-      if (whole_rounds) break;
+// 192x256 comes twice: W in three stages and A in two, and (stages 2) as a ring, which leads where rows lie a power of two apart
+// (2890 x 4096 x 4096: 0.956 of the time, 3001 x 4096 x 8192 0.961, K whole) and is level or behind elsewhere (1024 x 7680 x 2560 1.10, 2561 x 2560 x
+// 10240 1.07), so that only those rows look at it.
+
+// One row of the table against M x N x K (instantiated per row: the divisions by its extents are multiplications).
+struct Tile8Query {
+  int64_t M, N, K, ktiles;
+  int64_t steps[7];  // k tiles of the longest of p parts
+  bool in_table;
+  RowPitch pitch;
+  int tail_parts;    // 256x256: parts of the last round's tiles
+  int64_t tail_whole;
+};
+template <int I>
+inline void tile8_consider(const Tile8Query& q, double* best, dtas_config* out) {
+  constexpr Tile8Cost c = kTile8Cost[I];
+  constexpr int64_t kBig = c.bm > c.bn ? c.bm : c.bn, slots = c.bm * c.bn <= 64 * 64 ? 2 * kNumCU : kNumCU;
+  constexpr bool whole_rounds = c.bm == 256 && c.bn == 256;  // its split is of the last round's tiles (tail_split_256)
+  constexpr bool ring_192 = c.bm == 192 && c.stages == 2;
+  if (ring_192 && q.pitch != kPitchPow2) return;
+  const int64_t tm = ceil_div(q.M, c.bm), tn = ceil_div(q.N, c.bn), tiles = tm * tn;
+  if (!c.in_table && (q.in_table || (tm > 3 && q.M * 5 < tm * c.bm * 4))) return;
+  if (q.K * 2 * kBig >= (int64_t{1} << 31)) return;  // (32-bit tile offsets, describe_gemm)
+  if (tiles > 0x7fffffff / 8) return;
+  const double b = c.b * (q.pitch == kPitchSlow ? c.pitch : q.pitch == kPitchPow2 ? c.pow2 : 1.0) *
+                   (1.0 + c.few / static_cast<double>(tm) - c.pad * (1.0 - static_cast<double>(q.M) / static_cast<double>(tm * c.bm)));
+  const int most = whole_rounds || ring_192 ? 1 : q.in_table ? 4 : 6;
+  for (int parts = 1; parts <= most; ++parts) {
+    int last_parts = parts;
+    if (whole_rounds) {
+      last_parts = q.tail_parts;
+      // (inside dtas_gemm_f16_static: only as many partial tiles as there is room for)
+      if (!q.in_table && t_fixed_scratch && (tiles - q.tail_whole) * last_parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES) last_parts = 1;
+    } else if (parts > 1 && (tiles * parts > slots || q.ktiles < parts * (q.in_table ? 8 : 6) ||
+                             tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) {
+      break;  // (no more partial tiles than dtas_gemm_f16_static has room for)
+    }
+    const bool tail = whole_rounds && last_parts > 1;
+    const int64_t wgs = whole_rounds ? tiles : tiles * parts, full = wgs / slots, rem = wgs % slots;
+    const double steps = static_cast<double>(whole_rounds ? q.ktiles : q.steps[parts]);
+    const double share = static_cast<double>(wgs) / kNumCU;
+    double us = static_cast<double>(full) * (c.a + b * steps) + c.w * share;
+    const double fill = static_cast<double>(whole_rounds ? rem * last_parts : rem) / static_cast<double>(slots);
+    if (slots > kNumCU)  // (64x64: two or more workgroups share a CU)
+      us = c.a + b * steps * (wgs <= kNumCU ? c.r + (1.0 - c.r) * share : 0.75 * static_cast<double>(ceil_div(wgs, kNumCU))) + c.w * share;
+    else if (rem > 0) us += c.a + b * (whole_rounds ? static_cast<double>(q.steps[last_parts]) : steps) * (c.r + (1.0 - c.r) * fill);
+    if (last_parts > 1) {
+      const double crowd = whole_rounds ? fill : share;
+      us += c.h0 + c.h1 * last_parts + c.h2 * crowd * crowd * crowd * crowd;
+    }
+    if (!c.in_table && tm <= 2 && parts > 1) us += 0.46 * parts;
+    if (us < *best) {
+      *best = us;
+      *out = dtas_config{DTAS_GEMM_MFMA, c.block, 8, c.stages, {c.bm, c.bn, kBK}, tail ? 0 : parts, 0};
     }
   }
+}
+template <int... I>
+inline void tile8_consider_all(const Tile8Query& q, double* best, dtas_config* out, std::integer_sequence<int, I...>) {
+  (tile8_consider<I>(q, best, out), ...);
+}
+bool tile8_policy(int64_t M, int64_t N, int64_t K, bool in_table, dtas_config* out, double* us_out) {
+  Tile8Query q{M, N, K, ceil_div(K, kBK), {}, in_table, row_pitch(K), 1, 0};
+  q.steps[1] = q.ktiles;
+  q.steps[2] = ceil_div(q.ktiles, 2);
+  q.steps[3] = ceil_div(q.ktiles, 3);
+  q.steps[4] = ceil_div(q.ktiles, 4);
+  q.steps[5] = ceil_div(q.ktiles, 5);
+  q.steps[6] = ceil_div(q.ktiles, 6);
+  unsigned whole = 0;
+  tail_split_256(M, N, K, &q.tail_parts, &whole);
+  q.tail_whole = whole;
+  double best = 1e300;
+  tile8_consider_all(q, &best, out, std::make_integer_sequence<int, sizeof(kTile8Cost) / sizeof(kTile8Cost[0])>{});
   if (us_out) *us_out = best;
-  if (best == 1e300) return false;  // (nothing was written to *out)
-  // 192x256 against rows of W a multiple of 4 KiB apart: W in three stages and A in two, requested in the middle of a k tile,
-  // falls behind the ring of two (700 x 11008 x 4096 78.2 / 71.8 us, 1025 x 8192 x 2048 41.1 / 38.4; ahead elsewhere: 1400 x
-  // 4096 x 11008 152 / 178, 1025 x 7680 x 2560 50.7 / 53.9)
-  if (out->tile[0] == 192 && out->tile[1] == 256 && out->split_k == 1 && K % 2048 == 0) out->unroll = 2;
-  return true;
+  return best < 1e300;  // (else nothing was written to *out)
 }
 
 // What a call without a config runs: the bucket's row, or ahead of it a kernel chosen by M itself (what A costs it goes

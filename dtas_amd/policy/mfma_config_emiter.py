@@ -21,22 +21,23 @@ _TILES = [(4, 2), (2, 4), (2, 2), (1, 2), (2, 1), (1, 1)]
 _TILES8 = {(256, 256): (2, 4), (224, 256): (2, 4), (192, 256): (2, 4), (160, 256): (2, 4), (128, 256): (2, 4), (96, 256): (2, 4),
            (256, 128): (4, 2), (224, 128): (2, 4), (192, 128): (4, 2), (160, 128): (2, 4), (128, 128): (4, 2), (96, 128): (2, 4), (128, 64): (4, 2)}
 # the library's cost model beyond 128 rows (libdtas: kTile8Cost): tile, threads, stages, whether the table's rows name it, and
-# a, b, w, r, h0, h1, h2, pitch, few, pad
+# a, b, w, r, h0, h1, h2, pitch, pow2, few, pad
 _COST8 = [
-    (64, 64, 256, 4, True, 3.74, 0.243, 0.42, 0.71, 1, 1, 0.3, 1.03, 0.8, 0.16),
-    (128, 64, 512, 0, True, 4.02, 0.326, 0, 0.69, 3.14, 0.57, 0.51, 1.08, 0.65, 0.71),
-    (96, 128, 512, 0, False, 3.9, 0.435, 0, 0.68, 2.66, 0.96, 1.87, 1.12, 0.8, 0.53),
-    (128, 128, 512, 0, True, 4.06, 0.501, 0.21, 0.62, 2.59, 1.2, 2.98, 1.11, 0.8, 0.74),
-    (160, 128, 512, 0, False, 4.58, 0.599, 0, 0.64, 2.97, 1.41, 3.14, 1.1, 0.54, 0.71),
-    (192, 128, 512, 0, True, 4.52, 0.673, 0.49, 0.65, 2.68, 1.81, 3.93, 1.08, 0.46, 0.66),
-    (224, 128, 512, 0, False, 4.2, 0.755, 1.33, 0.63, 2.51, 2.3, 2.67, 1.06, 0.36, 0.59),
-    (256, 128, 512, 0, True, 4.1, 0.827, 1.96, 0.66, 2.03, 2.65, 3.96, 1.06, 0.26, 0.52),
-    (96, 256, 512, 0, False, 3.85, 0.717, 0.83, 0.7, 3.49, 1.73, 2.44, 1.16, 0.8, 0.16),
-    (128, 256, 512, 0, False, 3.71, 0.835, 2.06, 0.66, 3.25, 2.39, 3.21, 1.15, 0.71, 0.48),
-    (160, 256, 512, 0, False, 5.21, 1.02, 0.65, 0.57, 2.21, 3.07, 3.96, 1.11, 0.49, 0.48),
-    (192, 256, 512, 0, True, 5.19, 1.152, 2.05, 0.59, 2.39, 3.56, 3.96, 1.11, 0.37, 0.33),
-    (224, 256, 512, 0, False, 5.85, 1.317, 1.9, 0.56, 1.66, 4.2, 4.84, 1.05, 0.3, 0.36),
-    (256, 256, 512, 2, True, 6.98, 1.505, 0.41, 0.48, -4, 5.88, 5, 1.02, 0.28, 0.34),
+    (64, 64, 256, 4, True, 3.57, 0.29, 0.478, 0.717, 0.524, 0.734, 0.129, 1.088, 1.009, 0.574, 0.47),
+    (128, 64, 512, 0, True, 2.631, 0.403, 1.476, 0.909, 2.034, 0.637, 0.653, 1.108, 0.961, 0.203, 0.153),
+    (96, 128, 512, 0, False, 3.519, 0.476, 0.746, 0.809, 1.266, 0.975, 1.735, 1.107, 0.98, 0.614, 0.623),
+    (128, 128, 512, 0, True, 3.291, 0.544, 1.551, 0.823, 0.877, 1.463, 2.133, 1.071, 0.951, 0.485, 0.404),
+    (160, 128, 512, 0, False, 3.721, 0.611, 0.409, 0.902, 1.024, 1.727, 4.122, 1.08, 0.968, 0.377, 0.217),
+    (192, 128, 512, 0, True, 4.008, 0.677, 0.586, 0.909, 1.074, 2.066, 5.196, 1.085, 0.974, 0.301, 0.201),
+    (224, 128, 512, 0, False, 4.428, 0.766, 0, 0.849, 2.076, 2.391, 3.818, 1.088, 0.968, 0.232, 0.231),
+    (256, 128, 512, 0, True, 5.651, 0.874, 0, 0.737, 1.586, 2.705, 3.646, 1.051, 0.932, 0.223, 0.316),
+    (96, 256, 512, 0, False, 3.125, 0.722, 1.919, 0.88, 1.049, 1.981, 2.592, 1.096, 0.96, 0.948, 0.41),
+    (128, 256, 512, 0, False, 5.289, 0.846, 0, 0.692, 0.862, 2.651, 2.37, 1.081, 0.954, 0.889, 0.566),
+    (160, 256, 512, 0, False, 5.914, 0.99, 0.447, 0.675, -0.599, 3.146, 6.082, 1.054, 0.979, 0.584, 0.593),
+    (192, 256, 512, 0, True, 7.283, 1.152, 0.273, 0.69, 0.249, 2.667, 7.583, 1.039, 0.966, 0.497, 0.537),
+    (224, 256, 512, 0, False, 7.123, 1.294, 0.808, 0.652, 1.88, 2.796, 4.098, 1.025, 0.983, 0.407, 0.415),
+    (256, 256, 512, 2, True, 8.473, 1.449, 0.41, 0.613, -1.316, 4.31, 8.162, 1.011, 0.984, 0.311, 0.395),
+    (192, 256, 512, 2, True, 6.715, 1.142, 0.592, 0.663, 2.39, 3.56, 3.96, 1.063, 0.96, 0.508, 0.209),
 ]
 _LDS = 160 * 1024
 
@@ -54,24 +55,38 @@ class MFMAConfigEmiter(BaseConfigEmiter):
     def max_stages(tile_m: int, tile_n: int) -> int:
         return 2 if tile_m + tile_n >= 512 else 3 if tile_m + tile_n >= 384 else 4
 
+    @staticmethod
+    def row_pitch(K: int) -> str:
+        """How far apart rows of K lie, as the cost model sees it (libdtas: row_pitch): 'slow' 3 x 2^j or 5 x 2^j KiB, 'pow2' a
+        power of two from 4 KiB, '' otherwise."""
+        if K >= 2048 and K & (K - 1) == 0:
+            return "pow2"
+        odd = K
+        while odd and odd % 2 == 0:
+            odd //= 2
+        return "slow" if K % 512 == 0 and odd in (3, 5) else ""
+
     def tile8_policy(self, M: int, N: int, K: int):
         """(tile_m, tile_n, stages, split_k, threads) of the table's row beyond 128 rows: the cost model of the library's
         tile8_policy, over the tiles and splits the table's rows name (a host test keeps the two alike)."""
         cdiv = lambda a, b: -(-a // b)
         cus, ktiles = self.arch.num_sm, cdiv(K, 64)
-        odd_pitch = K % 1024 == 0 and (K // 1024) & (K // 1024 - 1) != 0
+        pitch_class = self.row_pitch(K)
         best_us, best = 1e300, None
-        for bm, bn, threads, stages, in_table, a, b0, w, r, h0, h1, h2, pitch, few, pad in _COST8:
+        for bm, bn, threads, stages, in_table, a, b0, w, r, h0, h1, h2, pitch, pow2, few, pad in _COST8:
             if not in_table or K * 2 * max(bm, bn) >= 1 << 31:
                 continue
             tm = cdiv(M, bm)
+            ring_192 = bm == 192 and stages == 2
+            if ring_192 and pitch_class != "pow2":
+                continue
             tiles = tm * cdiv(N, bn)
             if tiles > 0x7fffffff // 8:
                 continue
             whole_rounds = bm == 256 and bn == 256
             slots = 2 * cus if bm * bn <= 64 * 64 else cus
-            b = b0 * (pitch if odd_pitch else 1.0) * (1.0 + few / float(tm) - pad * (1.0 - float(M) / float(tm * bm)))
-            for parts in range(1, 5):
+            b = b0 * (pitch if pitch_class == 'slow' else pow2 if pitch_class == 'pow2' else 1.0) * (1.0 + few / float(tm) - pad * (1.0 - float(M) / float(tm * bm)))
+            for parts in range(1, 2 if ring_192 else 5):
                 last_parts = parts
                 if whole_rounds:
                     last_parts, _ = self.tail_split_256(M, N, K)
@@ -95,8 +110,6 @@ class MFMAConfigEmiter(BaseConfigEmiter):
                     best_us, best = us, (bm, bn, stages, 0 if tail else parts, threads)
                 if whole_rounds:
                     break
-        if best and best[:2] == (192, 256) and best[3] == 1 and K % 2048 == 0:
-            best = (192, 256, 2, 1, 512)
         self._model_us = best_us
         return best
 

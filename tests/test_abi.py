@@ -62,6 +62,25 @@ def test_select_bucket_uses_labelled_ranges():
     assert _lib.select_bucket(_lib.OP_GEMM_F16, 100000, 4096, 4096).index == 511
 
 
+@pytest.mark.parametrize("M,N,K,tile,split,unroll", [
+    # A read from memory, as it is between other kernels: the tiles of 256x256 in two parts, not whole smaller ones ...
+    (2048, 4096, 11008, (256, 256), 0, 2), (1900, 4096, 11008, (256, 256), 0, 2), (1280, 4096, 11008, (256, 256), 0, 2),
+    # ... while K = 8192 keeps these
+    (2048, 4096, 8192, (256, 128), 1, 0),
+    # the estimate is that of the kernel that runs: the ring only where rows lie a power of two apart
+    (4300, 2560, 10240, (192, 256), 1, 0), (2950, 4096, 4096, (192, 256), 1, 2),
+])
+def test_builtin_gemm_choice_with_operands_from_memory(M, N, K, tile, split, unroll):
+    c = _lib.builtin_gemm(M, N, K).config
+    assert (tuple(c.tile)[:2], c.split_k, c.unroll) == (tile, split, unroll)
+
+
+@pytest.mark.parametrize("M", [135, 150, 170, 192])
+def test_builtin_gemm_of_few_rows_against_a_long_k(M):
+    c = _lib.builtin_gemm(M, 2560, 10240).config    # (128x64 in three parts: 34 us with A from memory, 64x64 in two 30)
+    assert (c.tile[0], c.tile[1]) != (128, 64)
+
+
 def test_builtin_gemm_names_what_runs_without_a_config():
     # ahead of the bucket's row: a kernel chosen by M itself
     share = _lib.builtin_gemm(16, 4096, 4096)
