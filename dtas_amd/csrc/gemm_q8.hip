@@ -4,56 +4,72 @@
 // Few rows: the share kernel (gemm_share.hip) or the W-streaming kernel (gemm_stream.hip) on the bytes.  Otherwise the tile
 // kernel with the dequantiser in its W path (template flag WQ, instantiated here), or the dequantiser into a
 // library-owned fp16 buffer followed by the fp16 GEMM.
+#include <utility>
+
 #include "gemm_tile_kernel.h"
 
 namespace dtas {
 namespace {
 // The tiles that dequantise in their W path, by the estimate of tile8_policy (the 4-wavefront tiles, of which a CU holds several:
 // at r + (1 - r) x share of the chip up to one workgroup per CU, and at 0.75 (64x64) or 0.85 (128x64) per workgroup of the fullest
-// CU beyond).  Fitted to 300 sizes (65 .. 2048 rows against fourteen W of 2048 x 768 .. 14336 x 4096, W from memory) x up to 30 configurations:
-// 1.003 of the best one's time at 100 .. 1100 rows, 0.85 .. 0.91 of the time of the 4-wavefront tiles that ran before (203 x 10240 x 2560
-// 34.7 -> 28.0 us, 512 x 7680 x 2560 36.4 -> 30.3, 700 x 2560 x 10240 71.5 -> 55.4); h0 of the 8-wavefront tiles 1.5 us above the fit, as there.
+// CU beyond).  Fitted to 288 sizes (65 .. 2048 rows against 18 W of 1024 x 4096 .. 14336 x 4096) x up to 14 configurations, A, W and C all from
+// memory as there: 1.007 of the best one's time (held-out sizes 1.0075); 0.84 of the time of the 4-wavefront tiles that ran before over 121
+// sizes outside the fit (with one A for all launches: 203 x 10240 x 2560 34.7 -> 28.0 us, 512 x 7680 x 2560 36.4 -> 30.3, 700 x 2560 x 10240 71.5 -> 55.4).
 struct TileQ8Cost {
   int bm, bn, block, stages;
-  double a, b, w, r, h0, h1, h2, pitch, few, pad;
+  double a, b, w, r, h0, h1, h2, pitch, pow2, few, pad;
 };
 constexpr TileQ8Cost kTileQ8Cost[] = {
-    {64, 64, 256, 3, 4.53, 0.333, 0, 0.96, 0.85, 0.53, 0.04, 1, 0.48, 0.14},
-    {128, 64, 256, 3, 4.69, 0.474, 0.19, 0.86, 1.23, 0.67, 0.46, 1.02, 0.11, 0.05},
-    {96, 128, 512, 0, 4.72, 0.508, 0.35, 0.8, 2.45, 0.89, 0.55, 1.02, 0.37, 0.11},
-    {128, 128, 512, 0, 4.3, 0.57, 0.64, 0.75, 2.76, 1.15, 0.91, 1.01, 0.3, 0.17},
-    {160, 128, 512, 0, 3.74, 0.689, 1.35, 0.83, 2.92, 1.46, 1.13, 1.02, 0.15, 0.12},
-    {192, 128, 512, 0, 4.9, 0.789, 0, 0.73, 2.73, 1.87, 1.5, 1.01, 0.09, 0.15},
-    {256, 128, 512, 0, 4.95, 1.015, 0, 0.71, 2.92, 2.41, 1.98, 0.99, 0, 0.14},
+    {64, 64, 256, 3, 4.639, 0.359, 0, 1.012, 0.992, 0.517, 0.058, 1.025, 0.971, 0.424, 0.194},
+    {128, 64, 256, 3, 5.232, 0.483, 0, 0.816, 1.531, 0.623, 0.232, 1.013, 0.959, 0.164, 0.177},
+    {96, 128, 512, 0, 2.475, 0.614, 2.37, 0.981, 1.723, 0.886, 0.959, 1.007, 0.964, 0.183, 0.151},
+    {128, 128, 512, 0, 2.789, 0.648, 2.086, 0.975, 2.187, 1.157, 1.228, 1.024, 0.966, 0.148, 0.243},
+    {160, 128, 512, 0, 4.28, 0.728, 1.15, 0.931, 1.772, 1.527, 1.193, 1.038, 0.987, 0.088, 0.223},
+    {192, 128, 512, 0, 5.329, 0.795, 0.105, 0.875, 1.575, 1.905, 2.063, 1.035, 0.983, 0.081, 0.288},
+    {256, 128, 512, 0, 6.255, 1.019, 0.056, 0.76, 1.622, 2.452, 1.412, 1.042, 0.972, 0.025, 0.256},
 };
-double tile_q8_policy(int64_t M, int64_t N, int64_t K, dtas_config* out) {
-  const int64_t ktiles = ceil_div(K, kBK);
-  const bool odd_pitch = K % 1024 == 0 && ((K / 1024) & (K / 1024 - 1)) != 0;
-  double best = 1e300;
-  for (const TileQ8Cost& c : kTileQ8Cost) {
-    if (K * 2 * (c.bm > c.bn ? c.bm : c.bn) >= (int64_t{1} << 31)) continue;  // (32-bit tile offsets, describe_gemm)
-    const int64_t tm = ceil_div(M, c.bm), tn = ceil_div(N, c.bn), tiles = tm * tn, limit = c.block == 256 ? 2 * kNumCU : kNumCU;
-    if (tiles > 0x7fffffff / 8) continue;
-    const double b = c.b * (odd_pitch ? c.pitch : 1.0) *
-                     (1.0 + c.few / static_cast<double>(tm) - c.pad * (1.0 - static_cast<double>(M) / static_cast<double>(tm * c.bm)));
-    for (int parts = 1; parts <= 8; ++parts) {
-      // (K <= 768: a launch is mostly its start, and a hand-over costs what the shorter loop saves: 128 x 2048 x 768 8.6 us whole, 11.3 in three)
-      if (parts > 1 && (ktiles <= 12 || tiles * parts > limit || ktiles / parts < (c.block == 256 ? 4 : 6) ||
-                        tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) break;
-      const int64_t wgs = tiles * parts, full = wgs / kNumCU, rem = wgs % kNumCU;
-      const double steps = static_cast<double>(ceil_div(ktiles, parts)), share = static_cast<double>(wgs) / kNumCU;
-      double us = c.w * share;
-      if (c.block == 256)
-        us += c.a + b * steps * (wgs <= kNumCU ? c.r + (1.0 - c.r) * share : (c.bm == 64 ? 0.75 : 0.85) * static_cast<double>(ceil_div(wgs, kNumCU)));
-      else
-        us += static_cast<double>(full) * (c.a + b * steps) + (rem > 0 ? c.a + b * steps * (c.r + (1.0 - c.r) * static_cast<double>(rem) / kNumCU) : 0.0);
-      if (parts > 1) us += c.h0 + c.h1 * parts + c.h2 * share * share * share * share;
-      if (us < best) {
-        best = us;
-        *out = dtas_config{DTAS_GEMM_MFMA, c.block, 8, c.stages, {c.bm, c.bn, kBK}, parts, 0};
-      }
+// One row of the table against M x N x K (instantiated per row: the divisions by its extents are multiplications).
+struct TileQ8Query {
+  int64_t M, N, K, ktiles;
+  int64_t steps[9];  // k tiles of the longest of p parts
+  RowPitch pitch;
+};
+template <int I>
+inline void tile_q8_consider(const TileQ8Query& q, double* best, dtas_config* out) {
+  constexpr TileQ8Cost c = kTileQ8Cost[I];
+  constexpr int64_t kBig = c.bm > c.bn ? c.bm : c.bn, limit = c.block == 256 ? 2 * kNumCU : kNumCU;
+  if (q.K * 2 * kBig >= (int64_t{1} << 31)) return;  // (32-bit tile offsets, describe_gemm)
+  const int64_t tm = ceil_div(q.M, c.bm), tn = ceil_div(q.N, c.bn), tiles = tm * tn;
+  if (tiles > 0x7fffffff / 8) return;
+  const double b = c.b * (q.pitch == kPitchSlow ? c.pitch : q.pitch == kPitchPow2 ? c.pow2 : 1.0) *
+                   (1.0 + c.few / static_cast<double>(tm) - c.pad * (1.0 - static_cast<double>(q.M) / static_cast<double>(tm * c.bm)));
+  for (int parts = 1; parts <= 8; ++parts) {
+    // (K <= 768: a launch is mostly its start, and a hand-over costs what the shorter loop saves: 128 x 2048 x 768 8.6 us whole, 11.3 in three)
+    if (parts > 1 && (q.ktiles <= 12 || tiles * parts > limit || q.ktiles < parts * (c.block == 256 ? 4 : 6) ||
+                      tiles * parts * c.bm * c.bn * 4 > DTAS_STATIC_SCRATCH_PARTIAL_BYTES)) break;
+    const int64_t wgs = tiles * parts, full = wgs / kNumCU, rem = wgs % kNumCU;
+    const double steps = static_cast<double>(q.steps[parts]), share = static_cast<double>(wgs) / kNumCU;
+    double us = c.w * share;
+    if (c.block == 256)
+      us += c.a + b * steps * (wgs <= kNumCU ? c.r + (1.0 - c.r) * share : (c.bm == 64 ? 0.75 : 0.85) * static_cast<double>(ceil_div(wgs, kNumCU)));
+    else
+      us += static_cast<double>(full) * (c.a + b * steps) + (rem > 0 ? c.a + b * steps * (c.r + (1.0 - c.r) * static_cast<double>(rem) / kNumCU) : 0.0);
+    if (parts > 1) us += c.h0 + c.h1 * parts + c.h2 * share * share * share * share;
+    if (us < *best) {
+      *best = us;
+      *out = dtas_config{DTAS_GEMM_MFMA, c.block, 8, c.stages, {c.bm, c.bn, kBK}, parts, 0};
     }
   }
+}
+template <int... I>
+inline void tile_q8_consider_all(const TileQ8Query& q, double* best, dtas_config* out, std::integer_sequence<int, I...>) {
+  (tile_q8_consider<I>(q, best, out), ...);
+}
+double tile_q8_policy(int64_t M, int64_t N, int64_t K, dtas_config* out) {
+  const int64_t kt = ceil_div(K, kBK);
+  const TileQ8Query q{M, N, K, kt, {0, kt, ceil_div(kt, 2), ceil_div(kt, 3), ceil_div(kt, 4), ceil_div(kt, 5), ceil_div(kt, 6), ceil_div(kt, 7), ceil_div(kt, 8)}, row_pitch(K)};
+  double best = 1e300;
+  tile_q8_consider_all(q, &best, out, std::make_integer_sequence<int, sizeof(kTileQ8Cost) / sizeof(kTileQ8Cost[0])>{});
   return best;
 }
 }  // namespace
@@ -85,17 +101,16 @@ bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_o
     return true;
   }
   // Two routes.  (1) Dequantising in the W path of the tile kernel: no intermediate, W read once per row of tiles as bytes.
-  // (2) The dequantiser into a library-owned fp16 buffer, then the fp16 GEMM with every tile it has: ~5 us and 3 more bytes per
-  // weight through memory, worth it once the GEMM itself is long (7680 x 2560: from ~1300 rows, 10240 x 2560 ~900).  Its time
-  // against the fit's 300 sizes: 5.3 us + 0.415 per million weights + 0.907 of the fp16 GEMM's estimate (W comes from the cache); the
-  // lesser of the two estimates is the lesser time to 0.1 %.
+  // (2) The dequantiser into a library-owned fp16 buffer, then the fp16 GEMM with every tile it has: 3.4 us and 0.49 per million
+  // weights more, worth it once the GEMM itself is long (7680 x 2560: from ~1300 rows, 10240 x 2560 ~900).  Its time over
+  // the fit's sizes: these + the fp16 GEMM's estimate, to 5 %; the lesser of the two estimates is the lesser time to 0.1 %.
   cfg = dtas_config{DTAS_GEMM_MFMA, 256, 8, 3, {128, 128, kBK}, 1, 0};
   const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128);
   if (!vec_ok) return M <= 512 && t128 <= kNumCU;  // (the element kernel, or the two passes, whose second can run on whole vectors)
   const double us = tile_q8_policy(M, N, K, &cfg);
   dtas_config wide;
   double us16 = 0.;
-  return !(M > 128 && tile8_policy(M, N, K, false, &wide, &us16) && 5.3 + 0.415e-6 * static_cast<double>(N) * static_cast<double>(K) + 0.907 * us16 < us);
+  return !(M > 128 && tile8_policy(M, N, K, false, &wide, &us16) && 3.445 + 0.486e-6 * static_cast<double>(N) * static_cast<double>(K) + 1.002 * us16 < us);
 }
 }  // namespace dtas
 
