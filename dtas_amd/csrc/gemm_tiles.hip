@@ -308,7 +308,8 @@ int launch_tile_f16(const dtas_config& cfg, hipStream_t s, const half_t* a, cons
 // In the bucket table (`in_table`): the tiles marked so, K in up to 4 parts of 8 k tiles or more (1.036 of the best configuration's time on
 // average).  For a call without a config also the tiles between them, where no more than a fifth of their rows lie past M or
 // they make at most three rows of tiles, and up to 6 parts of 6 k tiles: 1.007 (1.026 with the fit to one A).  Up to two rows of tiles
-// those take K in parts only if they are ahead by 0.46 us a part: what is nearer is left to the table's tile (0.001 of the time).
+// those take K in parts of fewer than 24 k tiles only if they are ahead by 0.46 us a part: what is nearer is left to the table's
+// tile (0.001 of the time; longer parts as they come: 135 .. 192 x 2560 x 10240 on 96x128 in six 28.6 us, on 64x64 in two 30.4, in four 30.5 .. 32.6).
 struct Tile8Cost {
   int bm, bn, block, stages;
   bool in_table;
@@ -381,7 +382,7 @@ inline void tile8_consider(const Tile8Query& q, double* best, dtas_config* out) 
       const double crowd = whole_rounds ? fill : share;
       us += c.h0 + c.h1 * last_parts + c.h2 * crowd * crowd * crowd * crowd;
     }
-    if (!c.in_table && tm <= 2 && parts > 1) us += 0.46 * parts;
+    if (!c.in_table && tm <= 2 && parts > 1 && q.ktiles < 24 * parts) us += 0.46 * parts;
     if (us < *best) {
       *best = us;
       *out = dtas_config{DTAS_GEMM_MFMA, c.block, 8, c.stages, {c.bm, c.bn, kBK}, tail ? 0 : parts, 0};
