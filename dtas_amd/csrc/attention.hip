@@ -960,7 +960,9 @@ extern "C" int dtas_attn_pv_f16(const void* P, const void* V, void* out, int64_t
       // workgroups ends last.  V from memory, us, 32 heads of 80: 1024 / 2048 / 2250 keys 6.4 / 8.6 / 9.2, the row kernel
       // 6.6 / 9.9 / 11.2; 32 heads of 128 6.8 / 10.0, 7.3 / 12.1; 40 of 128 (4 pieces) against 300 / 600 / 2048 5.1 / 6.0 /
       // 10.8, 5.1 / 7.0 / 13.5; 64 of 80 (5) 7.7 / 11.2, 8.1 / 14.0; 96 of 128 (8) against 300 / 2048 5.6 / 15.4, 8.5 / 18.5.
-      // Fewer keys are level or lose by the sums' longer way through the LDS (32 heads of 80: 600 keys 5.4 / 5.2).
+      // Fewer keys are level or lose by the sums' longer way through the LDS (32 heads of 80: 600 keys 5.4 / 5.2).  In a decode layer
+      // replayed from a graph, two pieces against the row kernel, fp16 / 8-bit weights: 400 keys +0.4 / +0.5 us, 600 0.0 / 0.0, 800 -0.1 /
+      // +0.1, 900 -0.3 / -0.1, 1024 -0.3 / -0.4, 1400 -1.0 / -0.7, 2048 -1.9 / -1.2.
       int64_t shared_pieces = 1;
       if (n == 1 && heads * pieces > kNumCU && heads <= kNumCU) {
         shared_pieces = 2;

@@ -28,7 +28,8 @@ constexpr int largest_divisor(int n, int limit) {
 // transposing LDS read ds_read_b64_tr_b16 (4 wavefronts only).
 // WQ: W is 8-bit with an fp16 scale per 32 elements of a row (Wq bytes [N][K], ep.wscale [N][K/32]); its
 // tiles pass through registers and are dequantised on their way into the LDS.
-// M16: 8 wavefronts (256x256, 256x128, 128x256) on v_mfma_f32_16x16x32_f16 with one barrier per k tile (see the main loop).
+// M16: 8 wavefronts on v_mfma_f32_16x16x32_f16 with one barrier per k tile (see the main loop): NS = 2 the ring of five operand
+// units (256x256, 256x128, 128x256, 192x256, 192x128), NS >= 3 stages of their own (the twelve sizes of tile8_stages).
 template <int BM, int BN, int WM, int WN, int NS, bool WT = false, bool WQ = false, bool M16 = false>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* __restrict__ A,
                                                                  const half_t* __restrict__ W,
@@ -530,7 +531,10 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
     if constexpr (WQ) {
       // ---- 8-bit W on 8 wavefronts.  Every wavefront does the same: its blocks of A NS - 1 k tiles ahead, straight to the LDS, and
       // a 16-byte piece of W per lane (16 weights and their scale) three k tiles ahead of the stage it is dequantised into,
-      // one k tile before it is multiplied; the dequantiser's instructions issue under the MFMAs of the step before.
+      // one k tile before it is multiplied.  The dequantiser runs as one block behind the last MFMA of a step, ahead of the barrier
+      // (a scheduling fence stands between the MFMAs), in all eight wavefronts at the same time: what a SIMD's other wavefront
+      // could multiply meanwhile is not there.  41 .. 44 KB/us per CU (96x128: 12 KB of A and 8.5 of W and scales in 0.51 us, A in
+      // the caches) where the fp16 tiles move 59 .. 64.
       static_assert((NS - 2) * kQLoadsA + 4 <= 63, "outstanding loads must fit the vmcnt field");
       char* const w0 = lds + NS * kQStageA;
       int sa = 0;  // stage of A(kt)
