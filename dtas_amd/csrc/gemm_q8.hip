@@ -102,7 +102,7 @@ bool builtin_gemm_q8(int64_t M, int64_t N, int64_t K, bool stream_ok, bool vec_o
   }
   // Two routes.  (1) Dequantising in the W path of the tile kernel: no intermediate, W read once per row of tiles as bytes.
   // (2) The dequantiser into a library-owned fp16 buffer, then the fp16 GEMM with every tile it has: 3.4 us and 0.49 per million
-  // weights more, worth it once the GEMM itself is long (7680 x 2560: from ~1300 rows, 10240 x 2560 ~900).  Its time over
+  // weights more, worth it once the GEMM itself is long (7680 x 2560: from ~1000 rows, 10240 x 2560 ~770, 2560 x 10240 ~1540).  Its time over
   // the fit's sizes: these + the fp16 GEMM's estimate, to 5 %; the lesser of the two estimates is the lesser time to 0.1 %.
   cfg = dtas_config{DTAS_GEMM_MFMA, 256, 8, 3, {128, 128, kBK}, 1, 0};
   const int64_t t128 = ceil_div(M, 128) * ceil_div(N, 128);
