@@ -9,7 +9,9 @@
 // moves `vec` contiguous elements per access (up to 128 bit on the narrower side), a
 // wavefront's 64 accesses are one contiguous span, each thread keeps `unroll` accesses in
 // flight, a workgroup is 256 threads (4 wavefronts) and walks tiles of 256*unroll vectors
-// grid-stride.  Accesses are marked non-temporal: every byte is touched once.
+// grid-stride.  Loads are marked non-temporal: every byte is touched once.  Stores: store_out (dtas_device.h).
+#include <type_traits>
+
 #include "dtas_device.h"
 #include "dtas_host.h"
 
@@ -30,31 +32,31 @@ template <>
 struct Raw<1> {
   uint8_t d;
   static __device__ __forceinline__ Raw load(const void* p, int64_t i) { return {load_stream(static_cast<const uint8_t*>(p) + i)}; }
-  __device__ __forceinline__ void store(void* p, int64_t i) const { store_stream(d, static_cast<uint8_t*>(p) + i); }
+  __device__ __forceinline__ void store(void* p, int64_t i, bool through) const { store_out(d, static_cast<uint8_t*>(p) + i, through); }
 };
 template <>
 struct Raw<2> {
   uint16_t d;
   static __device__ __forceinline__ Raw load(const void* p, int64_t i) { return {load_stream(static_cast<const uint16_t*>(p) + i)}; }
-  __device__ __forceinline__ void store(void* p, int64_t i) const { store_stream(d, static_cast<uint16_t*>(p) + i); }
+  __device__ __forceinline__ void store(void* p, int64_t i, bool through) const { store_out(d, static_cast<uint16_t*>(p) + i, through); }
 };
 template <>
 struct Raw<4> {
   uint32_t d;
   static __device__ __forceinline__ Raw load(const void* p, int64_t i) { return {load_stream(static_cast<const uint32_t*>(p) + i)}; }
-  __device__ __forceinline__ void store(void* p, int64_t i) const { store_stream(d, static_cast<uint32_t*>(p) + i); }
+  __device__ __forceinline__ void store(void* p, int64_t i, bool through) const { store_out(d, static_cast<uint32_t*>(p) + i, through); }
 };
 template <>
 struct Raw<8> {
   u32x2 d;
   static __device__ __forceinline__ Raw load(const void* p, int64_t i) { return {load_stream(static_cast<const u32x2*>(p) + i)}; }
-  __device__ __forceinline__ void store(void* p, int64_t i) const { store_stream(d, static_cast<u32x2*>(p) + i); }
+  __device__ __forceinline__ void store(void* p, int64_t i, bool through) const { store_out(d, static_cast<u32x2*>(p) + i, through); }
 };
 template <>
 struct Raw<16> {
   u32x4 d;
   static __device__ __forceinline__ Raw load(const void* p, int64_t i) { return {load_stream(static_cast<const u32x4*>(p) + i)}; }
-  __device__ __forceinline__ void store(void* p, int64_t i) const { store_stream(d, static_cast<u32x4*>(p) + i); }
+  __device__ __forceinline__ void store(void* p, int64_t i, bool through) const { store_out(d, static_cast<u32x4*>(p) + i, through); }
 };
 template <>
 struct Raw<32> {
@@ -63,10 +65,10 @@ struct Raw<32> {
     const u32x4* q = static_cast<const u32x4*>(p) + 2 * i;
     return {{load_stream(q), load_stream(q + 1)}};
   }
-  __device__ __forceinline__ void store(void* p, int64_t i) const {
+  __device__ __forceinline__ void store(void* p, int64_t i, bool through) const {
     u32x4* q = static_cast<u32x4*>(p) + 2 * i;
-    store_stream(d[0], q);
-    store_stream(d[1], q + 1);
+    store_out(d[0], q, through);
+    store_out(d[1], q + 1, through);
   }
 };
 
@@ -83,7 +85,7 @@ struct AddOp {
   typedef T In;
   typedef T Out;
   static constexpr int kInputs = 2;
-  static constexpr bool kBytewise = false;
+  static constexpr bool kBytewise = false, kThrough = true;
   static __device__ __forceinline__ T apply(T a, T b) { return a + b; }
   static __device__ __forceinline__ uint32_t apply_word(uint32_t a, uint32_t) { return a; }  // (unused)
 };
@@ -92,7 +94,7 @@ struct AddOp<int8_t> {
   typedef int8_t In;
   typedef int8_t Out;
   static constexpr int kInputs = 2;
-  static constexpr bool kBytewise = true;
+  static constexpr bool kBytewise = true, kThrough = true;
   static __device__ __forceinline__ int8_t apply(int8_t a, int8_t b) {
     return static_cast<int8_t>(static_cast<uint8_t>(static_cast<uint8_t>(a) + static_cast<uint8_t>(b)));
   }
@@ -108,7 +110,7 @@ struct CopyOp {
   typedef Bits In;
   typedef Bits Out;
   static constexpr int kInputs = 1;
-  static constexpr bool kBytewise = sizeof(Bits) == 1;
+  static constexpr bool kBytewise = sizeof(Bits) == 1, kThrough = true;
   static __device__ __forceinline__ Bits apply(Bits a, Bits) { return a; }
   static __device__ __forceinline__ uint32_t apply_word(uint32_t a, uint32_t) { return a; }
 };
@@ -120,6 +122,9 @@ struct CastOp {
   typedef TO Out;
   static constexpr int kInputs = 1;
   static constexpr bool kBytewise = false;
+  // (to fp16 the cast streams its output: written through it takes 18.4 us over [4096, 4096] against 16.9, and the add that reads
+  // the result next 17.6 against 17.2 -- a pass over [1200, 4096] 45.3 / 44.7, [4096, 4096] 101.2 / 100.0)
+  static constexpr bool kThrough = sizeof(TO) > sizeof(TI);
   static __device__ __forceinline__ TO apply(TI a, TI) { return static_cast<TO>(a); }
   static __device__ __forceinline__ uint32_t apply_word(uint32_t a, uint32_t) { return a; }  // (unused)
 };
@@ -134,45 +139,51 @@ __global__ void __launch_bounds__(kBlock) elt_vector_kernel(const void* __restri
   typedef Raw<VEC * sizeof(TO)> RO;
   constexpr int64_t kTile = static_cast<int64_t>(kBlock) * U;
   const int64_t step = static_cast<int64_t>(gridDim.x) * kTile;
-  for (int64_t base = static_cast<int64_t>(blockIdx.x) * kTile; base < nvec; base += step) {
-    RI ra[U], rb[U];
-    const int64_t first = base + threadIdx.x;
-    const bool full = base + kTile <= nvec;
+  auto walk = [&](auto through) {
+    constexpr bool kThrough = decltype(through)::value;
+    for (int64_t base = static_cast<int64_t>(blockIdx.x) * kTile; base < nvec; base += step) {
+      RI ra[U], rb[U];
+      const int64_t first = base + threadIdx.x;
+      const bool full = base + kTile <= nvec;
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t i = first + u * kBlock;
-      if (full || i < nvec) {
-        ra[u] = RI::load(a, i);
-        if (Op::kInputs == 2) rb[u] = RI::load(b, i);
-      }
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      const int64_t i = first + u * kBlock;
-      if (full || i < nvec) {
-        RO ro;
-        if constexpr (Op::kBytewise && VEC % 4 == 0) {
-          // whole 32-bit words at once (byte by byte the compiler unpacks and repacks every element, and the launch is
-          // bound by that arithmetic: the int8 add over [8192, 4096] took 39.5 us at 8 vectors per thread, 18.0 at one)
-          uint32_t wa[VEC / 4], wb[VEC / 4], wo[VEC / 4];
-          __builtin_memcpy(wa, &ra[u], sizeof(wa));
-          if (Op::kInputs == 2) __builtin_memcpy(wb, &rb[u], sizeof(wb));
-#pragma unroll
-          for (int e = 0; e < VEC / 4; ++e) wo[e] = Op::apply_word(wa[e], Op::kInputs == 2 ? wb[e] : wa[e]);
-          __builtin_memcpy(&ro, wo, sizeof(ro));
-        } else {
-          Elems<TI, VEC> ea, eb;
-          Elems<TO, VEC> eo;
-          __builtin_memcpy(&ea, &ra[u], sizeof(ea));
-          if (Op::kInputs == 2) __builtin_memcpy(&eb, &rb[u], sizeof(eb)); else eb = ea;
-#pragma unroll
-          for (int e = 0; e < VEC; ++e) eo.v[e] = Op::apply(ea.v[e], eb.v[e]);
-          __builtin_memcpy(&ro, &eo, sizeof(ro));
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = first + u * kBlock;
+        if (full || i < nvec) {
+          ra[u] = RI::load(a, i);
+          if (Op::kInputs == 2) rb[u] = RI::load(b, i);
         }
-        ro.store(out, i);
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int64_t i = first + u * kBlock;
+        if (full || i < nvec) {
+          RO ro;
+          if constexpr (Op::kBytewise && VEC % 4 == 0) {
+            // whole 32-bit words at once (byte by byte the compiler unpacks and repacks every element, and the launch is
+            // bound by that arithmetic: the int8 add over [8192, 4096] took 39.5 us at 8 vectors per thread, 18.0 at one)
+            uint32_t wa[VEC / 4], wb[VEC / 4], wo[VEC / 4];
+            __builtin_memcpy(wa, &ra[u], sizeof(wa));
+            if (Op::kInputs == 2) __builtin_memcpy(wb, &rb[u], sizeof(wb));
+#pragma unroll
+            for (int e = 0; e < VEC / 4; ++e) wo[e] = Op::apply_word(wa[e], Op::kInputs == 2 ? wb[e] : wa[e]);
+            __builtin_memcpy(&ro, wo, sizeof(ro));
+          } else {
+            Elems<TI, VEC> ea, eb;
+            Elems<TO, VEC> eo;
+            __builtin_memcpy(&ea, &ra[u], sizeof(ea));
+            if (Op::kInputs == 2) __builtin_memcpy(&eb, &rb[u], sizeof(eb)); else eb = ea;
+#pragma unroll
+            for (int e = 0; e < VEC; ++e) eo.v[e] = Op::apply(ea.v[e], eb.v[e]);
+            __builtin_memcpy(&ro, &eo, sizeof(ro));
+          }
+          ro.store(out, i, kThrough);
+        }
       }
     }
-  }
+  };
+  // (one loop per kind of store: a choice at each store would wait for every load ahead of the first)
+  if (Op::kThrough && count <= kThroughBytes / static_cast<int64_t>(sizeof(TO))) walk(std::integral_constant<bool, Op::kThrough>{});
+  else walk(std::false_type{});
   // the last count % VEC elements, one per thread of workgroup 0
   if (blockIdx.x == 0) {
     const int64_t i = nvec * VEC + threadIdx.x;
@@ -292,7 +303,7 @@ __global__ void __launch_bounds__(kBlock) take_f16_kernel(const u32x4* __restric
        t += static_cast<int64_t>(gridDim.x) * blockDim.x) {
     int64_t row = ids[t / per_row];
     row = row < 0 ? 0 : row >= V ? V - 1 : row;
-    store_stream(A[row * per_row + t % per_row], out + t);
+    store_out(A[row * per_row + t % per_row], out + t, pieces <= kThroughBytes / 16);
   }
 }
 __global__ void __launch_bounds__(kBlock) take_f16_scalar_kernel(const half_t* __restrict__ A, const int* __restrict__ ids,
@@ -387,7 +398,7 @@ __global__ void __launch_bounds__(kBlock) rotary20_kernel(const half_t* __restri
       }
       raw = __builtin_bit_cast(u32x4, r);
     }
-    store_stream(raw, reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * d + 8 * v));
+    store_out(raw, reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * d + 8 * v), pieces <= kThroughBytes / 16);
     if (pieces - t <= step) break;   // (t + step might wrap in 32 bits)
   }
 }
@@ -423,7 +434,7 @@ __global__ void __launch_bounds__(kBlock) rotary16_kernel(const half_t* __restri
       }
       raw = __builtin_bit_cast(u32x4, r);
     }
-    store_stream(raw, reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * per_row * 8 + 8 * v));
+    store_out(raw, reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * per_row * 8 + 8 * v), pieces <= kThroughBytes / 16);
     if (pieces - t <= step) break;   // (t + step might wrap in 32 bits)
   }
 }
@@ -464,7 +475,7 @@ __global__ void __launch_bounds__(kBlock) rotary4_kernel(const half_t* __restric
       }
       raw = __builtin_bit_cast(u32x4, x);
     }
-    store_stream(raw, reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * per_row * 8 + j0));
+    store_out(raw, reinterpret_cast<u32x4*>(out + static_cast<int64_t>(row) * per_row * 8 + j0), pieces <= kThroughBytes / 16);
     if (pieces - t <= step) break;   // (t + step might wrap in 32 bits)
   }
 }
@@ -476,7 +487,7 @@ __global__ void __launch_bounds__(kBlock) rotary4_kernel(const half_t* __restric
 // lane) and 0..5 (words 0..2 of the lane before), piece 2 elements 6..9 (word 3 two lanes back, word 0 one back).
 // The tables' 8 elements come as one 16-byte load (piece 2: elements 12..19, of which it uses the upper four), asked
 // for together with the piece.  At n = 4096 (32 heads, d = 80): 9.2 us against 11.5 for the kernel above, which was
-// 12.2 before its stores became streaming ones; two or more chunks of rows per pass of a wavefront are slower.
+// 12.2 with plain stores; two or more chunks of rows per pass of a wavefront are slower.
 __global__ void __launch_bounds__(kBlock) rotary20_rows_kernel(const half_t* __restrict__ A, const half_t* __restrict__ cs,
                                                                const half_t* __restrict__ sn, half_t* __restrict__ out,
                                                                uint32_t rows, uint32_t heads, uint32_t per_row, int64_t pos0) {
@@ -529,7 +540,7 @@ __global__ void __launch_bounds__(kBlock) rotary20_rows_kernel(const half_t* __r
       }
       raw = __builtin_bit_cast(u32x4, r);
     }
-    if (on) store_stream(raw, reinterpret_cast<u32x4*>(out + at));
+    if (on) store_out(raw, reinterpret_cast<u32x4*>(out + at), static_cast<int64_t>(rows) * per_row <= kThroughBytes / 16);
   }
 }
 
@@ -562,7 +573,7 @@ __global__ void __launch_bounds__(kBlock) attn_mask_kernel(half_t* __restrict__ 
       }
     }
     if (total - t >= 8) {
-      store_stream(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(out + t));
+      store_out(__builtin_bit_cast(u32x4, v), reinterpret_cast<u32x4*>(out + t), total <= kThroughBytes / 2);
     } else {
 #pragma unroll
       for (int e = 0; e < 8; ++e)
@@ -583,7 +594,7 @@ __global__ void __launch_bounds__(kBlock) swap_axes_kernel(const u32x4* __restri
   for (I t = static_cast<I>(blockIdx.x) * kBlock + threadIdx.x; t < total; t += step) {
     const I r = t / per_row, p = t - r * per_row;   // output row r = ib * a + ia
     const I ib = r / a, ia = r - ib * a;
-    store_stream(A[(static_cast<int64_t>(ia) * b + ib) * per_row + p], out + t);
+    store_out(A[(static_cast<int64_t>(ia) * b + ib) * per_row + p], out + t, total <= kThroughBytes / 16);
     if (total - t <= step) break;   // (t + step might wrap in 32 bits)
   }
 }
@@ -592,7 +603,7 @@ __global__ void __launch_bounds__(kBlock) swap_axes_kernel(const u32x4* __restri
 // kSwapB consecutive ib in the order of the output, so that what it writes (kSwapB runs of kSwapA rows) and what it
 // reads (kSwapA runs of kSwapB rows) are both runs of whole 128-byte lines; addresses are a base per workgroup plus
 // 32-bit offsets, and a thread loads up to four pieces before it stores them.  At a = 4096, b = 32, d = 80: 8.8 us
-// against 9.6 for the kernel above (10.7 before its stores became streaming ones); at a = 1024 4.0 either way.
+// against 9.6 for the kernel above with streaming stores on both sides; written through 9.2, and at a = 2048 in a layer 5.6 -> 4.8.
 constexpr int kSwapA = 4, kSwapB = 8;
 __global__ void __launch_bounds__(kBlock) swap_axes_tile_kernel(const u32x4* __restrict__ A, u32x4* __restrict__ out, int64_t a,
                                                                 int64_t b, uint32_t per_row, uint32_t b_groups) {
@@ -617,9 +628,12 @@ __global__ void __launch_bounds__(kBlock) swap_axes_tile_kernel(const u32x4* __r
         to[k] = jb * out_plane + rem;
       }
     }
+    auto store = [&](auto through) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k)
-      if (u0 + k * kBlock < tile) store_stream(v[k], dst + to[k]);
+      for (int k = 0; k < 4; ++k)
+        if (u0 + k * kBlock < tile) store_out(v[k], dst + to[k], decltype(through)::value);
+    };
+    if (a * b * per_row <= kThroughBytes / 16) store(std::true_type{}); else store(std::false_type{});
   }
 }
 
@@ -635,7 +649,7 @@ __global__ void __launch_bounds__(kBlock) split3_kernel(const T* __restrict__ A,
     const I r = t / (3 * per_sec), c = t - r * (3 * per_sec);
     const I sec = c / per_sec, j = c - sec * per_sec;
     T* o = sec == 0 ? o0 : sec == 1 ? o1 : o2;
-    store_stream(A[t], o + static_cast<int64_t>(r) * per_sec + j);
+    store_out(A[t], o + static_cast<int64_t>(r) * per_sec + j, total <= kThroughBytes / static_cast<int64_t>(sizeof(T)));
     if (total - t <= step) break;   // (t + step might wrap in 32 bits)
   }
 }
@@ -644,7 +658,7 @@ __global__ void __launch_bounds__(kBlock) split3_kernel(const T* __restrict__ A,
 // of A and walks them section by section, so that its stores are three runs of kSplitRows x d elements, whole
 // 128-byte lines; the lines of A are read by the three walks within the one workgroup.  Addresses are a base per
 // workgroup plus 32-bit offsets, and a thread loads up to four pieces before it stores them.  At 131072 rows, d = 80:
-// 21.8 us against 23.1 for the kernel above (24.4 before its stores became streaming ones), at 32768 rows 7.1 / 7.7.
+// 21.8 us against 23.1 for the kernel above with streaming stores on both sides, at 32768 rows 7.1 / 7.7; written through 22.1 and 7.5.
 constexpr int kSplitRows = 8;
 __global__ void __launch_bounds__(kBlock) split3_tile_kernel(const u32x4* __restrict__ A, u32x4* __restrict__ o0, u32x4* __restrict__ o1,
                                                              u32x4* __restrict__ o2, int64_t rows, uint32_t per_sec) {
@@ -654,6 +668,7 @@ __global__ void __launch_bounds__(kBlock) split3_tile_kernel(const u32x4* __rest
   const u32x4* src = A + r0 * 3 * per_sec;
   for (uint32_t u0 = threadIdx.x; u0 < tile; u0 += 4 * kBlock) {
     u32x4 v[4];
+    u32x4* to[4];
 #pragma unroll
     for (int k = 0; k < 4; ++k) {
       const uint32_t u = u0 + k * kBlock;
@@ -661,17 +676,15 @@ __global__ void __launch_bounds__(kBlock) split3_tile_kernel(const u32x4* __rest
         const uint32_t sec = u / run, rem = u - sec * run;
         const uint32_t rr = rem / per_sec, j = rem - rr * per_sec;
         v[k] = src[(rr * 3 + sec) * per_sec + j];
+        to[k] = (sec == 0 ? o0 : sec == 1 ? o1 : o2) + r0 * per_sec + rem;
       }
     }
+    auto store = [&](auto through) {
 #pragma unroll
-    for (int k = 0; k < 4; ++k) {
-      const uint32_t u = u0 + k * kBlock;
-      if (u < tile) {
-        const uint32_t sec = u / run, rem = u - sec * run;
-        u32x4* o = sec == 0 ? o0 : sec == 1 ? o1 : o2;
-        store_stream(v[k], o + r0 * per_sec + rem);
-      }
-    }
+      for (int k = 0; k < 4; ++k)
+        if (u0 + k * kBlock < tile) store_out(v[k], to[k], decltype(through)::value);
+    };
+    if (rows * 3 * per_sec <= kThroughBytes / 16) store(std::true_type{}); else store(std::false_type{});
   }
 }
 

@@ -169,6 +169,31 @@ def test_every_vector_variant(oracle, op, vec, unroll):
     assert_bits_equal(out.check(), want)
 
 
+@pytest.mark.parametrize("vectors", [-1, 0, 1])
+def test_outputs_at_the_line_between_written_through_and_streamed(vectors):
+    """Outputs of 128 MiB and a vector less or more: exact against torch on the device, to the last element."""
+    gen = torch.Generator(device="cuda").manual_seed(vectors + 2)
+    count = (128 << 20) // 4 + 4 * vectors + 3                       # fp32 elements, a ragged tail behind the last vector
+    a32 = torch.randn(1, 1, count, device="cuda", generator=gen)
+    out32 = torch.empty_like(a32)
+    ops.copy(a32, out32)
+    assert torch.equal(a32, out32)
+    ops.add(a32, a32, out32)
+    assert torch.equal(a32 + a32, out32)
+    a16 = a32.half()
+    ops.cast(a16, out32)
+    assert torch.equal(a16.float(), out32)
+    a = (128 << 20) // 2 // (32 * 80) + vectors                      # rows of 80 elements: axis swap and split
+    rows = torch.randn(a, 32, 80, device="cuda", generator=gen).half()
+    swapped = torch.empty(32, a, 80, dtype=torch.float16, device="cuda")
+    ops.swap_axes(rows, swapped)
+    assert torch.equal(rows.transpose(0, 1), swapped)
+    fused = torch.randn(a // 3, 32, 240, device="cuda", generator=gen).half()
+    parts = [torch.empty(a // 3, 32, 80, dtype=torch.float16, device="cuda") for _ in range(3)]
+    ops.split3(fused, *parts)
+    assert all(torch.equal(p, w) for p, w in zip(parts, fused.split(80, dim=-1)))
+
+
 def test_grid_cap_makes_the_kernel_loop(oracle):
     rng = np.random.default_rng(4)
     a, b = rng.uniform(-1, 1, (300, 4096)).astype(np.float16), rng.uniform(-1, 1, (300, 4096)).astype(np.float16)
