@@ -241,3 +241,27 @@ def test_a_k_that_no_tile_holds_is_refused():
     for K in (1 << 24, 1 << 25):
         with pytest.raises(_lib.DtasError, match="too large"):
             _lib.builtin_gemm(300, 64, K)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", [256, 512])
+@pytest.mark.parametrize("M,N", [(1, 32), (129, 64), (300, 288), (300, 280), (257, 10240)])
+def test_rows_written_through_and_streamed_hold_the_same_bits(block, M, N):
+    """C on and off the 64-byte grid, N % 32 = 0 or not: the stores differ, the results do not."""
+    gen = torch.Generator(device="cuda").manual_seed(M * 7 + N)
+    A = torch.randn(M, 192, device="cuda", generator=gen).half()
+    W = (torch.randn(N, 192, device="cuda", generator=gen) * 0.05).half()
+    bias = torch.randn(N, device="cuda", generator=gen).half()
+    tile = cfg(variant=_lib.GEMM_MFMA, block=block, vec=8, unroll=2 if block == 256 else 0, tile=[128, 128, 64])
+    got = []
+    for offset in (0, 8, 32, 1):
+        raw = torch.full((M * N + 64 + offset,), 1234.5, dtype=torch.float16, device="cuda")
+        C = raw[offset:offset + M * N].view(M, N)
+        ops.gemm(A, W, bias, C, cfg=tile)
+        torch.cuda.synchronize()
+        assert bool((raw[:offset] == 1234.5).all()) and bool((raw[offset + M * N:] == 1234.5).all())
+        got.append(C.clone())
+    assert all(torch.equal(got[0], g) for g in got[1:])
+    # (the sum and the result are each rounded to fp16, 2^-11 of at most a few units)
+    want = (A.double() @ W.double().t()).half().double() + bias.double()
+    assert ((got[0].double() - want).abs() <= 2e-3 + 2e-3 * want.abs()).all()
