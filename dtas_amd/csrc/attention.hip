@@ -813,19 +813,21 @@ extern "C" int dtas_attn_scores_f16_f32(const void* Q, const void* Kmat, const v
                            static_cast<float*>(out), n, m, d, sc, tm, tn, static_cast<unsigned>(heads), pin);
       return check_launch("attn_scores");
     }
-    // ... or every row is cut at sectors of its own (attn_scores_sector_kernel), for continuations of up to 256 rows.  Tiles / own
-    // sectors, us, head dimension 80; in brackets with the softmax that reads them behind:
+    // ... or every row is cut at sectors of its own (attn_scores_sector_kernel), for continuations of up to 256 rows and for scores that
+    // a cache does not hold for the softmax.  Tiles / own sectors, us, head dimension 80; in brackets with the softmax that reads them behind:
     //  * keys: 32 heads, 203 x 601 11.2 / 12.0 (20.9 / 20.0), 256 x 601 11.8 / 11.9 (22.7 / 22.2); 203 x 703 12.6 / 12.3 (23.2 / 20.3), 256 x
     //    703 13.2 / 12.0 (24.8 / 24.0), 203 x 1031 15.7 / 13.8 (26.5 / 25.4), 130 x 2049 17.5 / 15.7 (29.3 / 27.4), 256 x 4095 49.5 / 37.3;
     //  * workgroups per CU, whose chains have to hide one another: 1.5, 32 heads, 65 x 1531 11.1 / 12.0, 100 x 1301 11.4 / 11.9, 24 heads,
     //    225 x 777 11.6 / 12.4; 1.75 and more, 32 heads, 203 x 777 14.0 / 12.5, 130 x 1031 13.8 / 11.8, 65 x 2049 13.1 / 11.9;
-    //  * rows: 64 heads, 225 x 1031 23.6 / 25.5 (41.5 / 42.8), 225 x 1301 26.5 / 28.9 (48.3 / 49.9), and level beyond 8192 rows in all with
-    //    32 heads (400 x 1031 21.9 / 22.4, 512 x 1301 30.6 / 29.2).  Prompts: launches of scores alone gain more (2047 x 2047 208 /
-    //    128), the layer around them nothing (1601: 636 / 642; 2047: 809 / 807).
+    //  * rows beyond 8192 in all, and 256: axis swaps, scores, softmax and P.V together.  Below 1100 keys level to 1 % behind (a layer of
+    //    1025 rows 374 / 376, of 777 298.4 / 300.1), and so are few scores (64 heads, 225 x 1301, 75 MB, 86.6 / 87.6); from 20 M scores on
+    //    the tiles' plain stores keep nothing for the softmax that the streaming ones here would lose: a layer of 500 rows after 2001
+    //    311 / 303, 700 after 2501 446 / 421, of 1250 rows 450 / 442, 1601 611 / 594, 2047 809 / 769; 64 heads, 1025 x 1301 300 / 271, 16
+    //    heads, 600 x 1301 64.5 / 61.6, 8 heads, 1500 x 3001 128 / 124.
     // Head dimensions of 64 and 128 pull more of K through the L1 than the tiles do (40 heads of 128, 1025 x 1025 57.6 / 98.9)
     const int64_t pieces = ceil_div(m, kSectorChunk), chunk = ceil_div(ceil_div(m, pieces), 16) * 16;
     const int64_t tm_s = ceil_div(n, kSectorRows), tn_s = ceil_div(m, chunk), tiles_s = tm_s * tn_s;
-    if (!whole_sectors && d > 64 && d <= 16 * kSectorSteps && n <= 256 && n * heads <= 8192 && m >= 700 && tiles_s * heads * 4 >= 7 * kNumCU) {
+    if (!whole_sectors && d > 64 && d <= 16 * kSectorSteps && ((n <= 256 && n * heads <= 8192 && m >= 700) || (m >= 1100 && n * m * heads >= 20000000)) && tiles_s * heads * 4 >= 7 * kNumCU) {
       const bool pin = n * m >= (int64_t{1} << 21);
       const int64_t wgs = pin ? kNumXCD * heads * ceil_div(tiles_s, kNumXCD) : tiles_s * heads;
       if (wgs > 0x7fffffff) return fail("attn_scores: too many tiles");

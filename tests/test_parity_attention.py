@@ -52,11 +52,12 @@ def test_scores_builtin_other_head_dims(oracle, heads, n, m, d):
     _check(out.check(), q, k, mask, oracle)
 
 
-@pytest.mark.parametrize("heads,n,m,d,at", [(32, 225, 700, 80, 1), (32, 225, 960, 80, 4), (32, 256, 1201, 72, 2), (4, 256, 8193, 80, 3)])
+@pytest.mark.parametrize("heads,n,m,d,at", [(32, 225, 700, 80, 1), (32, 225, 960, 80, 4), (32, 256, 1201, 72, 2), (4, 256, 8193, 80, 3),
+                                            (8, 1931, 1301, 80, 0), (64, 289, 1100, 80, 1), (5, 2047, 2047, 80, 0)])
 def test_scores_rows_cut_at_their_own_sectors(oracle, heads, n, m, d, at):
     # rows that are no whole 64-byte sectors, or an output `at` floats off one: chunks of up to 480 keys whose edges move with
     # the row (two to five of them; whole and partly filled blocks of 32 rows; head dimensions with and without an empty half
-    # k step; unequal spans per XCD from 2 M scores per head on).  Integer operands: every product and sum is exact, so the bits are the general kernel's
+    # k step; unequal spans per XCD from 2 M scores per head on; 20 M scores and more at any number of rows).  Integer operands: every product and sum is exact, so the bits are the general kernel's
     q, k, mask = _inputs(heads, n, m, d, n + m + d)
     buf = torch.full((heads * n * m + at + 16,), -7.0, dtype=torch.float32, device="cuda")
     out = buf[at:at + heads * n * m].view(heads, n, m)
