@@ -42,6 +42,19 @@ def test_rms_norm_other_row_lengths(oracle, H):
     _check(out.check(), oracle.c.rms_norm(x, w), oracle.np64.rms_norm(x, w))
 
 
+@pytest.mark.parametrize("n,H", [(156, 2560), (157, 2560), (3276, 2560), (3277, 2560), (488, 4096), (489, 4096), (4097, 4096)])
+def test_norms_at_the_lines_between_streamed_and_written_through(oracle, n, H):
+    # 400 k and 8 M elements (layer norm), 2 M and 16 M (RMS norm)
+    rng = np.random.default_rng(n + H)
+    x, w = rng.standard_normal((n, H)).astype(np.float16), rng.uniform(0.5, 1.5, H).astype(np.float16)
+    out = Guarded(x.shape, torch.float16)
+    ops.rms_norm(dev(x), dev(w), out.t)
+    _check(out.check(), oracle.c.rms_norm(x, w, threads=8), oracle.np64.rms_norm(x, w))
+    x32, g, b = x.astype(np.float32), w.astype(np.float32), rng.uniform(-0.2, 0.2, H).astype(np.float32)
+    ops.layer_norm(dev(x32), dev(g), dev(b), out.t)
+    _check(out.check(), oracle.c.layer_norm(x32, g, b, threads=8), oracle.np64.layer_norm(x32, g, b))
+
+
 # one n per branch of the built-in choice (rows per CU: up to 4, 4 .. 8, 8, 8 .. 12, 12 .. 16, 16 .. 24, beyond)
 REGIME_N = [1000, 1500, 2048, 3000, 4090, 6001, 8200]
 
