@@ -184,11 +184,17 @@ extern "C" int dtas_gemm_q8_f16_fused(const void* A, const void* Wq, const void*
   if (describe_gemm(M, N, K, cfg, la) != 0) return -1;
   const int bm = cfg.tile[0], bn = cfg.tile[1];
   if (cfg.block == 512 && bn == 128 && cfg.unroll == 0) {
-    if (bm == 96) return launch_mfma<96, 128, 2, 4, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
-    if (bm == 128) return launch_mfma<128, 128, 4, 2, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
-    if (bm == 160) return launch_mfma<160, 128, 2, 4, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
-    if (bm == 192) return launch_mfma<192, 128, 4, 2, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
-    if (bm == 256) return launch_mfma<256, 128, 4, 2, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk);
+    const bool quads = K % 64 == 0 && aligned(scale, 4);  // (a row's scales of four k tiles in one load)
+#define DTAS_Q8_CASE(BM_, WM_, WN_)                                                                                        \
+  if (bm == BM_)                                                                                                           \
+  return quads ? launch_mfma<BM_, 128, WM_, WN_, 4, false, true, true, true>(s, a, w, ep, C, M, N, K, sk)                   \
+               : launch_mfma<BM_, 128, WM_, WN_, 4, false, true, true>(s, a, w, ep, C, M, N, K, sk)
+    DTAS_Q8_CASE(96, 2, 4);
+    DTAS_Q8_CASE(128, 4, 2);
+    DTAS_Q8_CASE(160, 2, 4);
+    DTAS_Q8_CASE(192, 4, 2);
+    DTAS_Q8_CASE(256, 4, 2);
+#undef DTAS_Q8_CASE
   }
   if (bm == 128 && bn <= 128 && cfg.block != 256) return fail("gemm_q8: the %dx%d MFMA kernel uses 256 threads, got %d", bm, bn, cfg.block);
   if (bm == 256 && bn == 128 && cfg.unroll == 3) return launch_mfma<256, 128, 2, 2, 3, false, true>(s, a, w, ep, C, M, N, K, sk);

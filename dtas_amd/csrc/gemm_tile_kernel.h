@@ -30,7 +30,8 @@ constexpr int largest_divisor(int n, int limit) {
 // tiles pass through registers and are dequantised on their way into the LDS.
 // M16: 8 wavefronts on v_mfma_f32_16x16x32_f16 with one barrier per k tile (see the main loop): NS = 2 the ring of five operand
 // units (256x256, 256x128, 128x256, 192x256, 192x128), NS >= 3 stages of their own (the twelve sizes of tile8_stages).
-template <int BM, int BN, int WM, int WN, int NS, bool WT = false, bool WQ = false, bool M16 = false>
+// QS4: 8-bit W on 8 wavefronts, the scales of four k tiles of a row in one 16-byte load (K % 64 == 0, 4-byte aligned scales).
+template <int BM, int BN, int WM, int WN, int NS, bool WT = false, bool WQ = false, bool M16 = false, bool QS4 = false>
 __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* __restrict__ A,
                                                                  const half_t* __restrict__ W,
                                                                  GemmEpilogue ep, void* __restrict__ C, int64_t M,
@@ -231,8 +232,9 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   // The pieces come through buffer loads (out of range -> zeros), so every lane issues the same number of loads per tile
   // whatever its rows: the waits below count them.  Every row of the tile is written every time (rows past N as zeros).
   constexpr int kWtItems = WREG ? 4 * BN / (64 * NW) : 1;
-  constexpr int kWtSlots = WREG ? (M16 ? 3 : NS - 1) : 1;  // register sets: one per tile in flight
-  constexpr int kWtLoads = 2 * kWtItems;  // per lane and tile: a piece and its scale per item
+  static_assert(!QS4 || (WQ && M16 && kWtItems == 1), "scales by fours come with 8-bit W on 8 wavefronts");
+  constexpr int kWtSlots = WREG ? (M16 ? (QS4 ? 4 : 3) : NS - 1) : 1;  // register sets: one per tile in flight
+  constexpr int kWtLoads = QS4 ? 1 : 2 * kWtItems;  // per lane and tile: a piece and its scale per item
   u32x4 wt_reg[kWtSlots][kWtItems][1];
   unsigned short wq_scale[kWtSlots][kWtItems];
   const __amdgpu_buffer_rsrc_t rv = make_rsrc(W, WQ ? static_cast<unsigned>(K * N) : 0u);
@@ -245,16 +247,29 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       const int64_t row = n0 + r, k = static_cast<int64_t>(kt_abs(kt)) * kBK + c4 * 16;
       const bool in = row < N && k < K && (!M16 || kt < ktiles);  // K % 32 == 0: a piece and its scale group are all-in or all-out
       wt_reg[SLOT][i][0] = __builtin_amdgcn_raw_buffer_load_b128(rv, in ? static_cast<unsigned>(row * K + k) : kOob, 0, 0);
-      wq_scale[SLOT][i] = __builtin_amdgcn_raw_buffer_load_b16(rs, in ? static_cast<unsigned>((row * (K >> 5) + (k >> 5)) * 2) : kOob, 0, 0);
+      if constexpr (!QS4) wq_scale[SLOT][i] = __builtin_amdgcn_raw_buffer_load_b16(rs, in ? static_cast<unsigned>((row * (K >> 5) + (k >> 5)) * 2) : kOob, 0, 0);
     }
   };
-  auto wt_commit_at = [&](char* base, auto slot_tag) {
+  // QS4: word w of these are the two scales of k tile 4 quad + w, for the lower and the upper half of the tile (four lanes hold a row's;
+  // past the end of a row lie the next row's, which meet k tiles that are never multiplied; past the last row zeros)
+  [[maybe_unused]] u32x4 qs_cur, qs_next;
+  [[maybe_unused]] const unsigned qs_pick = (t & 2u) ? 0x03020302u : 0x01000100u;
+  [[maybe_unused]] auto qs_load = [&](int quad) -> u32x4 {
+    const int64_t row = n0 + (t >> 2);
+    return __builtin_amdgcn_raw_buffer_load_b128(rs, row < N ? static_cast<unsigned>((row * (K >> 5) + 2 * (kt0 + 4 * quad)) * 2) : kOob, 0, 0);
+  };
+  auto wt_commit_at = [&](char* base, auto slot_tag, [[maybe_unused]] unsigned scales = 0u) {
     constexpr int SLOT = decltype(slot_tag)::value;
 #pragma unroll
     for (int i = 0; i < kWtItems; ++i) {
       const unsigned item = t + i * 64 * NW, r = item >> 2, c4 = item & 3u;
-      const half_t sc = __builtin_bit_cast(half_t, wq_scale[SLOT][i]);
-      const f16x2 s2 = {sc, sc};
+      f16x2 s2;
+      if constexpr (QS4) {
+        s2 = __builtin_bit_cast(f16x2, __builtin_amdgcn_perm(scales, scales, qs_pick));
+      } else {
+        const half_t sc = __builtin_bit_cast(half_t, wq_scale[SLOT][i]);
+        s2 = f16x2{sc, sc};
+      }
       u32x4 out[2];
 #pragma unroll
       for (int w = 0; w < 4; ++w) {
@@ -472,14 +487,20 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       wt_load(0, std::integral_constant<int, 0>{});
       wt_load(1, std::integral_constant<int, 1>{});
       wt_load(2, std::integral_constant<int, 2>{});
+      if constexpr (QS4) {
+        wt_load(3, std::integral_constant<int, 3>{});
+        qs_cur = qs_load(0);
+        qs_next = qs_load(1);
+      }
       DTAS_SCHED_FENCE();
 #pragma unroll
       for (int p = 0; p < NS - 1; ++p) fetch_a_q(p, p);
       DTAS_SCHED_FENCE();
-      wt_commit_at(lds + NS * kQStageA, std::integral_constant<int, 0>{});
-      wt_load(3, std::integral_constant<int, 0>{});
+      wt_commit_at(lds + NS * kQStageA, std::integral_constant<int, 0>{}, QS4 ? qs_cur[0] : 0u);
+      wt_load(kWtSlots, std::integral_constant<int, 0>{});
       DTAS_SCHED_FENCE();
-      __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA + 2));
+      // (QS4: A's loads alone are counted on: the piece just requested is for the loop only, and the compiler moves its load there)
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA + (QS4 ? 0 : kWtLoads)));
     } else if constexpr (!kRing) {
       if (hi) {
 #pragma unroll
@@ -535,34 +556,56 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       // (a scheduling fence stands between the MFMAs), in all eight wavefronts at the same time: what a SIMD's other wavefront
       // could multiply meanwhile is not there.  41 .. 44 KB/us per CU (96x128: 12 KB of A and 8.5 of W and scales in 0.51 us, A in
       // the caches) where the fp16 tiles move 59 .. 64.
-      static_assert((NS - 2) * kQLoadsA + 4 <= 63, "outstanding loads must fit the vmcnt field");
+      // The scales one by one, two bytes of each of 16 rows per load and k tile, were a third of the L1's look-ups.  Those of four k tiles
+      // in one load (QS4): 203 x 7680 x 2560 21.3 -> 20.0 us, 203 x 10240 x 2560 28.3 -> 25.3, 203 x 2560 x 10240 31.1 -> 28.9, 450 x 10240 x
+      // 2560 35.1 -> 32.6, 700 x 2560 x 10240 55.4 -> 52.3 (without any scales, 26.5, 29.3, 32.9, 52.9 against 28.6, 31.4, 35.7, 56.1: all of it).
+      // K = 64 k + 32 and scales off the 4-byte grid keep the loop of three.
+      static_assert((NS - 2) * kQLoadsA + 2 * kWtLoads <= 63, "outstanding loads must fit the vmcnt field");
       char* const w0 = lds + NS * kQStageA;
       int sa = 0;  // stage of A(kt)
-      auto q_tile = [&](int kt, auto slot_tag) {  // (slot of W(kt + 1))
+      // (slot of W(kt + 1); QS4: of four, and the word of its scales.  `last`, QS4: of the last three k tiles, behind the loop -- nothing
+      // requests W any more, so the wait counts on A's loads alone)
+      auto q_tile = [&](int kt, auto slot_tag, auto last_tag) {
+        constexpr int SLOT = decltype(slot_tag)::value;
+        constexpr bool kLast = decltype(last_tag)::value;
         const int na = sa + 1 == NS ? 0 : sa + 1;
         char* const wc = w0 + (kt & 1) * (BN * kRowBytes);
         char* const w_next = w0 + ((kt & 1) ^ 1) * (BN * kRowBytes);
         fetch_a_q(sa == 0 ? NS - 1 : sa - 1, kt + NS - 1);  // into the stage that tile kt-1 left at the previous barrier
         DTAS_SCHED_FENCE();
         step16(0, lds + sa * kQStageA, wc, 1);
-        wt_commit_at(w_next, slot_tag);                          // W(kt+1), into the stage that W(kt-1) left
-        wt_load(kt + 4, slot_tag);
+        if constexpr (QS4 && SLOT == 0) qs_cur = qs_next;        // (kt + 1 begins the next four)
+        wt_commit_at(w_next, slot_tag, QS4 ? qs_cur[SLOT] : 0u); // W(kt+1), into the stage that W(kt-1) left
+        if constexpr (QS4 && SLOT == 0) qs_next = qs_load((kt + 1) / 4 + 1);
+        if constexpr (!kLast) wt_load(kt + 1 + kWtSlots, slot_tag);
         DTAS_SCHED_FENCE();
         // A(kt+1) has landed: behind it were requested A(kt+2) .. A(kt+NS-1) and two or more k tiles' pieces of W
-        __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA + 4));
+        __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA + (kLast ? 0 : 2 * kWtLoads)));
         __builtin_amdgcn_s_barrier();
         DTAS_SCHED_FENCE();
         step16(1, lds + na * kQStageA, w_next, 0);
         sa = na;
       };
       int kt = 0;
-      for (; kt + 2 < ktiles; kt += 3) {
-        q_tile(kt, std::integral_constant<int, 1>{});
-        q_tile(kt + 1, std::integral_constant<int, 2>{});
-        q_tile(kt + 2, std::integral_constant<int, 0>{});
+      if constexpr (QS4) {
+        for (; kt + 3 < ktiles; kt += 4) {
+          q_tile(kt, std::integral_constant<int, 1>{}, std::false_type{});
+          q_tile(kt + 1, std::integral_constant<int, 2>{}, std::false_type{});
+          q_tile(kt + 2, std::integral_constant<int, 3>{}, std::false_type{});
+          q_tile(kt + 3, std::integral_constant<int, 0>{}, std::false_type{});
+        }
+        if (kt < ktiles) q_tile(kt, std::integral_constant<int, 1>{}, std::true_type{});
+        if (kt + 1 < ktiles) q_tile(kt + 1, std::integral_constant<int, 2>{}, std::true_type{});
+        if (kt + 2 < ktiles) q_tile(kt + 2, std::integral_constant<int, 3>{}, std::true_type{});
+      } else {
+        for (; kt + 2 < ktiles; kt += 3) {
+          q_tile(kt, std::integral_constant<int, 1>{}, std::false_type{});
+          q_tile(kt + 1, std::integral_constant<int, 2>{}, std::false_type{});
+          q_tile(kt + 2, std::integral_constant<int, 0>{}, std::false_type{});
+        }
+        if (kt < ktiles) q_tile(kt, std::integral_constant<int, 1>{}, std::false_type{});
+        if (kt + 1 < ktiles) q_tile(kt + 1, std::integral_constant<int, 2>{}, std::false_type{});
       }
-      if (kt < ktiles) q_tile(kt, std::integral_constant<int, 1>{});
-      if (kt + 1 < ktiles) q_tile(kt + 1, std::integral_constant<int, 2>{});
     } else if constexpr (!kRing) {
       static_assert((NS - 1) * (kLoadsA > kLoadsW ? kLoadsA : kLoadsW) <= 63, "outstanding loads must fit the vmcnt field");
       int sa = 0, sw = 0;  // stages of A(kt), W(kt)
@@ -1130,7 +1173,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   }
 }
 
-template <int BM, int BN, int WM, int WN, int NS, bool WT = false, bool WQ = false, bool M16 = false>
+template <int BM, int BN, int WM, int WN, int NS, bool WT = false, bool WQ = false, bool M16 = false, bool QS4 = false>
 int launch_mfma(hipStream_t s, const half_t* A, const half_t* W, const GemmEpilogue& ep, void* C, int64_t M, int64_t N,
                 int64_t K, int nsplit, int batch = 1, unsigned unsplit = 0) {
   const unsigned tiles_m = static_cast<unsigned>(ceil_div(M, BM)), tiles_n = static_cast<unsigned>(ceil_div(N, BN));
@@ -1148,7 +1191,7 @@ int launch_mfma(hipStream_t s, const half_t* A, const half_t* W, const GemmEpilo
   GemmEpilogue batched = ep;
   batched.batches = static_cast<unsigned>(batch);
   batched.tiles_unsplit = unsplit;
-  hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, WM, WN, NS, WT, WQ, M16>), dim3(static_cast<unsigned>(wgs)), dim3(64 * WM * WN), 0,
+  hipLaunchKernelGGL((gemm_mfma_kernel<BM, BN, WM, WN, NS, WT, WQ, M16, QS4>), dim3(static_cast<unsigned>(wgs)), dim3(64 * WM * WN), 0,
                      s, A, W, batched, C, M, N, K, tiles_m, tiles_n, static_cast<unsigned>(nsplit), partials, arrivals);
   return check_launch("gemm");
 }

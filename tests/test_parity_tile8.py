@@ -106,6 +106,31 @@ def test_every_8_bit_tile_at_its_edges(oracle, bm, bn):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("bm,bn", Q8_TILES)
+def test_8_bit_tiles_with_the_scales_of_four_k_tiles_in_one_load(oracle, bm, bn):
+    # 1 .. 9 k tiles (none to two of the loop's four, none to three behind it), parts of K that begin at odd k tiles; scales off the
+    # 4-byte grid and K = 64 k + 32 take the loop that loads them one by one: the same bits from both on the same weights
+    for K, split in ((64, 1), (128, 1), (192, 1), (256, 1), (320, 1), (384, 1), (448, 1), (512, 1), (576, 1), (1088, 4), (2112, 7), (640, 2)):
+        M, N = bm + 5, bn + 7
+        a, _, bias = _inputs(M, N, K, K + bm)
+        wq, scale = _q8(N, K, K)
+        w = oracle.c.decode_q8(wq, scale, threads=8)
+        words = torch.from_numpy(wq.view(np.int32)).cuda()
+        out = Guarded((M, N), torch.float16)
+        ops.gemm_q8(dev(a), words, dev(scale), dev(bias), out.t, _cfg(bm, bn, 0, split))
+        got = out.check()
+        _check(got, oracle.c.gemm(a, w, bias, threads=8), oracle.np64.gemm(a, w, bias))
+        off = torch.zeros(N * (K // 32) + 1, dtype=torch.float16, device="cuda")
+        off[1:] = dev(scale).flatten()
+        ops.gemm_q8(dev(a), words, off[1:].view(N, K // 32), dev(bias), out.t, _cfg(bm, bn, 0, split))
+        assert_bits_equal(out.check(), got)
+        # what lies behind a row's scales is the next row's: infinities there stay with that row
+        scale[1::2, :6] = np.inf
+        ops.gemm_q8(dev(a), words, dev(scale), dev(bias), out.t, _cfg(bm, bn, 0, split))
+        assert_bits_equal(np.ascontiguousarray(out.check()[:, ::2]), np.ascontiguousarray(got[:, ::2]))
+
+
+@pytest.mark.gpu
 @pytest.mark.parametrize("epilogue", [_lib.EPI_BIAS, _lib.EPI_BIAS_ADD2, _lib.EPI_BIAS_ADD2_CAST_F32, _lib.EPI_BIAS_GELU])
 @pytest.mark.parametrize("M,N,K", [(97, 2560, 2560), (130, 768, 1024), (203, 520, 2080), (320, 2560, 10240), (450, 7680, 320), (700, 10240, 256), (900, 1000, 4096)])
 def test_8_bit_weights_without_a_config(M, N, K, epilogue):
