@@ -554,8 +554,9 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       // a 16-byte piece of W per lane (16 weights and their scale) three k tiles ahead of the stage it is dequantised into,
       // one k tile before it is multiplied.  The dequantiser runs as one block behind the last MFMA of a step, ahead of the barrier
       // (a scheduling fence stands between the MFMAs), in all eight wavefronts at the same time: what a SIMD's other wavefront
-      // could multiply meanwhile is not there.  41 .. 44 KB/us per CU (96x128: 12 KB of A and 8.5 of W and scales in 0.51 us, A in
-      // the caches) where the fp16 tiles move 59 .. 64.
+      // could multiply meanwhile is not there; yet a word of it behind each of four MFMAs takes 1 .. 8 % longer, and half of the
+      // wavefronts dequantising ahead of the step 0 .. 6 %.  45 KB/us per CU (96x128: 12 KB of A and 8.5 of W and scales in 0.46 us, A
+      // in the caches) where the fp16 tiles move 59 .. 64.
       // The scales one by one, two bytes of each of 16 rows per load and k tile, were a third of the L1's look-ups.  Those of four k tiles
       // in one load (QS4): 203 x 7680 x 2560 21.3 -> 20.0 us, 203 x 10240 x 2560 28.3 -> 25.3, 203 x 2560 x 10240 31.1 -> 28.9, 450 x 10240 x
       // 2560 35.1 -> 32.6, 700 x 2560 x 10240 55.4 -> 52.3 (without any scales, 26.5, 29.3, 32.9, 52.9 against 28.6, 31.4, 35.7, 56.1: all of it).
