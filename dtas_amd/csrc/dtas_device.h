@@ -193,14 +193,17 @@ __device__ __forceinline__ void store_stream(V v, V* p) { __builtin_nontemporal_
 // 125 us), seven calls over [4096, 4096] 107 -> 100, over [2000, 8192] 115 -> 104.  Alone, with an output that nobody reads, the
 // launch takes up to 0.9 us longer (copy of [1024, 4096] 4.3 / 5.1 us, of [4096, 4096] 11.6 / 12.2).
 // Outputs of more than half of the 256 MiB cache are streamed as before, and so are accesses of less than 8 bytes.
-// (s_nop: the data registers of a store of more than 8 bytes may not be written in the next cycle.)
+// The stores are the compiler's own: it keeps the two wait states that pass before a VALU instruction may write the data registers of
+// a store of more than 8 bytes, and counts the store among the outstanding ones.
 constexpr int64_t kThroughBytes = int64_t{128} << 20;
 template <typename V>
 __device__ __forceinline__ void store_out(V v, V* p, bool through) {
   static_assert(sizeof(V) <= 16, "one access");
   if (sizeof(V) >= 8 && through) {
-    if constexpr (sizeof(V) == 16) asm volatile("global_store_dwordx4 %0, %1, off sc1\n\ts_nop 0" ::"v"(p), "v"(v));
-    if constexpr (sizeof(V) == 8) asm volatile("global_store_dwordx2 %0, %1, off sc1" ::"v"(p), "v"(v));
+    if constexpr (sizeof(V) == 16)
+      __builtin_amdgcn_global_store_b128((__attribute__((address_space(1))) u32x4*)p, __builtin_bit_cast(u32x4, v), "agent");
+    if constexpr (sizeof(V) == 8)
+      __hip_atomic_store(reinterpret_cast<uint64_t*>(p), __builtin_bit_cast(uint64_t, v), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   } else {
     store_stream(v, p);
   }

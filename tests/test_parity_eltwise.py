@@ -194,6 +194,17 @@ def test_outputs_at_the_line_between_written_through_and_streamed(vectors):
     assert all(torch.equal(p, w) for p, w in zip(parts, fused.split(80, dim=-1)))
 
 
+@pytest.mark.parametrize("unroll", [1, 2, 4, 8])
+def test_a_cast_in_two_accesses_per_vector_on_both_sides_of_the_line(unroll):
+    """fp16 -> fp32 at 8 elements per vector, 32 bytes stored in two halves: written through up to 128 MiB, streamed beyond."""
+    gen = torch.Generator(device="cuda").manual_seed(unroll)
+    for count in ((128 << 20) // 4 - 8 * unroll, (128 << 20) // 4, (128 << 20) // 4 + 8):
+        a = torch.randn(1, count, device="cuda", generator=gen).half()
+        out = torch.full((1, count), -7.0, device="cuda")
+        ops.cast(a, out, cfg(variant=_lib.ELT_VECTOR, vec=8, unroll=unroll))
+        assert torch.equal(a.float(), out)
+
+
 def test_grid_cap_makes_the_kernel_loop(oracle):
     rng = np.random.default_rng(4)
     a, b = rng.uniform(-1, 1, (300, 4096)).astype(np.float16), rng.uniform(-1, 1, (300, 4096)).astype(np.float16)
