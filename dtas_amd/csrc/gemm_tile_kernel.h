@@ -497,10 +497,11 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       for (int p = 0; p < NS - 1; ++p) fetch_a_q(p, p);
       DTAS_SCHED_FENCE();
       wt_commit_at(lds + NS * kQStageA, std::integral_constant<int, 0>{}, QS4 ? qs_cur[0] : 0u);
-      wt_load(kWtSlots, std::integral_constant<int, 0>{});
       DTAS_SCHED_FENCE();
-      // (QS4: A's loads alone are counted on: the piece just requested is for the loop only, and the compiler moves its load there)
-      __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA + (QS4 ? 0 : kWtLoads)));
+      // (A's loads alone are counted on, and the piece is requested behind the wait: it is for the loop only, and the compiler would move
+      // its load there)
+      __builtin_amdgcn_s_waitcnt(waitcnt_imm((NS - 2) * kQLoadsA));
+      wt_load(kWtSlots, std::integral_constant<int, 0>{});
     } else if constexpr (!kRing) {
       if (hi) {
 #pragma unroll
@@ -564,8 +565,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
       static_assert((NS - 2) * kQLoadsA + 2 * kWtLoads <= 63, "outstanding loads must fit the vmcnt field");
       char* const w0 = lds + NS * kQStageA;
       int sa = 0;  // stage of A(kt)
-      // (slot of W(kt + 1); QS4: of four, and the word of its scales.  `last`, QS4: of the last three k tiles, behind the loop -- nothing
-      // requests W any more, so the wait counts on A's loads alone)
+      // (slot of W(kt + 1), of three; QS4: of four, and the word of its scales.  `last`: of the last two (three) k tiles, behind the loop --
+      // nothing requests W any more, so the wait counts on A's loads alone)
       auto q_tile = [&](int kt, auto slot_tag, auto last_tag) {
         constexpr int SLOT = decltype(slot_tag)::value;
         constexpr bool kLast = decltype(last_tag)::value;
@@ -604,8 +605,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
           q_tile(kt + 1, std::integral_constant<int, 2>{}, std::false_type{});
           q_tile(kt + 2, std::integral_constant<int, 0>{}, std::false_type{});
         }
-        if (kt < ktiles) q_tile(kt, std::integral_constant<int, 1>{}, std::false_type{});
-        if (kt + 1 < ktiles) q_tile(kt + 1, std::integral_constant<int, 2>{}, std::false_type{});
+        if (kt < ktiles) q_tile(kt, std::integral_constant<int, 1>{}, std::true_type{});
+        if (kt + 1 < ktiles) q_tile(kt + 1, std::integral_constant<int, 2>{}, std::true_type{});
       }
     } else if constexpr (!kRing) {
       static_assert((NS - 1) * (kLoadsA > kLoadsW ? kLoadsA : kLoadsW) <= 63, "outstanding loads must fit the vmcnt field");

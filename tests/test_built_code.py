@@ -1,0 +1,146 @@
+"""What the built kernels keep that no run can be relied on to show, read from the library's own code.
+
+ * A store of more than 8 bytes reads its data registers after it has issued: two wait states pass before a VALU instruction may
+   write them.  The compiler keeps them for the stores it knows, not for what stands in inline assembly.
+ * The 8-bit tiles on 8 wavefronts count the loads that may be outstanding when a stage of A is handed over.  A count that allows
+   for requests which the compiler drops or moves behind the wait is too large, and the stage is then read before it is whole.
+"""
+import os
+import re
+import shutil
+import subprocess
+
+import pytest
+
+from dtas_amd import _lib
+
+OBJDUMP = shutil.which("llvm-objdump", path="/opt/rocm/llvm/bin") or shutil.which("llvm-objdump")
+WIDE = re.compile(r"(?:global|flat|scratch)_store_dwordx[34] \S+ v\[(\d+):(\d+)\]|buffer_store_dwordx[34] v\[(\d+):(\d+)\]")
+WRITES = re.compile(r"v_\w+ v(?:(\d+)\b|\[(\d+):(\d+)\])")
+LINE = re.compile(r"\t(\w+)(.*)// ([0-9A-F]+):")
+JUMP = re.compile(r"s_c?branch\w* (\d+)")
+STATES = 2
+
+
+def instructions(text):
+    """[(instruction, address)] of a disassembly's lines, and the position of each address."""
+    code = [(m.group(1) + m.group(2).rstrip(), int(m.group(3), 16)) for m in map(LINE.match, text) if m]
+    return code, {address: i for i, (_, address) in enumerate(code)}
+
+
+def target(ins, address):
+    """Where a branch goes (None: not a branch)."""
+    jump = JUMP.match(ins)
+    return jump and address + 4 + 4 * (int(jump.group(1)) - (65536 if int(jump.group(1)) > 32767 else 0))
+
+
+def early_writes(text):
+    """Instructions that write a wide store's data registers with fewer than two wait states between, along branches too."""
+    code, index = instructions(text)
+
+    def following(at, states, lo, hi):
+        while states < STATES and at < len(code):
+            ins, address = code[at]
+            write = WRITES.match(ins)
+            if write and int(write.group(1) or write.group(2)) <= hi and int(write.group(1) or write.group(3)) >= lo:
+                yield ins
+            if ins.startswith("s_endpgm"):
+                return
+            nop, to = re.match(r"s_nop (\d+)", ins), target(ins, address)
+            states += int(nop.group(1)) + 1 if nop else 1
+            if to is not None:
+                yield from following(index[to], states, lo, hi)
+                if ins.startswith("s_branch"):
+                    return
+            at += 1
+
+    return [(ins, late) for at, (ins, _) in enumerate(code) if (store := WIDE.match(ins))
+            for late in following(at + 1, 0, *(int(x) for x in store.groups() if x is not None))]
+
+
+def most_outstanding(text):
+    """The most direct-to-LDS loads that can be outstanding at any s_barrier, over every path (loads and stores complete in order)."""
+    code, index = instructions(text)
+    most, seen, todo = 0, set(), [(0, ())]
+    while todo:
+        at, queue = todo.pop()
+        while at < len(code):
+            ins, address = code[at]
+            to = target(ins, address)
+            if to is not None or ins.startswith("s_barrier"):
+                if (at, queue) in seen:
+                    break
+                seen.add((at, queue))
+            if ins.startswith("s_endpgm"):
+                break
+            if re.match(r"(buffer|global|flat)_(load|store)", ins):
+                queue = (queue + (" lds" in ins,))[-63:]
+            wait = re.match(r"s_waitcnt.*vmcnt\((\d+)\)", ins)
+            if wait:
+                queue = queue[-int(wait.group(1)):] if int(wait.group(1)) else ()
+            if ins.startswith("s_barrier"):
+                most = max(most, sum(queue))
+            if to is not None:
+                todo.append((index[to], queue))
+                if ins.startswith("s_branch"):
+                    break
+            at += 1
+    return most
+
+
+def lines(*code):
+    return [f"\t{line}  // {4 * i:012X}: 00000000" for i, line in enumerate(code)]
+
+
+def test_the_rules_read_what_the_disassembler_prints():
+    def found(*code):
+        return len(early_writes(lines(*code)))
+
+    store, far, write = "global_store_dwordx4 v[24:25], v[16:19], off sc1", "v_add_u32_e32 v20, v1, v2", "v_lshl_add_u64 v[16:17], v[24:25], 0, s[2:3]"
+    assert found(store, write) == found(store, "s_nop 0", write) == found(store, far, "v_mov_b32_e32 v19, 0") == 1
+    assert found("buffer_store_dwordx4 v[16:19], v0, s[4:7], 0 offen", write) == found(store, "s_branch 1", far, write) == 1
+    assert found(store, "s_nop 1", write) == found(store, far, far, write) == found(store, "s_branch 1", write, far) == found(store, far) == 0
+    assert found(write, store, "s_cbranch_vccnz 65533", far, far) == 1
+
+    lds, load, wait, barrier = "buffer_load_dwordx4 v1, s[0:3], 0 offen lds", "buffer_load_dwordx4 v[2:5], v1, s[0:3], 0 offen", "s_waitcnt vmcnt(2)", "s_barrier"
+    assert most_outstanding(lines(lds, lds, lds, wait, barrier)) == most_outstanding(lines(lds, lds, load, "s_cbranch_scc1 1", wait, barrier)) == 2
+    assert most_outstanding(lines(lds, lds, load, load, wait, barrier)) == 0 and most_outstanding(lines(lds, barrier, "s_cbranch_scc1 65533", "s_endpgm")) == 63
+
+
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """{kernel symbol: lines of its disassembly} of the built library."""
+    if OBJDUMP is None:
+        pytest.skip("needs ROCm's llvm-objdump")
+    where = tmp_path_factory.mktemp("code")
+    shutil.copy(_lib.LIB_PATH, where / "lib.so")
+    subprocess.run([OBJDUMP, "--offloading", "lib.so"], cwd=where, check=True, capture_output=True)
+    found = {}
+    for name in (f for f in os.listdir(where) if f.endswith("gfx950")):
+        text = subprocess.run([OBJDUMP, "-d", "--no-show-raw-insn", "--no-leading-addr", name], cwd=where, check=True, capture_output=True, text=True).stdout
+        for line in text.splitlines():
+            symbol = re.match(r"[0-9a-f ]*<(\S+)>:", line)
+            if symbol:
+                body = found.setdefault((name, symbol.group(1)), [])
+            elif line.startswith("\t"):
+                body.append(line)
+    assert len(found) > 100
+    return found
+
+
+def test_no_wide_store_loses_its_data_registers(kernels):
+    assert sum(1 for body in kernels.values() for line in body if WIDE.match(line.strip())) > 500
+    found = [(name, *early) for name, body in kernels.items() for early in early_writes(body)]
+    assert not found, (len(found), found[:4])
+
+
+def test_a_stage_of_a_has_landed_where_an_8_bit_tile_hands_it_over(kernels):
+    # stages of A are requested NS - 1 k tiles ahead; at a barrier the one behind it is whole, NS - 2 may be on their way
+    tiles = {}
+    for (_, name), body in kernels.items():
+        kind = re.search(r"gemm_mfma_kernelILi(\d+)ELi128ELi\dELi\dELi(\d)ELb0ELb1ELb1ELb([01])E", name)
+        if kind:
+            rows, stages = int(kind.group(1)), int(kind.group(2))
+            loads = -(-rows // 64)  # per wavefront and stage: 8 wavefronts load 8 rows of 128 bytes each at a time
+            tiles[rows, kind.group(3)] = (most_outstanding(body), (stages - 2) * loads)
+    assert len(tiles) == 10 and all(most <= limit for most, limit in tiles.values()), tiles
