@@ -1058,12 +1058,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   // one access per lane to C and the residuals for every lane whose columns lie inside the row, at whatever
   // alignment the row has
   const bool vec_store = col + kVecC - 1 < N;
-  // C in one layer of the model (2560 / 7680 / 10240 columns), streamed / written through, us: 203 rows after 500 on 8-bit weights 179.4 / 176.1,
-  // 400 rows 183 / 179, 700 261 / 252, 1025 371 / 362, 1600 555 / 556, 2048 706 / 700; three products at 4096 / 11008 level up to 2000
-  // rows, 713 / 717 at 4000, 1394 / 1398 at 8192 (C of 33 .. 180 MB).  Launches whose C nobody reads: level to 5 % longer (2048 x 7680 x
-  // 2560 on 8-bit weights 75.2 / 78.9)
-  constexpr int64_t kThroughC = int64_t{48} << 20;
-  const bool through = N % 32 == 0 && M * N <= kThroughC / 2 && (reinterpret_cast<uintptr_t>(C) & 63u) == 0;
+  const bool through = writes_c_through(M, N, ep.batches, WT, reinterpret_cast<uintptr_t>(C));
   float bv[kVecC];
   cvec_t bvh;
 #pragma unroll
@@ -1153,8 +1148,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
         } else {
           half_t* dst = static_cast<half_t*>(C) + at;
           if (vec_store) {
-            // rows of whole sectors up to kThroughC: written through (store_out), for the launch that reads C next; beyond, and where
-            // rows share a sector, streamed past the operands in the L2
+            // (otherwise streamed past the operands in the L2)
             if (through) store_out(hv, reinterpret_cast<cvec_t*>(dst), true);
             else __builtin_nontemporal_store(hv, reinterpret_cast<cvec_a2*>(dst));
           } else {
