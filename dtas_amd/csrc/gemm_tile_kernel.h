@@ -1058,7 +1058,8 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   // one access per lane to C and the residuals for every lane whose columns lie inside the row, at whatever
   // alignment the row has
   const bool vec_store = col + kVecC - 1 < N;
-  const bool through = writes_c_through(M, N, ep.batches, WT, reinterpret_cast<uintptr_t>(C));
+  // (row-major W comes in a batch for the scores only, whose output is fp32)
+  const bool through = writes_c_through(M, N, WT ? ep.batches : 1, WT, reinterpret_cast<uintptr_t>(C));
   float bv[kVecC];
   cvec_t bvh;
 #pragma unroll
