@@ -4,6 +4,8 @@
    write them.  The compiler keeps them for the stores it knows, not for what stands in inline assembly.
  * The 8-bit tiles on 8 wavefronts count the loads that may be outstanding when a stage of A is handed over.  A count that allows
    for requests which the compiler drops or moves behind the wait is too large, and the stage is then read before it is whole.
+ * P.V reads V's fragments with transposing LDS reads in inline assembly.  The compiler takes their registers as written at once; nothing
+   may touch one until the wait for it, or the read that arrives late overwrites what stands there.
 """
 import os
 import re
@@ -88,6 +90,43 @@ def most_outstanding(text):
     return most
 
 
+def registers(ins):
+    """The vector registers an instruction names."""
+    return {r for m in re.finditer(r"\bv(?:(\d+)\b|\[(\d+):(\d+)\])", ins) for r in range(int(m.group(1) or m.group(2)), int(m.group(1) or m.group(3)) + 1)}
+
+
+def touched_in_flight(text):
+    """(transposing read, instruction of the k loop that names its registers before lgkmcnt(0)), over every path.
+
+    The k loop ends with the last MFMA.  Behind it no read is in flight: one is issued only where a further step follows, which waits
+    first.  (A path that skips that step is there in the code, with the loop's condition on it, but is never taken.)
+    """
+    code, index = instructions(text)
+    end = max((at for at, (ins, _) in enumerate(code) if ins.startswith("v_mfma")), default=-1)
+    found = []
+    for start, (read, _) in enumerate(code):
+        if not read.startswith("ds_read_b64_tr"):
+            continue
+        into, seen, todo = registers(read.split(",")[0]), set(), [start + 1]
+        while todo:
+            at = todo.pop()
+            if at in seen or at > end:
+                continue
+            seen.add(at)
+            ins, address = code[at]
+            if ins.startswith("s_endpgm") or re.match(r"s_waitcnt.*lgkmcnt\(0\)", ins):
+                continue
+            if registers(ins) & into:
+                found.append((read, ins))
+                continue
+            to = target(ins, address)
+            if to is not None:
+                todo.append(index[to])
+            if not ins.startswith("s_branch"):
+                todo.append(at + 1)
+    return found
+
+
 def lines(*code):
     return [f"\t{line}  // {4 * i:012X}: 00000000" for i, line in enumerate(code)]
 
@@ -105,6 +144,13 @@ def test_the_rules_read_what_the_disassembler_prints():
     lds, load, wait, barrier = "buffer_load_dwordx4 v1, s[0:3], 0 offen lds", "buffer_load_dwordx4 v[2:5], v1, s[0:3], 0 offen", "s_waitcnt vmcnt(2)", "s_barrier"
     assert most_outstanding(lines(lds, lds, lds, wait, barrier)) == most_outstanding(lines(lds, lds, load, "s_cbranch_scc1 1", wait, barrier)) == 2
     assert most_outstanding(lines(lds, lds, load, load, wait, barrier)) == 0 and most_outstanding(lines(lds, barrier, "s_cbranch_scc1 65533", "s_endpgm")) == 63
+
+    read, use, done = "ds_read_b64_tr_b16 v[2:3], v0 offset:64", "v_add_f32_e32 v3, v4, v5", "s_waitcnt lgkmcnt(0)"
+    mfma = "v_mfma_f32_32x32x16_f16 a[0:15], v[8:11], v[12:15], a[0:15]"
+    assert len(touched_in_flight(lines(read, use, mfma))) == len(touched_in_flight(lines(read, "s_cbranch_scc1 1", done, use, mfma))) == 1
+    assert len(touched_in_flight(lines(read, "s_waitcnt lgkmcnt(1)", use, mfma))) == len(touched_in_flight(lines(use, mfma, read, "s_cbranch_scc1 65532", mfma))) == 1
+    assert not touched_in_flight(lines(read, done, use, mfma)) and not touched_in_flight(lines(read, "s_waitcnt vmcnt(3) lgkmcnt(0)", use, mfma))
+    assert not touched_in_flight(lines(read, mfma, use))
 
 
 @pytest.fixture(scope="module")
@@ -144,6 +190,12 @@ def test_a_stage_of_a_has_landed_where_an_8_bit_tile_hands_it_over(kernels):
             loads = -(-rows // 64)  # per wavefront and stage: 8 wavefronts load 8 rows of 128 bytes each at a time
             tiles[rows, kind.group(3)] = (most_outstanding(body), (stages - 2) * loads)
     assert len(tiles) == 10 and all(most <= limit for most, limit in tiles.values()), tiles
+
+
+def test_nothing_touches_a_transposing_read_in_flight(kernels):
+    assert sum(1 for body in kernels.values() for line in body if "ds_read_b64_tr" in line) > 100
+    found = [(name, *pair) for (_, name), body in kernels.items() for pair in touched_in_flight(body)]
+    assert not found, (len(found), found[:4])
 
 
 def test_which_c_is_written_through_counts_every_problem_of_the_launch(tmp_path):
