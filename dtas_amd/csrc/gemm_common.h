@@ -34,17 +34,18 @@ struct GemmEpilogue {
 };
 
 // Whether the MFMA tile kernels write an fp16 C through the L2 (store_out) for the launch that reads it next: rows of whole 64-byte
-// sectors, up to 48 MiB over all problems of the launch, 10 MiB for P.V (k-major W).
+// sectors, up to 48 MiB, a row-major W.
 //  * C in one layer of the model (2560 / 7680 / 10240 columns), streamed / written through, us: 203 rows after 500 on 8-bit weights 179.4 / 176.1,
 //    400 rows 183 / 179, 700 261 / 252, 1025 371 / 362, 1600 555 / 556, 2048 706 / 700; three products at 4096 / 11008 level up to 2000
 //    rows, 713 / 717 at 4000, 1394 / 1398 at 8192 (C of 33 .. 180 MB).  Launches whose C nobody reads: level to 5 % longer (2048 x 7680 x
 //    2560 on 8-bit weights 75.2 / 78.9).
-//  * P.V with the axis swap that reads its output behind it: 32 heads of 128, n = m = 300 / 600 / 1024 (2.5 / 4.9 / 8.4 MB) 14.2 / 13.8, 18.8 /
-//    18.3, 26.4 / 26.3; 32 of 64, 2048 (8.4 MB) 67.5 / 66.8; 32 of 96, 2048 (12.6 MB) 67.1 / 67.8; 32 of 128, 2048 (16.8 MB) 72.4 / 73.5; 40 of
-//    128, 8192 x 1024 (84 MB) 195 / 203.
-constexpr bool writes_c_through(int64_t M, int64_t N, int64_t problems, bool k_major_w, uint64_t c_address) {
-  const int64_t limit = int64_t{k_major_w ? 10 : 48} << 20;
-  return N % 32 == 0 && c_address % 64 == 0 && M * N * problems <= limit / 2;
+//  * P.V (k-major W, a head per problem) streams its output.  The choice alone costs it 1 % where nothing is written through (32 heads of
+//    80, 203 x 703 14.20 -> 14.10 us without it, 512 x 512 9.55 -> 9.39).  With head dimensions that are multiples of 32, and the axis swap that reads
+//    the output behind it, written through / streamed: 32 heads of 128, 300 x 300 13.7 / 14.0, 1024 x 1024 26.0 / 25.7, 4096 x 4096
+//    233 / 226; 40 of 128, 8192 x 1024 200 / 193; 32 of 64, 2048 x 2048 66.4 / 66.1.
+constexpr bool writes_c_through(int64_t M, int64_t N, uint64_t c_address) {
+  constexpr int64_t kThroughC = int64_t{48} << 20;
+  return N % 32 == 0 && c_address % 64 == 0 && M * N <= kThroughC / 2;
 }
 
 // Attention scores, fused_NT_matmul1_divide_maximum_minimum_cast2 (before_dl.py:116-160):

@@ -1059,7 +1059,7 @@ __global__ void __launch_bounds__(64 * WM * WN) gemm_mfma_kernel(const half_t* _
   // alignment the row has
   const bool vec_store = col + kVecC - 1 < N;
   // (row-major W comes in a batch for the scores only, whose output is fp32)
-  const bool through = writes_c_through(M, N, WT ? ep.batches : 1, WT, reinterpret_cast<uintptr_t>(C));
+  const bool through = !WT && writes_c_through(M, N, reinterpret_cast<uintptr_t>(C));
   float bv[kVecC];
   cvec_t bvh;
 #pragma unroll
