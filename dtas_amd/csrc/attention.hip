@@ -813,17 +813,19 @@ extern "C" int dtas_attn_scores_f16_f32(const void* Q, const void* Kmat, const v
                            static_cast<float*>(out), n, m, d, sc, tm, tn, static_cast<unsigned>(heads), pin);
       return check_launch("attn_scores");
     }
-    // ... or every row is cut at sectors of its own (attn_scores_sector_kernel), for continuations of up to 256 rows and for scores that
-    // a cache does not hold for the softmax.  Tiles / own sectors, us, head dimension 80; in brackets with the softmax that reads them behind:
+    // ... or every row is cut at sectors of its own (attn_scores_sector_kernel), for continuations of up to 256 rows, and from 20 M scores
+    // against 1100 keys on: lines where the two measured level.  Tiles / own sectors, us, head dimension 80 where none is named (72 is the
+    // only other one the kernel takes); in brackets with the softmax that reads them behind:
     //  * keys: 32 heads, 203 x 601 11.2 / 12.0 (20.9 / 20.0), 256 x 601 11.8 / 11.9 (22.7 / 22.2); 203 x 703 12.6 / 12.3 (23.2 / 20.3), 256 x
     //    703 13.2 / 12.0 (24.8 / 24.0), 203 x 1031 15.7 / 13.8 (26.5 / 25.4), 130 x 2049 17.5 / 15.7 (29.3 / 27.4), 256 x 4095 49.5 / 37.3;
     //  * workgroups per CU, whose chains have to hide one another: 1.5, 32 heads, 65 x 1531 11.1 / 12.0, 100 x 1301 11.4 / 11.9, 24 heads,
     //    225 x 777 11.6 / 12.4; 1.75 and more, 32 heads, 203 x 777 14.0 / 12.5, 130 x 1031 13.8 / 11.8, 65 x 2049 13.1 / 11.9;
     //  * rows beyond 8192 in all, and 256: axis swaps, scores, softmax and P.V together.  Below 1100 keys level to 1 % behind (a layer of
     //    1025 rows 374 / 376, of 777 298.4 / 300.1), and so are few scores (64 heads, 225 x 1301, 75 MB, 86.6 / 87.6); from 20 M scores on
-    //    the tiles' plain stores keep nothing for the softmax that the streaming ones here would lose: a layer of 500 rows after 2001
+    //    what the tiles' plain stores leave in the caches for the softmax is worth less than their partial sectors cost: a layer of 500 rows after 2001
     //    311 / 303, 700 after 2501 446 / 421, of 1250 rows 450 / 442, 1601 611 / 594, 2047 809 / 769; 64 heads, 1025 x 1301 300 / 271, 16
-    //    heads, 600 x 1301 64.5 / 61.6, 8 heads, 1500 x 3001 128 / 124.
+    //    heads, 600 x 1301 64.5 / 61.6, 8 heads, 1500 x 3001 128 / 124.  Head dimension 72: 32 heads, 600 x 2001 141.8 / 134.4, 1301 x 1301
+    //    181.8 / 181.3, 2047 x 2047 398.7 / 357.5, 16 heads, 1200 x 1201 90.5 / 88.3, 600 x 2101 92.9 / 87.5.
     // Head dimensions of 64 and 128 pull more of K through the L1 than the tiles do (40 heads of 128, 1025 x 1025 57.6 / 98.9)
     const int64_t pieces = ceil_div(m, kSectorChunk), chunk = ceil_div(ceil_div(m, pieces), 16) * 16;
     const int64_t tm_s = ceil_div(n, kSectorRows), tn_s = ceil_div(m, chunk), tiles_s = tm_s * tn_s;

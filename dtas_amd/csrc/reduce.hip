@@ -183,8 +183,12 @@ __global__ void __launch_bounds__(ITERS * R > 8 ? 512 : 1024) row_reg_kernel(
   half_t* out = static_cast<half_t*>(outp);
   // Norms of a middle size are written through the L2 for the launch that reads them (store_out), us, streamed / through: a layer of
   // 203 rows after 500 on 8-bit weights 176.6 / 173.0, 400 rows 181.6 / 178.3, 1025 level, 130 138.4 / 139.4; seven calls over
-  // [1200, 4096] 45.9 / 45.0 by either norm, [2400, 4096] 71.5 / 69.2 by the RMSNorm, [2000, 8192] 104.5 / 105.2 by the LayerNorm, three
-  // products of 200 rows 111.5 / 112.0 by the RMSNorm.  The softmax's rows are streamed: of whole sectors level (2048 x 2048 with the
+  // [1200, 4096] 45.9 / 45.0 by either norm, [2000, 8192] 104.5 / 105.2 by the LayerNorm, three products of 200 rows 111.5 / 112.0 by the
+  // RMSNorm.  The RMSNorm's upper part, seven calls: [2400, 4096] 69.5 / 67.7, [3000, 4096] 77.7 / 76.4, [4096, 4096] 99.6 / 98.8, [3276, 5120]
+  // 104.6 / 103.6, three products of 600 .. 4000 rows level; beyond 16 M elements products of 4200 .. 8192 rows are level to 0.2 % ahead written
+  // through (8192: 1374 / 1371) and are streamed.  A launch whose output nobody reads takes 4 .. 9 % longer ([4096, 4096] 11.1 / 11.7), the
+  // cast that reads it 8 .. 10 % less with it (29.8 / 27.4).
+  // The softmax's rows are streamed: of whole sectors level (2048 x 2048 with the
   // P.V behind 190 / 187), ragged ones written through part of a sector at a time 7.7 / 11.0 (203 x 703)
   constexpr int64_t kThroughFrom = OP == kRms ? 2000000 : 400000, kThroughTo = OP == kRms ? 16 << 20 : 8 << 20;  // elements
   const bool through = (OP == kRms || OP == kLayerNorm) && rows * cols >= kThroughFrom && rows * cols <= kThroughTo;
