@@ -188,10 +188,50 @@ def test_outputs_at_the_line_between_written_through_and_streamed(vectors):
     swapped = torch.empty(32, a, 80, dtype=torch.float16, device="cuda")
     ops.swap_axes(rows, swapped)
     assert torch.equal(rows.transpose(0, 1), swapped)
-    fused = torch.randn(a // 3, 32, 240, device="cuda", generator=gen).half()
-    parts = [torch.empty(a // 3, 32, 80, dtype=torch.float16, device="cuda") for _ in range(3)]
+    r = (128 << 20) // 2 // (32 * 240) + vectors                     # the split's three outputs together
+    assert (r * 32 * 240 * 2 <= 128 << 20) == (a * 32 * 80 * 2 <= 128 << 20) == (vectors <= 0)
+    fused = torch.randn(r, 32, 240, device="cuda", generator=gen).half()
+    parts = [torch.empty(r, 32, 80, dtype=torch.float16, device="cuda") for _ in range(3)]
     ops.split3(fused, *parts)
     assert all(torch.equal(p, w) for p, w in zip(parts, fused.split(80, dim=-1)))
+
+
+@pytest.mark.parametrize("heads,d,rot", [(32, 80, 20), (64, 520, 20), (32, 128, 128), (40, 96, 24)])
+def test_rotary_at_the_line_between_written_through_and_streamed(heads, d, rot):
+    """128 MiB and a position less or more: every kernel the shape has gives the bits of the one for any rotated width."""
+    row = heads * d * 2
+    last = (128 << 20) // row                                        # the last number of positions within the line
+    gen = torch.Generator(device="cuda").manual_seed(d)
+    angle = torch.rand(last + 1, rot, device="cuda", generator=gen) * 6.28
+    cos, sin = angle.cos().half(), angle.sin().half()
+    for n in (last - 1, last, last + 1):
+        assert (n * row <= 128 << 20) == (n <= last)
+        a = torch.randn(1, n, heads, d, device="cuda", generator=gen).half()
+        want, out = torch.empty_like(a), torch.empty_like(a)
+        ops.rotary(a, cos, sin, want, n, cfg(variant=_lib.ELT_VECTOR, block=256, vec=8, unroll=2))
+        for unroll in (0, 1):
+            out.fill_(-7.0)
+            ops.rotary(a, cos, sin, out, n, cfg(variant=_lib.ELT_VECTOR, block=256, vec=8, unroll=unroll))
+            assert torch.equal(out, want)
+
+
+@pytest.mark.parametrize("more", [-1, 0, 1])
+def test_take_and_mask_at_the_line_between_written_through_and_streamed(more):
+    gen = torch.Generator(device="cuda").manual_seed(more + 5)
+    n = (128 << 20) // (2560 * 2) + more
+    assert (n * 2560 * 2 <= 128 << 20) == (more <= 0)
+    table = torch.randn(500, 2560, device="cuda", generator=gen).half()
+    ids = torch.randint(-3, 510, (n,), device="cuda", generator=gen, dtype=torch.int32)     # (clipped to the table)
+    out = torch.empty(n, 2560, dtype=torch.float16, device="cuda")
+    ops.take(table, ids, out)
+    assert torch.equal(out, table[ids.long().clamp(0, 499)])
+    rows, cols = 8192, 8192 + more                                   # (8192 x 8192 fp16: 128 MiB to the byte)
+    if more < 0:
+        rows, cols = 8191, 8192
+    mask = torch.empty(1, 1, rows, cols, dtype=torch.float16, device="cuda")
+    ops.attn_mask(mask)
+    i, j = torch.arange(rows, device="cuda", dtype=torch.int32)[:, None], torch.arange(cols, device="cuda", dtype=torch.int32)[None, :]
+    assert torch.equal(mask[0, 0], torch.where(j - (cols - rows) > i, -65504.0, 65504.0).half())
 
 
 @pytest.mark.parametrize("unroll", [1, 2, 4, 8])

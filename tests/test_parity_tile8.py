@@ -290,3 +290,25 @@ def test_rows_written_through_and_streamed_hold_the_same_bits(block, M, N):
     # (the sum and the result are each rounded to fp16, 2^-11 of at most a few units)
     want = (A.double() @ W.double().t()).half().double() + bias.double()
     assert ((got[0].double() - want).abs() <= 2e-3 + 2e-3 * want.abs()).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("block", [256, 512])
+@pytest.mark.parametrize("M,N", [(2457, 10240), (2458, 10240), (786432, 32), (786433, 32)])
+def test_c_at_the_line_between_written_through_and_streamed(block, M, N):
+    """48 MiB and a row more, on the 64-byte grid (by the size) and off it (streamed): the same bits."""
+    assert (M * N * 2 <= 48 << 20) == (M in (2457, 786432))
+    gen = torch.Generator(device="cuda").manual_seed(M + N)
+    A = torch.randn(M, 64, device="cuda", generator=gen).half()
+    W = (torch.randn(N, 64, device="cuda", generator=gen) * 0.05).half()
+    tile = cfg(variant=_lib.GEMM_MFMA, block=block, vec=8, unroll=2 if block == 256 else 0, tile=[128, 128, 64])
+    got = []
+    for offset in (0, 8):
+        raw = torch.full((M * N + 64,), 1234.5, dtype=torch.float16, device="cuda")
+        ops.gemm(A, W, None, raw[offset:offset + M * N].view(M, N), cfg=tile)
+        assert bool((raw[:offset] == 1234.5).all()) and bool((raw[offset + M * N:] == 1234.5).all())
+        got.append(raw[offset:offset + M * N].view(M, N))
+    assert torch.equal(*got)
+    want = A.double() @ W.double().t()
+    # (fp32 sums of 64 products of magnitude 1e-1 and one rounding to fp16: 2^-11 of the value)
+    assert ((got[0].double() - want).abs() <= 1e-5 + 2 ** -11 * 1.01 * want.abs()).all()
